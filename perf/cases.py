@@ -258,3 +258,48 @@ def tolerance(case):
         return {"rel": 1e-4, "max": 0.25}
     # z of up to 50 in exp(-z) at fp32: a relative error of 3e-6 against float64 for saturated groups, 5e-7 else
     return {"rel": 1.2e-5, "max": 1.3e-4}
+
+
+def exact(case, seed):
+    """Gradients of a layer in float64 from their closed form: per add group G (a kernel column, a channel, or a block
+    of channels and a kernel column) and rail, z = sum over G of x w, value 1 - exp(-z).  The values ``y`` are counts
+    over a power of two; the networks' results go through 8-bit roundings: neither has a 64-bit value of its own."""
+    if case["kind"] not in ("func", "layer"):
+        return None
+    st = prepare(case, seed)
+    if case["kind"] == "layer":
+        x, w = _q7(st["x"]).double(), _q7(st["layer"].weight_org).double()
+    else:
+        x, w = st["x"].double(), st["w"].double()
+    n, c_out, wo, ho = _out_shape(case)
+    k_w, k_h, pad = case["k_w"], case["k_h"], case["pad"]
+    grad_x, grad_w = torch.empty_like(x), [torch.zeros_like(w), torch.zeros_like(w)]
+    rails = (w.clamp(0, 100), (-w).clamp(0, 100))
+    if case["mode"] == "z_bin":
+        groups = [(slice(c, c + 1), range(k_h)) for c in range(case["c_in"])]
+    else:
+        step = case["z_unit"] if case["mode"] == "yz_bin" else case["c_in"]
+        groups = [(slice(c, min(c + step, case["c_in"])), [v]) for c in range(0, case["c_in"], step) for v in range(k_h)]
+    items = max(1, 2 ** 27 // (wo * ho * max(c_out, case["c_in"] * k_w)))
+    for n0 in range(0, n, items):
+        xp = torch.nn.functional.pad(x[n0:n0 + items], (pad, pad, pad, pad))
+        g = st["up"][n0:n0 + items].double().permute(1, 0, 2, 3).reshape(c_out, -1)
+        gxp = torch.zeros_like(xp)
+        for c, columns in groups:
+            taps = [(u, v) for u in range(k_w) for v in columns]
+            # (tap, channel, item, a, b) of the group, as rows of one matrix
+            col = torch.stack([xp[:, c, u:u + wo, v:v + ho].transpose(0, 1) for u, v in taps])
+            shape, col = col.shape, col.reshape(-1, g.shape[1])
+            dcol = torch.zeros_like(col)
+            for rail, sign, into in ((rails[0], 1, grad_w[0]), (rails[1], -1, grad_w[1])):
+                wm = torch.cat([rail[:, c, u, v] for u, v in taps], 1)
+                e = g * torch.exp(-(wm @ col)) * sign
+                dcol += wm.t() @ e
+                dw = (e @ col.t()).reshape(c_out, len(taps), -1)
+                for t, (u, v) in enumerate(taps):
+                    into[:, c, u, v] += dw[:, t]
+            for t, (u, v) in enumerate(taps):
+                gxp[:, c, u:u + wo, v:v + ho] += dcol.reshape(shape)[t].transpose(0, 1)
+        grad_x[n0:n0 + items] = gxp[:, :, pad:pad + case["w"], pad:pad + case["h"]]
+    grad_w = grad_w[0] * (w >= 0) - grad_w[1] * (w <= 0)
+    return dict(y=None, grad_x=grad_x, grad_w=grad_w)
