@@ -542,8 +542,8 @@ def main():
         "roofline": {
             "bound": "valu",
             "kernel": ("the rail-skipping convolution kernel (v_and_or_b32 on register-indexed accumulators: one "
-                       "and-or per activation word and weight; k_conv_fwd_rail_lds where activation words are "
-                       "shared through LDS)" if rail else "k_conv_fwd (v_and_or_b32 / v_bcnt_u32_b32, both rails)"),
+                       "and-or per activation word and weight; k_conv_fwd_tile_rail at the headline"
+                       ")" if rail else "k_conv_fwd (v_and_or_b32 / v_bcnt_u32_b32, both rails)"),
             # work no kernel can avoid (one and-or per activation word and weight, plus the popcount-adds) per
             # second of the kernel's average launch duration, against lanes x clock
             "achieved": achieved / 1e12,

@@ -93,12 +93,15 @@ int make_geometry(const geo_sc_conv_desc* d, Geometry* g)
     }
     g->seed_wrap = g->mode == GEO_SC_ACC_YZ ? (size_t)g->z_unit * wi * hi : (size_t)plane;
     {
-        // waves the position-parallel kernel could start at most (one (pack, add group) pair per
-        // wave) against the 1024 SIMDs; members of one OR group against the 64 lanes
+        // Lanes over the members of an OR group instead of over output positions: where positions are too few
+        // and no launch shares an OR group out over waves (outputs with a single row, kernel widths without
+        // rail-packed weights).  Waves the position-parallel kernel could start at most (one (pack, add group)
+        // pair per wave) against the 1024 SIMDs; members of one OR group against the 64 lanes
         const long long pos_waves = (((long long)d->n * wo * ho + 63) / 64) * g->n_cotile * g->packs * g->add_outer *
                                     g->add_inner;
         const long long members = (long long)g->or_rows * g->or_ch_per_group * d->w_k;
-        g->thin = pos_waves < 2048 && members >= 64;
+        const bool shared_or = wo >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5);
+        g->thin = pos_waves < 2048 && members >= 64 && !shared_or;
     }
     g->act_item_inner = !g->thin && g->mode == GEO_SC_ACC_Y && g->generator == GEO_SC_GEN_LFSR && wo == 1 && d->n >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5) &&
                         (unsigned long long)g->act_words * 4 < 0xffffffffull;  // its kernel addresses the buffer with 32-bit byte offsets

@@ -14,6 +14,7 @@
 // Consecutive workgroups take the c_out tiles of the same positions.
 #include "sc_common.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace geo_sc {
@@ -38,6 +39,7 @@ struct FwdParams {
     int add_outer, add_inner, or_ch_total, or_ch_per_group;
     unsigned add_stride, or_stride;
     int or_rows;  // kernel rows OR-ed together before the popcount (1, or h_k for the full OR)
+    int or_shares, pairs_per_slot;  // k_conv_fwd_tile_rail: waves per OR group, pairs one after the other
     int keep_touches;  // always 0; k_conv_fwd_items_rail_wg: makes the values of its cache touches count as used
 };
 
@@ -352,20 +354,20 @@ __global__ __launch_bounds__(64) void k_conv_fwd_split(FwdParams q)
 }
 
 // Layers with few output positions and large OR groups (classifier layers: 64 x 4 x 4 -> 10 at
-// batch 256 has 2560 outputs of 1024 products each): one wave per (output position, c_out tile,
+// batch 256 has 2560 outputs of 1024 products each): one wave per (two output positions, c_out tile,
 // pack, add group); the lanes run over the members of the OR group, each with its own weight
-// line in VGPRs, and the 2 x 16 partial OR words are combined across the wave with xor shuffles.
+// line in VGPRs (read once for both positions), and the 2 x 32 partial OR words are combined across the
+// wave by halving: in the step of lane bit k every lane hands the half of its words that its partner
+// keeps to that partner, so 32 + 16 + 8 + 4 + 2 + 1 shuffles leave one finished word per lane (bit 5: position,
+// bit 4: rail, bits 3 - 0: channel) where a full xor reduction of every word takes 64 x 6.
 // Results are added into the zeroed y with integer atomics.  Activation layout [n][P][c_in][wi][hi].
-__global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q)
+constexpr int kThinPositions = 2;
+__global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q, long long positions)
 {
-    constexpr int C = kCoTile;
+    constexpr int C = kCoTile, R = kThinPositions;
     const int lane = threadIdx.x;
     const int cot = blockIdx.x % q.n_cotile;
-    const long long m = blockIdx.x / q.n_cotile;
-    const int b = (int)(m % q.ho);
-    const long long t = m / q.ho;
-    const int a = (int)(t % q.wo);
-    const long long n = t / q.wo;
+    const long long m0 = (long long)(blockIdx.x / q.n_cotile) * R;
     const int groups = q.add_outer * q.add_inner;
     const int p = blockIdx.y / groups, g = blockIdx.y - p * groups;
     const int go = g / q.add_inner, gi = g - go * q.add_inner;
@@ -374,17 +376,29 @@ __global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q)
     const int members = q.or_rows * chs * q.w_k;
     const size_t lines_per_pack = (size_t)q.or_rows * q.add_inner * q.or_ch_total * q.w_k;
     const size_t line0 = p * lines_per_pack + (size_t)ch0 * q.add_inner * q.w_k + (size_t)gi * chs * q.w_k;
-    const uint32_t* ap0 = q.act + ((size_t)n * q.packs + p) * q.act_plane + (size_t)gi * q.add_stride +
-                          (size_t)ch0 * q.or_stride + (size_t)a * q.hi + b;
-
-    uint32_t orp[C], orn[C];
+    const uint32_t* ap0[R];
 #pragma unroll
-    for (int c = 0; c < C; c++) orp[c] = orn[c] = 0u;
+    for (int r = 0; r < R; r++) {
+        const long long m = m0 + r < positions ? m0 + r : m0;  // a position past the end is never stored
+        const int b = (int)(m % q.ho);
+        const long long t = m / q.ho;
+        const int a = (int)(t % q.wo);
+        const long long n = t / q.wo;
+        ap0[r] = q.act + ((size_t)n * q.packs + p) * q.act_plane + (size_t)gi * q.add_stride +
+                 (size_t)ch0 * q.or_stride + (size_t)a * q.hi + b;
+    }
+
+    uint32_t acc[R * 2 * C];  // [position][rail][channel]
+#pragma unroll
+    for (int i = 0; i < R * 2 * C; i++) acc[i] = 0u;
     for (int j = lane; j < members; j += 64) {
         // member j = (kernel row of the OR, channel of the group, tap u), u fastest
         const int u = j % q.w_k, t2 = j / q.w_k;
         const int ch = t2 % chs, row = t2 / chs;
-        const uint32_t aw = ap0[(size_t)ch * q.or_stride + (size_t)u * q.hi + row];
+        const size_t off = (size_t)ch * q.or_stride + (size_t)u * q.hi + row;
+        uint32_t aw[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) aw[r] = ap0[r][off];
         const uint4* wl = reinterpret_cast<const uint4*>(q.wgt + ((line0 + j) * q.n_cotile + cot) * (2 * C));
         uint32_t wv[2 * C];
 #pragma unroll
@@ -396,25 +410,30 @@ __global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q)
             wv[4 * v4 + 3] = w4.w;
         }
 #pragma unroll
-        for (int c = 0; c < C; c++) {
-            orp[c] |= aw & wv[c];
-            orn[c] |= aw & wv[C + c];
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int c = 0; c < 2 * C; c++) acc[r * 2 * C + c] |= aw[r] & wv[c];
+    }
+    static_assert(R * 2 * C == 64, "one finished word per lane");
+#pragma unroll
+    for (int half = 32; half >= 1; half >>= 1) {
+        const bool upper = (lane & half) != 0;
+#pragma unroll
+        for (int i = 0; i < half; i++) {
+            const uint32_t keep = upper ? acc[i + half] : acc[i], give = upper ? acc[i] : acc[i + half];
+            acc[i] = keep | (uint32_t)__shfl_xor((int)give, half);
         }
     }
-    int mine = 0;
-#pragma unroll
-    for (int c = 0; c < C; c++) {
-        uint32_t vp = orp[c], vn = orn[c];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            vp |= (uint32_t)__shfl_xor((int)vp, off);
-            vn |= (uint32_t)__shfl_xor((int)vn, off);
-        }
-        if (lane == c) mine = __popc(vp) - __popc(vn);
-    }
-    const int co = cot * C + lane;
-    if (lane < C && co < q.c_out)
-        atomicAdd(q.y + (((size_t)n * q.c_out + co) * q.wo + a) * q.ho + b, mine);
+    const int mine = __popc(acc[0]);
+    const int other = __shfl_xor(mine, C);  // the channel's other rail
+    const long long m = m0 + (lane >> 5);
+    const int co = cot * C + (lane & (C - 1));
+    if ((lane & C) || m >= positions || co >= q.c_out) return;
+    const int b = (int)(m % q.ho);
+    const long long t = m / q.ho;
+    const int a = (int)(t % q.wo);
+    const long long n = t / q.wo;
+    atomicAdd(q.y + (((size_t)n * q.c_out + co) * q.wo + a) * q.ho + b, mine - other);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -614,135 +633,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     }
 }
 
-// k_conv_fwd_rail for 3-wide kernels with the activation words staged through LDS.  The waves of the
-// c_out tiles of one position tile read the same four activation words per lane and channel; here
-// NWV of them form a workgroup, every wave fetches 8 / NWV channels of a chunk of 8 and leaves them in
-// LDS as 16 bytes per lane, and all read them back with one ds_read_b128 per channel: an eighth (a
-// quarter) of the global loads per wave, and the wait in front of a channel's 96 vector instructions is
-// for LDS and the scalar cache instead of the vector memory path.  The chunks are double-buffered:
-// the loads of chunk t + 1 are issued before chunk t is computed and written to LDS after it, one
-// barrier per chunk.  NPT position tiles (NWV waves each, staged separately) share the workgroup and
-// its barrier.  Needs c_in % 8 == 0 and n_cotile % NWV == 0 (the launcher checks).
-constexpr int kStageChannels = 8;
-template <int NWV, int NPT>
-__global__ __launch_bounds__(64 * NWV * NPT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_fwd_rail_lds(FwdParams q)
-{
-    constexpr int C = kCoTile, R = 2, WK = 3, NW = R + WK - 1, CH = kStageChannels, CPW = CH / NWV;
-    static_assert(NW == 4 && CH % NWV == 0, "a lane's words of one channel are one uint4");
-    __shared__ uint4 stage_all[2][NPT][CH][64];
-    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int wave = wave_all % NWV, pt = wave_all / NWV;  // c_out tile and position tile inside the workgroup
-    const int cot_groups = q.n_cotile / NWV;
-    const int cot = (blockIdx.x % cot_groups) * NWV + wave;
-    const long long slot0 = ((long long)(blockIdx.x / cot_groups) * NPT + pt) * 64 + lane;
-    const bool live = slot0 < q.slots;
-    const long long slot = live ? slot0 : 0;
-    const int b = (int)(slot % q.ho);
-    const long long t = slot / q.ho;
-    const int a0 = (int)(t % q.row_groups) * R;
-    const long long n = t / q.row_groups;
-    const unsigned item_stride = (unsigned)q.packs * q.act_plane;
-    // byte offsets of the lane's four rows in the stream buffer (under 4 GB: the launcher checks), read
-    // with buffer loads: the chunk's and channel's offset is the scalar operand
-    unsigned voff[NW];
-#pragma unroll
-    for (int j = 0; j < NW; j++) {
-        const int row = a0 + j < q.wi ? a0 + j : q.wi - 1;
-        voff[j] = 4u * ((unsigned)n * item_stride + (unsigned)b + (unsigned)row * q.hi);
-    }
-    const unsigned ch_b = 4u * (unsigned)q.wi * q.hi;
-    const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(q.act), 0, (int)(4u * (unsigned)q.n * item_stride), 0x00020000);
-    const int chunks_per_pass = q.c_in / CH;
-    // this launch row's share of the (pack, kernel row) passes; with more than one row the partial sums
-    // are added to the zeroed y with integer atomics
-    const int pass_begin = blockIdx.y * q.pv_per_block;
-    const int passes = min(q.packs * q.h_k, pass_begin + q.pv_per_block);
-    const int total = (passes - pass_begin) * chunks_per_pass;
-
-    int sum[2 * C];  // [2 c + r]
-#pragma unroll
-    for (int i = 0; i < 2 * C; i++) sum[i] = 0;
-
-    // this wave's channels of chunk (pass, cc): wave + NWV * i
-    uint4 fetched[CPW];
-    auto fetch = [&](int pass, int cc) {
-        const int p = pass / q.h_k, v = pass - p * q.h_k;
-        const unsigned so = 4u * ((unsigned)p * q.act_plane + (unsigned)v) + (unsigned)(cc * CH + wave) * ch_b;
-#pragma unroll
-        for (int i = 0; i < CPW; i++) {
-            const int sc = (int)(so + (unsigned)(NWV * i) * ch_b);
-            fetched[i] = make_uint4(__builtin_amdgcn_raw_buffer_load_b32(act, (int)voff[0], sc, 0),
-                                    __builtin_amdgcn_raw_buffer_load_b32(act, (int)voff[1], sc, 0),
-                                    __builtin_amdgcn_raw_buffer_load_b32(act, (int)voff[2], sc, 0),
-                                    __builtin_amdgcn_raw_buffer_load_b32(act, (int)voff[3], sc, 0));
-        }
-    };
-    auto commit = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < CPW; i++) stage_all[buf][pt][wave + NWV * i][lane] = fetched[i];
-    };
-
-    const size_t line0 = (size_t)cot * q.rail_lines + (size_t)pass_begin * q.c_in * WK;
-    const uint32_t* wp = q.wgt_rail + line0 * C;
-    const uint32_t* ip = q.wgt_rail_idx + line0 * (C / 2);
-    fetch(pass_begin, 0);
-    commit(0);
-    __syncthreads();
-    int tc = 0;
-    for (int pass = pass_begin; pass < passes; pass++) {
-        u32x16 p0 = 0u, p1 = 0u, n0 = 0u, n1 = 0u;
-        for (int cc = 0; cc < chunks_per_pass; cc++, tc++) {
-            const int buf = tc & 1;
-            // the chunk after this one may belong to the next pass
-            const bool last_of_pass = cc + 1 == chunks_per_pass;
-            const bool more = tc + 1 < total;
-            if (more) fetch(last_of_pass ? pass + 1 : pass, last_of_pass ? 0 : cc + 1);
-            for (int ch = 0; ch < CH; ch++) {
-                const uint4 aw = stage_all[buf][pt][ch][lane];
-                uint32_t wv[WK][C], iv[WK][C / 2];
-#pragma unroll
-                for (int l = 0; l < WK; l++) {
-#pragma unroll
-                    for (int c = 0; c < C; c++) wv[l][c] = wp[l * C + c];
-#pragma unroll
-                    for (int c = 0; c < C / 2; c++) iv[l][c] = ip[l * (C / 2) + c];
-                }
-                rail_line(p0, p1, n0, n1, wv[0], iv[0], aw.x, aw.y);
-                rail_line(p0, p1, n0, n1, wv[1], iv[1], aw.y, aw.z);
-                rail_line(p0, p1, n0, n1, wv[2], iv[2], aw.z, aw.w);
-                wp += WK * C;
-                ip += WK * (C / 2);
-            }
-            if (more) commit(buf ^ 1);
-            __syncthreads();
-        }
-        // end of a (pack, kernel row) pass: binary add across kernel rows and packs
-#pragma unroll
-        for (int i = 0; i < C; i++) {
-            sum[i] += __popc(p0[i]) - __popc(n0[i]);
-            sum[C + i] += __popc(p1[i]) - __popc(n1[i]);
-        }
-    }
-
-    if (!live) return;
-    const size_t out_plane = (size_t)q.wo * q.ho;
-#pragma unroll
-    for (int c = 0; c < C; c++) {
-        const int co = cot * C + c;
-        if (co >= q.c_out) break;
-        int32_t* yo = q.y + ((size_t)n * q.c_out + co) * out_plane + (size_t)a0 * q.ho + b;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            if (a0 + r >= q.wo) continue;
-            if (gridDim.y == 1)
-                yo[(size_t)r * q.ho] = sum[2 * c + r];
-            else
-                atomicAdd(yo + (size_t)r * q.ho, sum[2 * c + r]);  // integer adds: order does not matter
-        }
-    }
-}
-
 // The rail-skipping form of k_conv_fwd_split<2, WK, 1, false>: launches split over blockIdx.y and
 // the accumulation modes other than y, position-major activation streams, two output rows per lane.
 // Partial sums are added to the zeroed y with integer atomics.
@@ -878,66 +768,63 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     }
 }
 
-// k_conv_fwd_split_rail for launches in which every wave sums exactly one (pack, add group) pair (blockIdx.y =
-// the pair): small layers split as far as they go.  Without running sums a wave needs 96 registers instead of
-// 128 - the 64 accumulators sit at v[32:95], the counts go from the popcounts straight into the atomics - so
-// five waves fit a SIMD instead of four: 5120 waves (the 32 -> 64 5 x 5 layer at 8 x 8, batch 256) are one
-// round instead of two, of which the second would run a quarter full and bound by load latency.
-// Two waves per workgroup, each with a tile of its own: a CU takes at most 16 workgroups, which single-wave
-// workgroups would hit at four waves per SIMD.
-// WG: the pairs of one tile as the waves of one workgroup (at most 16 pairs): their counts meet in LDS
-// (ds_add_u32) and the workgroup stores the sums - no zeroing launch over y and no global atomics, whose
-// drain is what such a launch otherwise ends with (the 32 -> 64 layer: waves live 59 us of the 88 us that
-// the launch with atomics takes).
-constexpr int kPairWaves = 2, kPairWgMax = 16;
-template <int WK, int CU, bool WG = false>
-__global__ __launch_bounds__(WG ? 64 * kPairWgMax : 64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(5, 5)))
-void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
-{
-    constexpr int C = kCoTile, R = 2, NW = R + WK - 1;
-    __shared__ int red[WG ? 2 * C * 64 : 1];  // [2 c + r][lane]
-    const int wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned tile = WG ? blockIdx.x : blockIdx.x * kPairWaves + wave_in_wg;
-    if (!WG && tile >= n_tiles) return;
-    if constexpr (WG) {
-        for (int i = threadIdx.x; i < 2 * C * 64; i += blockDim.x) red[i] = 0;
-        __syncthreads();
-    }
-    const int cot = tile % q.n_cotile;
-    const long long slot0 = (long long)(tile / q.n_cotile) * 64 + (threadIdx.x & 63);
-    const bool live = slot0 < q.slots;
-    const long long slot = live ? slot0 : 0;
-    const int b = (int)(slot % q.ho);
-    const long long t = slot / q.ho;
-    const int a0 = (int)(t % q.row_groups) * R;
-    const long long n = t / q.row_groups;
-    const unsigned item_stride = (unsigned)q.packs * q.act_plane;
+// The five-wave kernels (accumulators at v[32:95], 96 registers): launches in which a wave keeps no running sums.
+// A lane's position and the byte offsets of its rows in the stream buffer (the launcher keeps the buffer under
+// 4 GB); rows past the end (partial last group) are clamped to valid ones: they only feed outputs that are never
+// stored.
+template <int NW>
+struct PairLane {
+    bool live;
+    int a0, b;
+    long long n;
     unsigned voff[NW];
+    __device__ __forceinline__ PairLane(const FwdParams& q, long long slot0)
+    {
+        live = slot0 < q.slots;
+        const long long slot = live ? slot0 : 0;
+        b = (int)(slot % q.ho);
+        const long long t = slot / q.ho;
+        a0 = (int)(t % q.row_groups) * 2;
+        n = t / q.row_groups;
 #pragma unroll
-    for (int j = 0; j < NW; j++) {
-        const int row = a0 + j < q.wi ? a0 + j : q.wi - 1;
-        voff[j] = 4u * ((unsigned)n * item_stride + (unsigned)b + (unsigned)row * q.hi);
+        for (int j = 0; j < NW; j++) {
+            const int row = a0 + j < q.wi ? a0 + j : q.wi - 1;
+            voff[j] = 4u * ((unsigned)n * (unsigned)q.packs * q.act_plane + (unsigned)b + (unsigned)row * q.hi);
+        }
     }
-    const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(q.act), 0, (int)(4u * (unsigned)q.n * item_stride), 0x00020000);
-    const unsigned plane_b = 4u * q.act_plane, add_b = 4u * q.add_stride, or_b = 4u * q.or_stride;
+};
 
+// Weight lines as constant memory (no launch that reads them writes them): where LDS atomics and barriers sit
+// in the same loop the compiler reads a plain global pointer with vector loads.
+typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+
+// OR of one (pack, add group) pair over share `share` of `shares` of the group's channels, assigned to the
+// accumulators; false where the share has no channels (nothing is assigned then).
+template <int WK, int CU>
+__device__ __forceinline__ bool or_pair(const FwdParams& q, __amdgpu_buffer_rsrc_t act, const unsigned (&voff)[WK + 1],
+                                        int cot, int pv, int share, int shares, u32x16& p0, u32x16& p1, u32x16& n0,
+                                        u32x16& n1)
+{
+    constexpr int C = kCoTile, NW = WK + 1;
+    const unsigned plane_b = 4u * q.act_plane, add_b = 4u * q.add_stride, or_b = 4u * q.or_stride;
     const int groups = q.add_outer * q.add_inner;
-    const int pv = WG ? wave_in_wg : blockIdx.y;
     const int p = pv / groups;
     const int go = (pv - p * groups) / q.add_inner;
     const int gi = pv - p * groups - go * q.add_inner;
     const int ch0 = go * q.or_ch_per_group;
     const int chs = min(q.or_ch_per_group, q.or_ch_total - ch0);
+    const int chunk = (chs + shares - 1) / shares;
+    const int c_begin = min(chs, chunk * share), c_end = min(chs, chunk * (share + 1));
+    if (c_begin == c_end) return false;
     const size_t lines_per_pack = (size_t)q.or_rows * q.add_inner * q.or_ch_total * q.w_k;
     const size_t line = (size_t)cot * q.rail_lines + p * lines_per_pack + (size_t)ch0 * q.add_inner * q.w_k +
                         (size_t)gi * chs * q.w_k;
-    const uint32_t* wp = q.wgt_rail + line * C;
-    const uint32_t* ip = q.wgt_rail_idx + line * (C / 2);
-    u32x16 p0, p1, n0, n1;  // written by the group's first line
     bool first = true;
-    const unsigned group_off = (unsigned)p * plane_b + (unsigned)gi * add_b + (unsigned)ch0 * or_b;
+    const unsigned group_off = (unsigned)p * plane_b + (unsigned)gi * add_b + (unsigned)(ch0 + c_begin) * or_b;
     for (int row = 0; row < q.or_rows; row++) {
+        const size_t line_row = line + ((size_t)row * chs + c_begin) * WK;
+        ConstWords wp = (ConstWords)(q.wgt_rail + line_row * C);
+        ConstWords ip = (ConstWords)(q.wgt_rail_idx + line_row * (C / 2));
         unsigned ch_off = group_off + 4u * (unsigned)row;  // next kernel row: one word further
         auto channels_of = [&](auto cu_tag, auto first_tag) {
             constexpr int N = decltype(cu_tag)::value;
@@ -976,33 +863,40 @@ void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
                 channels_of(cu_tag, std::false_type());
             first = false;
         };
-        int ci = 0;
-        for (; ci + CU <= chs; ci += CU) channels(std::integral_constant<int, CU>());
+        int ci = c_begin;
+        for (; ci + CU <= c_end; ci += CU) channels(std::integral_constant<int, CU>());
         if constexpr (CU > 1)
-            for (; ci < chs; ci++) channels(std::integral_constant<int, 1>());
+            for (; ci < c_end; ci++) channels(std::integral_constant<int, 1>());
     }
+    return true;
+}
+
+// k_conv_fwd_split_rail for launches in which every wave sums exactly one (pack, add group) pair (blockIdx.y =
+// the pair) and which are more than a round of waves.  Without running sums a wave needs 96 registers instead of
+// 128 - the 64 accumulators sit at v[32:95], the counts go from the popcounts straight into the atomics - so
+// five waves fit a SIMD instead of four.
+// Two waves per workgroup, each with a tile of its own: a CU takes at most 16 workgroups, which single-wave
+// workgroups would hit at four waves per SIMD.
+constexpr int kPairWaves = 2;
+template <int WK, int CU>
+__global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(5, 5)))
+void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
+{
+    constexpr int C = kCoTile;
+    const int wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned tile = blockIdx.x * kPairWaves + wave_in_wg;
+    if (tile >= n_tiles) return;
+    const int cot = tile % q.n_cotile;
+    const PairLane<WK + 1> at(q, (long long)(tile / q.n_cotile) * 64 + (threadIdx.x & 63));
+    const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(q.act), 0, (int)(4u * (unsigned)q.n * (unsigned)q.packs * q.act_plane), 0x00020000);
+    u32x16 p0, p1, n0, n1;  // written by the group's first line
+    or_pair<WK, CU>(q, act, at.voff, cot, blockIdx.y, 0, 1, p0, p1, n0, n1);
+    if (!at.live) return;
     const size_t out_plane = (size_t)q.wo * q.ho;
-    int32_t* yo = q.y + ((size_t)n * q.c_out + (size_t)cot * C) * out_plane + (size_t)a0 * q.ho + b;
-    const bool row1 = a0 + 1 < q.wo;
+    int32_t* yo = q.y + ((size_t)at.n * q.c_out + (size_t)cot * C) * out_plane + (size_t)at.a0 * q.ho + at.b;
+    const bool row1 = at.a0 + 1 < q.wo;
     // accumulator (channel c, row r) is element 2 c + r of the 32: p0 / n0 hold channels 0 - 7, p1 / n1 8 - 15
-    if constexpr (WG) {
-        const int lane = threadIdx.x & 63;
-#pragma unroll
-        for (int e = 0; e < 2 * C; e++) {
-            const u32x16& pv16 = e < C ? p0 : p1;
-            const u32x16& nv16 = e < C ? n0 : n1;
-            atomicAdd(&red[e * 64 + lane], __popc(pv16[e % C]) - __popc(nv16[e % C]));  // result unused: ds_add_u32
-        }
-        __syncthreads();
-        if (!live) return;
-        const int n_waves = blockDim.x >> 6;
-        for (int e = wave_in_wg; e < 2 * C; e += n_waves) {
-            const int c = e >> 1, r = e & 1;
-            if (cot * C + c < q.c_out && (r == 0 || row1)) yo[(size_t)c * out_plane + (size_t)r * q.ho] = red[e * 64 + lane];
-        }
-        return;
-    }
-    if (!live) return;
 #pragma unroll
     for (int c = 0; c < C; c++) {
         if (cot * C + c >= q.c_out) break;
@@ -1011,6 +905,94 @@ void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
         const int e = 2 * (c % (C / 2));
         atomicAdd(yo + (size_t)c * out_plane, __popc(pv16[e]) - __popc(nv16[e]));  // integer adds: order does not matter
         if (row1) atomicAdd(yo + (size_t)c * out_plane + q.ho, __popc(pv16[e + 1]) - __popc(nv16[e + 1]));
+    }
+}
+
+// The kernel of most launches: a workgroup owns one tile (64 lane slots x 16 channels) and works on
+// blockDim / (64 or_shares) pairs at a time, `or_shares` waves to a pair, `pairs_per_slot` pairs one after the other.
+// Bound by the issue rate of v_and_or_b32 where the launch fills the GPU; what decides then is the number of
+// waves a SIMD can choose from, as every wave waits ~1800 cycles for its channel's words and weight lines and
+// then issues 96 (3 lines) x 4.4 cycles: the counts are summed in LDS (ds_add_u32) instead of in 32 registers, so
+// that five waves fit a SIMD.  128 -> 128 channels, 3 x 3, 16 x 16, batch 256, L 128: 1.155 ms; with the sums in
+// registers (four waves) 1.38, and 1.29 with the activation words of four c_out tiles staged through LDS besides,
+// which this kernel replaced; 64 -> 64 at 56 x 56, L 256, batch 30: 0.95 -> 0.87.
+// or_shares > 1, for launches with too few (tile, pair) waves: an OR can be cut anywhere, so every wave of a pair
+// takes a share of the channels and the partial words meet in LDS (ds_or_b32).  512 -> 512 channels, L 128:
+// 4 x 4 images, batch 50: 474 -> 300 us, batch 128: 924 -> 605; 2 x 2, batch 50: 1760 -> 190 (where lanes ran
+// over the members); 32 -> 32, 5 x 5, 16 x 16, one image: 27 -> 12.
+// With one row of blocks the sums are stored (no zeroing launch, no global atomics); with more they are added to
+// the zeroed y.
+// Dynamic LDS: 32 x 64 sums, and with or_shares > 1 a 64 x 64 OR buffer per pair in flight.
+constexpr int kTileWaves = 16;
+template <int WK, int CU>
+__global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu(5, 5)))
+void k_conv_fwd_tile_rail(FwdParams q)
+{
+    constexpr int C = kCoTile;
+    extern __shared__ uint32_t tile_lds[];
+    int* red = reinterpret_cast<int*>(tile_lds);  // [2 c + r][lane]
+    uint32_t* orb = tile_lds + 2 * C * 64;        // [pair][rail][2 c + r][lane]
+    const int waves = blockDim.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int shares = q.or_shares, in_flight = waves / shares;
+    const int mine = wave / shares, share = wave - mine * shares;
+    const int lds_words = 2 * C * 64 + (shares > 1 ? in_flight * 4 * C * 64 : 0);
+    for (int i = threadIdx.x; i < lds_words; i += blockDim.x) tile_lds[i] = 0;
+    __syncthreads();
+    const int cot = blockIdx.x % q.n_cotile;
+    const PairLane<WK + 1> at(q, (long long)(blockIdx.x / q.n_cotile) * 64 + lane);
+    const __amdgpu_buffer_rsrc_t act = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(q.act), 0, (int)(4u * (unsigned)q.n * (unsigned)q.packs * q.act_plane), 0x00020000);
+    const int pairs = q.packs * q.add_outer * q.add_inner;
+    for (int it = 0; it < q.pairs_per_slot; it++) {
+        const int pv = (blockIdx.y * q.pairs_per_slot + it) * in_flight + mine;
+        u32x16 p0, p1, n0, n1;  // written by the group's first line
+        if (pv < pairs && or_pair<WK, CU>(q, act, at.voff, cot, pv, share, shares, p0, p1, n0, n1)) {
+            if (shares == 1) {
+#pragma unroll
+                for (int e = 0; e < C; e++) {  // results unused: ds_add_u32
+                    atomicAdd(&red[e * 64 + lane], __popc(p0[e]) - __popc(n0[e]));
+                    atomicAdd(&red[(C + e) * 64 + lane], __popc(p1[e]) - __popc(n1[e]));
+                }
+            } else {
+                uint32_t* o = orb + mine * (4 * C * 64) + lane;
+#pragma unroll
+                for (int e = 0; e < C; e++) {
+                    atomicOr(o + e * 64, p0[e]);
+                    atomicOr(o + (C + e) * 64, p1[e]);
+                    atomicOr(o + (2 * C + e) * 64, n0[e]);
+                    atomicOr(o + (3 * C + e) * 64, n1[e]);
+                }
+            }
+        }
+        if (shares > 1) {
+            __syncthreads();
+            // element e of the 32 belongs to one wave: it counts, sums and clears for the next pairs
+            for (int e = wave; e < 2 * C; e += waves) {
+                int d = red[e * 64 + lane];
+                for (int s = 0; s < in_flight; s++) {
+                    uint32_t* o = orb + s * (4 * C * 64) + e * 64 + lane;
+                    d += __popc(o[0]) - __popc(o[2 * C * 64]);
+                    o[0] = 0;
+                    o[2 * C * 64] = 0;
+                }
+                red[e * 64 + lane] = d;
+            }
+            if (it + 1 < q.pairs_per_slot) __syncthreads();
+        }
+    }
+    __syncthreads();
+    if (!at.live) return;
+    const size_t out_plane = (size_t)q.wo * q.ho;
+    int32_t* yo = q.y + ((size_t)at.n * q.c_out + (size_t)cot * C) * out_plane + (size_t)at.a0 * q.ho + at.b;
+    for (int e = wave; e < 2 * C; e += waves) {
+        const int c = e >> 1, r = e & 1;
+        if (cot * C + c >= q.c_out || at.a0 + r >= q.wo) continue;
+        int32_t* dst = yo + (size_t)c * out_plane + (size_t)r * q.ho;
+        if (gridDim.y == 1)
+            *dst = red[e * 64 + lane];
+        else
+            atomicAdd(dst, red[e * 64 + lane]);  // integer adds: order does not matter
     }
 }
 
@@ -1386,37 +1368,32 @@ __global__ __launch_bounds__(256) void k_zero_i32(int32_t* __restrict__ p, size_
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = 0;
 }
 
-// How a position-parallel launch (R accumulator rows per lane, kernel extent WK in dim 2, 0: run-time) is cut:
+// How a position-parallel launch (R accumulator rows per lane) is cut whose waves keep their sums in registers:
 // waves of 64 lane slots per c_out tile, and the (pack, add group) pairs shared out over blockIdx.y.
 struct SplitPlan {
     int row_groups;
     long long slots, tiles, waves;
     int pv, splits, pv_per_block;
-    bool lds;  // the kernel that shares activation words through LDS
 };
-SplitPlan plan_splits(const Geometry& g, int R, int WK, bool rows_in_n)
+SplitPlan plan_splits(const Geometry& g, int R, bool rows_in_n)
 {
     SplitPlan sp;
     sp.row_groups = rows_in_n ? (g.n + R - 1) / R : (g.wo + R - 1) / R;
     sp.slots = rows_in_n ? (long long)sp.row_groups * g.ho : (long long)g.n * sp.row_groups * g.ho;
     sp.tiles = (sp.slots + 63) / 64;
     sp.waves = sp.tiles * g.n_cotile;
-    // Fewer than four waves per SIMD (small layers, the SC-linear mapping): split the (pack, add
-    // group) sum over blockIdx.y until about twelve waves per SIMD exist, so that three resident
-    // waves per SIMD stay available through the tail; the partial sums meet in y through integer
-    // atomics.  Measured on MI355X: 4096x4096 linear at batch 1024 7.05 -> 6.24 ms.
+    // Fewer than four waves per SIMD (small layers): split the (pack, add group) sum over blockIdx.y until
+    // about twelve waves per SIMD exist, so that three resident waves per SIMD stay available through the tail;
+    // the partial sums meet in y through integer atomics.
     sp.pv = g.packs * g.add_outer * g.add_inner;
     int splits = 1;
-    // the LDS-staged kernel: y mode, 3-wide kernels, whole chunks of 8 channels, 4 or 8 c_out tiles
-    sp.lds = R == 2 && WK == 3 && !rows_in_n && g.rail && g.mode == GEO_SC_ACC_Y &&
-             g.c_in % kStageChannels == 0 && g.n_cotile % 4 == 0;
     if (sp.waves < 4096) {
         splits = (int)((12288 + sp.waves - 1) / sp.waves);
         if (splits > sp.pv) splits = sp.pv;
     } else if (g.rail && !rows_in_n) {
         // Equal waves run in rounds of 4096 (four per SIMD): 3.06 rounds take the time of 4.  Splitting the
-        // passes 2-, 3- or 4-fold makes the rounds shorter and the last one fuller (C5: 12544 waves, 0.77 ->
-        // 0.94 of the rounded-up time); taken when it gains more than the atomics cost.
+        // passes 2-, 3- or 4-fold makes the rounds shorter and the last one fuller; taken when it gains more than
+        // the atomics cost.
         auto fill = [&](int k) { const double r = (double)sp.waves * k / 4096.0; return r / (double)(long long)(r + 0.999999); };
         double best = fill(1) * 1.08;
         for (int k = 2; k <= 4; k++)
@@ -1430,22 +1407,81 @@ SplitPlan plan_splits(const Geometry& g, int R, int WK, bool rows_in_n)
     return sp;
 }
 
+// The rail-skipping launches with two output rows per lane (position-major streams).
+enum RailKernel { kRailPlain, kRailSplit, kRailPair, kRailTile };
+struct RailPlan {
+    RailKernel kernel;
+    int shares, in_flight, per_slot;  // kRailTile
+    int splits;                       // blockIdx.y
+};
+constexpr long long kPairRound = 5 * 4 * 256;  // waves of a round with five waves per SIMD
+RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
+{
+    const long long lines = (long long)g.or_rows * g.or_ch_per_group * g.w_k;  // of an OR group
+    const long long tiles = sp.waves, pairs = tiles * sp.pv;                   // (tile, pair) waves
+    const int pv = sp.pv;
+    RailPlan p = {kRailTile, 1, 4, 1, 1};
+    // Short groups, where the 32 LDS additions at the end of a group weigh most, keep their sums in registers
+    // once four waves per SIMD exist without splitting a tile (3 -> 32, 5 x 5, 32 x 32, batch 256, L 64: 64 us
+    // against 72), or with so many groups per tile that the tile kernel's per-group work shows (z mode, 3 x 3, 1320
+    // groups of 309 tiles: 395 against 439 us; 1220 groups of 116 tiles: 146 against 162).
+    if (g.mode == GEO_SC_ACC_Y && tiles >= 4096 && lines <= 24) return {kRailPlain, 0, 0, 0, 1};
+    if (lines <= 12 && pairs >= 100000) return {kRailSplit, 0, 0, 0, sp.splits};
+    // Long groups, few of them per tile, in launches whose waves fill their rounds: the counts of a pair go
+    // straight to y (64 -> 64, 3 x 3, 32 x 32, batch 128, L 64: 327 us against 336).  With twelve pairs per tile, or
+    // with image rows shorter than 16 (more lines per atomic), the atomics cost more than that gains.
+    const long long rounds = (pairs + kPairRound - 1) / kPairRound;
+    if (pv <= 10 && g.w_k >= 3 && lines >= 96 && g.ho >= 16 && pairs > 4096 && pairs * 5 >= rounds * kPairRound * 4)
+        return {kRailPair, 0, 0, 0, pv};
+    if (lines >= 48 && g.or_ch_per_group >= 16 && !(pairs >= 8192 && (pv >= 12 || g.w_k == 1))) {
+        // Too few waves: the OR of a group shared out over four, eight or sixteen of them (a workgroup of a
+        // multiple of four waves loads the four SIMDs alike: 512 -> 512 at 4 x 4, batch 50: 4 shares 300 us, 3: 337,
+        // 6: 392)
+        p.in_flight = 1;
+        p.shares = pairs * 4 >= 2048 || g.or_ch_per_group < 32   ? 4
+                   : pairs * 8 >= 2048 || g.or_ch_per_group < 64 ? 8
+                                                                 : 16;
+        p.splits = pv;
+        // a round of waves without splitting the tiles, groups short enough for the atomics to show: all pairs
+        // of a tile in one workgroup (32 -> 64, 5 x 5, 8 x 8, batch 256, L 64: 76 us; 88 with one pair each)
+        if (p.shares == 4 && tiles >= 512 && lines < 256 && pv <= 16) {
+            p.in_flight = 2;
+            p.per_slot = (pv + 1) / 2;
+            p.splits = 1;
+        }
+        return p;
+    }
+    if (lines <= 48 && tiles < 1024 && pv <= 24) {
+        // few short groups: all pairs of a tile in one workgroup where that leaves enough of them
+        p.in_flight = pv <= 4 ? 4 : pv <= 8 || pv > 16 || tiles >= 128 ? 8 : 16;
+        p.per_slot = tiles >= 128 ? (pv + p.in_flight - 1) / p.in_flight : 1;
+    } else {
+        // pairs one after the other: fewer additions to y against a longer last round
+        const int most = (pv + 3) / 4;
+        int want = lines >= 256 ? 2 : lines >= 80 ? 4 : lines >= 20 ? (int)(160 / lines) : 8;
+        if (want > most) want = most;
+        while (want > 1 && tiles * ((most + want - 1) / want) < kPairRound / 4) want--;
+        p.per_slot = want;
+    }
+    if (pv / p.in_flight / p.per_slot >= 32768) p.per_slot = pv / p.in_flight / 32768 + 1;  // a grid's limit in y
+    const int per_block = p.in_flight * p.per_slot;
+    p.splits = (pv + per_block - 1) / per_block;
+    return p;
+}
+
 template <int R, int WK, int CU, bool ROWS_IN_N>
 int launch(const Geometry& g, FwdParams q, hipStream_t s)
 {
-    const SplitPlan sp = plan_splits(g, R, WK, ROWS_IN_N);
+    const SplitPlan sp = plan_splits(g, R, ROWS_IN_N);
     q.row_groups = sp.row_groups;
     q.slots = sp.slots;
-    const long long tiles = sp.tiles, blocks = sp.waves, waves = sp.waves;
+    const long long tiles = sp.tiles, blocks = sp.waves;
     if (blocks <= 0 || blocks > 0x7fffffffLL) return GEO_SC_ERR_INVALID_ARGUMENT;
     // per-lane word offsets are 32-bit
     if ((unsigned long long)R * g.packs * g.act_plane >= 0xffffffffull) return GEO_SC_ERR_UNSUPPORTED;
     if (ROWS_IN_N != g.act_item_inner) return GEO_SC_ERR_INVALID_ARGUMENT;
     const int pv = sp.pv;
-    int splits = sp.splits;
-    const bool lds = sp.lds;
     q.pv_per_block = sp.pv_per_block;
-    const bool plain = splits == 1 && g.mode == GEO_SC_ACC_Y && !ROWS_IN_N;
     if constexpr (ROWS_IN_N) {
         static_assert(R == 2 && WK > 0, "item-innermost launches take two items per lane");
         // the kernel addresses the whole stream buffer with 32-bit byte offsets; y mode only
@@ -1467,55 +1503,45 @@ int launch(const Geometry& g, FwdParams q, hipStream_t s)
         hipLaunchKernelGGL((k_conv_fwd_items_rail_wg<WK, CU, S>), dim3((unsigned)blocks), dim3(64 * S), 0, s, q);
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
-    // one (pack, add group) pair per wave and more than a round of waves: the form with five waves per SIMD,
-    // with the pairs of a tile in one workgroup where they are few enough
-    const bool pair = g.rail && R == 2 && WK > 0 && !lds && !plain && q.pv_per_block == 1 && waves * splits > 4096;
-    // (in one round of five waves per SIMD only: with a second round, whole workgroups wait for ten free wave
-    // slots of one CU, and the 32 -> 32 layer at 16 x 16 takes 161 us instead of 135 us)
-    const bool pair_wg = pair && splits <= kPairWgMax && waves * splits <= 5 * 4 * 256;
-    if (!plain && !pair_wg) {
+    auto clear_y = [&]() {
         const size_t n_out = (size_t)g.n * g.c_out * g.wo * g.ho;
-        size_t zb = (n_out + 255) / 256;
+        const size_t zb = (n_out + 255) / 256;
         hipLaunchKernelGGL(k_zero_i32, dim3((unsigned)(zb > 4096 ? 4096 : zb)), dim3(256), 0, s, q.y, n_out);
-    }
-    const dim3 grid((unsigned)blocks, (unsigned)(plain ? 1 : splits));
+    };
     if (g.rail) {
         if constexpr (R == 2 && WK > 0) {
             // two channels per trip for 1-wide kernels: with three, the six address pairs push the 32
             // sums out of the 128 registers
             constexpr int CR = WK == 1 ? 2 : 1;
-            if (lds) {
-                // c_out tiles of one position tile share their activation words through LDS
-                // Four c_out tiles per workgroup.  With eight tiles or more, four position tiles share the
-                // workgroup and its barrier (16 waves, the whole CU in step): the four waves of a c_out tile
-                // read the same weight lines at the same time, which the scalar cache then serves once
-                // (C3 1.38 -> 1.29 ms; 8 c_out tiles x 2 position tiles 1.31, 2 x 8 1.33).  With four tiles
-                // in all the common barrier costs more than that saves (C5).
-                const int nwv = 4;
-                const int npt = g.n_cotile % 8 == 0 ? 4 : 1;
-                const long long tile_sets = (tiles + npt - 1) / npt;
-                const dim3 grid_lds((unsigned)(tile_sets * (g.n_cotile / nwv)), (unsigned)splits);
-                if (npt == 4)
-                    hipLaunchKernelGGL((k_conv_fwd_rail_lds<4, 4>), grid_lds, dim3(1024), 0, s, q);
-                else
-                    hipLaunchKernelGGL((k_conv_fwd_rail_lds<4, 1>), grid_lds, dim3(256), 0, s, q);
-            } else if (plain)
+            const RailPlan rp = plan_rail(g, sp);
+            if (rp.splits > 1 || rp.kernel == kRailSplit) clear_y();
+            const dim3 grid((unsigned)blocks, (unsigned)rp.splits);
+            if (rp.kernel == kRailPlain)
                 hipLaunchKernelGGL((k_conv_fwd_rail<WK, CR>), grid, dim3(64), 0, s, q);
-            else if (pair_wg)
-                hipLaunchKernelGGL((k_conv_fwd_pair_rail<WK, CR, true>), dim3((unsigned)blocks), dim3(64 * splits), 0, s, q,
-                                   (unsigned)blocks);
-            else if (pair)
-                hipLaunchKernelGGL((k_conv_fwd_pair_rail<WK, CR>),
-                                   dim3((unsigned)((blocks + kPairWaves - 1) / kPairWaves), (unsigned)splits),
-                                   dim3(64 * kPairWaves), 0, s, q, (unsigned)blocks);
-            else
+            else if (rp.kernel == kRailSplit)
                 hipLaunchKernelGGL((k_conv_fwd_split_rail<WK, CR>), grid, dim3(64), 0, s, q);
+            else if (rp.kernel == kRailPair)
+                hipLaunchKernelGGL((k_conv_fwd_pair_rail<WK, CR>),
+                                   dim3((unsigned)((blocks + kPairWaves - 1) / kPairWaves), (unsigned)rp.splits),
+                                   dim3(64 * kPairWaves), 0, s, q, (unsigned)blocks);
+            else {
+                q.or_shares = rp.shares;
+                q.pairs_per_slot = rp.per_slot;
+                const size_t lds = sizeof(uint32_t) * 64 * kCoTile * (2 + (rp.shares > 1 ? 4 * rp.in_flight : 0));
+                hipLaunchKernelGGL((k_conv_fwd_tile_rail<WK, CR>), grid,
+                                   dim3((unsigned)(64 * rp.shares * rp.in_flight)), lds, s, q);
+            }
         } else
             return GEO_SC_ERR_INVALID_ARGUMENT;  // make_geometry sets rail for two-row launches only
-    } else if (plain)
+        return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
+    }
+    const dim3 grid((unsigned)blocks, (unsigned)sp.splits);
+    if (sp.splits == 1 && g.mode == GEO_SC_ACC_Y)
         hipLaunchKernelGGL((k_conv_fwd<R, WK, CU, false>), grid, dim3(64), 0, s, q);
-    else
+    else {
+        clear_y();
         hipLaunchKernelGGL((k_conv_fwd_split<R, WK, CU, false>), grid, dim3(64), 0, s, q);
+    }
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
 
@@ -1529,10 +1555,10 @@ double conv_forward_cost(const Geometry& g)
         const double waves = ((double)g.n * g.wo * g.ho / 128.0 + 1.0) * g.n_cotile;
         return waves * pv / 4096.0;
     }
-    const int wk = g.w_k == 1 || g.w_k == 3 || g.w_k == 5 ? g.w_k : 0;
-    const SplitPlan sp = plan_splits(g, wk ? 2 : 1, wk, false);
-    const double rounds = (double)((sp.waves * sp.splits + 4095) / 4096);
-    return rounds * sp.pv_per_block;
+    // waves of one pair in rounds of five per SIMD; workgroups retire by themselves, so a round is not all or nothing
+    const SplitPlan sp = plan_splits(g, g.rail ? 2 : 1, false);
+    const double fifths = std::ceil((double)sp.waves * pv / (kPairRound / 5));
+    return fifths < 5 ? 1.0 : fifths / 5;
 }
 
 int launch_rail_pack(const Geometry& g, uint32_t* wgt, hipStream_t s, bool from_generator)
@@ -1569,6 +1595,7 @@ int launch_conv_forward(const Geometry& g, const uint32_t* act, const uint32_t* 
     q.act_plane = (unsigned)g.act_plane;
     q.row_groups = 0;
     q.keep_touches = 0;
+    q.or_shares = q.pairs_per_slot = 0;
     q.slots = 0;
     q.n = g.n;
     q.add_outer = g.add_outer;
@@ -1580,13 +1607,14 @@ int launch_conv_forward(const Geometry& g, const uint32_t* act, const uint32_t* 
     q.or_stride = g.mode == GEO_SC_ACC_Z ? 1u : ch_plane;
     q.or_rows = g.or_rows;
     if (g.thin) {
-        const long long blocks = (long long)g.n * g.wo * g.ho * g.n_cotile;
+        const long long positions = (long long)g.n * g.wo * g.ho;
+        const long long blocks = (positions + kThinPositions - 1) / kThinPositions * g.n_cotile;
         const long long pv = (long long)g.packs * g.add_outer * g.add_inner;
         if (blocks > 0x7fffffffLL || pv > 65535 || g.act_item_inner) return GEO_SC_ERR_INVALID_ARGUMENT;
         const size_t n_out = (size_t)g.n * g.c_out * g.wo * g.ho;
         size_t zb = (n_out + 255) / 256;
         hipLaunchKernelGGL(k_zero_i32, dim3((unsigned)(zb > 4096 ? 4096 : zb)), dim3(256), 0, s, q.y, n_out);
-        hipLaunchKernelGGL(k_conv_fwd_thin, dim3((unsigned)blocks, (unsigned)pv), dim3(64), 0, s, q);
+        hipLaunchKernelGGL(k_conv_fwd_thin, dim3((unsigned)blocks, (unsigned)pv), dim3(64), 0, s, q, positions);
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
     // Two accumulator rows per lane halve the weight traffic per instruction.  Outputs with

@@ -415,11 +415,11 @@ def test_long_kernels_use_the_row_chunked_weight_generator(capi, so, sx, sw, pad
     ((128, 5, 32, 32), (49, 5, 1, 1), (0, 0), 128, (7, 8, 1, 1), "lfsr"),   # 1 x 1
     ((128, 4, 32, 32), (65, 4, 3, 2), (1, 0), 8, (7, 8, 1, 1), "lfsr"),     # L = 8, even kernel extent in dim 3
     ((128, 3, 32, 32), (50, 3, 3, 3), (1, 1), 64, (7, 8, 1, 1), "acc"),     # random generators: same kernel
-    # 3-wide kernels with c_in % 8 == 0 and 4 or 8 c_out tiles: activation words staged through LDS
-    ((128, 8, 33, 32), (50, 8, 3, 3), (1, 1), 32, (7, 8, 1, 1), "lfsr"),    # four c_out tiles (one position tile per workgroup), odd row count, partial c_out tile
-    ((73, 16, 30, 31), (113, 16, 3, 3), (1, 1), 64, (7, 2, 2, 2), "lfsr"),  # eight c_out tiles, two packs, 531 position tiles (not a multiple of the four per workgroup), the last one ragged
+    # whole chunks of 8 channels
+    ((128, 8, 33, 32), (50, 8, 3, 3), (1, 1), 32, (7, 8, 1, 1), "lfsr"),    # four c_out tiles, odd row count, partial c_out tile
+    ((73, 16, 30, 31), (113, 16, 3, 3), (1, 1), 64, (7, 2, 2, 2), "lfsr"),  # eight c_out tiles, two packs, 531 position tiles, the last one ragged
     ((128, 8, 32, 32), (128, 8, 3, 2), (1, 0), 128, (7, 8, 1, 1), "lfsr"),  # two kernel rows, four packs
-    ((144, 24, 32, 32), (64, 24, 3, 1), (0, 0), 16, (7, 8, 1, 1), "acc"),   # three chunks of channels per pass
+    ((144, 24, 32, 32), (64, 24, 3, 1), (0, 0), 16, (7, 8, 1, 1), "acc"),   # one kernel row
 ])
 def test_large_y_mode_launches_skip_the_zero_rail(capi, so, shape_x, shape_w, pad, L, loading, gen):
     """Launches of at least 4096 waves in y mode run the kernel that processes only the non-zero rail of
@@ -455,7 +455,7 @@ def test_large_y_mode_launches_skip_the_zero_rail(capi, so, shape_x, shape_w, pa
 
 # ------------------------------------------------------------------ launches split over (pack, kernel row) pairs
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,loading", [
-    ((256, 32, 8, 8), (64, 32, 5, 5), (2, 2), 64, (7, 2, 2, 2)),     # 5120 waves, one pair each: the pairs of a tile in one workgroup
+    ((256, 32, 8, 8), (64, 32, 5, 5), (2, 2), 64, (7, 2, 2, 2)),     # 512 tiles: the pairs of a tile in one workgroup, an OR shared out over four waves
     ((250, 32, 8, 8), (60, 32, 5, 5), (2, 2), 64, (7, 8, 1, 1)),     # the same with a ragged last tile and a partial c_out tile
     ((256, 32, 16, 16), (32, 32, 5, 5), (2, 2), 64, (7, 2, 2, 2)),   # 10240 waves: two rounds, one pair per wave with atomics
     ((200, 16, 8, 9), (48, 16, 3, 3), (1, 1), 256, (7, 8, 1, 1)),    # 24 pairs: more than a workgroup takes
@@ -476,6 +476,39 @@ def test_split_launches_match_oracle(capi, so, shape_x, shape_w, pad, L, loading
         capi.conv2d_add_partial_from_streams(act, wgt, d, out=y)
         assert np.array_equal(y.cpu().numpy(), exp)
     assert np.array_equal(capi.conv2d_add_partial_forward(x.cuda(), w.cuda(), L, pad, tw, lw, ww, wa).cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("shape_x,shape_w,pad,L,mode,zu", [
+    ((2, 70, 5, 6), (20, 70, 3, 3), (1, 1), 32, "y", 1),       # an OR shared out over 16 waves, the last two without a channel
+    ((2, 37, 6, 7), (17, 37, 3, 3), (1, 1), 64, "y", 1),       # over 8, the last share short
+    ((1, 64, 2, 2), (16, 64, 5, 5), (2, 2), 256, "y", 1),      # two lane slots
+    ((8, 130, 7, 9), (33, 130, 1, 1), (0, 0), 128, "y", 1),    # 1-wide, shares of an odd number of channels
+    ((40, 20, 16, 16), (40, 20, 3, 3), (1, 1), 128, "y", 1),   # over 4, one pair per workgroup
+    ((128, 33, 16, 16), (33, 33, 3, 3), (1, 1), 32, "y", 1),   # three pairs of a tile two at a time in one workgroup
+    ((4, 20, 9, 8), (18, 20, 3, 3), (1, 1), 64, "full", 1),    # OR over kernel rows as well
+    ((3, 5, 9, 9), (20, 5, 3, 3), (1, 1), 128, "y", 1),        # short groups: 12 pairs in 16 waves
+    ((33, 3, 31, 32), (32, 3, 3, 3), (1, 1), 64, "y", 1),      # 6 pairs in 8 waves
+    ((40, 4, 16, 16), (33, 4, 5, 5), (2, 2), 128, "y", 1),     # 20 pairs, 8 waves, three rounds of them
+    ((16, 60, 12, 12), (40, 60, 3, 3), (1, 1), 128, "z", 1),   # 240 groups of nine lines
+    ((60, 45, 13, 15), (83, 45, 3, 3), (1, 1), 64, "yz", 32),  # ragged last channel block
+    ((100, 256, 8, 8), (256, 256, 1, 1), (0, 0), 32, "z", 1),  # 204800 one-line groups
+    ((5, 64, 4, 5), (10, 64, 4, 4), (0, 0), 64, "y", 1),       # lanes over the members, an even number of positions
+    ((3, 80, 1, 1), (18, 80, 1, 1), (0, 0), 128, "y", 1),      # and an odd one
+])
+def test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode, zu):
+    """Every way the position-parallel launches cut their (pack, add group) pairs and OR groups over waves,
+    at the edges of the rule that chooses it: bit for bit, twice (the second call finds counts in y)."""
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=shape_w[0] + L)
+    w.view(-1)[::7] = 0.0
+    gen = "rand" if mode == "full" else "lfsr"
+    exp = (so.conv2d_general(x.numpy(), w.numpy(), L, pad, mode, 1, gen, 3) if mode == "full" else
+           so.conv2d_modes(x.numpy(), w.numpy(), L, pad, mode, zu))
+    d = capi.make_desc(x.shape, w.shape, L, pad, accumulate=mode, z_unit=zu, generator=gen, seed=3)
+    y = torch.full(capi.output_shape(d), 12345, dtype=torch.int32, device="cuda")
+    act, wgt = capi.act_streams(x.cuda(), d), capi.weight_streams(w.cuda(), d)
+    for _ in range(2):
+        capi.conv2d_add_partial_from_streams(act, wgt, d, out=y)
+        assert np.array_equal(y.cpu().numpy(), exp)
 
 
 # ------------------------------------------------------------------ batches cut into chunks
