@@ -285,6 +285,25 @@ def bn_fixed_from_counts(counts, bit_length, gamma, beta, eps, running_mean=None
     return mean, var, w_n, b_n, invstd, scale
 
 
+BN_EVAL_CHANNELS = 4096
+
+
+def bn_fixed_eval(x, mean, var, gamma, beta, eps, stream=None):
+    """geo_sc_bn_fixed_eval: (y, scale) of a fixed-point batch norm on given statistics; ``x``: contiguous fp32 GPU
+    tensor (n, c, ...), the rest contiguous fp32 of c entries on the same GPU (gamma / beta may be None)."""
+    n, c = x.shape[:2]
+    for t in (x, mean, var, gamma, beta):
+        if t is not None and not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == x.device
+                                  and (t is x or t.numel() == c)):
+            raise ValueError("x, statistics and parameters must be contiguous float32 tensors on one GPU")
+    y = torch.empty_like(x)
+    scale = torch.empty((), dtype=torch.float32, device=x.device)
+    _check(_native.lib().geo_sc_bn_fixed_eval(_ptr(x), n, c, x.numel() // (n * c), _ptr(mean), _ptr(var), _ptr(gamma),
+                                              _ptr(beta), float(eps), _ptr(y), _ptr(scale), _stream_ptr(stream)),
+           "geo_sc_bn_fixed_eval")
+    return y, scale
+
+
 def quantize_many(tensors, prec, stream=None):
     """geo_sc_quantize_many: quantize() of every tensor of the list (contiguous fp32 GPU tensors) in one launch;
     returns the new tensors."""

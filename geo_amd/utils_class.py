@@ -4,6 +4,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import utils_functional
 
@@ -42,6 +43,31 @@ def _fixed_affine(module, x, mean, var):
     return w_n, b_n
 
 
+def _fixed_eval(module, x, dims):
+    """The value of ``BatchNorm*_fixed`` in eval mode as one kernel, or None where the chain of operations has to run:
+    whenever something besides the value is asked for (gradients, forward-mode tangents, function transforms,
+    tracing), and for layouts, types and devices that the kernel does not take."""
+    if module.training or torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dim() != dims:
+        return None
+    if not (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and 0 < x.numel() < 2 ** 31
+            and x.shape[1] == module.num_features):
+        return None
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 \
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0:
+        return None
+    from . import capi
+    mean, var = module.running_mean, module.running_var
+    gamma, beta = (module.weight, module.bias) if module.affine else (None, None)
+    if mean is None or var is None or module.num_features > capi.BN_EVAL_CHANNELS \
+            or x.device.index != torch.cuda.current_device():
+        return None
+    for t in (mean, var, gamma, beta):
+        if t is not None and not (t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()):
+            return None
+    y, module.scale = capi.bn_fixed_eval(x, mean, var, gamma, beta, module.eps)
+    return y
+
+
 class BatchNorm2d_fixed(nn.BatchNorm2d):
     """2-d batch norm whose value is the fixed-point affine; gradients are those of the
     ordinary batch norm (utils_class.py:37-65)."""
@@ -51,6 +77,9 @@ class BatchNorm2d_fixed(nn.BatchNorm2d):
         self.register_buffer("scale", None)
 
     def forward(self, x):
+        out = _fixed_eval(self, x, 4)
+        if out is not None:
+            return out
         out = F.batch_norm(x, self.running_mean, self.running_var, self.weight, self.bias, training=self.training)
         if self.training:
             mean, var = x.mean(dim=(0, 2, 3)), x.var(dim=(0, 2, 3), unbiased=False)
@@ -69,6 +98,9 @@ class BatchNorm1d_fixed(nn.BatchNorm1d):
         self.register_buffer("scale", None)
 
     def forward(self, x):
+        out = _fixed_eval(self, x, 2)
+        if out is not None:
+            return out
         out = F.batch_norm(x, self.running_mean, self.running_var, self.weight, self.bias, training=self.training)
         if self.training:
             mean, var = x.mean(dim=0), x.var(dim=0, unbiased=False)

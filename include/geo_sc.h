@@ -377,6 +377,16 @@ GEO_SC_API int geo_sc_bn_fixed_from_counts(const int32_t* counts, int n, int c, 
                                            size_t workspace_bytes, geo_sc_stream_t stream);
 
 /*
+ * BatchNorm2d_fixed / BatchNorm1d_fixed on given statistics, for inference, in one launch (utils_class.py:49-64):
+ * y = x * w_n + b_n with w_n, b_n as geo_sc_bn_fixed_affine forms them from mean and var (c floats each); gamma /
+ * beta may be NULL (1 / 0).  x, y: (n, c, plane) contiguous floats, y may be x; scale receives one float; c at
+ * most 4096 and fewer than 2^31 elements (GEO_SC_ERR_UNSUPPORTED otherwise).
+ */
+GEO_SC_API int geo_sc_bn_fixed_eval(const float* x, int n, int c, int plane, const float* mean, const float* var,
+                                    const float* gamma, const float* beta, float eps, float* y, float* scale,
+                                    geo_sc_stream_t stream);
+
+/*
  * quantize (utils_functional.py:33-39) in one pass: dst = clamp(round(src * 2^prec), -(2^prec - 1), 2^prec - 1)
  * / 2^prec, rounding half to even as torch.round does; prec 1..23.  The layer applies it to its input
  * and to weight_org on every call (utils_class.py:32-33).  n fp32 elements on the device; dst may be src.

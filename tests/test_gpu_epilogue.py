@@ -171,6 +171,46 @@ def test_bn_fixed_affine_matches_torch_ops(capi, c, affine):
     assert torch.allclose(rm, exp_rm, rtol=1e-6, atol=1e-7) and torch.allclose(rv, exp_rv, rtol=1e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("shape,affine,spoil", [
+    ((256, 32, 32, 32), True, None), ((3, 10), True, None), ((1, 1, 1, 1), True, None), ((5, 7, 3, 5), False, None),
+    ((2, 700, 2, 2), True, None), ((1, 4097, 2, 2), True, None), ((50, 300), False, None),
+    ((4, 6, 4, 4), True, "nan"), ((4, 6, 4, 4), True, "inf"), ((4, 6, 4, 4), True, "negative"), ((4, 6, 4, 4), True, "zero")])
+def test_fixed_batch_norm_in_eval_mode_equals_the_op_chain(shape, affine, spoil):
+    """BatchNorm*_fixed without gradients (one kernel) against the same module with gradients enabled (the chain of
+    operations): value and ``scale`` bit for bit, NaN for NaN."""
+    from geo_amd import utils_class
+    g = torch.Generator().manual_seed(shape[1])
+    c = shape[1]
+    bn = (utils_class.BatchNorm2d_fixed if len(shape) == 4 else utils_class.BatchNorm1d_fixed)(c, affine=affine).cuda().eval()
+    with torch.no_grad():
+        bn.running_mean.copy_(torch.rand(c, generator=g) - 0.3)
+        bn.running_var.copy_(torch.rand(c, generator=g) * 0.5 + 0.01)
+        if affine:
+            bn.weight.copy_(torch.rand(c, generator=g) + 0.5)
+            bn.bias.copy_(torch.rand(c, generator=g) - 0.5)
+        x = torch.rand(shape, generator=g).cuda() * 2 - 1
+        if spoil == "nan":
+            bn.running_mean[1] = float("nan")
+            x.view(-1)[5] = float("nan")
+        elif spoil == "inf":
+            bn.running_mean[1] = float("inf")
+            x.view(-1)[5] = float("inf")
+        elif spoil == "negative":   # the logarithm of a negative mean
+            bn.weight.neg_()
+        elif spoil == "zero":       # scale 0
+            bn.weight.zero_()
+    with torch.enable_grad():
+        exp, exp_scale = bn(x.clone()).detach(), bn.scale.clone()
+    with torch.no_grad():
+        got = bn(x.clone())
+    eq = lambda a, b: torch.equal(torch.nan_to_num(a, 123.0, 1e30, -1e30), torch.nan_to_num(b, 123.0, 1e30, -1e30))
+    assert got.shape == exp.shape and eq(got, exp) and eq(bn.scale, exp_scale) and bn.scale.shape == exp_scale.shape
+    with torch.no_grad():           # strides and sizes the kernel does not take
+        if len(shape) == 4:
+            assert eq(bn(x.contiguous(memory_format=torch.channels_last)), exp)
+        assert bn(x[:0]).shape == x[:0].shape
+
+
 def test_quantize_kernel_equals_the_torch_op_chain():
     """geo_sc_quantize against (x * 2^p).round().clamp(+-(2^p - 1)) / 2^p (utils_functional.py:33-39):
     bit for bit, including ties (half to even), the clamp ends, zeros' signs aside, and NaN."""
