@@ -1425,7 +1425,8 @@ RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
     // once four waves per SIMD exist without splitting a tile (3 -> 32, 5 x 5, 32 x 32, batch 256, L 64: 64 us
     // against 72), or with so many groups per tile that the tile kernel's per-group work shows (z mode, 3 x 3, 1320
     // groups of 309 tiles: 395 against 439 us; 1220 groups of 116 tiles: 146 against 162).
-    if (g.mode == GEO_SC_ACC_Y && tiles >= 4096 && lines <= 24) return {kRailPlain, 0, 0, 0, 1};
+    if (g.mode == GEO_SC_ACC_Y && tiles >= 4096 && lines <= 24)
+        return {sp.splits == 1 ? kRailPlain : kRailSplit, 0, 0, 0, sp.splits};
     if (lines <= 12 && pairs >= 100000) return {kRailSplit, 0, 0, 0, sp.splits};
     // Long groups, few of them per tile, in launches whose waves fill their rounds: the counts of a pair go
     // straight to y (64 -> 64, 3 x 3, 32 x 32, batch 128, L 64: 327 us against 336).  With twelve pairs per tile, or
