@@ -17,8 +17,10 @@
 //     dcol[k][m] = sum_j Wd[j][k]  * E[m][j]           Wd = (wp ; -wn)
 // All three run on MFMA kernels (fp32 in, fp32 accumulate, fp32 out) that take each operand either
 // K-major or I-major: k_gemm_split forms every fp32 product from six bf16 MFMA products of a three-way
-// split of the operands (aligned operands; k_gemm_big is the same product with eight waves on tiles of
-// up to 256 x 256 for the large results), k_gemm_f32 uses v_mfma_f32_32x32x2_f32 (any alignment);
+// split of the operands; k_gemm_big is the same product with eight waves on tiles of up to 256 x 256 for
+// the large results.  Rows of col and E are padded to 16 bytes so that sizes that are no multiples of four take
+// these kernels too (77 items of 45 x 27 x 19 -> 83 channels, z_unit 32: weight gradient 216 us on
+// fp32 MFMAs with element-wise loads, 97 here; input gradient 136, 83);
 // exp and the product with g are fused into the first GEMM's epilogue; the second is split over m
 // and reduced deterministically.
 //
@@ -52,7 +54,6 @@ __device__ __forceinline__ float exp_neg(float z) { return __expf(-z); }
 
 constexpr int kTile = 128;   // block tile in I and J
 constexpr int kChunk = 16;   // K per LDS stage
-constexpr int kLd = 132;     // LDS row stride in floats: rows stay 16-byte aligned for float4 stores
 
 enum Epilogue { EPI_STORE = 0, EPI_EXP_TIMES_G = 1, EPI_EXP_TIMES_G_PLANES = 2, EPI_STORE_ITEMS = 3 };
 
@@ -136,63 +137,6 @@ __device__ __forceinline__ void gemm_tile_of(const GemmParams& q, int w, int& it
     }
 }
 
-// Staging of one kChunk x kTile operand tile for the fp32 kernel, split in two so that the global
-// loads of chunk c+1 are in flight while the MFMAs of chunk c run: fetch() reads 8 elements per
-// thread into registers, commit() writes them to LDS as s[k][i].
-//   K-major operand: element (k, i) at p[k*ld + i]
-//   I-major operand: element (k, i) at p[i*ld + k]
-// Guarded scalar loads for operands of any alignment and extent (lanes outside the operand read a valid
-// dummy address and are zeroed by a select, no divergent branches); aligned operands take k_gemm_split.
-template <bool KMAJOR>
-struct Stager {
-    const float* p;      // this thread's first element of the current chunk
-    const float* dummy;  // any valid address of the operand
-    long long ld;
-    int kk0, ii;         // first k (inside the chunk) and first i (inside the tile) of this thread
-    bool i_ok;
-    unsigned ok;         // bit c: element c of the last fetch lies inside the operand
-
-    // element c (0..7) of this thread sits at (k, i) = (kk0 + kdelta(c), ii)
-    static __device__ __forceinline__ int kdelta(int c) { return KMAJOR ? c * 2 : c; }
-
-    __device__ __forceinline__ void init(const float* base, long long ld_, int i0, int k_begin, int I)
-    {
-        const int t = threadIdx.x;
-        ld = ld_;
-        dummy = base;
-        if (KMAJOR) {
-            kk0 = t >> 7;  // rows kk0, kk0 + 2, ..., kk0 + 14, one i
-            ii = t & 127;
-            p = base + (long long)(k_begin + kk0) * ld + i0 + ii;
-        } else {
-            ii = t >> 1;
-            kk0 = (t & 1) * 8;  // eight consecutive k of one i
-            p = base + (long long)(i0 + ii) * ld + k_begin + kk0;
-        }
-        i_ok = i0 + ii < I;
-    }
-    // k_left = k_end - k0 of the chunk being fetched.  Only the loads are issued here; lanes outside
-    // the operand are zeroed in commit(), after the MFMAs of the chunk in flight, so that nothing
-    // waits for the loads before those MFMAs.
-    __device__ __forceinline__ void fetch(float (&r)[8], int k_left)
-    {
-        ok = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const bool okc = i_ok && kk0 + kdelta(c) < k_left;
-            const float* qq = okc ? p + (KMAJOR ? (long long)kdelta(c) * ld : (long long)c) : dummy;
-            r[c] = *qq;
-            ok |= okc ? 1u << c : 0u;
-        }
-        p += KMAJOR ? (long long)kChunk * ld : (long long)kChunk;
-    }
-    __device__ __forceinline__ void commit(float (*s)[kLd], float (&r)[8]) const
-    {
-#pragma unroll
-        for (int c = 0; c < 8; c++) s[kk0 + kdelta(c)][ii] = (ok >> c & 1u) ? r[c] : 0.0f;
-    }
-};
-
 // Epilogue of one wave: accumulator register r of lane l holds C[8*(r/4) + 4*(l/32) + r%4][l%32] of a
 // 32 x 32 block; (iw, jw) is the wave's corner in the result.  No branches around the loads of the
 // upstream gradient: they go out 16 at a time from clamped addresses, then the exponentials, then
@@ -273,109 +217,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& q, const floatx16 (
     }
 }
 
-// The K loop and the epilogue of one wave that owns the first NX x NY of its 2 x 2 blocks of
-// 32 x 32 (edge tiles and narrow operands leave blocks without results; NX = 0: none, the wave only
-// stages).  A function of its own per (NX, NY), entered through a wave-uniform switch: the
-// accumulators then live in one variant from zeroing to store and every MFMA is unconditional.
-// Conditions on single blocks inside one loop make the compiler copy all accumulators between
-// register classes on every trip.
-// v_mfma_f32_32x32x2_f32: lane l feeds A[i = l%32][k = l/32] and B[k = l/32][j = l%32].
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int NX, int NY>
-__device__ __forceinline__ void gemm_wave(const GemmParams& q, float (*as)[kChunk][kLd], float (*bs)[kChunk][kLd], int i0,
-                                          int j0, int batch, int split, int k_begin, int k_end, int wi, int wj, int l32,
-                                          int lk)
-{
-    floatx16 acc[NX ? NX : 1][NY ? NY : 1];
-#pragma unroll
-    for (int x = 0; x < NX; x++)
-#pragma unroll
-        for (int y = 0; y < NY; y++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[x][y][r] = 0.0f;
-
-    Stager<A_KMAJOR> sa;
-    Stager<B_KMAJOR> sb;
-    sa.init(q.a + batch * q.a_batch_stride, q.lda, i0, k_begin, min(q.I, i0 + q.tile_i));
-    sb.init(q.b + batch * q.b_batch_stride, q.ldb, j0, k_begin, min(q.J, j0 + q.tile_j));
-    float ra[8], rb[8];
-    if (k_begin < k_end) {
-        sa.fetch(ra, k_end - k_begin);
-        sb.fetch(rb, k_end - k_begin);
-        sa.commit(as[0], ra);
-        sb.commit(bs[0], rb);
-    }
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = k_begin; k0 < k_end; k0 += kChunk) {
-        const bool more = k0 + kChunk < k_end;
-        if (more) {
-            sa.fetch(ra, k_end - k0 - kChunk);
-            sb.fetch(rb, k_end - k0 - kChunk);
-        }
-#pragma unroll
-        for (int kk = 0; kk < kChunk; kk += 2) {
-            float a[NX ? NX : 1], b[NY ? NY : 1];
-#pragma unroll
-            for (int x = 0; x < NX; x++) a[x] = as[buf][kk + lk][wi + 32 * x + l32];
-#pragma unroll
-            for (int y = 0; y < NY; y++) b[y] = bs[buf][kk + lk][wj + 32 * y + l32];
-#pragma unroll
-            for (int x = 0; x < NX; x++)
-#pragma unroll
-                for (int y = 0; y < NY; y++)
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x], b[y], acc[x][y], 0, 0, 0);
-        }
-        if (more) {
-            // the other buffer was last read one trip ago, before that trip's barrier
-            sa.commit(as[buf ^ 1], ra);
-            sb.commit(bs[buf ^ 1], rb);
-        }
-        __syncthreads();
-        buf ^= 1;
-    }
-
-    store_tile<EPI, NX, NY>(q, acc, q.c + batch * q.c_batch_stride + split * q.c_split_stride, i0 + wi, j0 + wj, l32, lk);
-}
-
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI>
-// four waves per SIMD (at most 128 registers: four workgroups per CU)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gemm_f32(GemmParams q)
-{
-    __shared__ __attribute__((aligned(16))) float as[2][kChunk][kLd];
-    __shared__ __attribute__((aligned(16))) float bs[2][kChunk][kLd];
-    int it, jt, z;
-    gemm_tile_of(q, blockIdx.x, it, jt, z);
-    const int i0 = it * q.tile_i, j0 = jt * q.tile_j;
-    const int batch = z / q.splits, split = z - batch * q.splits;
-    const int k_begin = split * q.k_per_split;
-    const int k_end = min(q.K, k_begin + q.k_per_split);
-    // the wave index through readfirstlane: the compiler then knows that everything derived from it
-    // (tile corner, block choice) is uniform and branches on it with scalar instructions
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    // this wave's corner in the tile: 2 x 2 waves of 64 x 64; with a tile of 64 in one dimension
-    // (results that are narrow there) the four waves line up along the other, 32 x 64 (or 64 x 32) each
-    const bool narrow_j = q.tile_j < kTile, narrow_i = q.tile_i < kTile;
-    const int wi = narrow_j ? wave * 32 : narrow_i ? 0 : (wave >> 1) * 64;
-    const int wj = narrow_j ? 0 : narrow_i ? wave * 32 : (wave & 1) * 64;
-    const int l32 = lane & 31, lk = lane >> 5;
-    // which of this wave's (up to) four 32 x 32 blocks lie inside the result
-    const bool x0 = i0 + wi < q.I, x1 = !narrow_j && i0 + wi + 32 < q.I;
-    const bool y0 = j0 + wj < q.J, y1 = !narrow_i && j0 + wj + 32 < q.J;
-    const int blocks_xy = (x0 && y0) ? 2 * (int)x1 + (int)y1 : -1;
-#define GEO_SC_GEMM_WAVE(NX, NY)                                                                                        \
-    gemm_wave<A_KMAJOR, B_KMAJOR, EPI, NX, NY>(q, as, bs, i0, j0, batch, split, k_begin, k_end, wi, wj, l32, lk)
-    // every variant runs the same staging and the same number of barriers
-    switch (blocks_xy) {
-    case 3: GEO_SC_GEMM_WAVE(2, 2); break;
-    case 2: GEO_SC_GEMM_WAVE(2, 1); break;
-    case 1: GEO_SC_GEMM_WAVE(1, 2); break;
-    case 0: GEO_SC_GEMM_WAVE(1, 1); break;
-    default: GEO_SC_GEMM_WAVE(0, 0); break;
-    }
-#undef GEO_SC_GEMM_WAVE
-}
-
-// ---- the same GEMM on the bf16 matrix cores, fp32 results ----
+// ---- the GEMM: fp32 operands and results on the bf16 matrix cores ----
 // Every fp32 operand element is split into three bf16 terms (x = hi + mid + lo to 2^-27 |x|: each
 // term is the round-to-nearest bf16 of what the previous ones leave) and a product is formed from
 // the six term products of relative size >= 2^-18 (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi),
@@ -1238,12 +1080,12 @@ __host__ __device__ inline void group_of(const Groups& G, int ci, int u, int v, 
 // col[g][k][m] = x~[n, ci, a+u, b+v] for groups g0 + blockIdx.z, (ci, u, v) = member k of the
 // group, m = (n, a, b); x~ is the zero-padded activation, read straight from the unpadded
 // tensor.  blockIdx.y selects kIm2colMembers consecutive members; a thread reads its position's
-// table entry once and moves those members.  Reads and writes run along m.
+// table entry once and moves those members.  Reads and writes run along m; rows are ld elements apart.
 constexpr int kIm2colMembers = 12;
 __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x, float* __restrict__ col,
                                                      const int* __restrict__ base, const int* __restrict__ arow,
-                                                     const int* __restrict__ bcol, int g0, int m_total, Groups G,
-                                                     int w_in, int h_in, size_t g_stride)
+                                                     const int* __restrict__ bcol, int g0, int m_total, int ld,
+                                                     Groups G, int w_in, int h_in, size_t g_stride)
 {
     const int g = g0 + blockIdx.z;
     const int k0 = blockIdx.y * kIm2colMembers;
@@ -1265,7 +1107,7 @@ __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x
         }
 #pragma unroll
         for (int q = 0; q < kIm2colMembers; q++)
-            if (k0 + q < k1) colg[(size_t)(k0 + q) * m_total + m] = vals[q];
+            if (k0 + q < k1) colg[(size_t)(k0 + q) * ld + m] = vals[q];
     }
 }
 
@@ -2467,13 +2309,10 @@ int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
         } else {
             hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, true>), grid, dim3(256), 0, s, q);
         }
-    } else if constexpr (AK && BK) {
-        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI>), grid, dim3(256), 0, s, q);
     } else {
-        if (a_vec && b_vec)
-            hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI>), grid, dim3(256), 0, s, q);
-        else
-            hipLaunchKernelGGL((k_gemm_f32<AK, BK, EPI>), grid, dim3(256), 0, s, q);
+        // (the scratch layout aligns the rows)
+        if (!a_vec || !b_vec) return GEO_SC_ERR_UNSUPPORTED;
+        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI>), grid, dim3(256), 0, s, q);
     }
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
@@ -2508,6 +2347,8 @@ size_t view_floats(const Geometry& g)
 {
     return (size_t)g.h_k * g.c_in * g.n * (g.w_in + 2 * g.pad_w) * g.ho + (size_t)g.w_k * g.ho;
 }
+
+inline long long pad4(long long v) { return (v + 3) & ~3LL; }
 
 BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
 {
@@ -2563,8 +2404,9 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     b.splits = (int)((b.m_total + b.m_per_split - 1) / b.m_per_split);
     // per-row scratch, each row's part padded to 64 floats so that float4 staging stays aligned
     auto pad64 = [](size_t v) { return (v + 63) & ~(size_t)63; };
-    b.col_v = pad64((size_t)b.m_total * K);
-    b.e_v = pad64((size_t)b.m_total * 2 * g.c_out);
+    // (rows of col and of E start on 16-byte boundaries: the products that read them along a row do so four at a time)
+    b.col_v = pad64((size_t)pad4(b.m_total) * K);
+    b.e_v = pad64((size_t)b.m_total * pad4(2 * g.c_out));
     b.part_v = pad64((size_t)(b.fused_k && b.fused_splits > b.splits ? b.fused_splits : b.splits) * K * 2 * g.c_out);
     b.w_v = pad64((size_t)K * 2 * g.c_out);
     // the fused kernel needs neither col nor E
@@ -2651,6 +2493,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
     float* wd = (float*)(ws + L.off_wd);
     const Groups& G = L.G;
     const int M = (int)L.m_total, K = G.n_members, J = 2 * g.c_out;
+    const int col_ld = (int)pad4(M), e_ld = (int)pad4(J);  // row strides of col and E
     const long long x_total = (long long)g.n * g.c_in * g.w_in * g.h_in;
     if (x_total > 0x7fffffffLL || K > 65535 * kIm2colMembers) return GEO_SC_ERR_UNSUPPORTED;
     if ((long long)g.n * g.c_out * g.wo * g.ho > 0x7fffffffLL) return GEO_SC_ERR_UNSUPPORTED;
@@ -2792,7 +2635,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         } else {
             hipLaunchKernelGGL(k_im2col_rows,
                                dim3(m_blocks > 1024 ? 1024 : m_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
-                               dim3(256), 0, s, x, col, pos_base, pos_arow, pos_bcol, v0, M, G, g.w_in, g.h_in, L.col_v);
+                               dim3(256), 0, s, x, col, pos_base, pos_arow, pos_bcol, v0, M, col_ld, G, g.w_in, g.h_in, L.col_v);
         }
         const bool dx_taps = gx && L.dx_taps;
         const bool dx_rows = dx_taps || (gx && L.dx_rows && ((uintptr_t)gx & 15) == 0);
@@ -2816,7 +2659,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         GemmParams q1 = {};
         q1.a = col; q1.b = wcat; q1.c = e;
         q1.I = M; q1.J = J; q1.K = K;
-        q1.lda = M; q1.ldb = J; q1.ldc = J;
+        q1.lda = col_ld; q1.ldb = J; q1.ldc = e_ld;
         q1.splits = 1; q1.k_per_split = K; q1.c_split_stride = 0;
         q1.a_batch_stride = (long long)L.col_v; q1.b_batch_stride = (long long)L.w_v;
         q1.c_batch_stride = (long long)L.e_v;
@@ -2830,7 +2673,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             GemmParams q2 = {};
             q2.a = col; q2.b = e; q2.c = part;
             q2.I = K; q2.J = J; q2.K = M;
-            q2.lda = M; q2.ldb = J; q2.ldc = J;
+            q2.lda = col_ld; q2.ldb = e_ld; q2.ldc = J;
             q2.splits = L.splits; q2.k_per_split = L.m_per_split; q2.c_split_stride = (long long)K * J;
             q2.a_batch_stride = (long long)L.col_v; q2.b_batch_stride = (long long)L.e_v;
             q2.c_batch_stride = (long long)L.part_v;
@@ -2851,7 +2694,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             GemmParams q3 = {};
             q3.a = wd; q3.b = e; q3.c = gx;
             q3.I = g.c_in; q3.J = (int)m2; q3.K = k9;
-            q3.lda = g.c_in; q3.ldb = J; q3.ldc = m2;
+            q3.lda = g.c_in; q3.ldb = e_ld; q3.ldc = m2;
             q3.splits = 1; q3.k_per_split = k9; q3.c_split_stride = 0;
             q3.a_batch_stride = 0; q3.b_batch_stride = (long long)L.e_v; q3.c_batch_stride = 0;
             q3.sh_zero = zero; q3.sh_j = J; q3.sh_wo = g.wo; q3.sh_ho = g.ho; q3.sh_win = g.w_in; q3.sh_hin = g.h_in;
@@ -2871,7 +2714,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             GemmParams q3 = {};
             q3.a = wd; q3.b = e; q3.c = dcol;
             q3.I = g.c_in; q3.J = (int)m2; q3.K = k3;
-            q3.lda = g.c_in; q3.ldb = J; q3.ldc = m2;
+            q3.lda = g.c_in; q3.ldb = e_ld; q3.ldc = m2;
             q3.splits = 1; q3.k_per_split = k3; q3.c_split_stride = 0;
             q3.a_batch_stride = (long long)L.w_v; q3.b_batch_stride = (long long)L.e_v;
             q3.c_batch_stride = (long long)g.c_in * m2;
@@ -2887,8 +2730,8 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         GemmParams q3 = {};
         q3.a = wd; q3.b = e; q3.c = dcol;
         q3.I = K; q3.J = M; q3.K = J;
-        q3.lda = K; q3.ldb = J; q3.ldc = M;
-        q3.splits = 1; q3.k_per_split = J; q3.c_split_stride = 0;
+        q3.lda = K; q3.ldb = e_ld; q3.ldc = M;
+        q3.splits = 1; q3.k_per_split = e_ld; q3.c_split_stride = 0;
         q3.a_batch_stride = (long long)L.w_v; q3.b_batch_stride = (long long)L.e_v;
         q3.c_batch_stride = (long long)L.col_v;
         if ((rc = launch_gemm<true, false, EPI_STORE>(q3, nv, s)) != GEO_SC_OK) return rc;
