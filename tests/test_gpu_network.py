@@ -194,6 +194,35 @@ def test_tail_backward_matches_torch_autograd():
             assert err < 2e-5, (shape, err)
 
 
+@pytest.mark.parametrize("shape,pool", [((3, 1, 16, 16), False), ((9, 300, 9, 7), False), ((130, 512, 2, 2), False),
+                                        ((40, 513, 6, 6), True), ((17, 129, 16, 2), False), ((2, 2048, 1, 1), False),
+                                        ((70, 33, 16, 16), True)])
+def test_tail_backward_sums_of_any_number_of_channels(shape, pool):
+    """One to 32 partial sums per channel, channels that are no multiple of what a workgroup adds at a time: without
+    masks the gradient is linear, its sums in float64 are the oracle.  fp32 sums of at most 2^14 random terms stay
+    within 2^-24 * 2^7 of the result's scale."""
+    from geo_amd import capi
+    n, c, w, h = shape
+    g = torch.Generator().manual_seed(c)
+    counts = torch.randint(-64, 65, shape, generator=g, dtype=torch.int32)
+    go = torch.randn((n, c, w // 2, h // 2) if pool else shape, generator=g)
+    mean, invstd, gamma = torch.randn(c, generator=g), torch.rand(c, generator=g) + 0.5, torch.rand(c, generator=g) + 0.5
+    one, zero = torch.ones(c), torch.zeros(c)
+    gy, gg, gb = capi.layer_tail_backward(counts.cuda(), go.cuda(), 64, one.cuda(), zero.cuda(), mean.cuda(), invstd.cuda(),
+                                          gamma.cuda(), False, pool, False)
+    per = lambda t: t.double().view(1, c, 1, 1)
+    d = go.double()
+    if pool:
+        d = d.repeat_interleave(2, 2).repeat_interleave(2, 3) / 4
+    xhat = (counts.double() / 64 - per(mean)) * per(invstd)
+    rb, rg = d.sum((0, 2, 3)), (d * xhat).sum((0, 2, 3))
+    m = n * w * h
+    ry = per(gamma) * per(invstd) * (d - per(rb) / m - xhat * per(rg) / m)
+    for got, ref in ((gy, ry), (gg, rg), (gb, rb)):
+        assert got.shape == ref.shape
+        assert (got.cpu().double() - ref).abs().max() <= 2.0 ** -17 * ref.abs().max()
+
+
 def test_count_stats_are_the_correctly_rounded_channel_statistics():
     """geo_sc_count_stats against float64 mean and biased variance of counts / L (utils_class.py:52-56):
     equal to the float64 result rounded to fp32, for whole-quad planes, ragged planes, an unaligned
