@@ -470,3 +470,27 @@ def test_backward_small_groups_at_the_headline_shape(capi, mode, zu):
     check(f"{mode} z_unit {zu} (batch 64) grad_w", gw, rw)
     gx2, gw2 = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), accumulate=mode, z_unit=zu)
     assert torch.equal(gx2, gx) and torch.equal(gw2, gw)   # deterministic
+
+
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((8, 64, 8, 8), (128, 64, 3, 3), 1, "y", 1),      # a product per kernel column with few tiles
+    ((16, 512, 4, 4), (520, 512, 3, 3), 1, "y", 1),   # ragged channel tile; one partial dL/dw
+    ((128, 512, 4, 4), (512, 512, 3, 3), 1, "y", 1),  # three partial dL/dw
+    ((9, 40, 7, 8), (72, 40, 5, 5), 2, "y", 1),       # odd rows, ragged tiles
+    ((8, 300, 5, 5), (200, 300, 3, 3), 1, "yz", 32),  # dL/dw in tiles over a ragged last channel block
+])
+def test_backward_of_many_channels_at_few_positions(capi, shape_x, shape_w, pad, mode, zu):
+    """Partial weight gradients added in tiles of 32 weights x 32 channels, and the products around them, against float64 autograd on the GPU; repeated calls give the same bits."""
+    x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=5)
+    w.view(-1)[::7] = 0.0
+    n, c_out = shape_x[0], shape_w[0]
+    wo, ho = shape_x[2] + 2 * pad - shape_w[2] + 1, shape_x[3] + 2 * pad - shape_w[3] + 1
+    g = torch.randn((n, c_out, wo, ho), generator=torch.Generator().manual_seed(8))
+    kw = dict(accumulate=mode, z_unit=zu)
+    gx, gw = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), **kw)
+    rx, rw = _fp64_reference_on_gpu(x, w, g, pad, mode, zu)
+    check(f"{shape_x} * {shape_w} {mode} grad_x", gx, rx)
+    check(f"{shape_x} * {shape_w} {mode} grad_w", gw, rw)
+    assert float(rx.abs().max()) > 0 and float(rw.abs().max()) > 0
+    gx2, gw2 = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), **kw)
+    assert torch.equal(gx2, gx) and torch.equal(gw2, gw)
