@@ -460,7 +460,7 @@ def probe_mfma_forward(torch):
             "slices_per_cu": slices, "tile": "128 positions x 256 rail-columns x 384 members", "times": t,
             "fp4_tflops_mfma_only": 2 * macs / (t["mfma_only_ms"] * 1e-3) / 1e12,
             "fp4_tflops_with_threshold": 2 * macs / (t["with_threshold_and_count_ms"] * 1e-3) / 1e12,
-            "note": "operands arrive expanded to one fp4 value per stream bit; the vector-ALU kernel takes 1.30 ms for "
+            "note": "operands arrive expanded to one fp4 value per stream bit; the vector-ALU kernel takes 1.155 ms for "
                     "the same layer from bit-packed streams"}
 
 
@@ -542,8 +542,8 @@ def main():
         "roofline": {
             "bound": "valu",
             "kernel": ("the rail-skipping convolution kernel (v_and_or_b32 on register-indexed accumulators: one "
-                       "and-or per activation word and weight; k_conv_fwd_tile_rail at the headline"
-                       ")" if rail else "k_conv_fwd (v_and_or_b32 / v_bcnt_u32_b32, both rails)"),
+                       "and-or per activation word and weight; k_conv_fwd_tile_rail at the headline)"
+                       if rail else "k_conv_fwd (v_and_or_b32 / v_bcnt_u32_b32, both rails)"),
             # work no kernel can avoid (one and-or per activation word and weight, plus the popcount-adds) per
             # second of the kernel's average launch duration, against lanes x clock
             "achieved": achieved / 1e12,
