@@ -1413,6 +1413,8 @@ struct RailPlan {
     RailKernel kernel;
     int shares, in_flight, per_slot;  // kRailTile
     int splits;                       // blockIdx.y
+    // the launch adds to y (several blocks or waves hold a part of a count each): y is zeroed in front of it
+    bool adds() const { return kernel == kRailSplit || kernel == kRailPair || splits > 1; }
 };
 constexpr long long kPairRound = 5 * 4 * 256;  // waves of a round with five waves per SIMD
 RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
@@ -1515,7 +1517,7 @@ int launch(const Geometry& g, FwdParams q, hipStream_t s)
             // sums out of the 128 registers
             constexpr int CR = WK == 1 ? 2 : 1;
             const RailPlan rp = plan_rail(g, sp);
-            if (rp.splits > 1 || rp.kernel == kRailSplit) clear_y();
+            if (rp.adds()) clear_y();
             const dim3 grid((unsigned)blocks, (unsigned)rp.splits);
             if (rp.kernel == kRailPlain)
                 hipLaunchKernelGGL((k_conv_fwd_rail<WK, CR>), grid, dim3(64), 0, s, q);

@@ -511,6 +511,18 @@ def test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode
         assert np.array_equal(y.cpu().numpy(), exp)
 
 
+@pytest.mark.parametrize("shape_x,shape_w,pad,L,mode", [
+    ((320, 32, 16, 16), (128, 32, 3, 1), (0, 0), 32, "y"),    # one (pack, add group) pair per tile, 4480 tiles
+    ((256, 11, 16, 16), (140, 11, 3, 3), (1, 1), 32, "full"), # the same, an OR over kernel rows as well
+    ((160, 32, 16, 16), (128, 32, 3, 1), (0, 0), 64, "y"),    # two pairs per tile
+    ((64, 20, 16, 16), (64, 20, 5, 5), (2, 2), 64, "y"),      # ten, one round of waves exactly
+])
+def test_launches_with_one_wave_per_pair_write_every_count(capi, so, shape_x, shape_w, pad, L, mode):
+    """Long OR groups, at most ten pairs per tile and full rounds of waves: one wave per pair, counts added to y.  y holds other
+    values before the call, as freshly allocated memory does: they must not show, in the first call or the second."""
+    test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode, 1)
+
+
 # ------------------------------------------------------------------ batches cut into chunks
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,kw", [
     ((11, 6, 9, 8), (20, 6, 3, 3), (1, 1), 64, {}),                                   # position-major, 3-wide
