@@ -95,12 +95,13 @@ int make_geometry(const geo_sc_conv_desc* d, Geometry* g)
     {
         // Lanes over the members of an OR group instead of over output positions: where positions are too few
         // and no launch shares an OR group out over waves (outputs with a single row, kernel widths without
-        // rail-packed weights).  Waves the position-parallel kernel could start at most (one (pack, add group)
+        // rail-packed weights, stream buffers from 4 GiB on).  Waves the position-parallel kernel could start at most (one (pack, add group)
         // pair per wave) against the 1024 SIMDs; members of one OR group against the 64 lanes
         const long long pos_waves = (((long long)d->n * wo * ho + 63) / 64) * g->n_cotile * g->packs * g->add_outer *
                                     g->add_inner;
         const long long members = (long long)g->or_rows * g->or_ch_per_group * d->w_k;
-        const bool shared_or = wo >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5);
+        const bool shared_or = wo >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5) &&
+                               (unsigned long long)g->act_words * 4 < 0xffffffffull;
         g->thin = pos_waves < 2048 && members >= 64 && !shared_or;
     }
     g->act_item_inner = !g->thin && g->mode == GEO_SC_ACC_Y && g->generator == GEO_SC_GEN_LFSR && wo == 1 && d->n >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5) &&

@@ -1417,7 +1417,7 @@ struct RailPlan {
     bool adds() const { return kernel == kRailSplit || kernel == kRailPair || splits > 1; }
 };
 constexpr long long kPairRound = 5 * 4 * 256;  // waves of a round with five waves per SIMD
-RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
+RailPlan plan_rail_unbounded(const Geometry& g, const SplitPlan& sp)
 {
     const long long lines = (long long)g.or_rows * g.or_ch_per_group * g.w_k;  // of an OR group
     const long long tiles = sp.waves, pairs = tiles * sp.pv;                   // (tile, pair) waves
@@ -1469,6 +1469,14 @@ RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
     if (pv / p.in_flight / p.per_slot >= 32768) p.per_slot = pv / p.in_flight / 32768 + 1;  // a grid's limit in y
     const int per_block = p.in_flight * p.per_slot;
     p.splits = (pv + per_block - 1) / per_block;
+    return p;
+}
+RailPlan plan_rail(const Geometry& g, const SplitPlan& sp)
+{
+    const RailPlan p = plan_rail_unbounded(g, sp);
+    // a grid has at most 2^32 - 1 threads in x (from 2^24 tiles of four waves on, 137 GB of counts): one wave per tile
+    if (p.kernel == kRailTile && sp.waves * 64 * p.shares * p.in_flight > 0xffffffffLL)
+        return {g.mode == GEO_SC_ACC_Y && sp.splits == 1 ? kRailPlain : kRailSplit, 0, 0, 0, sp.splits};
     return p;
 }
 

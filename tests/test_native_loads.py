@@ -109,6 +109,20 @@ def test_descriptors_around_four_gib_of_activation_streams():
     assert max(sizes) - min(sizes) <= 8 * item  # chunk sizes may differ by a few items, not by the batch
 
 
+def test_few_positions_with_streams_beyond_32_bit_offsets_are_not_refused():
+    """A stage call on few positions whose activation streams the kernels with 32-bit offsets cannot address runs with the
+    lanes over the members of its OR groups: the call gets as far as its launch, which fails without a GPU."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("GPU present: the pointers below are never to be read")
+    import ctypes as ct
+    from geo_amd import _native, capi
+    fake = ct.c_void_p(256)
+    for c_in, L in ((1 << 23, 256), (1 << 25, 32)):
+        d = capi.make_desc((1, c_in, 6, 6), (4, c_in, 3, 3), L)
+        assert _native.lib().geo_sc_conv2d_add_partial_from_streams(ct.byref(d), fake, fake, fake, None) == 4
+
+
 def test_stream_tables_are_constants_of_the_library():
     """The comparison tables the generators read (evaluated at compile time) against the oracle's register:
     posp1 inverts the cycle from state 1, thr[code] holds [code > state] along the doubled cycle."""
