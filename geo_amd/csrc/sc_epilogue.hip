@@ -354,6 +354,10 @@ __global__ __launch_bounds__(256) void k_tail_bwd_apply(TailParams q, const floa
         }
 }
 
+// Correctly rounded (sqrtf is, as compiled here, and equals torch.sqrt on every float; __fsqrt_rn is the hardware's
+// approximate root, off by up to two units in the last place).
+__device__ __forceinline__ float sqrt_rn(float v) { return sqrtf(v); }
+
 // Inference form of BatchNorm*_fixed (utils_class.py:49-64): y = x * w_n + b_n with w_n, b_n quantised from the
 // running statistics.  Bound by the 8 bytes per element; as PyTorch operations it is an (unused) batch norm, 24
 // launches on tensors of c elements and two passes over x.  Every workgroup forms the c affine pairs itself (c is
@@ -385,7 +389,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* __restrict__
     __shared__ double red[256];
     double part = 0.0;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
-        const float inv = __fsqrt_rn(__fadd_rn(var[ch], eps));
+        const float inv = sqrt_rn(__fadd_rn(var[ch], eps));
         const float gm = gamma ? gamma[ch] : 1.0f, bt = beta ? beta[ch] : 0.0f;
         const float w = __fdiv_rn(gm, inv);
         pairs[ch] = make_float2(w, __fsub_rn(bt, __fdiv_rn(__fmul_rn(mean[ch], gm), inv)));
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
     }
     double part = 0.0;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
-        const float inv = __fsqrt_rn(__fadd_rn(var[ch], eps));
+        const float inv = sqrt_rn(__fadd_rn(var[ch], eps));
         const float gm = gamma ? gamma[ch] : 1.0f;
         part += (double)__fdiv_rn(gm, inv);
     }
@@ -479,7 +483,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
     const float scale = scale_s;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
         const float mu = mean[ch], vr = var[ch];
-        const float inv = __fsqrt_rn(__fadd_rn(vr, eps));
+        const float inv = sqrt_rn(__fadd_rn(vr, eps));
         const float gm = gamma ? gamma[ch] : 1.0f, bt = beta ? beta[ch] : 0.0f;
         const float w = __fdiv_rn(gm, inv);
         const float b = __fsub_rn(bt, __fdiv_rn(__fmul_rn(mu, gm), inv));
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
         const float qb = fminf(fmaxf(rintf(__fmul_rn(__fdiv_rn(b, scale), 128.0f)), -127.0f), 127.0f);
         w_n[ch] = __fmul_rn(__fdiv_rn(qw, 128.0f), scale);
         b_n[ch] = __fmul_rn(__fdiv_rn(qb, 128.0f), scale);
-        if (invstd) invstd[ch] = 1.0f / __fsqrt_rn(__fadd_rn(vr, eps_grad));
+        if (invstd) invstd[ch] = 1.0f / sqrt_rn(__fadd_rn(vr, eps_grad));
         if (running_mean) running_mean[ch] = __fadd_rn(__fmul_rn(running_mean[ch], 0.9f), __fmul_rn(mu, 0.1f));
         if (running_var)
             running_var[ch] = __fadd_rn(__fmul_rn(running_var[ch], 0.9f), __fmul_rn(__fmul_rn(vr, unbias), 0.1f));

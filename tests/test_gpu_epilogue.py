@@ -211,6 +211,20 @@ def test_fixed_batch_norm_in_eval_mode_equals_the_op_chain(shape, affine, spoil)
         assert bn(x[:0]).shape == x[:0].shape
 
 
+def test_fixed_affine_rounds_every_operation_once(capi):
+    """w_n, b_n of two million channels against the operations of utils_class.py:52-62: a root or quotient that is off in the
+    last place moves some of them across a boundary of the 8-bit rounding."""
+    from geo_amd import utils_functional as uf
+    c = 1 << 21
+    g = torch.Generator(device="cuda").manual_seed(6)
+    mean, var, gamma, beta = (torch.rand(c, generator=g, device="cuda") + 0.01 for _ in range(4))
+    inv = torch.sqrt(var + 1e-5)
+    exp_w, exp_scale = uf.quantize_shift(gamma / inv)
+    exp_b, _ = uf.quantize_shift(beta - mean * gamma / inv, exp_scale)
+    w_n, b_n, _, scale = capi.bn_fixed_affine(mean, var, gamma, beta, 1e-5, 100)
+    assert torch.equal(scale, exp_scale) and torch.equal(w_n, exp_w) and torch.equal(b_n, exp_b)
+
+
 def test_quantize_kernel_equals_the_torch_op_chain():
     """geo_sc_quantize against (x * 2^p).round().clamp(+-(2^p - 1)) / 2^p (utils_functional.py:33-39):
     bit for bit, including ties (half to even), the clamp ends, zeros' signs aside, and NaN."""
