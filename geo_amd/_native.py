@@ -70,6 +70,8 @@ C_API = {
     "geo_sc_bn_fixed_from_counts": (ctypes.c_int, [_P] + [ctypes.c_int] * 5 + [_P, _P, ctypes.c_float, ctypes.c_float] +
                                     [_P] * 9 + [ctypes.c_size_t, _P]),
     "geo_sc_bn_fixed_eval": (ctypes.c_int, [_P] + [ctypes.c_int] * 3 + [_P] * 4 + [ctypes.c_float] + [_P] * 3),
+    "geo_sc_bn_eval_weight": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_float, _P, _P]),
+    "geo_sc_bn_fixed_eval_mean": (ctypes.c_int, [_P] + [ctypes.c_int] * 3 + [_P] * 4 + [ctypes.c_float] + [_P] * 4),
     "geo_sc_quantize_many": (ctypes.c_int, [ctypes.c_int, _P, _P, _P, ctypes.c_int, _P]),
     "geo_sc_copy_back_clamp": (ctypes.c_int, [ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, ctypes.c_float, _P]),
     "geo_sc_conv2d_add_partial_forward_q7": (ctypes.c_int, [_D, _P, _P, _P, _P, ctypes.c_size_t, _P]),

@@ -288,19 +288,33 @@ def bn_fixed_from_counts(counts, bit_length, gamma, beta, eps, running_mean=None
 BN_EVAL_CHANNELS = 4096
 
 
-def bn_fixed_eval(x, mean, var, gamma, beta, eps, stream=None):
-    """geo_sc_bn_fixed_eval: (y, scale) of a fixed-point batch norm on given statistics; ``x``: contiguous fp32 GPU
-    tensor (n, c, ...), the rest contiguous fp32 of c entries on the same GPU (gamma / beta may be None)."""
+def bn_eval_weight(var, gamma, eps, stream=None):
+    """geo_sc_bn_eval_weight: gamma / sqrt(var + eps) per channel (contiguous fp32 GPU tensors of one size; gamma may be
+    None)."""
+    for t in (var, gamma):
+        if t is not None and not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == var.device
+                                  and t.numel() == var.numel()):
+            raise ValueError("variance and weight must be contiguous float32 tensors of one size on one GPU")
+    w = torch.empty(var.numel(), dtype=torch.float32, device=var.device)
+    _check(_native.lib().geo_sc_bn_eval_weight(_ptr(var), _ptr(gamma), var.numel(), float(eps), _ptr(w), _stream_ptr(stream)),
+           "geo_sc_bn_eval_weight")
+    return w
+
+
+def bn_fixed_eval(x, mean, var, gamma, beta, eps, w_mean=None, stream=None):
+    """geo_sc_bn_fixed_eval_mean: (y, scale) of a fixed-point batch norm on given statistics; ``x``: contiguous fp32 GPU
+    tensor (n, c, ...), the rest contiguous fp32 of c entries on the same GPU (gamma / beta may be None).  ``w_mean``: one
+    float, the mean of ``bn_eval_weight`` that the scale is taken from (None: formed in double precision)."""
     n, c = x.shape[:2]
-    for t in (x, mean, var, gamma, beta):
+    for t, size in ((x, x.numel()), (mean, c), (var, c), (gamma, c), (beta, c), (w_mean, 1)):
         if t is not None and not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == x.device
-                                  and (t is x or t.numel() == c)):
+                                  and t.numel() == size):
             raise ValueError("x, statistics and parameters must be contiguous float32 tensors on one GPU")
     y = torch.empty_like(x)
     scale = torch.empty((), dtype=torch.float32, device=x.device)
-    _check(_native.lib().geo_sc_bn_fixed_eval(_ptr(x), n, c, x.numel() // (n * c), _ptr(mean), _ptr(var), _ptr(gamma),
-                                              _ptr(beta), float(eps), _ptr(y), _ptr(scale), _stream_ptr(stream)),
-           "geo_sc_bn_fixed_eval")
+    _check(_native.lib().geo_sc_bn_fixed_eval_mean(_ptr(x), n, c, x.numel() // (n * c), _ptr(mean), _ptr(var), _ptr(gamma),
+                                                   _ptr(beta), float(eps), _ptr(w_mean), _ptr(y), _ptr(scale),
+                                                   _stream_ptr(stream)), "geo_sc_bn_fixed_eval_mean")
     return y, scale
 
 

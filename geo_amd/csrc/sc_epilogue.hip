@@ -360,10 +360,15 @@ __device__ __forceinline__ float sqrt_rn(float v) { return sqrtf(v); }
 
 // Inference form of BatchNorm*_fixed (utils_class.py:49-64): y = x * w_n + b_n with w_n, b_n quantised from the
 // running statistics.  Bound by the 8 bytes per element; as PyTorch operations it is an (unused) batch norm, 24
-// launches on tensors of c elements and two passes over x.  Every workgroup forms the c affine pairs itself (c is
-// at most a few hundred: two divisions per thread, under the latency of the first loads of x) and keeps them in LDS,
-// so there is one launch: 256 x 32 x 32 x 32 158 us of kernels as operations, 12.4 us here.
+// launches on tensors of c elements and two passes over x.  Every workgroup forms the c affine pairs itself (two
+// divisions per channel, 16 channels per thread at the most; one or two at the networks' 10 to 512, under the latency
+// of the first loads of x) and keeps them in LDS.
+// 256 x 32 x 32 x 32: 158 us of kernels as operations, 12.4 us here.
 // Arithmetic of k_bn_fixed_affine, except that NaN passes the clamp as it passes torch.clamp.
+// w_mean (optional): the channel mean of w that the scale is taken from.  The scale is a power of two, so where
+// 3 mean(w) lies next to one, the order in which the mean's sum is formed decides about a factor of two: a caller that
+// has to meet another implementation's scale hands in that implementation's mean (a float); without it the sum is
+// formed in double precision.
 constexpr int kBnEvalChannels = 4096;
 __device__ __forceinline__ float fixed8(float v, float scale)
 {
@@ -378,11 +383,19 @@ __device__ __forceinline__ float mul_then_add(float x, float2 wb)
     const float p = x * wb.x;
     return p + wb.y;
 }
+// w = gamma / sqrt(var + eps): what that mean is taken of
+__global__ __launch_bounds__(256) void k_bn_eval_weight(const float* __restrict__ var, const float* __restrict__ gamma, int c,
+                                                        float eps, float* __restrict__ w)
+{
+    const int ch = blockIdx.x * 256 + threadIdx.x;
+    if (ch < c) w[ch] = __fdiv_rn(gamma ? gamma[ch] : 1.0f, sqrt_rn(__fadd_rn(var[ch], eps)));
+}
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* __restrict__ x, float* __restrict__ y, unsigned items,
                                                        unsigned plane, int c, const float* __restrict__ mean,
-                                                       const float* __restrict__ var, const float* __restrict__ gamma,
-                                                       const float* __restrict__ beta, float eps,
+                                                       const float* __restrict__ var,
+                                                       const float* __restrict__ gamma, const float* __restrict__ beta,
+                                                       float eps, const float* __restrict__ w_mean,
                                                        float* __restrict__ scale_out)
 {
     extern __shared__ float2 pairs[];  // [c]: w_n, b_n
@@ -395,13 +408,20 @@ __global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* __restrict__
         pairs[ch] = make_float2(w, __fsub_rn(bt, __fdiv_rn(__fmul_rn(mean[ch], gm), inv)));
         part += (double)w;
     }
-    red[threadIdx.x] = part;
-    __syncthreads();
-    for (int step = 128; step >= 1; step >>= 1) {
-        if ((int)threadIdx.x < step) red[threadIdx.x] += red[threadIdx.x + step];
+    float m;
+    if (w_mean) {
+        m = *w_mean;
+    } else {
+        red[threadIdx.x] = part;
         __syncthreads();
+        for (int step = 128; step >= 1; step >>= 1) {
+            if ((int)threadIdx.x < step) red[threadIdx.x] += red[threadIdx.x + step];
+            __syncthreads();
+        }
+        m = (float)(red[0] / (double)c);
     }
-    const float scale = exp2f(ceilf(log2f(__fmul_rn((float)(red[0] / (double)c), 3.0f))));
+    // (powf as torch's 2 ** t: from 2^16 on and below 2^-33 it is not always the power of two itself)
+    const float scale = powf(2.0f, ceilf(log2f(__fmul_rn(m, 3.0f))));
     if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
     for (int ch = threadIdx.x; ch < c; ch += 256)
         pairs[ch] = make_float2(fixed8(pairs[ch].x, scale), fixed8(pairs[ch].y, scale));
@@ -846,23 +866,39 @@ extern "C" int geo_sc_bn_fixed_from_counts(const int32_t* counts, int n, int c, 
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
 
-extern "C" int geo_sc_bn_fixed_eval(const float* x, int n, int c, int plane, const float* mean, const float* var,
-                                    const float* gamma, const float* beta, float eps, float* y, float* scale,
-                                    geo_sc_stream_t stream)
+extern "C" int geo_sc_bn_eval_weight(const float* var, const float* gamma, int c, float eps, float* w,
+                                     geo_sc_stream_t stream)
+{
+    if (!var || !w || c < 1) return GEO_SC_ERR_INVALID_ARGUMENT;
+    hipLaunchKernelGGL(k_bn_eval_weight, dim3((unsigned)(((long long)c + 255) / 256)), dim3(256), 0, (hipStream_t)stream, var,
+                       gamma, c, eps, w);
+    return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
+}
+
+extern "C" int geo_sc_bn_fixed_eval_mean(const float* x, int n, int c, int plane, const float* mean, const float* var,
+                                         const float* gamma, const float* beta, float eps, const float* w_mean, float* y,
+                                         float* scale, geo_sc_stream_t stream)
 {
     if (!x || !y || !mean || !var || !scale || n < 1 || c < 1 || plane < 1) return GEO_SC_ERR_INVALID_ARGUMENT;
     if (c > kBnEvalChannels) return GEO_SC_ERR_UNSUPPORTED;  // the affine pairs sit in LDS
     const size_t elements = (size_t)n * c * plane;
     if (elements > 0x7fffffffu) return GEO_SC_ERR_UNSUPPORTED;  // 32-bit indices
     const bool vec = plane % 4 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15u) == 0;
-    // four to sixteen vectors per thread where there are that many
+    // four items (vectors, or elements) per thread; from 2M items on 2048 workgroups, each thread with more
     const unsigned items = (unsigned)(elements / (vec ? 4 : 1));
     size_t blocks = ((size_t)items + 1023) / 1024;
     if (blocks > 2048) blocks = 2048;
     auto kernel = vec ? k_bn_fixed_eval<true> : k_bn_fixed_eval<false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), sizeof(float2) * c, (hipStream_t)stream, x, y, items,
-                       (unsigned)plane, c, mean, var, gamma, beta, eps, scale);
+                       (unsigned)plane, c, mean, var, gamma, beta, eps, w_mean, scale);
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
+}
+
+extern "C" int geo_sc_bn_fixed_eval(const float* x, int n, int c, int plane, const float* mean, const float* var,
+                                    const float* gamma, const float* beta, float eps, float* y, float* scale,
+                                    geo_sc_stream_t stream)
+{
+    return geo_sc_bn_fixed_eval_mean(x, n, c, plane, mean, var, gamma, beta, eps, nullptr, y, scale, stream);
 }
 
 extern "C" int geo_sc_quantize(const float* src, float* dst, size_t n, int prec, geo_sc_stream_t stream)

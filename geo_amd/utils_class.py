@@ -44,7 +44,7 @@ def _fixed_affine(module, x, mean, var):
 
 
 def _fixed_eval(module, x, dims):
-    """The value of ``BatchNorm*_fixed`` in eval mode as one kernel, or None where the chain of operations has to run:
+    """The value of ``BatchNorm*_fixed`` in eval mode as one pass over ``x``, or None where the chain of operations has to run:
     whenever something besides the value is asked for (gradients, forward-mode tangents, function transforms,
     tracing), and for layouts, types and devices that the kernel does not take."""
     if module.training or torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dim() != dims:
@@ -64,7 +64,10 @@ def _fixed_eval(module, x, dims):
     for t in (mean, var, gamma, beta):
         if t is not None and not (t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()):
             return None
-    y, module.scale = capi.bn_fixed_eval(x, mean, var, gamma, beta, module.eps)
+    # the channel mean as the chain takes it (quantize_shift): with another order of additions the scale can be another
+    # power of two
+    w_mean = torch.mean(capi.bn_eval_weight(var, gamma, module.eps))
+    y, module.scale = capi.bn_fixed_eval(x, mean, var, gamma, beta, module.eps, w_mean=w_mean)
     return y
 
 

@@ -381,10 +381,20 @@ GEO_SC_API int geo_sc_bn_fixed_from_counts(const int32_t* counts, int n, int c, 
  * y = x * w_n + b_n with w_n, b_n as geo_sc_bn_fixed_affine forms them from mean and var (c floats each); gamma /
  * beta may be NULL (1 / 0).  x, y: (n, c, plane) contiguous floats, y may be x; scale receives one float; c at
  * most 4096 and fewer than 2^31 elements (GEO_SC_ERR_UNSUPPORTED otherwise).
+ * The scale is 2 ** ceil(log2(mean(w) * 3)), w = gamma / sqrt(var + eps).  mean(w) is formed in double precision here
+ * and rounded once; the reference's is an fp32 reduction, whose order decides about a factor of two of the scale where
+ * 3 mean(w) lies within its rounding error of a power of two.  A caller that has to meet such a mean takes w from
+ * geo_sc_bn_eval_weight (c floats), reduces it as the other side does, and hands the result (one float on the device)
+ * to geo_sc_bn_fixed_eval_mean, which is geo_sc_bn_fixed_eval with that mean (NULL: the double-precision one).
  */
 GEO_SC_API int geo_sc_bn_fixed_eval(const float* x, int n, int c, int plane, const float* mean, const float* var,
                                     const float* gamma, const float* beta, float eps, float* y, float* scale,
                                     geo_sc_stream_t stream);
+GEO_SC_API int geo_sc_bn_eval_weight(const float* var, const float* gamma, int c, float eps, float* w,
+                                     geo_sc_stream_t stream);
+GEO_SC_API int geo_sc_bn_fixed_eval_mean(const float* x, int n, int c, int plane, const float* mean, const float* var,
+                                         const float* gamma, const float* beta, float eps, const float* w_mean, float* y,
+                                         float* scale, geo_sc_stream_t stream);
 
 /*
  * quantize (utils_functional.py:33-39) in one pass: dst = clamp(round(src * 2^prec), -(2^prec - 1), 2^prec - 1)

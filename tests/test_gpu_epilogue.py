@@ -225,6 +225,36 @@ def test_fixed_affine_rounds_every_operation_once(capi):
     assert torch.equal(scale, exp_scale) and torch.equal(w_n, exp_w) and torch.equal(b_n, exp_b)
 
 
+def _chain(monkeypatch, f):
+    """``f()`` with the one-pass form of the eval-mode batch norm switched off: the chain of operations alone."""
+    from geo_amd import utils_class
+    with monkeypatch.context() as m:
+        m.setattr(utils_class, "_fixed_eval", lambda *a: None)
+        return f()
+
+
+@pytest.mark.parametrize("top", [4.0, 2.0, 1.0, 2.0 ** 20, 2.0 ** -36])
+def test_eval_batch_norm_scale_next_to_a_power_of_two(top, monkeypatch):
+    """The scale is 2 ** ceil(log2(3 mean(w))): with 3 w within a rounding error of a power of two in every channel the
+    order in which the mean's sum is formed decides about a factor of two.  Value and ``scale`` are those of the chain."""
+    from geo_amd import utils_class
+    scales = set()
+    for c in [*range(1, 130, 3), 200, 300, 512, 700, 1000, 2048, 3000, 4096]:
+        bn = utils_class.BatchNorm2d_fixed(c).cuda().eval()
+        x = torch.rand((2, c, 2, 2), generator=torch.Generator().manual_seed(c)).cuda()
+        w = torch.tensor(top / 3)
+        for ulps in (-1, 0, 1):
+            with torch.no_grad():
+                bn.running_var.fill_(1 - 1e-5)   # sqrt(var + eps) = 1
+                bn.weight.fill_(torch.nextafter(w, w + ulps).item() if ulps else w.item())
+                exp = _chain(monkeypatch, lambda: bn(x.clone()))
+                exp_scale = bn.scale.clone()
+                got = bn(x.clone())
+            assert torch.equal(bn.scale, exp_scale) and torch.equal(got, exp), (c, ulps, bn.scale, exp_scale)
+            scales.add(float(exp_scale))
+    assert len(scales) == (2 if top in (1.0, 2.0, 4.0) else 1)   # both sides of the step; further out the logarithm rounds to one
+
+
 def test_quantize_kernel_equals_the_torch_op_chain():
     """geo_sc_quantize against (x * 2^p).round().clamp(+-(2^p - 1)) / 2^p (utils_functional.py:33-39):
     bit for bit, including ties (half to even), the clamp ends, zeros' signs aside, and NaN."""
