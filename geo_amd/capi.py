@@ -301,16 +301,17 @@ def bn_eval_weight(var, gamma, eps, stream=None):
     return w
 
 
-def bn_fixed_eval(x, mean, var, gamma, beta, eps, w_mean=None, stream=None):
+def bn_fixed_eval(x, mean, var, gamma, beta, eps, w_mean=None, out=None, stream=None):
     """geo_sc_bn_fixed_eval_mean: (y, scale) of a fixed-point batch norm on given statistics; ``x``: contiguous fp32 GPU
     tensor (n, c, ...), the rest contiguous fp32 of c entries on the same GPU (gamma / beta may be None).  ``w_mean``: one
-    float, the mean of ``bn_eval_weight`` that the scale is taken from (None: formed in double precision)."""
+    float, the mean of ``bn_eval_weight`` that the scale is taken from (None: formed in double precision).  ``out``: where
+    y goes (may be ``x``)."""
     n, c = x.shape[:2]
-    for t, size in ((x, x.numel()), (mean, c), (var, c), (gamma, c), (beta, c), (w_mean, 1)):
+    for t, size in ((x, x.numel()), (mean, c), (var, c), (gamma, c), (beta, c), (w_mean, 1), (out, x.numel())):
         if t is not None and not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == x.device
                                   and t.numel() == size):
             raise ValueError("x, statistics and parameters must be contiguous float32 tensors on one GPU")
-    y = torch.empty_like(x)
+    y = torch.empty_like(x) if out is None else out
     scale = torch.empty((), dtype=torch.float32, device=x.device)
     _check(_native.lib().geo_sc_bn_fixed_eval_mean(_ptr(x), n, c, x.numel() // (n * c), _ptr(mean), _ptr(var), _ptr(gamma),
                                                    _ptr(beta), float(eps), _ptr(w_mean), _ptr(y), _ptr(scale),

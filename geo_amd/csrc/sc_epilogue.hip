@@ -390,10 +390,10 @@ __global__ __launch_bounds__(256) void k_bn_eval_weight(const float* __restrict_
     const int ch = blockIdx.x * 256 + threadIdx.x;
     if (ch < c) w[ch] = __fdiv_rn(gamma ? gamma[ch] : 1.0f, sqrt_rn(__fadd_rn(var[ch], eps)));
 }
+// (y may be x: no __restrict__ on the two; a thread writes what it has read)
 template <bool VEC>
-__global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* __restrict__ x, float* __restrict__ y, unsigned items,
-                                                       unsigned plane, int c, const float* __restrict__ mean,
-                                                       const float* __restrict__ var,
+__global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* x, float* y, unsigned items, unsigned plane, int c,
+                                                       const float* __restrict__ mean, const float* __restrict__ var,
                                                        const float* __restrict__ gamma, const float* __restrict__ beta,
                                                        float eps, const float* __restrict__ w_mean,
                                                        float* __restrict__ scale_out)

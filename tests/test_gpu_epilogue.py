@@ -255,6 +255,28 @@ def test_eval_batch_norm_scale_next_to_a_power_of_two(top, monkeypatch):
     assert len(scales) == (2 if top in (1.0, 2.0, 4.0) else 1)   # both sides of the step; further out the logarithm rounds to one
 
 
+def test_eval_batch_norm_kernel_in_place_and_over_2048_workgroups(capi):
+    """geo_sc_bn_fixed_eval_mean: y may be x; more vectors (and elements) than four for each thread of the largest grid;
+    without a mean the scale comes from a sum in double precision, as geo_sc_bn_fixed_affine forms it."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for shape in ((40, 65, 57, 64), (9, 33, 87, 89), (3, 4096, 1, 1)):
+        c = shape[1]
+        x = torch.rand(shape, generator=g, device="cuda") - 0.5
+        mean, var, gamma, beta = (torch.rand(c, generator=g, device="cuda") + 0.1 for _ in range(4))
+        w_n, b_n, _, scale = capi.bn_fixed_affine(mean, var, gamma, beta, 1e-5, 100)
+        exp = x * w_n.view(1, c, 1, 1) + b_n.view(1, c, 1, 1)
+        y, s = capi.bn_fixed_eval(x, mean, var, gamma, beta, 1e-5)
+        assert torch.equal(y, exp) and torch.equal(s, scale)
+        z = x.clone()
+        out, _ = capi.bn_fixed_eval(z, mean, var, gamma, beta, 1e-5, out=z)
+        assert out is z and torch.equal(z, exp)
+        _, s2 = capi.bn_fixed_eval(x, mean, var, gamma, beta, 1e-5, w_mean=torch.full((), float(scale) * 0.75, device="cuda"))
+        assert float(s2) == 4 * float(scale)     # ceil(log2(2.25 scale))
+        assert torch.equal(capi.bn_eval_weight(var, gamma, 1e-5), gamma / torch.sqrt(var + 1e-5))
+    with pytest.raises(capi.GeoScError):
+        capi.bn_fixed_eval(torch.zeros(1, 4097, 1, 1, device="cuda"), *([torch.ones(4097, device="cuda")] * 4), 1e-5)
+
+
 def test_quantize_kernel_equals_the_torch_op_chain():
     """geo_sc_quantize against (x * 2^p).round().clamp(+-(2^p - 1)) / 2^p (utils_functional.py:33-39):
     bit for bit, including ties (half to even), the clamp ends, zeros' signs aside, and NaN."""
