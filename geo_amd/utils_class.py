@@ -44,16 +44,18 @@ def _fixed_affine(module, x, mean, var):
 
 
 def _fixed_eval(module, x, dims):
-    """The value of ``BatchNorm*_fixed`` in eval mode as one pass over ``x``, or None where the chain of operations has to run:
-    whenever something besides the value is asked for (gradients, forward-mode tangents, function transforms,
-    tracing), and for layouts, types and devices that the kernel does not take."""
+    """The value of ``BatchNorm*_fixed`` in eval mode as one pass over ``x``, or None where the chain of operations has to
+    run: whenever something besides the value is asked for or somebody watches the operations (gradients, forward-mode
+    tangents, function transforms, tracing, dispatch and function modes, tensor subclasses), and for layouts, types, sizes
+    and devices that the kernel does not take."""
     if module.training or torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dim() != dims:
         return None
     if not (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and 0 < x.numel() < 2 ** 31
-            and x.shape[1] == module.num_features):
+            and x.shape[1] == module.num_features and not x.is_neg()):
         return None
     if torch.jit.is_tracing() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 \
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0:
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0 \
+            or torch._C._len_torch_function_stack() > 0:
         return None
     from . import capi
     mean, var = module.running_mean, module.running_var
@@ -62,7 +64,9 @@ def _fixed_eval(module, x, dims):
             or x.device.index != torch.cuda.current_device():
         return None
     for t in (mean, var, gamma, beta):
-        if t is not None and not (t.device == x.device and t.dtype == torch.float32 and t.is_contiguous()):
+        if t is not None and not (type(t) in (torch.Tensor, nn.Parameter) and t.device == x.device
+                                  and t.dtype == torch.float32 and t.shape == (module.num_features,) and t.is_contiguous()
+                                  and not t.is_neg()):
             return None
     # the channel mean as the chain takes it (quantize_shift): with another order of additions the scale can be another
     # power of two

@@ -277,6 +277,62 @@ def test_eval_batch_norm_kernel_in_place_and_over_2048_workgroups(capi):
         capi.bn_fixed_eval(torch.zeros(1, 4097, 1, 1, device="cuda"), *([torch.ones(4097, device="cuda")] * 4), 1e-5)
 
 
+def test_eval_batch_norm_leaves_transforms_modes_and_subclasses_to_the_op_chain(monkeypatch):
+    """Whatever looks at the operations themselves sees them: forward-mode tangents, tracing, function transforms, dispatch
+    and function modes, tensor subclasses, views whose values are not what lies in memory."""
+    import torch.autograd.forward_ad as fw
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from geo_amd import utils_class
+    g = torch.Generator().manual_seed(1)
+    bn = utils_class.BatchNorm2d_fixed(6).cuda().eval()
+    x = torch.rand((4, 6, 4, 4), generator=g).cuda()
+
+    class Tagged(torch.Tensor):
+        pass
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatches(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        bn.running_mean.copy_(torch.rand(6, generator=g) - 0.3)
+        bn.running_var.copy_(torch.rand(6, generator=g) + 0.1)
+        bn.weight.copy_(torch.rand(6, generator=g) + 0.5)
+        exp = bn(x)
+        assert torch.equal(exp, _chain(monkeypatch, lambda: bn(x)))
+        with fw.dual_level():
+            out = fw.unpack_dual(bn(fw.make_dual(x, torch.ones_like(x))))
+            assert torch.equal(out.primal, exp) and out.tangent is not None
+        assert "batch_norm" in str(torch.jit.trace(bn, (x,), check_trace=False).inlined_graph)
+        assert "batch_norm" in make_fx(bn)(x).code
+        for transform in (lambda: torch.func.vmap(bn)(x.view(2, 2, 6, 4, 4)),
+                          lambda: torch.func.jvp(bn, (x,), (torch.ones_like(x),))):
+            with pytest.raises(RuntimeError, match="data"):   # the chain's write to .data is refused there
+                transform()
+        for mode in (Functions, Dispatches):
+            seen = []
+            with mode():
+                assert torch.equal(bn(x), exp)
+            assert any("batch_norm" in n for n in seen), mode
+        assert torch.equal(bn(torch._neg_view(-x)), exp)
+        for name in ("weight", "running_var"):
+            t = getattr(bn, name).detach()
+            out = torch.func.functional_call(bn, {name: t.as_subclass(Tagged)}, (x,))
+            assert type(out) is Tagged and torch.equal(out.as_subclass(torch.Tensor), exp)
+            assert torch.equal(torch.func.functional_call(bn, {name: torch._neg_view(-t)}, (x,)), exp)
+            with pytest.raises(RuntimeError):                 # refused by F.batch_norm
+                torch.func.functional_call(bn, {name: t[:5]}, (x,))
+        assert torch.equal(bn(x), exp)
+
+
 def test_quantize_kernel_equals_the_torch_op_chain():
     """geo_sc_quantize against (x * 2^p).round().clamp(+-(2^p - 1)) / 2^p (utils_functional.py:33-39):
     bit for bit, including ties (half to even), the clamp ends, zeros' signs aside, and NaN."""
