@@ -225,6 +225,9 @@ __device__ __forceinline__ void store_tile(const GemmParams& q, const floatx16 (
 // (mid lo, lo mid, lo lo) are below 2^-26 of the product, less than the rounding of an fp32
 // multiply.  Six bf16 MFMAs of 16 k take 6 x 8 passes where eight fp32 MFMAs of 2 k take
 // 8 x 16.  The split happens once per element, when a staged chunk is written to LDS.
+// Range: an operand above 3.39e38 is infinite to it, and an infinite one makes its products NaN (WgradOperands); the
+// terms of one below 2^-109 reach into bf16's subnormal numbers and are exact to 2^-134 only, a hundredth of the smallest
+// normal float.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -1225,12 +1228,34 @@ __global__ __launch_bounds__(256) void k_weight_operands(const float* __restrict
     }
 }
 
+// What a weight gradient is formed again from where its partial sums came out NaN (col NULL: nothing is; M positions,
+// rows of col and E col_ld and e_ld apart, groups col_v and e_v).  An infinite element of E, or one that rounds to a
+// bf16 infinity (above 3.39e38), is inf + (inf - inf) after its split into three bf16 terms: the product is NaN where an
+// fp32 product is infinite (or finite).  The sizes whose rows are no whole quads, which an fp32 product would serve, take
+// the split as well, so theirs is put right here: col E in fp32, one multiply-add after the other.  A sum that is NaN
+// by its operands ends at the element that makes it so.
+struct WgradOperands {
+    const float* col;
+    const float* e;
+    long long m, col_ld, e_ld;
+    size_t col_v, e_v;
+};
+__device__ __forceinline__ float wgrad_again(const WgradOperands& o, int group, int k, int j, long long begin, long long end)
+{
+    const float* c = o.col + group * o.col_v + k * o.col_ld;
+    const float* e = o.e + group * o.e_v + j;
+    float sum = 0.0f;
+#pragma unroll 1
+    for (long long m = begin; m < end && sum == sum; m++) sum = fmaf(c[m], e[m * o.e_ld], sum);
+    return sum;
+}
+
 // dL/dw of the members of group g0 + blockIdx.y from the split partial sums part[g][s][k][j].  A
 // block takes 32 consecutive (k, co) entries; 8 sets of threads each sum every 8th split, the
 // sets are then added in a fixed order, so the result does not depend on scheduling.
 __global__ __launch_bounds__(256) void k_reduce_wgrad(const float* __restrict__ part, const float* __restrict__ w,
                                                       float* __restrict__ gw, int g0, int splits, int c_out, Groups G,
-                                                      size_t g_stride)
+                                                      size_t g_stride, WgradOperands again)
 {
     __shared__ float red[2][8][32];
     const int K = G.n_members;
@@ -1251,14 +1276,26 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad(const float* __restrict__ 
     red[0][grp][lane] = sp;
     red[1][grp][lane] = sn;
     __syncthreads();
-    const Member mb = member_of(G, g, k);
-    if (grp == 0 && ok && mb.ok) {
+    auto add_sets = [&]() {
         sp = sn = 0.0f;
 #pragma unroll
         for (int gidx = 0; gidx < 8; gidx++) {
             sp += red[0][gidx][lane];
             sn += red[1][gidx][lane];
         }
+    };
+    add_sets();
+    // (every set holds the same 32 sums here: all waves agree)
+    if (again.col && __any(ok && (sp != sp || sn != sn))) {
+        __syncthreads();
+        const long long share = (again.m + 7) / 8, begin = min(again.m, grp * share), end = min(again.m, begin + share);
+        red[0][grp][lane] = ok && sp != sp ? wgrad_again(again, blockIdx.y, k, co, begin, end) : grp ? 0.0f : sp;
+        red[1][grp][lane] = ok && sn != sn ? wgrad_again(again, blockIdx.y, k, c_out + co, begin, end) : grp ? 0.0f : sn;
+        __syncthreads();
+        add_sets();
+    }
+    const Member mb = member_of(G, g, k);
+    if (grp == 0 && ok && mb.ok) {
         const long long wi = (((long long)co * G.c_in + mb.ci) * G.w_k + mb.u) * G.h_k + mb.v;
         const float wv = w[wi];
         float r = 0.0f;
@@ -1410,7 +1447,7 @@ __global__ __launch_bounds__(256) void k_weight_cat_tiled(const float* __restric
 // written in 128-byte runs along the weights of one channel.
 __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restrict__ part, const float* __restrict__ w,
                                                             float* __restrict__ gw, int g0, int ng, int splits, int c_out,
-                                                            Groups G, size_t g_stride)
+                                                            Groups G, size_t g_stride, WgradOperands again)
 {
     __shared__ float tp[32][33], tn[32][33];  // [weight][channel]
     const int per_channel = G.c_in * G.w_k * G.h_k;
@@ -1430,6 +1467,8 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restr
                     sp += src[s0 * stride];
                     sn += src[s0 * stride + c_out];
                 }
+                if (again.col && sp != sp) sp = wgrad_again(again, g - g0, k, co, 0, again.m);
+                if (again.col && sn != sn) sn = wgrad_again(again, g - g0, k, c_out + co, 0, again.m);
             }
         }
         tp[q][tx] = sp;
@@ -2599,10 +2638,10 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                 // few partial sums (wide layers): coalesced tiles; many: the kernel that adds eight splits side by side
                 if (L.fused_splits <= 4)
                     hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, L.fused_splits,
-                                       g.c_out, G, L.part_v);
+                                       g.c_out, G, L.part_v, WgradOperands{});
                 else
                     hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                       L.fused_splits, g.c_out, G, L.part_v);
+                                       L.fused_splits, g.c_out, G, L.part_v, WgradOperands{});
             }
             if (gx && L.dcol_slices > 1)
                 hipLaunchKernelGGL(k_sum_slices, dim3(grid1d((long long)((size_t)nv * L.col_v / 4))), dim3(256), 0, s, dcol,
@@ -2680,16 +2719,18 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             q2.a_rows = view_rows; q2.a_rows_batch = L.view_k_pad; q2.a_item = g.wo * g.ho; q2.a_skip = (g.w_k - 1) * g.ho;
             rc = view ? launch_gemm<false, true, EPI_STORE, true>(q2, nv, s) : launch_gemm<false, true, EPI_STORE>(q2, nv, s);
             if (rc != GEO_SC_OK) return rc;
+            WgradOperands again = {};
+            if (!view) again = {col, e, M, col_ld, e_ld, L.col_v, L.e_v};
             // Few partial sums and many weights: coalesced tiles (512 -> 512, 3 x 3, three partial sums: 50 -> 15.6 us;
             // the other kernel reads w and writes dL/dw one element per line).  Not where eight splits side by side are
             // what fills the GPU.
             const dim3 w_tiles((g.c_in * g.w_k * g.h_k + 31) / 32, (g.c_out + 31) / 32);
             if (L.splits <= 8 && (long long)w_tiles.x * w_tiles.y >= 512 && w_tiles.y <= 65535)
                 hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, L.splits, g.c_out,
-                                   G, L.part_v);
+                                   G, L.part_v, again);
             else
                 hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                   L.splits, g.c_out, G, L.part_v);
+                                   L.splits, g.c_out, G, L.part_v, again);
         }
         if (!gx) continue;
         if (dx_taps) {

@@ -494,3 +494,42 @@ def test_backward_of_many_channels_at_few_positions(capi, shape_x, shape_w, pad,
     assert float(rx.abs().max()) > 0 and float(rw.abs().max()) > 0
     gx2, gw2 = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), **kw)
     assert torch.equal(gx2, gx) and torch.equal(gw2, gw)
+
+
+@pytest.mark.parametrize("shape_x,shape_w", [
+    ((3, 20, 5, 7), (45, 20, 3, 3)),   # 105 positions, 90 rail columns: neither in whole quads
+    ((3, 20, 5, 7), (46, 20, 3, 3)),   # odd positions
+    ((4, 20, 6, 6), (45, 20, 3, 3)),   # odd rail columns
+    ((9, 40, 11, 13), (71, 40, 3, 3)), # several tiles and splits of each product
+    ((3, 150, 5, 7), (360, 150, 3, 3)),  # partial sums added in tiles of weights x channels
+])
+def test_infinite_and_largest_gradients_at_sizes_of_no_whole_quads(capi, shape_x, shape_w):
+    """An infinite element of the upstream gradient makes its channel's weight gradient infinite, not NaN, and leaves the
+    other channels' bits alone; a NaN stays one; a finite gradient that a bf16 would round to infinity stays finite."""
+    from oracle import surrogate
+    x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_w[0])
+    x = (x * 0.9 + 0.05).contiguous()
+    w = (w * 2).contiguous()
+    w.view(-1)[::7] = 0.0
+    w[9] = 0.0
+    pad = (1, 1)
+    back = lambda gy: capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, pad)
+    g = torch.randn((shape_x[0], shape_w[0]) + shape_x[2:], generator=torch.Generator().manual_seed(4))
+    gx, gw = back(g)
+    near = torch.zeros(shape_x, dtype=torch.bool)
+    near[1, :, 1:4, 2:5] = True
+    others = [c for c in range(shape_w[0]) if c != 7]
+    for value in (float("inf"), -float("inf"), float("nan")):
+        # away from the border: every activation it meets is positive
+        gi = g.clone()
+        gi[1, 7, 2, 3] = value
+        ix, iw = back(gi)
+        assert torch.equal(iw[others], gw[others])
+        assert bool((iw[7] == value).all() if value == value else torch.isnan(iw[7]).all()), value
+        assert torch.equal(ix.cpu()[~near], gx.cpu()[~near]) and not bool(torch.isfinite(ix.cpu()[near]).any())
+    # without weights E is the gradient itself
+    gb = g * 0
+    gb[1, 9, 2, 3] = 3.4e38
+    _, rw, _ = surrogate.surrogate_autograd(x * 0.04, w, gb, pad)
+    _, bw = capi.conv2d_add_partial_backward((x * 0.04).cuda(), w.cuda(), gb.cuda(), 128, pad)
+    check("grad_w of a gradient of 3.4e38", bw, rw)
