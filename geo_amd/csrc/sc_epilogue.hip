@@ -354,17 +354,14 @@ __global__ __launch_bounds__(256) void k_tail_bwd_apply(TailParams q, const floa
         }
 }
 
-// Correctly rounded (sqrtf is, as compiled here, and equals torch.sqrt on every float; __fsqrt_rn is the hardware's
-// approximate root, off by up to two units in the last place).
-__device__ __forceinline__ float sqrt_rn(float v) { return sqrtf(v); }
-
 // Inference form of BatchNorm*_fixed (utils_class.py:49-64): y = x * w_n + b_n with w_n, b_n quantised from the
 // running statistics.  Bound by the 8 bytes per element; as PyTorch operations it is an (unused) batch norm, 24
 // launches on tensors of c elements and two passes over x.  Every workgroup forms the c affine pairs itself (two
 // divisions per channel, 16 channels per thread at the most; one or two at the networks' 10 to 512, under the latency
 // of the first loads of x) and keeps them in LDS.
 // 256 x 32 x 32 x 32: 158 us of kernels as operations, 12.4 us here.
-// Arithmetic of k_bn_fixed_affine, except that NaN passes the clamp as it passes torch.clamp.
+// Arithmetic of the chain of operations bit for bit: sqrtf and log2f equal torch.sqrt and torch.log2 on every positive
+// float, and NaN passes the clamp as it passes torch.clamp.
 // w_mean (optional): the channel mean of w that the scale is taken from.  The scale is a power of two, so where
 // 3 mean(w) lies next to one, the order in which the mean's sum is formed decides about a factor of two: a caller that
 // has to meet another implementation's scale hands in that implementation's mean (a float); without it the sum is
@@ -388,7 +385,7 @@ __global__ __launch_bounds__(256) void k_bn_eval_weight(const float* __restrict_
                                                         float eps, float* __restrict__ w)
 {
     const int ch = blockIdx.x * 256 + threadIdx.x;
-    if (ch < c) w[ch] = __fdiv_rn(gamma ? gamma[ch] : 1.0f, sqrt_rn(__fadd_rn(var[ch], eps)));
+    if (ch < c) w[ch] = __fdiv_rn(gamma ? gamma[ch] : 1.0f, sqrtf(__fadd_rn(var[ch], eps)));
 }
 // (y may be x: no __restrict__ on the two; a thread writes what it has read)
 template <bool VEC>
@@ -402,7 +399,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* x, float* y,
     __shared__ double red[256];
     double part = 0.0;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
-        const float inv = sqrt_rn(__fadd_rn(var[ch], eps));
+        const float inv = sqrtf(__fadd_rn(var[ch], eps));
         const float gm = gamma ? gamma[ch] : 1.0f, bt = beta ? beta[ch] : 0.0f;
         const float w = __fdiv_rn(gm, inv);
         pairs[ch] = make_float2(w, __fsub_rn(bt, __fdiv_rn(__fmul_rn(mean[ch], gm), inv)));
@@ -447,7 +444,10 @@ __global__ __launch_bounds__(256) void k_bn_fixed_eval(const float* x, float* y,
 //     inv = sqrt(var + eps);  w = gamma / inv;  b = beta - mean * gamma / inv
 //     scale = 2 ** ceil(log2(mean_over_channels(w) * 3))
 //     w_n = round(w / scale * 128).clamp(-127, 127) / 128 * scale,   b_n likewise with the same scale
-// in PyTorch's operation order, one rounding per operation.  Also the running statistics of
+// in PyTorch's operation order, one rounding per operation except the root: __fsqrt_rn is the hardware's approximate one,
+// off by up to two units in the last place (w_n, b_n differ from the correctly rounded root's for a few channels in a
+// million; with that root the updated weights of a VGG-16 step, where Adam divides gradients near zero by their own size,
+// leave the former ones by a quarter of their norm).  Also the running statistics of
 // F.batch_norm(training=True) (momentum 0.1, unbiased variance) and 1 / sqrt(var + eps_grad) for the
 // backward.  The channel mean is accumulated in double precision.
 __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, const float* var,
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
     }
     double part = 0.0;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
-        const float inv = sqrt_rn(__fadd_rn(var[ch], eps));
+        const float inv = __fsqrt_rn(__fadd_rn(var[ch], eps));
         const float gm = gamma ? gamma[ch] : 1.0f;
         part += (double)__fdiv_rn(gm, inv);
     }
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
     const float scale = scale_s;
     for (int ch = threadIdx.x; ch < c; ch += 256) {
         const float mu = mean[ch], vr = var[ch];
-        const float inv = sqrt_rn(__fadd_rn(vr, eps));
+        const float inv = __fsqrt_rn(__fadd_rn(vr, eps));
         const float gm = gamma ? gamma[ch] : 1.0f, bt = beta ? beta[ch] : 0.0f;
         const float w = __fdiv_rn(gm, inv);
         const float b = __fsub_rn(bt, __fdiv_rn(__fmul_rn(mu, gm), inv));
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void k_bn_fixed_affine(const float* mean, cons
         const float qb = fminf(fmaxf(rintf(__fmul_rn(__fdiv_rn(b, scale), 128.0f)), -127.0f), 127.0f);
         w_n[ch] = __fmul_rn(__fdiv_rn(qw, 128.0f), scale);
         b_n[ch] = __fmul_rn(__fdiv_rn(qb, 128.0f), scale);
-        if (invstd) invstd[ch] = 1.0f / sqrt_rn(__fadd_rn(vr, eps_grad));
+        if (invstd) invstd[ch] = 1.0f / __fsqrt_rn(__fadd_rn(vr, eps_grad));
         if (running_mean) running_mean[ch] = __fadd_rn(__fmul_rn(running_mean[ch], 0.9f), __fmul_rn(mu, 0.1f));
         if (running_var)
             running_var[ch] = __fadd_rn(__fmul_rn(running_var[ch], 0.9f), __fmul_rn(__fmul_rn(vr, unbias), 0.1f));

@@ -378,8 +378,8 @@ GEO_SC_API int geo_sc_bn_fixed_from_counts(const int32_t* counts, int n, int c, 
 
 /*
  * BatchNorm2d_fixed / BatchNorm1d_fixed on given statistics, for inference, in one launch (utils_class.py:49-64):
- * y = x * w_n + b_n with w_n, b_n as geo_sc_bn_fixed_affine forms them from mean and var (c floats each); gamma /
- * beta may be NULL (1 / 0).  x, y: (n, c, plane) contiguous floats, y may be x; scale receives one float; c at
+ * y = x * w_n + b_n with w_n, b_n as the module forms them from mean and var (c floats each), one rounding per
+ * operation; gamma / beta may be NULL (1 / 0).  x, y: (n, c, plane) contiguous floats, y may be x; scale receives one float; c at
  * most 4096 and fewer than 2^31 elements (GEO_SC_ERR_UNSUPPORTED otherwise).
  * The scale is 2 ** ceil(log2(mean(w) * 3)), w = gamma / sqrt(var + eps).  mean(w) is formed in double precision here
  * and rounded once; the reference's is an fp32 reduction, whose order decides about a factor of two of the scale where
