@@ -285,9 +285,6 @@ def bn_fixed_from_counts(counts, bit_length, gamma, beta, eps, running_mean=None
     return mean, var, w_n, b_n, invstd, scale
 
 
-BN_EVAL_CHANNELS = 4096
-
-
 def bn_eval_weight(var, gamma, eps, stream=None):
     """geo_sc_bn_eval_weight: gamma / sqrt(var + eps) per channel (contiguous fp32 GPU tensors of one size; gamma may be
     None)."""

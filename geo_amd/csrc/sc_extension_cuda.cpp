@@ -60,6 +60,39 @@ at::Tensor conv2d_or_acc(torch::Tensor input, torch::Tensor weight, int64_t bit_
     return forward_on_device(input, weight, d);
 }
 
+// The value and the scale of BatchNorm*_fixed on given statistics (utils_class.py:49-64): the weight, its mean as
+// PyTorch reduces it (which the chain of operations takes the scale from), the pass over x.  Nothing where the kernel does
+// not take the tensors.  In C++ because it is three launches for what was one ctypes call: host time of the 4-layer
+// CNN's forward on one image 515 us with ctypes calls, 393 here (423 with the one launch and a mean in double precision).
+std::optional<std::tuple<at::Tensor, at::Tensor>> bn_fixed_eval(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var,
+                                                                const std::optional<at::Tensor>& gamma,
+                                                                const std::optional<at::Tensor>& beta, double eps)
+{
+    const auto plain = [&](const at::Tensor& t) {
+        return t.is_cuda() && t.device() == x.device() && t.scalar_type() == at::kFloat && t.layout() == at::kStrided &&
+               t.is_contiguous() && !t.is_neg();
+    };
+    if (x.dim() < 2 || !plain(x) || x.numel() < 1 || x.numel() > 0x7fffffff || x.size(1) > 4096) return std::nullopt;
+    const int64_t c = x.size(1);
+    const auto per_channel = [&](const at::Tensor& t) { return plain(t) && t.dim() == 1 && t.size(0) == c; };
+    if (!per_channel(mean) || !per_channel(var) || (gamma && !per_channel(*gamma)) || (beta && !per_channel(*beta)))
+        return std::nullopt;
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    geo_sc_stream_t stream = (geo_sc_stream_t)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index()).stream();
+    const float* gm = gamma ? gamma->const_data_ptr<float>() : nullptr;
+    const float* bt = beta ? beta->const_data_ptr<float>() : nullptr;
+    const at::Tensor w = at::empty({c}, x.options());
+    check_status(geo_sc_bn_eval_weight(var.const_data_ptr<float>(), gm, (int)c, (float)eps, w.data_ptr<float>(), stream),
+                 "batch norm weight");
+    const at::Tensor w_mean = at::mean(w);
+    at::Tensor y = at::empty_like(x), scale = at::empty({}, x.options());
+    check_status(geo_sc_bn_fixed_eval_mean(x.const_data_ptr<float>(), (int)x.size(0), (int)c, (int)(x.numel() / (x.size(0) * c)),
+                                           mean.const_data_ptr<float>(), var.const_data_ptr<float>(), gm, bt, (float)eps,
+                                           w_mean.const_data_ptr<float>(), y.data_ptr<float>(), scale.data_ptr<float>(), stream),
+                 "batch norm in eval mode");
+    return std::make_tuple(y, scale);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("conv2d_add_partial_variable_acc", &conv2d_add_partial_variable_acc,
@@ -69,4 +102,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("conv2d_add_partial_acc_acc", &conv2d_add_partial_acc_acc,
           "SC forward conv2d partial bin add, accurate random generator");
     m.def("conv2d_or_acc", &conv2d_or_acc, "SC forward conv2d or add, random generator");
+    m.def("_bn_fixed_eval", &bn_fixed_eval, "fixed-point batch norm on given statistics: (y, scale), or None");
 }

@@ -6,7 +6,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd import forward_ad
 
-from . import utils_functional
+from . import _native, utils_functional
 
 
 class Conv2d_Add_Partial(nn.Conv2d):
@@ -48,30 +48,26 @@ def _fixed_eval(module, x, dims):
     run: whenever something besides the value is asked for or somebody watches the operations (gradients, forward-mode
     tangents, function transforms, tracing, dispatch and function modes, tensor subclasses), and for layouts, types, sizes
     and devices that the kernel does not take."""
-    if module.training or torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dim() != dims:
-        return None
-    if not (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and 0 < x.numel() < 2 ** 31
-            and x.shape[1] == module.num_features and not x.is_neg()):
+    if module.training or torch.is_grad_enabled() or type(x) is not torch.Tensor or not x.is_cuda or x.dim() != dims:
         return None
     if torch.jit.is_tracing() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 \
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0 \
             or torch._C._len_torch_function_stack() > 0:
         return None
-    from . import capi
     mean, var = module.running_mean, module.running_var
     gamma, beta = (module.weight, module.bias) if module.affine else (None, None)
-    if mean is None or var is None or module.num_features > capi.BN_EVAL_CHANNELS \
-            or x.device.index != torch.cuda.current_device():
-        return None
-    for t in (mean, var, gamma, beta):
-        if t is not None and not (type(t) in (torch.Tensor, nn.Parameter) and t.device == x.device
-                                  and t.dtype == torch.float32 and t.shape == (module.num_features,) and t.is_contiguous()
-                                  and not t.is_neg()):
+    for t in (mean, var):
+        if type(t) not in (torch.Tensor, nn.Parameter):
             return None
-    # the channel mean as the chain takes it (quantize_shift): with another order of additions the scale can be another
-    # power of two
-    w_mean = torch.mean(capi.bn_eval_weight(var, gamma, module.eps))
-    y, module.scale = capi.bn_fixed_eval(x, mean, var, gamma, beta, module.eps, w_mean=w_mean)
+    for t in (gamma, beta):
+        if t is not None and type(t) not in (torch.Tensor, nn.Parameter):
+            return None
+    if x.shape[1] != module.num_features:
+        return None
+    out = _native.module("sc_extension_cuda")._bn_fixed_eval(x, mean, var, gamma, beta, module.eps)
+    if out is None:
+        return None
+    y, module.scale = out
     return y
 
 
