@@ -93,8 +93,8 @@ int launch_weight_streams(const Geometry& g, const float* w, uint32_t* streams, 
                           bool rail_only = false);
 int launch_conv_forward(const Geometry& g, const uint32_t* act, const uint32_t* wgt, int32_t* y, hipStream_t s);
 // Predicted duration of that launch in units of one wave walking one (pack, add group) pair on a full GPU:
-// what the forward compares when it cuts a batch into chunks (waves run in rounds of four per SIMD, so a
-// chunk whose waves fill whole rounds costs less per item).
+// what the forward compares when it cuts a batch into chunks (waves run in rounds of five per SIMD, so a
+// chunk of less than a round costs as much as a round; beyond one the cost is proportional).
 double conv_forward_cost(const Geometry& g);
 // fills the rail-packed part of a weight stream buffer from its two-rail lines (no-op unless g.wgt_rail;
 // with from_generator also where launch_weight_streams has written that part itself)

@@ -361,10 +361,13 @@ __global__ __launch_bounds__(64) void k_conv_fwd_split(FwdParams q)
 // keeps to that partner, so 32 + 16 + 8 + 4 + 2 + 1 shuffles leave one finished word per lane (bit 5: position,
 // bit 4: rail, bits 3 - 0: channel) where a full xor reduction of every word takes 64 x 6.
 // Results are added into the zeroed y with integer atomics.  Activation layout [n][P][c_in][wi][hi].
-constexpr int kThinPositions = 2;
+// R positions per wave: two, with fewer than a wave per CU one (the halving then starts with an OR of the two half waves):
+// bound by the latency of a wave's loads and shuffles there, 206 -> 45 channels, full OR over 3 x 3, four positions: 25.6
+// us with two, 17.2 with one; from two waves per SIMD on two positions take half the time.
+template <int R>
 __global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q, long long positions)
 {
-    constexpr int C = kCoTile, R = kThinPositions;
+    constexpr int C = kCoTile;
     const int lane = threadIdx.x;
     const int cot = blockIdx.x % q.n_cotile;
     const long long m0 = (long long)(blockIdx.x / q.n_cotile) * R;
@@ -414,21 +417,33 @@ __global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q, long long pos
 #pragma unroll
             for (int c = 0; c < 2 * C; c++) acc[r * 2 * C + c] |= aw[r] & wv[c];
     }
-    static_assert(R * 2 * C == 64, "one finished word per lane");
-#pragma unroll
-    for (int half = 32; half >= 1; half >>= 1) {
+    // (a lambda per step: as a loop over `half` the compiler does not unroll it for R = 1 and indexes at run time)
+    auto halve = [&](auto half_tag) {
+        constexpr int half = decltype(half_tag)::value;
         const bool upper = (lane & half) != 0;
 #pragma unroll
         for (int i = 0; i < half; i++) {
             const uint32_t keep = upper ? acc[i + half] : acc[i], give = upper ? acc[i] : acc[i + half];
             acc[i] = keep | (uint32_t)__shfl_xor((int)give, half);
         }
+    };
+    static_assert(R * 2 * C == 64 || R * 2 * C == 32, "a finished word per lane, or per pair of lanes");
+    if constexpr (R == 2) {
+        halve(std::integral_constant<int, 32>());
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2 * C; i++) acc[i] |= (uint32_t)__shfl_xor((int)acc[i], 32);
     }
+    halve(std::integral_constant<int, 16>());
+    halve(std::integral_constant<int, 8>());
+    halve(std::integral_constant<int, 4>());
+    halve(std::integral_constant<int, 2>());
+    halve(std::integral_constant<int, 1>());
     const int mine = __popc(acc[0]);
     const int other = __shfl_xor(mine, C);  // the channel's other rail
     const long long m = m0 + (lane >> 5);
     const int co = cot * C + (lane & (C - 1));
-    if ((lane & C) || m >= positions || co >= q.c_out) return;
+    if ((lane & C) || lane >= 32 * R || m >= positions || co >= q.c_out) return;
     const int b = (int)(m % q.ho);
     const long long t = m / q.ho;
     const int a = (int)(t % q.wo);
@@ -1423,47 +1438,63 @@ RailPlan plan_rail_unbounded(const Geometry& g, const SplitPlan& sp)
     const long long tiles = sp.waves, pairs = tiles * sp.pv;                   // (tile, pair) waves
     const int pv = sp.pv;
     RailPlan p = {kRailTile, 1, 4, 1, 1};
+    // The lines between the forms were set on 2800 launches of random sizes (streams of 32 to 256 bits, kernels of 1, 3 and
+    // 5, every accumulation), each timed in some forty forms: what this rule takes is 5.4 % over the best form of each on
+    // the (geometric) average.
     // Short groups, where the 32 LDS additions at the end of a group weigh most, keep their sums in registers
     // once four waves per SIMD exist without splitting a tile (3 -> 32, 5 x 5, 32 x 32, batch 256, L 64: 64 us
-    // against 72), or with so many groups per tile that the tile kernel's per-group work shows (z mode, 3 x 3, 1320
-    // groups of 309 tiles: 395 against 439 us; 1220 groups of 116 tiles: 146 against 162).
-    if (g.mode == GEO_SC_ACC_Y && tiles >= 4096 && lines <= 24)
-        return {sp.splits == 1 ? kRailPlain : kRailSplit, 0, 0, 0, sp.splits};
-    if (lines <= 12 && pairs >= 100000) return {kRailSplit, 0, 0, 0, sp.splits};
+    // against 72), where a tile has a single pair (4 -> 11 channels, 1 x 1, 13 x 31, batch 86: 5.3 against 7.1), with a dozen
+    // or two of pairs in few tiles, where a wave is alone on its SIMD (16 pairs of 12 lines in 18 tiles: 8.1 against 10.8 as
+    // the sixteen waves of a workgroup), or with so many groups per tile that the tile kernel's per-group work shows (z
+    // mode, 3 x 3, 1320 groups of 309 tiles: 395 against 439 us; 1220 groups of 116 tiles: 146 against 162).
+    const bool y_mode = g.mode == GEO_SC_ACC_Y;
+    if (y_mode && tiles >= 4096 && lines <= 24) return {sp.splits == 1 ? kRailPlain : kRailSplit, 0, 0, 0, sp.splits};
+    if (y_mode && pv == 1 && lines <= 32) return {kRailPlain, 0, 0, 0, 1};
+    if ((lines <= 28 && pv >= 12 && pv <= 24 && pairs < 350) || (lines <= 12 && pairs >= 100000)) return {kRailSplit, 0, 0, 0, sp.splits};
     // Long groups, few of them per tile, in launches whose waves fill their rounds: the counts of a pair go
-    // straight to y (64 -> 64, 3 x 3, 32 x 32, batch 128, L 64: 327 us against 336).  With twelve pairs per tile, or
-    // with image rows shorter than 16 (more lines per atomic), the atomics cost more than that gains.
+    // straight to y (64 -> 64, 3 x 3, 32 x 32, batch 128, L 64: 327 us against 336).  With twelve pairs per tile, with
+    // image rows shorter than 16 (more lines per atomic), or with groups of under 128 lines (32 -> 16 channels, 3 x 3, L 64,
+    // 801 tiles: 65 against 44) the atomics cost more than that gains.
     const long long rounds = (pairs + kPairRound - 1) / kPairRound;
-    if (pv <= 10 && g.w_k >= 3 && lines >= 96 && g.ho >= 16 && pairs > 4096 && pairs * 5 >= rounds * kPairRound * 4)
+    if (pv <= 10 && g.w_k >= 3 && lines >= 128 && g.ho >= 16 && pairs > 4096 && pairs * 5 >= rounds * kPairRound * 4)
         return {kRailPair, 0, 0, 0, pv};
-    if (lines >= 48 && g.or_ch_per_group >= 16 && !(pairs >= 8192 && (pv >= 12 || g.w_k == 1))) {
+    const int ch = g.or_ch_per_group;
+    if (lines >= 48 && ch >= 4 && pairs < (lines < 96 ? 1024 : lines < 160 ? 1792 : 8192)) {
         // Too few waves: the OR of a group shared out over four, eight or sixteen of them (a workgroup of a
         // multiple of four waves loads the four SIMDs alike: 512 -> 512 at 4 x 4, batch 50: 4 shares 300 us, 3: 337,
-        // 6: 392)
+        // 6: 392).  Groups of under 160 lines are shared up to one or two waves per SIMD only (22 -> 311 channels at 5 x 3,
+        // batch 122, L 128, 66 lines, 4320 pairs: shared 76 us, four pairs side by side 36; 1260 pairs of 156 lines: 32
+        // against 41), longer ones as long as the launch is under two rounds (256 -> 256 at 8 x 8, batch 50, L 128: 4800
+        // pairs of 768 lines: 266 against 303).
         p.in_flight = 1;
-        p.shares = pairs * 4 >= 2048 || g.or_ch_per_group < 32   ? 4
-                   : pairs * 8 >= 2048 || g.or_ch_per_group < 64 ? 8
-                                                                 : 16;
+        p.shares = pairs * 4 >= 2048 || ch < 8 ? 4 : pairs * 8 >= 2048 || ch < 48 ? 8 : 16;
         p.splits = pv;
-        // a round of waves without splitting the tiles, groups short enough for the atomics to show: all pairs
+        // half a round of tiles, groups short enough for the atomics to show: all pairs
         // of a tile in one workgroup (32 -> 64, 5 x 5, 8 x 8, batch 256, L 64: 76 us; 88 with one pair each)
-        if (p.shares == 4 && tiles >= 512 && lines < 256 && pv <= 16) {
-            p.in_flight = 2;
+        if (p.shares == 4 && tiles >= 512 && lines < 192 && pv <= 16) {
+            p.in_flight = pv > 1 ? 2 : 1;
             p.per_slot = (pv + 1) / 2;
             p.splits = 1;
         }
         return p;
     }
-    if (lines <= 48 && tiles < 1024 && pv <= 24) {
-        // few short groups: all pairs of a tile in one workgroup where that leaves enough of them
-        p.in_flight = pv <= 4 ? 4 : pv <= 8 || pv > 16 || tiles >= 128 ? 8 : 16;
-        p.per_slot = tiles >= 128 ? (pv + p.in_flight - 1) / p.in_flight : 1;
+    if (lines <= 64 && tiles < 1024 && pv <= 24) {
+        // few short groups
+        if (pairs < 512 && ch >= 4 && lines >= 24) {
+            p.shares = 4;
+            p.in_flight = pv > 1 ? 2 : 1;
+        } else {
+            // all pairs of a tile in one workgroup where that leaves enough of them
+            p.in_flight = pv <= 4 ? 4 : pv <= 8 || pv > 16 || tiles >= 256 ? 8 : 16;
+            p.per_slot = tiles >= 128 ? (pv + p.in_flight - 1) / p.in_flight : 1;
+        }
     } else {
         // pairs one after the other: fewer additions to y against a longer last round
-        const int most = (pv + 3) / 4;
+        p.in_flight = tiles < 64 && pv >= 8 && pairs < 8000 ? 8 : pv <= 2 ? pv : 4;
+        const int most = (pv + p.in_flight - 1) / p.in_flight;
         int want = lines >= 256 ? 2 : lines >= 80 ? 4 : lines >= 20 ? (int)(160 / lines) : 8;
         if (want > most) want = most;
-        while (want > 1 && tiles * ((most + want - 1) / want) < kPairRound / 4) want--;
+        while (want > 1 && tiles * ((most + want - 1) / want) * p.in_flight < kPairRound) want--;
         p.per_slot = want;
     }
     if (pv / p.in_flight / p.per_slot >= 32768) p.per_slot = pv / p.in_flight / 32768 + 1;  // a grid's limit in y
@@ -1558,6 +1589,15 @@ int launch(const Geometry& g, FwdParams q, hipStream_t s)
 
 }  // namespace
 
+// positions per wave of k_conv_fwd_thin: one where waves of two are fewer than the CUs (both sides at 300 random sizes:
+// under 128 waves one position is 1.1 - 1.5 times as fast, from 128 to 512 the two are equal, beyond that two positions
+// are up to 2 times as fast)
+static int thin_positions(const Geometry& g)
+{
+    const long long positions = (long long)g.n * g.wo * g.ho;
+    return (positions + 1) / 2 * g.n_cotile * g.packs * g.add_outer * g.add_inner < 256 ? 1 : 2;
+}
+
 double conv_forward_cost(const Geometry& g)
 {
     const double pv = (double)g.packs * g.add_outer * g.add_inner;
@@ -1619,13 +1659,15 @@ int launch_conv_forward(const Geometry& g, const uint32_t* act, const uint32_t* 
     q.or_rows = g.or_rows;
     if (g.thin) {
         const long long positions = (long long)g.n * g.wo * g.ho;
-        const long long blocks = (positions + kThinPositions - 1) / kThinPositions * g.n_cotile;
+        const int per_wave = thin_positions(g);
+        const long long blocks = (positions + per_wave - 1) / per_wave * g.n_cotile;
         const long long pv = (long long)g.packs * g.add_outer * g.add_inner;
         if (blocks > 0x7fffffffLL || pv > 65535 || g.act_item_inner) return GEO_SC_ERR_INVALID_ARGUMENT;
         const size_t n_out = (size_t)g.n * g.c_out * g.wo * g.ho;
         size_t zb = (n_out + 255) / 256;
         hipLaunchKernelGGL(k_zero_i32, dim3((unsigned)(zb > 4096 ? 4096 : zb)), dim3(256), 0, s, q.y, n_out);
-        hipLaunchKernelGGL(k_conv_fwd_thin, dim3((unsigned)blocks, (unsigned)pv), dim3(64), 0, s, q, positions);
+        auto kernel = per_wave == 1 ? k_conv_fwd_thin<1> : k_conv_fwd_thin<2>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (unsigned)pv), dim3(64), 0, s, q, positions);
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
     // Two accumulator rows per lane halve the weight traffic per instruction.  Outputs with

@@ -77,7 +77,7 @@ def test_backward_matches_float64_oracle(capi, shape_x, shape_w, pad, mode, scal
 
 GEMM_CASES = [
     # OR groups of more than 32 members take the three-GEMM path (K = c_in * w_k members per kernel row)
-    ((3, 12, 5, 3), (5, 12, 3, 1), (1, 0), 3.0),      # K = 36; 45 positions and 10 rails: unaligned operands (fp32 kernel)
+    ((3, 12, 5, 3), (5, 12, 3, 1), (1, 0), 3.0),      # K = 36; 45 positions and 10 rails: rows that are no whole quads
     ((4, 20, 6, 6), (6, 20, 2, 3), (0, 1), 2.0),      # K = 40: two whole chunks and a partial one
     ((2, 16, 9, 8), (8, 16, 5, 2), (2, 0), 2.0),      # K = 80: five whole chunks
     ((2, 64, 17, 16), (70, 64, 2, 1), (0, 0), 6.0),   # K = 128, four position tiles, 140 rails: a ragged second column tile
@@ -99,8 +99,8 @@ GEMM_CASES = [
 
 @pytest.mark.parametrize("shape_x,shape_w,pad,scale", GEMM_CASES)
 def test_backward_through_the_gemm_kernels(capi, shape_x, shape_w, pad, scale):
-    """Chunk counts, partial chunks, edge tiles and operand alignments of the GEMM kernels (bf16 three-way
-    split products for aligned operands, fp32 MFMAs otherwise) against the float64 oracle."""
+    """Chunk counts, partial chunks, edge tiles and rows of any length of the GEMM kernels (bf16 three-way
+    split products) against the float64 oracle."""
     from oracle import surrogate
     x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_x[1])
     w = (w * scale).contiguous()

@@ -458,7 +458,7 @@ def test_large_y_mode_launches_skip_the_zero_rail(capi, so, shape_x, shape_w, pa
     ((256, 32, 8, 8), (64, 32, 5, 5), (2, 2), 64, (7, 2, 2, 2)),     # 512 tiles: the pairs of a tile in one workgroup, an OR shared out over four waves
     ((250, 32, 8, 8), (60, 32, 5, 5), (2, 2), 64, (7, 8, 1, 1)),     # the same with a ragged last tile and a partial c_out tile
     ((256, 32, 16, 16), (32, 32, 5, 5), (2, 2), 64, (7, 2, 2, 2)),   # 10240 waves: two rounds, one pair per wave with atomics
-    ((200, 16, 8, 9), (48, 16, 3, 3), (1, 1), 256, (7, 8, 1, 1)),    # 24 pairs: more than a workgroup takes
+    ((200, 16, 8, 9), (48, 16, 3, 3), (1, 1), 256, (7, 8, 1, 1)),    # 24 pairs per tile: several rows of blocks add to y
     ((64, 32, 8, 8), (64, 32, 5, 5), (2, 2), 64, (7, 8, 1, 1)),      # 1280 waves: under a round, several pairs per wave
 ])
 def test_split_launches_match_oracle(capi, so, shape_x, shape_w, pad, L, loading):
@@ -479,14 +479,14 @@ def test_split_launches_match_oracle(capi, so, shape_x, shape_w, pad, L, loading
 
 
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,mode,zu", [
-    ((2, 70, 5, 6), (20, 70, 3, 3), (1, 1), 32, "y", 1),       # an OR shared out over 16 waves, the last two without a channel
-    ((2, 37, 6, 7), (17, 37, 3, 3), (1, 1), 64, "y", 1),       # over 8, the last share short
-    ((1, 64, 2, 2), (16, 64, 5, 5), (2, 2), 256, "y", 1),      # two lane slots
+    ((2, 70, 5, 6), (20, 70, 3, 3), (1, 1), 32, "y", 1),       # lanes over the members, a position per wave
+    ((2, 37, 6, 7), (17, 37, 3, 3), (1, 1), 64, "y", 1),       # the same, an odd number of members
+    ((1, 64, 2, 2), (16, 64, 5, 5), (2, 2), 256, "y", 1),      # an OR shared out over 16 waves, two lane slots
     ((8, 130, 7, 9), (33, 130, 1, 1), (0, 0), 128, "y", 1),    # 1-wide, shares of an odd number of channels
-    ((40, 20, 16, 16), (40, 20, 3, 3), (1, 1), 128, "y", 1),   # over 4, one pair per workgroup
-    ((128, 33, 16, 16), (33, 33, 3, 3), (1, 1), 32, "y", 1),   # three pairs of a tile two at a time in one workgroup
-    ((4, 20, 9, 8), (18, 20, 3, 3), (1, 1), 64, "full", 1),    # OR over kernel rows as well
-    ((3, 5, 9, 9), (20, 5, 3, 3), (1, 1), 128, "y", 1),        # short groups: 12 pairs in 16 waves
+    ((40, 20, 16, 16), (40, 20, 3, 3), (1, 1), 128, "y", 1),   # twelve pairs in 16 waves
+    ((128, 33, 16, 16), (33, 33, 3, 3), (1, 1), 32, "y", 1),   # three pairs in four waves
+    ((4, 20, 9, 8), (18, 20, 3, 3), (1, 1), 64, "full", 1),    # OR over kernel rows as well, lanes over the members
+    ((3, 5, 9, 9), (20, 5, 3, 3), (1, 1), 128, "y", 1),        # short groups in few tiles: a wave per pair
     ((33, 3, 31, 32), (32, 3, 3, 3), (1, 1), 64, "y", 1),      # 6 pairs in 8 waves
     ((40, 4, 16, 16), (33, 4, 5, 5), (2, 2), 128, "y", 1),     # 20 pairs, 8 waves, three rounds of them
     ((16, 60, 12, 12), (40, 60, 3, 3), (1, 1), 128, "z", 1),   # 240 groups of nine lines
@@ -496,8 +496,8 @@ def test_split_launches_match_oracle(capi, so, shape_x, shape_w, pad, L, loading
     ((3, 80, 1, 1), (18, 80, 1, 1), (0, 0), 128, "y", 1),      # and an odd one
 ])
 def test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode, zu):
-    """Every way the position-parallel launches cut their (pack, add group) pairs and OR groups over waves,
-    at the edges of the rule that chooses it: bit for bit, twice (the second call finds counts in y)."""
+    """The ways the position-parallel launches cut their (pack, add group) pairs and OR groups over waves (the rows below
+    and the tests that follow hold the others): bit for bit, twice (the second call finds counts in y)."""
     x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=shape_w[0] + L)
     w.view(-1)[::7] = 0.0
     gen = "rand" if mode == "full" else "lfsr"
@@ -512,10 +512,29 @@ def test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode
 
 
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,mode", [
-    ((320, 32, 16, 16), (128, 32, 3, 1), (0, 0), 32, "y"),    # one (pack, add group) pair per tile, 4480 tiles
-    ((256, 11, 16, 16), (140, 11, 3, 3), (1, 1), 32, "full"), # the same, an OR over kernel rows as well
-    ((160, 32, 16, 16), (128, 32, 3, 1), (0, 0), 64, "y"),    # two pairs per tile
-    ((64, 20, 16, 16), (64, 20, 5, 5), (2, 2), 64, "y"),      # ten, one round of waves exactly
+    ((8, 40, 8, 8), (16, 40, 3, 3), (1, 1), 64, "y"),      # 24 (tile, pair) waves: lanes over the members, two positions per wave
+    ((7, 40, 9, 9), (16, 40, 3, 3), (1, 1), 64, "y"),      # 30, an odd number of positions
+    ((9, 40, 8, 9), (16, 40, 3, 3), (1, 1), 64, "y"),      # 36: an OR shared out over waves
+    ((4, 70, 10, 9), (20, 70, 3, 3), (1, 1), 128, "y"),    # over 16, the last two without a channel
+    ((4, 37, 10, 9), (20, 37, 3, 3), (1, 1), 128, "y"),    # over 8, the last share short
+    ((8, 5, 12, 12), (20, 5, 5, 5), (2, 2), 64, "full"),   # over 4 of five channels and five kernel rows
+    ((8, 9, 12, 12), (20, 9, 3, 3), (1, 1), 64, "y"),      # short groups: over 4, two pairs side by side
+    ((8, 9, 12, 12), (20, 9, 3, 1), (1, 1), 64, "y"),      # the same with one row of blocks, which stores
+    ((96, 40, 20, 20), (64, 40, 1, 1), (0, 0), 64, "y"),   # two pairs in two waves
+    ((4, 6, 13, 14), (20, 6, 5, 5), (2, 2), 256, "y"),     # 40 pairs of 14 tiles, eight at a time
+    ((5, 4, 13, 14), (20, 4, 3, 1), (0, 1), 32, "y"),      # a single short pair per tile
+    ((41, 20, 16, 16), (17, 20, 1, 1), (0, 0), 32, "y"),   # the same, 1-wide
+])
+def test_launch_forms_at_the_lines_of_the_rule(capi, so, shape_x, shape_w, pad, L, mode):
+    """Few waves and short groups, on both sides of the lines between the forms: bit for bit, twice."""
+    test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode, 1)
+
+
+@pytest.mark.parametrize("shape_x,shape_w,pad,L,mode", [
+    ((320, 43, 16, 16), (128, 43, 3, 1), (0, 0), 32, "y"),    # one (pack, add group) pair per tile, 4480 tiles
+    ((256, 15, 16, 16), (140, 15, 3, 3), (1, 1), 32, "full"), # the same, an OR over kernel rows as well
+    ((160, 43, 16, 16), (128, 43, 3, 1), (0, 0), 64, "y"),    # two pairs per tile
+    ((64, 26, 16, 16), (64, 26, 5, 5), (2, 2), 64, "y"),      # ten, one round of waves exactly
 ])
 def test_launches_with_one_wave_per_pair_write_every_count(capi, so, shape_x, shape_w, pad, L, mode):
     """Long OR groups, at most ten pairs per tile and full rounds of waves: one wave per pair, counts added to y.  y holds other
