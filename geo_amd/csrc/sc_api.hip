@@ -93,19 +93,22 @@ int make_geometry(const geo_sc_conv_desc* d, Geometry* g)
     }
     g->seed_wrap = g->mode == GEO_SC_ACC_YZ ? (size_t)g->z_unit * wi * hi : (size_t)plane;
     {
-        // Lanes over the members of an OR group instead of over output positions, where positions are too few.
+        // Lanes over the members of an OR group instead of over output positions, where positions are too few; members
+        // of one OR group against the 64 lanes.
         // Launches that share an OR group out over waves (two output rows per lane, rail-packed weights, stream buffers
-        // under 4 GiB) need fewer of them: with under 32 (tile, pair) waves the lanes over members take 0.4 - 0.9 of
-        // their time, with 64 to 128 already 1 - 3 times it.  The others (outputs with a single row, other kernel widths):
-        // waves the position-parallel kernel could start at most (one (pack, add group) pair per wave) against the
-        // 1024 SIMDs.  Members of one OR group against the 64 lanes
-        const long long pairs = (long long)g->n_cotile * g->packs * g->add_outer * g->add_inner;
+        // under 4 GiB) need it with fewer than 48 (tile, pair) waves whose work is under 6000 steps of 64 members (a step is
+        // for two positions): 0.75 of the best other form's time on the average of 169 random sizes, 9 of them over 1.05;
+        // with more steps in as many waves up to 2.2 times it.  The others (outputs with a single row, other kernel
+        // widths): waves the position-parallel kernel could start at most (one (pack, add group) pair per wave) against
+        // the 1024 SIMDs.
+        const long long positions = (long long)d->n * wo * ho;
+        const long long pairs = (long long)g->n_cotile * g->packs * g->add_outer * g->add_inner;  // per tile of 64 slots
         const long long members = (long long)g->or_rows * g->or_ch_per_group * d->w_k;
         const bool shared_or = wo >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5) &&
                                (unsigned long long)g->act_words * 4 < 0xffffffffull;
-        const long long waves = shared_or ? ((long long)d->n * ((wo + 1) / 2) * ho + 63) / 64 * pairs
-                                          : ((long long)d->n * wo * ho + 63) / 64 * pairs;
-        g->thin = members >= 64 && waves < (shared_or ? 32 : 2048);
+        g->thin = members >= 64 && (shared_or ? ((long long)d->n * ((wo + 1) / 2) * ho + 63) / 64 * pairs < 48 &&
+                                                    (positions + 1) / 2 * pairs * ((members + 63) / 64) < 6000
+                                              : (positions + 63) / 64 * pairs < 2048);
     }
     g->act_item_inner = !g->thin && g->mode == GEO_SC_ACC_Y && g->generator == GEO_SC_GEN_LFSR && wo == 1 && d->n >= 2 && (d->w_k == 1 || d->w_k == 3 || d->w_k == 5) &&
                         (unsigned long long)g->act_words * 4 < 0xffffffffull;  // its kernel addresses the buffer with 32-bit byte offsets

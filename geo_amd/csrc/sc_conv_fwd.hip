@@ -1459,13 +1459,13 @@ RailPlan plan_rail_unbounded(const Geometry& g, const SplitPlan& sp)
     if (pv <= 10 && g.w_k >= 3 && lines >= 128 && g.ho >= 16 && pairs > 4096 && pairs * 5 >= rounds * kPairRound * 4)
         return {kRailPair, 0, 0, 0, pv};
     const int ch = g.or_ch_per_group;
-    if (lines >= 48 && ch >= 4 && pairs < (lines < 96 ? 1024 : lines < 160 ? 1792 : 8192)) {
+    if (lines >= 48 && ch >= 4 && pairs < (lines < 96 ? 1024 : lines < 160 ? 1792 : lines >= 256 && pv <= 8 && g.w_k >= 3 ? 11000 : 8192)) {
         // Too few waves: the OR of a group shared out over four, eight or sixteen of them (a workgroup of a
         // multiple of four waves loads the four SIMDs alike: 512 -> 512 at 4 x 4, batch 50: 4 shares 300 us, 3: 337,
         // 6: 392).  Groups of under 160 lines are shared up to one or two waves per SIMD only (22 -> 311 channels at 5 x 3,
         // batch 122, L 128, 66 lines, 4320 pairs: shared 76 us, four pairs side by side 36; 1260 pairs of 156 lines: 32
         // against 41), longer ones as long as the launch is under two rounds (256 -> 256 at 8 x 8, batch 50, L 128: 4800
-        // pairs of 768 lines: 266 against 303).
+        // pairs of 768 lines: 266 against 303; 193 -> 360 at 9 x 9, batch 87, L 64: 8556 pairs of 579 lines: 356 against 494).
         p.in_flight = 1;
         p.shares = pairs * 4 >= 2048 || ch < 8 ? 4 : pairs * 8 >= 2048 || ch < 48 ? 8 : 16;
         p.splits = pv;

@@ -481,7 +481,7 @@ def test_split_launches_match_oracle(capi, so, shape_x, shape_w, pad, L, loading
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,mode,zu", [
     ((2, 70, 5, 6), (20, 70, 3, 3), (1, 1), 32, "y", 1),       # lanes over the members, a position per wave
     ((2, 37, 6, 7), (17, 37, 3, 3), (1, 1), 64, "y", 1),       # the same, an odd number of members
-    ((1, 64, 2, 2), (16, 64, 5, 5), (2, 2), 256, "y", 1),      # an OR shared out over 16 waves, two lane slots
+    ((1, 64, 2, 2), (16, 64, 5, 5), (2, 2), 256, "y", 1),      # the same, four positions
     ((8, 130, 7, 9), (33, 130, 1, 1), (0, 0), 128, "y", 1),    # 1-wide, shares of an odd number of channels
     ((40, 20, 16, 16), (40, 20, 3, 3), (1, 1), 128, "y", 1),   # twelve pairs in 16 waves
     ((128, 33, 16, 16), (33, 33, 3, 3), (1, 1), 32, "y", 1),   # three pairs in four waves
@@ -512,12 +512,13 @@ def test_rail_launch_forms_match_oracle(capi, so, shape_x, shape_w, pad, L, mode
 
 
 @pytest.mark.parametrize("shape_x,shape_w,pad,L,mode", [
-    ((8, 40, 8, 8), (16, 40, 3, 3), (1, 1), 64, "y"),      # 24 (tile, pair) waves: lanes over the members, two positions per wave
+    ((8, 40, 8, 8), (16, 40, 3, 3), (1, 1), 64, "y"),      # 24 (tile, pair) waves: lanes over the members, two positions to a wave
     ((7, 40, 9, 9), (16, 40, 3, 3), (1, 1), 64, "y"),      # 30, an odd number of positions
-    ((9, 40, 8, 9), (16, 40, 3, 3), (1, 1), 64, "y"),      # 36: an OR shared out over waves
+    ((14, 40, 8, 9), (16, 40, 3, 3), (1, 1), 64, "y"),     # 48: an OR shared out over waves
+    ((5, 200, 8, 8), (16, 200, 3, 3), (1, 1), 64, "y"),    # 18 with many members: the same
     ((4, 70, 10, 9), (20, 70, 3, 3), (1, 1), 128, "y"),    # over 16, the last two without a channel
     ((4, 37, 10, 9), (20, 37, 3, 3), (1, 1), 128, "y"),    # over 8, the last share short
-    ((8, 5, 12, 12), (20, 5, 5, 5), (2, 2), 64, "full"),   # over 4 of five channels and five kernel rows
+    ((24, 5, 12, 12), (20, 5, 5, 5), (2, 2), 64, "full"),  # over 4 of five channels and five kernel rows
     ((8, 9, 12, 12), (20, 9, 3, 3), (1, 1), 64, "y"),      # short groups: over 4, two pairs side by side
     ((8, 9, 12, 12), (20, 9, 3, 1), (1, 1), 64, "y"),      # the same with one row of blocks, which stores
     ((96, 40, 20, 20), (64, 40, 1, 1), (0, 0), 64, "y"),   # two pairs in two waves
