@@ -354,16 +354,17 @@ __global__ __launch_bounds__(64) void k_conv_fwd_split(FwdParams q)
 }
 
 // Layers with few output positions and large OR groups (classifier layers: 64 x 4 x 4 -> 10 at
-// batch 256 has 2560 outputs of 1024 products each): one wave per (two output positions, c_out tile,
+// batch 256 has 2560 outputs of 1024 products each): one wave per (R output positions, c_out tile,
 // pack, add group); the lanes run over the members of the OR group, each with its own weight
-// line in VGPRs (read once for both positions), and the 2 x 32 partial OR words are combined across the
+// line in VGPRs (read once for all R positions), and the R x 32 partial OR words are combined across the
 // wave by halving: in the step of lane bit k every lane hands the half of its words that its partner
-// keeps to that partner, so 32 + 16 + 8 + 4 + 2 + 1 shuffles leave one finished word per lane (bit 5: position,
-// bit 4: rail, bits 3 - 0: channel) where a full xor reduction of every word takes 64 x 6.
+// keeps to that partner, so with R = 2 32 + 16 + 8 + 4 + 2 + 1 shuffles leave one finished word per lane (bit 5:
+// position, bit 4: rail, bits 3 - 0: channel) where a full xor reduction of every word takes 64 x 6.  With R = 1 the
+// two half waves are ORed first (32 shuffles) and then hold the same words.
 // Results are added into the zeroed y with integer atomics.  Activation layout [n][P][c_in][wi][hi].
-// R positions per wave: two, with fewer than a wave per CU one (the halving then starts with an OR of the two half waves):
-// bound by the latency of a wave's loads and shuffles there, 206 -> 45 channels, full OR over 3 x 3, four positions: 25.6
-// us with two, 17.2 with one; from two waves per SIMD on two positions take half the time.
+// Bound by the latency of a wave's loads and shuffles, so with few waves R = 1 (see thin_positions).  64 x 4 x 4 -> 10,
+// against one position and a full reduction per wave: batch 256, L 64: 15.9 -> 10.7 us, L 128: 24.2 -> 14.7 (R = 2); one
+// image, L 128: 7.6 -> 6.4 (7.9 with R = 2), batch 16: 8.1 -> 7.0 (8.3).
 template <int R>
 __global__ __launch_bounds__(64) void k_conv_fwd_thin(FwdParams q, long long positions)
 {
@@ -926,8 +927,8 @@ void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
 // The kernel of most launches: a workgroup owns one tile (64 lane slots x 16 channels) and works on
 // blockDim / (64 or_shares) pairs at a time, `or_shares` waves to a pair, `pairs_per_slot` pairs one after the other.
 // Bound by the issue rate of v_and_or_b32 where the launch fills the GPU; what decides then is the number of
-// waves a SIMD can choose from, as every wave waits ~1800 cycles for its channel's words and weight lines and
-// then issues 96 (3 lines) x 4.4 cycles: the counts are summed in LDS (ds_add_u32) instead of in 32 registers, so
+// waves a SIMD can choose from, as every wave waits for its channel's words and weight lines before it can issue
+// their 96 and-ors (3 lines): the counts are summed in LDS (ds_add_u32) instead of in 32 registers, so
 // that five waves fit a SIMD.  128 -> 128 channels, 3 x 3, 16 x 16, batch 256, L 128: 1.155 ms; with the sums in
 // registers (four waves) 1.38, and 1.29 with the activation words of four c_out tiles staged through LDS besides,
 // which this kernel replaced; 64 -> 64 at 56 x 56, L 256, batch 30: 0.95 -> 0.87.
