@@ -266,6 +266,34 @@ def test_eval_batch_norm_kernel_in_place_and_over_2048_workgroups(capi):
         capi.bn_fixed_eval(torch.zeros(1, 4097, 1, 1, device="cuda"), *([torch.ones(4097, device="cuda")] * 4), 1e-5)
 
 
+@pytest.mark.parametrize("c", [1, 700, 4096])
+def test_eval_batch_norm_in_a_captured_graph(c):
+    """Every replay reads what its input, weights and statistics hold then; eager work in between."""
+    from geo_amd import utils_class
+    g = torch.Generator(device="cuda").manual_seed(c)
+    bn = utils_class.BatchNorm2d_fixed(c).cuda().eval()
+    x = torch.rand((3, c, 4, 5), generator=g, device="cuda")
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            bn(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = bn(x)
+            scale = bn.scale
+        for _ in range(4):
+            x.copy_(torch.rand(x.shape, generator=g, device="cuda") - 0.5)
+            for t in (bn.weight, bn.bias, bn.running_mean, bn.running_var):
+                t.copy_(torch.rand(c, generator=g, device="cuda") * 3 + 0.1)
+            graph.replay()
+            got, got_scale = y.clone(), scale.clone()
+            exp = bn(x)
+            assert torch.equal(got, exp) and torch.equal(got_scale, bn.scale)
+            torch.cuda.synchronize()
+
+
 def test_eval_batch_norm_leaves_transforms_modes_and_subclasses_to_the_op_chain(monkeypatch):
     """Whatever looks at the operations themselves sees them: forward-mode tangents, tracing, function transforms, dispatch
     and function modes, tensor subclasses, views whose values are not what lies in memory."""
