@@ -46,8 +46,8 @@ struct Geometry {
     size_t act_words;    // n * packs * act_plane
     // Weight stream buffer: lines [packs][h_k][k_or][n_cotile] of 2 x kCoTile words (both rails), then,
     // with rail, the same lines once more in the rail-packed form the plain y-mode kernel reads:
-    // at wgt_rail_off kCoTile words per line (the non-zero rail's word), at wgt_rail_idx_off
-    // kCoTile / 2 words per line (16 bits per channel: which rail), both ordered [n_cotile][line]
+    // at wgt_rail_off kCoTile words per line (the non-zero rail's word, zero words in front), at wgt_rail_idx_off
+    // kCoTile / 2 words per line (16 bits per word: rail_field), both ordered [n_cotile][line]
     // with wgt_rail_lines lines per tile.
     // Behind the rail-packed copy: wgt_flag_off, one word that the packing kernel sets when a caller's
     // line carries two non-zero rails for one channel (which the rail-packed form cannot hold), then
@@ -59,6 +59,35 @@ struct Geometry {
     // property of the weights' shape alone); rail: this geometry's launch reads it.
     bool wgt_rail, rail;
 };
+
+// A rail-packed line holds its 16 channels with the zero words in front, in channel order on either side; live: bit c set
+// where channel c's word is not zero.  A wave that accumulates the line jumps over the zero words.
+__device__ __forceinline__ int rail_slot(uint32_t live, int c)
+{
+    const uint32_t below = (1u << c) - 1u;
+    return (live >> c) & 1u ? kCoTile - __popc(live >> c) : __popc(~live & below);
+}
+// The 16-bit field of channel c at slot `at`: bits 7:0 the register offset of its accumulators (2 c for the positive rail and
+// for zero weights, 32 + 2 c for the negative one), bits 15:12 the SRC2 and DST enables of the VGPR index mode.  But for four
+// slots, whose bits 15:8 or 11:8 say how a wave reads the line (index mode ignores bits 11:8 of M0, and the kernels set
+// the enables of slots 0 and 8 themselves):
+//   slot 0, 15:8: five times the zero words to jump over (at most 15) in the line, or in its left half where that has others;
+//   slot 1, 11:8: the line's zero words, at most 15;
+//   slot 8, 15:8: five times the zero words to jump over in the right half (at most 7);
+//   slot 9, 8   : 1 where the left half holds words that are not zero.
+// (Five: a slot's code is five words long.  A line or half without any other ORs one zero word.)
+__device__ __forceinline__ uint32_t rail_field(uint32_t live, int at, int c, bool negative)
+{
+    constexpr int H = kCoTile / 2;
+    const int zeros = min(kCoTile - __popc(live), kCoTile - 1);
+    uint32_t high = 0xC0u;
+    if (at == 0) high = 5u * (uint32_t)zeros;
+    if (at == 1) high |= (uint32_t)zeros;
+    if (at == H) high = zeros < H ? 0u : 5u * (uint32_t)(zeros - H);
+    if (at == H + 1) high |= zeros < H ? 1u : 0u;
+    return high << 8 | ((negative ? 2u * kCoTile : 0u) + 2u * (uint32_t)c);
+}
+static_assert(kCoTile == 16, "rail-packed lines hold 16 channels");
 
 // Stream tables (one per stream length, constant data of the code object):
 //   posp1[r], r < L-1 : 1 + index in the LFSR cycle of state r+1  (cycle[0] = 1)
@@ -99,13 +128,8 @@ double conv_forward_cost(const Geometry& g);
 // fills the rail-packed part of a weight stream buffer from its two-rail lines (no-op unless g.wgt_rail;
 // with from_generator also where launch_weight_streams has written that part itself)
 int launch_rail_pack(const Geometry& g, uint32_t* wgt, hipStream_t s, bool from_generator);
-// the LFSR weight generators of the y-mode line order write the rail-packed copy (and clear the flag area)
-// themselves; kernels long in dim 3 take the row-chunked one
-inline bool generator_packs_rails(const Geometry& g)
-{
-    return g.generator == GEO_SC_GEN_LFSR && (g.mode == GEO_SC_ACC_Y || g.mode == GEO_SC_ACC_FULL);
-}
-inline bool weight_rows_generator(const Geometry& g) { return generator_packs_rails(g) && g.h_k >= 16; }
+// the LFSR weight generator writes the rail-packed copy (and clears the flag area) itself
+inline bool generator_packs_rails(const Geometry& g) { return g.generator == GEO_SC_GEN_LFSR; }
 size_t backward_workspace_bytes(const Geometry& g, int groups_per_round);
 // GEO_SC_ERR_WORKSPACE when workspace_bytes is below backward_workspace_bytes(g, groups_per_round)
 int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x, const float* w, const float* gy,

@@ -480,6 +480,8 @@ typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 // M0 of a channel from its 16-bit field: index in bits 7:0, the SRC2 and DST enables in bits 15:12
 #define GEO_SC_RAIL_LO(I) "s_and_b32 m0, %[" I "], 0xffff\n"
 #define GEO_SC_RAIL_HI(I) "s_lshr_b32 m0, %[" I "], 16\n"
+// slots 0 and 8: bits 15:8 of their fields are not the enables (rail_field)
+#define GEO_SC_RAIL_ON(I) "s_set_gpr_idx_on %[" I "], gpr_idx(SRC2,DST)\n"
 #define GEO_SC_RAIL_OPERANDS                                                                                           \
     [w0] "s"(w[0]), [w1] "s"(w[1]), [w2] "s"(w[2]), [w3] "s"(w[3]), [w4] "s"(w[4]), [w5] "s"(w[5]), [w6] "s"(w[6]),     \
         [w7] "s"(w[7]), [w8] "s"(w[8]), [w9] "s"(w[9]), [w10] "s"(w[10]), [w11] "s"(w[11]), [w12] "s"(w[12]),           \
@@ -489,7 +491,7 @@ typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 #define GEO_SC_RAIL_16(PAIR)                                                                                           \
     PAIR("w0", "") PAIR("w1", GEO_SC_RAIL_HI("i0")) PAIR("w2", GEO_SC_RAIL_LO("i1")) PAIR("w3", GEO_SC_RAIL_HI("i1"))   \
     PAIR("w4", GEO_SC_RAIL_LO("i2")) PAIR("w5", GEO_SC_RAIL_HI("i2")) PAIR("w6", GEO_SC_RAIL_LO("i3"))                  \
-    PAIR("w7", GEO_SC_RAIL_HI("i3")) PAIR("w8", GEO_SC_RAIL_LO("i4")) PAIR("w9", GEO_SC_RAIL_HI("i4"))                  \
+    PAIR("w7", GEO_SC_RAIL_HI("i3")) PAIR("w8", GEO_SC_RAIL_ON("i4")) PAIR("w9", GEO_SC_RAIL_HI("i4"))                  \
     PAIR("w10", GEO_SC_RAIL_LO("i5")) PAIR("w11", GEO_SC_RAIL_HI("i5")) PAIR("w12", GEO_SC_RAIL_LO("i6"))               \
     PAIR("w13", GEO_SC_RAIL_HI("i6")) PAIR("w14", GEO_SC_RAIL_LO("i7")) PAIR("w15", GEO_SC_RAIL_HI("i7"))
 
@@ -545,6 +547,7 @@ GEO_SC_DEFINE_RAIL_LINES(rail_line_lo, rail_line_first_lo, "v32", "v33", "v[32:4
 #undef GEO_SC_RAIL_16
 #undef GEO_SC_RAIL_OPERANDS
 #undef GEO_SC_RAIL_LO
+#undef GEO_SC_RAIL_ON
 #undef GEO_SC_RAIL_HI
 
 // sum += popcount(pos) - popcount(neg) in three instructions (the compiler's form takes four)
@@ -814,6 +817,287 @@ struct PairLane {
 // in the same loop the compiler reads a plain global pointer with vector loads.
 typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
 
+// ---- the OR of consecutive channels of an add group, as one asm block for 3- and 5-wide kernels ----
+// How many of a line's words are zero is a property of the weights: streams of a small code are mostly zero words (the initial
+// weights of a 64-channel layer at L 256: two thirds), and so are the channels that pad the last tile.  The channels
+// of a group go through one of three loops, picked by the zero words of the group's first lines:
+//   DENSE (fewer than kSkipZeros per line)  every word of a line;
+//   SKIP                                    a jump over the line's zero words, which its packing has put in front;
+//   HALF  (kHalfZeros or more)              only the right halves of the lines (slots 8 - 15) are loaded, so that two
+//                                           stages of lines fit the scalar registers and one is in flight while the other is
+//                                           ORed; the left half of a line with more than eight words is loaded where it is met.
+// What bounds them: DENSE the issue of v_and_or_b32; HALF the scalar instructions, one per SIMD and four cycles like
+// the vector ones, of which a line takes one per word and three for its jump.
+// One block with its loads and waits inside, registers assigned by hand: scalar loads return out of order, so only
+// lgkmcnt(0) says that a line has arrived and the next stage's loads must be issued behind that wait, an order that the
+// compiler does not keep; and 64 pinned accumulators that live across its branches it spills.
+// Scalar registers (s32 is the compiler's): DENSE and SKIP: words of three lines in s[36:51], s[52:67], s[68:83], their fields
+// in s[84:91], s[92:99], s[24:31].  HALF: words of stage A's three lines in s[36:59], of stage B's in s[60:83], fields in
+// s[84:95] and s[96:99], s[24:31]; addresses of the lines' first slots in s[18:23] (low) and vcc_hi (high).  s33: temporary;
+// s[34:35]: temporary, and the zero words of the first lines.
+// Index mode stays on between the loads of a channel and the next one's: nothing but the slots' vector instructions is issued.
+#define GEO_SC_SLOT(SET, W, I, X0, X1)                                                                                 \
+    SET "v_and_or_b32 v32, s[" #W "+" #I "], %[" X0 "], v32\n"                                                          \
+        "v_and_or_b32 v33, s[" #W "+" #I "], %[" X1 "], v33\n"
+#define GEO_SC_SLOT_FIRST(SET, W, I, X0, X1)                                                                           \
+    SET "v_and_b32 v32, s[" #W "+" #I "], %[" X0 "]\n"                                                                  \
+        "v_and_b32 v33, s[" #W "+" #I "], %[" X1 "]\n"                                                                  \
+        "s_xor_b32 m0, m0, 32\n"                                                                                       \
+        "v_mov_b32 v32, 0\n"                                                                                           \
+        "v_mov_b32 v33, 0\n"
+#define GEO_SC_M0_ON(F) "s_set_gpr_idx_on s[" #F "+0], gpr_idx(SRC2,DST)\n"
+#define GEO_SC_M0_LO(F, J) "s_mov_b32 m0, s[" #F "+" #J "]\n"
+#define GEO_SC_M0_HI(F, J) "s_lshr_b32 m0, s[" #F "+" #J "], 16\n"
+#define GEO_SC_EIGHT(SLOT, W, F, X0, X1)                                                                               \
+    SLOT(GEO_SC_M0_ON(F), W, 0, X0, X1) SLOT(GEO_SC_M0_HI(F, 0), W, 1, X0, X1)                                         \
+    SLOT(GEO_SC_M0_LO(F, 1), W, 2, X0, X1) SLOT(GEO_SC_M0_HI(F, 1), W, 3, X0, X1)                                      \
+    SLOT(GEO_SC_M0_LO(F, 2), W, 4, X0, X1) SLOT(GEO_SC_M0_HI(F, 2), W, 5, X0, X1)                                      \
+    SLOT(GEO_SC_M0_LO(F, 3), W, 6, X0, X1) SLOT(GEO_SC_M0_HI(F, 3), W, 7, X0, X1)
+#define GEO_SC_INDEX_ON "s_set_gpr_idx_on 0, gpr_idx(SRC2,DST)\n"
+#define GEO_SC_INDEX_OFF "s_set_gpr_idx_off\n"
+// Over zero words: a slot is five words of code, and bits 15:8 of the first field hold five times the zero words.
+// s_getpc_b64 gives the address of the s_lshl2_add_u32, three words in front of the first slot but one for s_addk_i32.
+#define GEO_SC_JUMP(F)                                                                                                 \
+    "s_bfe_u32 s33, s[" #F "+0], 0x80008\n"                                                                            \
+    "s_addk_i32 s33, 3\n"                                                                                              \
+    "s_getpc_b64 s[34:35]\n"                                                                                           \
+    "s_lshl2_add_u32 s34, s33, s34\n"                                                                                  \
+    "s_addc_u32 s35, s35, 0\n"                                                                                         \
+    "s_setpc_b64 s[34:35]\n"
+// the same with the address of the first slot in BASE and vcc_hi (GEO_SC_BASE; no carry between the slots)
+#define GEO_SC_JUMP_FROM(BASE, F)                                                                                      \
+    "s_bfe_u32 s33, s[" #F "+0], 0x80008\n"                                                                            \
+    "s_lshl2_add_u32 vcc_lo, s33, " BASE "\n"                                                                          \
+    "s_setpc_b64 vcc\n"
+#define GEO_SC_DENSE(W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W + 8, F + 4, X0, X1)
+#define GEO_SC_FIRST(W, F, X0, X1)                                                                                     \
+    GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W + 8, F + 4, X0, X1)
+#define GEO_SC_SKIP(W, F, X0, X1) GEO_SC_JUMP(F) GEO_SC_DENSE(W, F, X0, X1)
+// a line's right half; LABEL marks its first slot
+#define GEO_SC_HALF(LABEL, BASE, W, F, X0, X1)                                                                         \
+    GEO_SC_JUMP_FROM(BASE, F) ".Lsc_" LABEL "_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)
+#define GEO_SC_BASE(LABEL, BASE) "s_add_u32 " BASE ", vcc_lo, .Lsc_" LABEL "_%=-.Lsc_pc_%=\n"
+// Bit 24 of a line's fifth field word: its left half holds words too.  Lines of a stage with the flag, out of line:
+#define GEO_SC_ANY_LEFT2(LABEL, F0, F1)                                                                                \
+    "s_or_b32 s33, s[" #F0 "+0], s[" #F1 "+0]\n"                                                                       \
+    "s_bitcmp1_b32 s33, 24\n"                                                                                          \
+    "s_cbranch_scc1 .Lsc_" LABEL "_%=\n"                                                                               \
+    ".Lsc_" LABEL "_back_%=:\n"
+#define GEO_SC_ANY_LEFT3(LABEL, F0, F1, F2)                                                                            \
+    "s_or_b32 s33, s[" #F0 "+0], s[" #F1 "+0]\n"                                                                       \
+    "s_or_b32 s33, s33, s[" #F2 "+0]\n"                                                                                \
+    "s_bitcmp1_b32 s33, 24\n"                                                                                          \
+    "s_cbranch_scc1 .Lsc_" LABEL "_%=\n"                                                                               \
+    ".Lsc_" LABEL "_back_%=:\n"
+#define GEO_SC_LEFT(W, F, X0, X1, L)                                                                                   \
+    "s_bitcmp1_b32 s[" #F "+0], 24\n"                                                                                  \
+    "s_cbranch_scc0 2f\n"                                                                                              \
+    "s_lshr_b32 s33, %[wo], 1\n"                                                                                       \
+    "s_load_dwordx8 s[" #W ":" #W "+7], %[wp], %[wo] offset:64*" #L "\n"                                               \
+    "s_load_dwordx4 s[" #F ":" #F "+3], %[ip], s33 offset:32*" #L "\n"                                                 \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                           \
+    GEO_SC_JUMP(F) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                             \
+    "2:\n"
+// loads of line L of the channel AT bytes behind %[wo] (in the words; half of it in the fields, s33)
+#define GEO_SC_FIELD_OFFSET "s_lshr_b32 s33, %[wo], 1\n"
+#define GEO_SC_LOAD(W, F, L)                                                                                           \
+    "s_load_dwordx16 s[" #W ":" #W "+15], %[wp], %[wo] offset:64*" #L "\n"                                             \
+    "s_load_dwordx8 s[" #F ":" #F "+7], %[ip], s33 offset:32*" #L "\n"
+#define GEO_SC_LOAD_HALF(W, F, L, AT)                                                                                  \
+    "s_load_dwordx8 s[" #W ":" #W "+7], %[wp], %[wo] offset:" #AT "+64*" #L "+32\n"                                    \
+    "s_load_dwordx4 s[" #F ":" #F "+3], %[ip], s33 offset:" #AT "/2+32*" #L "+16\n"
+// (the next channel's line: not behind the last one)
+#define GEO_SC_LOAD_NEXT(W, F, L)                                                                                      \
+    "s_cmp_lt_u32 %[left], 2\n"                                                                                        \
+    "s_cbranch_scc1 1f\n"                                                                                              \
+    GEO_SC_FIELD_OFFSET GEO_SC_LOAD(W, F, L) "1:\n"
+#define GEO_SC_WAIT_ALL "s_waitcnt vmcnt(0) lgkmcnt(0)\n"
+#define GEO_SC_WAIT_LINES "s_waitcnt lgkmcnt(0)\n"
+#define GEO_SC_FETCH(X, V) "buffer_load_dword %[" X "], %[" V "], %[act], %[co] offen\n"
+#define GEO_SC_FETCH4(X) GEO_SC_FETCH(X "0", "v0") GEO_SC_FETCH(X "1", "v1") GEO_SC_FETCH(X "2", "v2") GEO_SC_FETCH(X "3", "v3")
+#define GEO_SC_FETCH6(X) GEO_SC_FETCH4(X) GEO_SC_FETCH(X "4", "v4") GEO_SC_FETCH(X "5", "v5")
+// to the next channel and its activation words, if there is one; B: bytes of a channel's lines
+#define GEO_SC_AHEAD(B, FETCHES)                                                                                       \
+    "s_cmp_lt_u32 %[left], 2\n"                                                                                        \
+    "s_cbranch_scc1 1f\n"                                                                                              \
+    "s_add_u32 %[co], %[co], %[orb]\n"                                                                                 \
+    "s_addk_i32 %[wo], " #B "\n"                                                                                       \
+    FETCHES "1:\n"
+#define GEO_SC_NEXT_OR_END                                                                                             \
+    "s_sub_u32 %[left], %[left], 1\n"                                                                                  \
+    "s_cmp_eq_u32 %[left], 0\n"                                                                                        \
+    "s_cbranch_scc1 99f\n"
+// One channel with its words in X, the next one's to Y.
+#define GEO_SC_CHANNEL3(LINE, X, Y)                                                                                    \
+    GEO_SC_WAIT_ALL GEO_SC_INDEX_OFF GEO_SC_AHEAD(192, GEO_SC_FETCH4(Y)) GEO_SC_INDEX_ON                               \
+    LINE(36, 84, X "0", X "1") GEO_SC_LOAD_NEXT(36, 84, 0)                                                             \
+    LINE(52, 92, X "1", X "2") GEO_SC_LOAD_NEXT(52, 92, 1)                                                             \
+    LINE(68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                             \
+    GEO_SC_NEXT_OR_END
+// (lines 3 and 4 take the place of lines 0 and 1)
+#define GEO_SC_CHANNEL5(LINE, X, Y)                                                                                    \
+    GEO_SC_WAIT_ALL GEO_SC_INDEX_ON                                                                                    \
+    LINE(36, 84, X "0", X "1") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3)                                              \
+    LINE(52, 92, X "1", X "2") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(52, 92, 4)                                              \
+    GEO_SC_INDEX_OFF GEO_SC_AHEAD(320, GEO_SC_FETCH6(Y)) GEO_SC_INDEX_ON                                               \
+    LINE(68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                             \
+    GEO_SC_WAIT_LINES                                                                                                  \
+    LINE(36, 84, X "3", X "4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                             \
+    LINE(52, 92, X "4", X "5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                             \
+    GEO_SC_NEXT_OR_END
+#define GEO_SC_LOOP(LABEL, CHANNEL, LINE, LOADS)                                                                       \
+    LABEL "0:\n" LOADS LABEL "1:\n" CHANNEL(LINE, "x", "y") CHANNEL(LINE, "y", "x") "s_branch " LABEL "1b\n"
+// the first lines' zero words (bits 27:24 of the first field word) pick the loop for the channels behind the first
+#define GEO_SC_COUNT_ZEROS                                                                                             \
+    "s_bfe_u32 s35, s84, 0x40018\n"                                                                                    \
+    "s_bfe_u32 s33, s92, 0x40018\n"                                                                                    \
+    "s_add_u32 s35, s35, s33\n"                                                                                        \
+    "s_bfe_u32 s33, s24, 0x40018\n"                                                                                    \
+    "s_add_u32 s35, s35, s33\n"
+#define GEO_SC_LOADS_FULL GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 0) GEO_SC_LOAD(52, 92, 1) GEO_SC_LOAD(68, 24, 2)
+#define GEO_SC_LOADS_HALF_A(AT)                                                                                        \
+    GEO_SC_LOAD_HALF(36, 84, 0, AT) GEO_SC_LOAD_HALF(44, 88, 1, AT) GEO_SC_LOAD_HALF(52, 92, 2, AT)
+// the first channel (its first line assigns where `row` is 0), then the loops
+#define GEO_SC_OR_CHANNELS(B, FETCHES, REST_OF_FIRST, CHANNEL, BASES, HALF_LOOP, LEFT_HALVES)                          \
+    "s_nop 4\n" /* the compiler may have written an operand of the loads with a vector instruction just before */      \
+    GEO_SC_LOADS_FULL FETCHES GEO_SC_WAIT_ALL GEO_SC_COUNT_ZEROS GEO_SC_INDEX_ON                                       \
+    "s_cmp_lg_u32 %[row], 0\n"                                                                                         \
+    "s_cbranch_scc1 3f\n"                                                                                              \
+    GEO_SC_FIRST(36, 84, "x0", "x1")                                                                                   \
+    "s_branch 4f\n"                                                                                                    \
+    "3:\n" GEO_SC_DENSE(36, 84, "x0", "x1") "4:\n"                                                                     \
+    GEO_SC_DENSE(52, 92, "x1", "x2") GEO_SC_DENSE(68, 24, "x2", "x3") REST_OF_FIRST                                    \
+    GEO_SC_NEXT_OR_END GEO_SC_INDEX_OFF                                                                                \
+    "s_add_u32 %[co], %[co], %[orb]\n"                                                                                 \
+    "s_addk_i32 %[wo], " #B "\n"                                                                                       \
+    FETCHES                                                                                                            \
+    "s_cmp_ge_u32 s35, %[zhalf]\n"                                                                                     \
+    "s_cbranch_scc1 30f\n"                                                                                             \
+    "s_cmp_ge_u32 s35, %[zskip]\n"                                                                                     \
+    "s_cbranch_scc1 20f\n"                                                                                             \
+    GEO_SC_LOOP("1", CHANNEL, GEO_SC_DENSE, GEO_SC_LOADS_FULL)                                                         \
+    GEO_SC_LOOP("2", CHANNEL, GEO_SC_SKIP, GEO_SC_LOADS_FULL)                                                          \
+    "30:\n"                                                                                                            \
+    "s_getpc_b64 vcc\n"                                                                                                \
+    ".Lsc_pc_%=:\n"                                                                                                    \
+    /* all slots between here and 99 in one 4 GB: a carry takes the other loop */                                      \
+    "s_add_u32 s33, vcc_lo, 99f-.Lsc_pc_%=\n"                                                                          \
+    "s_cbranch_scc1 20b\n"                                                                                             \
+    GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(0) BASES                                                                   \
+    "31:\n" HALF_LOOP LEFT_HALVES                                                                                      \
+    "99:\n" GEO_SC_INDEX_OFF
+#define GEO_SC_OR_OPERANDS                                                                                             \
+    [wp] "s"(wp), [ip] "s"(ip), [act] "s"(act), [orb] "s"(or_b), [row] "s"(row), [zskip] "n"(3 * kSkipZeros),          \
+        [zhalf] "n"(3 * kHalfZeros), [v0] "v"(voff[0]), [v1] "v"(voff[1]), [v2] "v"(voff[2]), [v3] "v"(voff[3])
+#define GEO_SC_OR_CLOBBERS                                                                                            \
+    "m0", "scc", "vcc", "memory", "s18", "s19", "s20", "s21", "s22", "s23", "s24", "s25", "s26", "s27", "s28",         \
+    "s29", "s30", "s31", "s33", "s34", "s35", "s36", "s37", "s38", "s39", "s40", "s41", "s42", "s43", "s44",           \
+    "s45", "s46", "s47", "s48", "s49", "s50", "s51", "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59",           \
+    "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74",           \
+    "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89",           \
+    "s90", "s91", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "s99"
+// Mean zero words per line from which the loops are taken.  Below two the jump costs what it saves (uniform weights: one
+// line in three has a zero word, and jumping over it took the 128 -> 128 layer at L 128 from 1.154 to 1.197 ms).  HALF from 7,
+// 9 or 11 zero words on: the 4-layer CNN at batch 256 562 / 566 / 583 us, 64 -> 64 at 56 x 56 (step, L 256) 4.36 / 4.37 / 4.42 ms.
+constexpr int kSkipZeros = 2, kHalfZeros = 7;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// chs >= 1 channels, the first at byte offset ch_off of the stream buffer `act`, or_b bytes apart; wp, ip: their lines.
+// row 0: the accumulators are assigned, otherwise added to.
+__device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigned (&voff)[4], unsigned ch_off, unsigned or_b,
+                                                 ConstWords wp, ConstWords ip, int chs, int row, u32x16& p0, u32x16& p1,
+                                                 u32x16& n0, u32x16& n1)
+{
+    uint32_t x0, x1, x2, x3, y0, y1, y2, y3;
+    unsigned wo = 0, left = (unsigned)chs;
+// even channels in stage A, odd ones in stage B; the next channel's lines to the other stage
+#define GEO_SC_HALF_CHANNEL3(LOADS, FETCHES)                                                                           \
+    GEO_SC_WAIT_ALL GEO_SC_INDEX_OFF                                                                                   \
+    "s_cmp_lt_u32 %[left], 2\n"                                                                                        \
+    "s_cbranch_scc1 1f\n"                                                                                              \
+    "s_add_u32 %[co], %[co], %[orb]\n"                                                                                 \
+    GEO_SC_FIELD_OFFSET LOADS FETCHES                                                                                  \
+    "1:\n" GEO_SC_INDEX_ON
+    asm volatile(
+        GEO_SC_OR_CHANNELS(192, GEO_SC_FETCH4("x"), "", GEO_SC_CHANNEL3,
+            GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
+            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22") GEO_SC_BASE("b2", "s23"),
+            GEO_SC_HALF_CHANNEL3(GEO_SC_LOAD_HALF(60, 96, 0, 192) GEO_SC_LOAD_HALF(68, 24, 1, 192)
+                                 GEO_SC_LOAD_HALF(76, 28, 2, 192), GEO_SC_FETCH4("y"))
+            GEO_SC_HALF("a0", "s18", 36, 84, "x0", "x1") GEO_SC_HALF("a1", "s19", 44, 88, "x1", "x2")
+            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3") GEO_SC_ANY_LEFT3("left_a", 84, 88, 92)
+            "s_addk_i32 %[wo], 192\n" GEO_SC_NEXT_OR_END
+            GEO_SC_HALF_CHANNEL3(GEO_SC_LOADS_HALF_A(192), GEO_SC_FETCH4("x"))
+            GEO_SC_HALF("b0", "s21", 60, 96, "y0", "y1") GEO_SC_HALF("b1", "s22", 68, 24, "y1", "y2")
+            GEO_SC_HALF("b2", "s23", 76, 28, "y2", "y3") GEO_SC_ANY_LEFT3("left_b", 96, 24, 28)
+            "s_addk_i32 %[wo], 192\n" GEO_SC_NEXT_OR_END
+            "s_branch 31b\n",
+            ".Lsc_left_a_%=:\n"
+            GEO_SC_LEFT(36, 84, "x0", "x1", 0) GEO_SC_LEFT(44, 88, "x1", "x2", 1) GEO_SC_LEFT(52, 92, "x2", "x3", 2)
+            "s_branch .Lsc_left_a_back_%=\n"
+            ".Lsc_left_b_%=:\n"
+            GEO_SC_LEFT(60, 96, "y0", "y1", 0) GEO_SC_LEFT(68, 24, "y1", "y2", 1) GEO_SC_LEFT(76, 28, "y2", "y3", 2)
+            "s_branch .Lsc_left_b_back_%=\n")
+        : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
+          [x2] "=&v"(x2), [x3] "=&v"(x3), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2), [y3] "=&v"(y3),
+          [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
+        : GEO_SC_OR_OPERANDS
+        : GEO_SC_OR_CLOBBERS);
+}
+
+__device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigned (&voff)[6], unsigned ch_off, unsigned or_b,
+                                                 ConstWords wp, ConstWords ip, int chs, int row, u32x16& p0, u32x16& p1,
+                                                 u32x16& n0, u32x16& n1)
+{
+    uint32_t x0, x1, x2, x3, x4, x5, y0, y1, y2, y3, y4, y5;
+    unsigned wo = 0, left = (unsigned)chs;
+    // HALF: lines 0 - 2 of a channel in stage A, lines 3 and 4 in stage B; the channel's words in x, the next one's to y
+    asm volatile(
+        GEO_SC_OR_CHANNELS(320, GEO_SC_FETCH6("x"),
+            GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3) GEO_SC_LOAD(52, 92, 4) GEO_SC_WAIT_LINES
+            GEO_SC_DENSE(36, 84, "x3", "x4") GEO_SC_DENSE(52, 92, "x4", "x5"),
+            GEO_SC_CHANNEL5,
+            GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
+            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22"),
+            GEO_SC_WAIT_ALL
+            GEO_SC_FIELD_OFFSET GEO_SC_LOAD_HALF(60, 96, 3, 0) GEO_SC_LOAD_HALF(68, 24, 4, 0)
+            "s_cmp_lt_u32 %[left], 2\n"
+            "s_cbranch_scc1 1f\n"
+            "s_add_u32 %[co], %[co], %[orb]\n"
+            GEO_SC_FETCH6("y")
+            "1:\n" GEO_SC_INDEX_ON
+            GEO_SC_HALF("a0", "s18", 36, 84, "x0", "x1") GEO_SC_HALF("a1", "s19", 44, 88, "x1", "x2")
+            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3") GEO_SC_ANY_LEFT3("left_a", 84, 88, 92)
+            GEO_SC_WAIT_LINES
+            "s_cmp_lt_u32 %[left], 2\n"
+            "s_cbranch_scc1 1f\n"
+            GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(320)
+            "1:\n"
+            GEO_SC_HALF("b0", "s21", 60, 96, "x3", "x4") GEO_SC_HALF("b1", "s22", 68, 24, "x4", "x5")
+            GEO_SC_ANY_LEFT2("left_b", 96, 24)
+            "s_addk_i32 %[wo], 320\n" GEO_SC_NEXT_OR_END
+            GEO_SC_INDEX_OFF
+            "s_waitcnt vmcnt(0)\n"
+            "v_mov_b32 %[x0], %[y0]\n"
+            "v_mov_b32 %[x1], %[y1]\n"
+            "v_mov_b32 %[x2], %[y2]\n"
+            "v_mov_b32 %[x3], %[y3]\n"
+            "v_mov_b32 %[x4], %[y4]\n"
+            "v_mov_b32 %[x5], %[y5]\n"
+            "s_branch 31b\n",
+            ".Lsc_left_a_%=:\n"
+            GEO_SC_LEFT(36, 84, "x0", "x1", 0) GEO_SC_LEFT(44, 88, "x1", "x2", 1) GEO_SC_LEFT(52, 92, "x2", "x3", 2)
+            "s_branch .Lsc_left_a_back_%=\n"
+            ".Lsc_left_b_%=:\n"
+            GEO_SC_LEFT(60, 96, "x3", "x4", 3) GEO_SC_LEFT(68, 24, "x4", "x5", 4)
+            "s_branch .Lsc_left_b_back_%=\n")
+        : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
+          [x2] "=&v"(x2), [x3] "=&v"(x3), [x4] "=&v"(x4), [x5] "=&v"(x5), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2),
+          [y3] "=&v"(y3), [y4] "=&v"(y4), [y5] "=&v"(y5), [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
+        : GEO_SC_OR_OPERANDS, [v4] "v"(voff[4]), [v5] "v"(voff[5])
+        : GEO_SC_OR_CLOBBERS);
+}
+
 // OR of one (pack, add group) pair over share `share` of `shares` of the group's channels, assigned to the
 // accumulators; false where the share has no channels (nothing is assigned then).
 template <int WK, int CU>
@@ -832,6 +1116,10 @@ __device__ __forceinline__ bool or_pair(const FwdParams& q, __amdgpu_buffer_rsrc
     const int chunk = (chs + shares - 1) / shares;
     const int c_begin = min(chs, chunk * share), c_end = min(chs, chunk * (share + 1));
     if (c_begin == c_end) return false;
+    // the buffer resource as words, for the asm blocks
+    const unsigned long long act_base = (unsigned long long)q.act;
+    const u32x4 act_words = {(uint32_t)act_base, (uint32_t)(act_base >> 32), 4u * (unsigned)q.n * (unsigned)q.packs * q.act_plane,
+                             0x00020000u};
     const size_t lines_per_pack = (size_t)q.or_rows * q.add_inner * q.or_ch_total * q.w_k;
     const size_t line = (size_t)cot * q.rail_lines + p * lines_per_pack + (size_t)ch0 * q.add_inner * q.w_k +
                         (size_t)gi * chs * q.w_k;
@@ -842,6 +1130,10 @@ __device__ __forceinline__ bool or_pair(const FwdParams& q, __amdgpu_buffer_rsrc
         ConstWords wp = (ConstWords)(q.wgt_rail + line_row * C);
         ConstWords ip = (ConstWords)(q.wgt_rail_idx + line_row * (C / 2));
         unsigned ch_off = group_off + 4u * (unsigned)row;  // next kernel row: one word further
+        if constexpr (WK == 3 || WK == 5) {
+            or_channels_rail(act_words, voff, ch_off, or_b, wp, ip, c_end - c_begin, row, p0, p1, n0, n1);
+            continue;
+        }
         auto channels_of = [&](auto cu_tag, auto first_tag) {
             constexpr int N = decltype(cu_tag)::value;
             constexpr bool FIRST = decltype(first_tag)::value;
@@ -1345,36 +1637,28 @@ void k_conv_fwd_items_rail_lds(FwdParams q)
     }
 }
 
-// Rail-packed weight lines from the two-rail lines [line][cot][2][16]: word = pos | neg (at most one
-// is non-zero), stored [cot][line][16]; per channel a 16-bit field with what the rail kernels move
-// into M0: bits 7:0 the register offset of the channel's accumulators, 2 c for the positive rail
-// (and for zero weights), 32 + 2 c for the negative one, bits 15:12 the SRC2 and DST enables of
-// the VGPR index mode; stored [cot][line][8].  One thread per (line, tile).
+// Rail-packed weight lines from the two-rail lines [line][cot][2][16]: word = pos | neg (at most one is non-zero), stored
+// [cot][line][slot] with the zero words in front, and a 16-bit field per slot with what the rail kernels move into M0 (rail_slot,
+// rail_field).  A thread per channel, so that a line is read and written by 16 consecutive lanes (random generator,
+// 17 -> 441 channels, 3 x 3, L 128: 5 us less than a thread per line).
 // `both` (one word, cleared by the launcher) is set when a channel of a line has two non-zero rails.
 __global__ __launch_bounds__(256) void k_rail_pack(const uint32_t* __restrict__ lines2, uint32_t* __restrict__ words,
-                                                   uint32_t* __restrict__ idx, size_t n_lines, int n_cotile,
+                                                   uint16_t* __restrict__ fields, size_t n_lines, int n_cotile,
                                                    uint32_t* __restrict__ both)
 {
     constexpr int C = kCoTile;
-    const size_t total = n_lines * n_cotile;
+    const size_t total = n_lines * n_cotile * C;  // whole lines: the lanes of a line take every step together
+    const int c = threadIdx.x & (C - 1);
     bool two_rails = false;
-    for (size_t l = (size_t)blockIdx.x * 256 + threadIdx.x; l < total; l += (size_t)gridDim.x * 256) {
-        const size_t cot = l % n_cotile, line = l / n_cotile;
-        const size_t dst = cot * n_lines + line;
-        const uint32_t* src = lines2 + l * 2 * C;
-        uint32_t packed[C / 2];
-#pragma unroll
-        for (int c2 = 0; c2 < C / 2; c2++) packed[c2] = 0;
-#pragma unroll
-        for (int c = 0; c < C; c++) {
-            const uint32_t wp = src[c], wn = src[C + c];
-            two_rails |= wp != 0u && wn != 0u;
-            words[dst * C + c] = wp | wn;
-            const uint32_t field = 0xC000u | ((wn != 0u ? 2u * C : 0u) + 2u * c);
-            packed[c >> 1] |= field << (16 * (c & 1));
-        }
-#pragma unroll
-        for (int c2 = 0; c2 < C / 2; c2++) idx[dst * (C / 2) + c2] = packed[c2];
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (size_t)gridDim.x * 256) {
+        const size_t l = e / C, line = l / n_cotile, cot = l - line * n_cotile;
+        const uint32_t wp = lines2[l * 2 * C + c], wn = lines2[l * 2 * C + C + c];
+        two_rails |= wp != 0u && wn != 0u;
+        const uint32_t live = (uint32_t)(__ballot((wp | wn) != 0u) >> (threadIdx.x & 48)) & 0xffffu;
+        const int at = rail_slot(live, c);
+        const size_t dst = (cot * n_lines + line) * C + at;
+        words[dst] = wp | wn;
+        fields[dst] = (uint16_t)rail_field(live, at, c, wn != 0u);
     }
     if (two_rails) atomicOr(both, 1u);
 }
@@ -1619,9 +1903,10 @@ int launch_rail_pack(const Geometry& g, uint32_t* wgt, hipStream_t s, bool from_
     if (from_generator && generator_packs_rails(g)) return GEO_SC_OK;  // written, flag area included, by the generator
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(256), 0, s, reinterpret_cast<int32_t*>(wgt + g.wgt_flag_off), (size_t)64);
     const size_t lines = g.wgt_rail_lines;
-    size_t blocks = (lines * g.n_cotile + 255) / 256;
+    size_t blocks = (lines * g.n_cotile * kCoTile + 255) / 256;
     hipLaunchKernelGGL(k_rail_pack, dim3((unsigned)(blocks > 4096 ? 4096 : blocks)), dim3(256), 0, s, wgt,
-                       wgt + g.wgt_rail_off, wgt + g.wgt_rail_idx_off, lines, g.n_cotile, wgt + g.wgt_flag_off);
+                       wgt + g.wgt_rail_off, reinterpret_cast<uint16_t*>(wgt + g.wgt_rail_idx_off), lines, g.n_cotile,
+                       wgt + g.wgt_flag_off);
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
 

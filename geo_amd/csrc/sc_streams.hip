@@ -11,6 +11,8 @@
 // table.
 #include "sc_common.h"
 
+#include <algorithm>
+
 namespace geo_sc {
 
 namespace {
@@ -212,179 +214,110 @@ __global__ __launch_bounds__(kGenThreads) void k_act_streams(const XT* __restric
     }
 }
 
-// Weight streams, tiled layout [P][h_k][k][cotile][rail][16]; one thread per
-// (h, k, padded c_out), c_out fastest so that a wave writes whole tiles.
-// rail_words / rail_fields: the rail-packed copy in the same pass, [c_out tile][line][channel] with
-// line = (pack, kernel row, member): the non-zero rail's word and the 16-bit M0 field of the channel's rail
-// (see k_rail_pack); the first block also clears the buffer's flag area.  two_rail = 0 leaves the two-rail
-// lines unwritten (a caller whose convolution kernel reads the rail-packed copy only).
-__global__ __launch_bounds__(kGenThreads) void k_weight_streams(const float* __restrict__ w,
-                                                               uint32_t* __restrict__ streams,
+// Weight streams, lines in the order the convolution kernels consume them: [P][outer add group][inner add group][OR channel
+// of the group][w_k], each line [cotile][rail][16].  z_mode: inner group = input channel, OR channel = kernel row, seed
+// index u*h_k + v (sc_cuda_kernel.cu:322-324).  Otherwise: outer group = block of zu input channels (all of them in
+// y mode), inner group = kernel row, seed index (channel within the block)*w_k + u (:232, sc.cpp:345-346).
+// rail_words / rail_fields: the rail-packed copy in the same pass, [c_out tile][line][slot]: the non-zero rail's word and its
+// 16-bit field, zero words in front (rail_slot, rail_field); the first block also clears the buffer's flag area.
+// two_rail = 0 leaves the two-rail lines unwritten (a caller whose convolution kernel reads the rail-packed copy only).
+//
+// A block takes 16 output channels x 16 members (input channel, u) x `rows` kernel rows (ROWS, or run-time where that is 0).
+// The weights come in through LDS, read in runs along the kernel rows and, where `rows` is all of them, the members: with
+// lanes along c_out every lane read a cache line of its own.  Then a thread keeps one (channel, member) and walks the rows; the
+// lines of consecutive members are neighbours, so a block writes them in 1 KB runs, their fields in 512 bytes.
+template <int ROWS>
+__global__ __launch_bounds__(kGenThreads) void k_weight_streams(const float* __restrict__ w, uint32_t* __restrict__ streams,
                                                                GenParams gp, int c_out, int c_in, int w_k, int h_k,
-                                                               int n_cotile, uint32_t* __restrict__ rail_words,
-                                                               uint16_t* __restrict__ rail_fields, size_t rail_lines,
+                                                               int n_cotile, int z_mode, int zu, int rows_arg,
+                                                               size_t lines_per_pack, uint32_t* __restrict__ rail_words,
+                                                               uint16_t* __restrict__ rail_fields,
                                                                uint32_t* __restrict__ flags, int two_rail)
 {
     extern __shared__ uint32_t lds[];
-    load_tables_to_lds(lds, gp.L, gp.wpc);
-    const uint32_t* posp1 = lds;
-    const uint32_t* thr = lds + gp.L;
-    if (flags && blockIdx.x == 0 && threadIdx.x < 64) flags[threadIdx.x] = 0u;
-    const int k_or = c_in * w_k;
-    const int co_pad = n_cotile * kCoTile;
-    const size_t total = (size_t)h_k * k_or * co_pad;
-    const size_t pack_stride = (size_t)h_k * k_or * n_cotile * 2 * kCoTile;
-    const float Lf = (float)gp.L, top = (float)(gp.L - 1);
-    for (size_t e = (size_t)blockIdx.x * kGenThreads + threadIdx.x; e < total; e += (size_t)gridDim.x * kGenThreads) {
-        const int co = (int)(e % co_pad);
-        const size_t r = e / co_pad;
-        const int k = (int)(r % k_or);
-        const int v = (int)(r / k_or);
-        const int ci = k / w_k, u = k % w_k;
-        int cp = 0, cn = 0;
-        if (co < c_out) {
-            const float wv = w[(((size_t)co * c_in + ci) * w_k + u) * h_k + v];
-            const float t = wv * Lf;
-            cp = (int)ceilf(fminf(fmaxf(t, 0.0f), top));    // sc.cpp:303
-            cn = (int)ceilf(-fminf(fmaxf(t, -top), 0.0f));  // sc.cpp:304
-        }
-        const int op = (int)posp1[(67 + k) % (gp.L - 1)];  // sc.cpp:345
-        const int on = (int)posp1[(37 + k) % (gp.L - 1)];  // sc.cpp:346
-        const int cot = co / kCoTile, co_l = co % kCoTile;
-        const size_t base = (((size_t)v * k_or + k) * n_cotile + cot) * (2 * kCoTile) + co_l;
-        for (int pk = 0; pk < gp.packs; pk++) {
-            const uint32_t wp = cp ? stream_word(thr, cp, op, pk, gp) : 0u;
-            const uint32_t wn = cn ? stream_word(thr, cn, on, pk, gp) : 0u;
-            if (two_rail) {
-                streams[pk * pack_stride + base] = wp;
-                streams[pk * pack_stride + base + kCoTile] = wn;
-            }
-            if (rail_words) {
-                const size_t dst = ((size_t)cot * rail_lines + ((size_t)pk * h_k + v) * k_or + k) * kCoTile + co_l;
-                rail_words[dst] = wp | wn;
-                rail_fields[dst] = (uint16_t)(0xC000u | ((cn ? 2u * kCoTile : 0u) + 2u * co_l));
-            }
-        }
-    }
-}
-
-// Weight streams of kernels long in dim 3 (the SC linear layer's 1 x 256 rows): a block takes a
-// tile of 16 output channels x 16 OR members x 16 kernel rows.  The weights come in through LDS (w is
-// read in 64-byte runs along the kernel row), then a thread keeps one (channel, member) and walks the
-// 16 rows: the lines of consecutive members are neighbours in the rail-packed copy, so a block writes
-// it in 1 KB runs.  rail_words / rail_fields: the rail-packed copy in the same pass (these tensors are
-// large: a separate pass would read all lines back): [c_out tile][line][channel], the non-zero rail's
-// word and the 16-bit M0 field of the channel's rail.  two_rail = 0 leaves the two-rail lines unwritten
-// (a caller whose convolution kernel reads the rail-packed copy only).
-__global__ __launch_bounds__(kGenThreads) void k_weight_streams_rows(const float* __restrict__ w,
-                                                                    uint32_t* __restrict__ streams,
-                                                                    GenParams gp, int c_out, int c_in, int w_k,
-                                                                    int h_k, int n_cotile,
-                                                                    int v_chunks, uint32_t* __restrict__ rail_words,
-                                                                    uint16_t* __restrict__ rail_fields,
-                                                                    size_t rail_lines, uint32_t* __restrict__ flags,
-                                                                    int two_rail)
-{
-    extern __shared__ uint32_t lds[];
-    load_tables_to_lds(lds, gp.L, gp.wpc);
-    if (flags && blockIdx.x == 0 && threadIdx.x < 64) flags[threadIdx.x] = 0u;
+    const int rows = ROWS ? ROWS : rows_arg;
     const uint32_t* posp1 = lds;
     const uint32_t* thr = lds + gp.L;
     float* wt = reinterpret_cast<float*>(lds + gp.L + gp.L * gp.wpc);  // [row][member][channel], rows of 17
-    const int k_or = c_in * w_k;
-    const int k_chunks = (k_or + 15) / 16;
-    const size_t pack_stride = (size_t)h_k * k_or * n_cotile * 2 * kCoTile;
+    const int members = c_in * w_k, k_chunks = (members + 15) / 16, v_chunks = (h_k + rows - 1) / rows;
     const float Lf = (float)gp.L, top = (float)(gp.L - 1);
-    const size_t n_blocks = (size_t)v_chunks * k_chunks * n_cotile;
+    const unsigned n_blocks = (unsigned)v_chunks * k_chunks * n_cotile;
+    const size_t rail_lines = lines_per_pack * gp.packs;
     const int co_l = threadIdx.x & 15, k_l = threadIdx.x >> 4;
-    for (size_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
-        const int cot = (int)(blk % n_cotile);
-        const size_t r = blk / n_cotile;
-        const int k0 = (int)(r % k_chunks) * 16, v0 = (int)(r / k_chunks) * 16;
-        __syncthreads();  // the previous tile has been read
-        // element e = (channel e / 256, member (e / 16) % 16, row e % 16): 16 consecutive threads read 64 bytes
-#pragma unroll 4
-        for (int i = 0; i < 16; i++) {
-            const int vl = threadIdx.x & 15, kl = threadIdx.x >> 4;
-            const int co = cot * kCoTile + i, k = k0 + kl, v = v0 + vl;
-            const bool ok = co < c_out && k < k_or && v < h_k;
-            const float val = w[ok ? ((size_t)co * k_or + k) * h_k + v : 0];
-            wt[(vl * 16 + kl) * 17 + i] = ok ? val : 0.0f;
+    int cot, k0, v0;
+    auto tile_of = [&](unsigned blk) {
+        const unsigned r = blk / (unsigned)n_cotile, c = r / (unsigned)k_chunks;
+        cot = (int)(blk - r * n_cotile);
+        k0 = (int)(r - c * k_chunks) * 16;
+        v0 = (int)c * rows;
+    };
+    // element e = 256 i + thread = (channel, member, row) of the tile, row fastest; of a single row the thread's own
+    auto fetch = [&](int i, int& slot) {
+        const int e = i * kGenThreads + threadIdx.x, m = e / rows;
+        const int vl = e - m * rows, kl = ROWS == 1 ? k_l : m & 15, cl = ROWS == 1 ? co_l : m >> 4;
+        const int co = cot * kCoTile + cl, k = k0 + kl, v = v0 + vl;
+        const bool ok = co < c_out && k < members && v < h_k;
+        const float val = w[ok ? ((size_t)co * members + k) * h_k + v : 0];
+        slot = (vl * 16 + kl) * 17 + cl;
+        return ok ? val : 0.0f;
+    };
+    // the first elements are under way while the tables go to LDS
+    tile_of(blockIdx.x);
+    int slot0;
+    float first = fetch(0, slot0);
+    load_tables_to_lds(lds, gp.L, gp.wpc);
+    if (flags && blockIdx.x == 0 && threadIdx.x < 64) flags[threadIdx.x] = 0u;
+    if (ROWS != 1) wt[slot0] = first;
+    for (unsigned blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
+        if (blk != blockIdx.x) {
+            tile_of(blk);
+            if (ROWS == 1)
+                first = fetch(0, slot0);
+            else
+                __syncthreads();  // the previous tile has been read
         }
-        __syncthreads();
+        if (ROWS != 1) {
+#pragma unroll 4
+            for (int i = blk == blockIdx.x ? 1 : 0; i < rows; i++) {
+                int slot;
+                const float val = fetch(i, slot);
+                wt[slot] = val;
+            }
+            __syncthreads();
+        }
         const int k = k0 + k_l;
-        if (k >= k_or) continue;
-        const int op = (int)posp1[(67 + k) % (gp.L - 1)];
-        const int on = (int)posp1[(37 + k) % (gp.L - 1)];
-        for (int vl = 0; vl < 16 && v0 + vl < h_k; vl++) {
+        if (k >= members) continue;
+        const int ci = k / w_k, u = k - ci * w_k;
+        // line and seed index of row 0, their steps per row
+        const int ch0 = z_mode ? 0 : ci / zu * zu, cl = z_mode ? 0 : ci - ch0, chs = z_mode ? h_k : min(zu, c_in - ch0);
+        const size_t line0 = z_mode ? (size_t)ci * h_k * w_k + u : (size_t)ch0 * h_k * w_k + (size_t)cl * w_k + u;
+        const int line_step = z_mode ? w_k : chs * w_k;
+        const int seed0 = z_mode ? u * h_k : cl * w_k + u, seed_step = z_mode ? 1 : 0;
+        for (int vl = 0; vl < rows && v0 + vl < h_k; vl++) {
             const int v = v0 + vl;
-            const float t = wt[(vl * 16 + k_l) * 17 + co_l] * Lf;
-            const int cp = (int)ceilf(fminf(fmaxf(t, 0.0f), top));
-            const int cn = (int)ceilf(-fminf(fmaxf(t, -top), 0.0f));
-            const size_t base = (((size_t)v * k_or + k) * n_cotile + cot) * (2 * kCoTile) + co_l;
+            const float t = (ROWS == 1 ? first : wt[(vl * 16 + k_l) * 17 + co_l]) * Lf;
+            const int cp = (int)ceilf(fminf(fmaxf(t, 0.0f), top));    // sc.cpp:303
+            const int cn = (int)ceilf(-fminf(fmaxf(t, -top), 0.0f));  // sc.cpp:304; one of the two is 0
+            const int code = cp | cn;
+            const int o = (int)posp1[((cn ? 37 : 67) + seed0 + v * seed_step) % (gp.L - 1)];
+            const size_t line = line0 + (size_t)v * line_step;
+            const size_t base = (line * n_cotile + cot) * (2 * kCoTile) + co_l;
             for (int pk = 0; pk < gp.packs; pk++) {
-                const uint32_t wp = cp ? stream_word(thr, cp, op, pk, gp) : 0u;
-                const uint32_t wn = cn ? stream_word(thr, cn, on, pk, gp) : 0u;
+                const uint32_t word = code ? stream_word(thr, code, o, pk, gp) : 0u;
                 if (two_rail) {
-                    streams[pk * pack_stride + base] = wp;
-                    streams[pk * pack_stride + base + kCoTile] = wn;
+                    uint32_t* dst = streams + pk * lines_per_pack * n_cotile * (2 * kCoTile) + base;
+                    dst[0] = cp ? word : 0u;
+                    dst[kCoTile] = cn ? word : 0u;
                 }
                 if (rail_words) {
-                    const size_t dst = ((size_t)cot * rail_lines + ((size_t)pk * h_k + v) * k_or + k) * kCoTile + co_l;
-                    rail_words[dst] = wp | wn;
-                    rail_fields[dst] = (uint16_t)(0xC000u | ((cn ? 2u * kCoTile : 0u) + 2u * co_l));
+                    // the line's 16 channels are 16 consecutive lanes
+                    const uint32_t live = (uint32_t)(__ballot(word != 0u) >> (threadIdx.x & 48)) & 0xffffu;
+                    const int at = rail_slot(live, co_l);
+                    const size_t dst = ((size_t)cot * rail_lines + pk * lines_per_pack + line) * kCoTile + at;
+                    rail_words[dst] = word;
+                    rail_fields[dst] = (uint16_t)rail_field(live, at, co_l, cn != 0);
                 }
             }
-        }
-    }
-}
-
-// Weight streams of the grouped accumulation modes, same line format, lines ordered as the
-// convolution kernel consumes them: [P][outer add group][inner add group][OR channel of the
-// group][w_k].  z_mode: inner group = input channel, OR channel = kernel row, seed index
-// u*h_k + v (sc_cuda_kernel.cu:322-324).  Otherwise: outer group = block of zu input channels,
-// inner group = kernel row, seed index (channel within the block)*w_k + u (:232).
-__global__ __launch_bounds__(kGenThreads) void k_weight_streams_grouped(
-    const float* __restrict__ w, uint32_t* __restrict__ streams, GenParams gp, int c_out, int c_in, int w_k, int h_k, int n_cotile, int z_mode, int add_outer, int add_inner, int or_ch_total,
-    int zu)
-{
-    extern __shared__ uint32_t lds[];
-    load_tables_to_lds(lds, gp.L, gp.wpc);
-    const uint32_t* posp1 = lds;
-    const uint32_t* thr = lds + gp.L;
-    const int co_pad = n_cotile * kCoTile;
-    const size_t total = (size_t)add_outer * add_inner * zu * w_k * co_pad;
-    const size_t pack_stride = (size_t)add_inner * or_ch_total * w_k * n_cotile * 2 * kCoTile;
-    const float Lf = (float)gp.L, top = (float)(gp.L - 1);
-    for (size_t e = (size_t)blockIdx.x * kGenThreads + threadIdx.x; e < total; e += (size_t)gridDim.x * kGenThreads) {
-        const int co = (int)(e % co_pad);
-        size_t r = e / co_pad;
-        const int u = (int)(r % w_k);
-        r /= w_k;
-        const int cl = (int)(r % zu);
-        r /= zu;
-        const int gi = (int)(r % add_inner);
-        const int go = (int)(r / add_inner);
-        const int ch0 = go * zu;
-        const int chs = min(zu, or_ch_total - ch0);
-        if (cl >= chs) continue;  // ragged last group: no padding lines
-        const int ci = z_mode ? gi : ch0 + cl;
-        const int v = z_mode ? cl : gi;
-        const int sidx = z_mode ? u * h_k + v : cl * w_k + u;
-        int cp = 0, cn = 0;
-        if (co < c_out) {
-            const float wv = w[(((size_t)co * c_in + ci) * w_k + u) * h_k + v];
-            const float t = wv * Lf;
-            cp = (int)ceilf(fminf(fmaxf(t, 0.0f), top));
-            cn = (int)ceilf(-fminf(fmaxf(t, -top), 0.0f));
-        }
-        const int op = (int)posp1[(67 + sidx) % (gp.L - 1)];
-        const int on = (int)posp1[(37 + sidx) % (gp.L - 1)];
-        const size_t line = (size_t)ch0 * add_inner * w_k + (size_t)gi * chs * w_k + (size_t)cl * w_k + u;
-        const size_t base = (line * n_cotile + co / kCoTile) * (2 * kCoTile) + (co % kCoTile);
-        for (int pk = 0; pk < gp.packs; pk++) {
-            streams[pk * pack_stride + base] = cp ? stream_word(thr, cp, op, pk, gp) : 0u;
-            streams[pk * pack_stride + base + kCoTile] = cn ? stream_word(thr, cn, on, pk, gp) : 0u;
         }
     }
 }
@@ -666,32 +599,26 @@ int launch_weight_streams(const Geometry& g, const float* w, uint32_t* streams, 
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
     const GenParams gp = gen_params(g, g.load_wait_w);
-    if (g.mode != GEO_SC_ACC_Y && g.mode != GEO_SC_ACC_FULL) {
-        const size_t padded =
-            (size_t)g.add_outer * g.add_inner * g.or_ch_per_group * g.w_k * g.n_cotile * kCoTile;
-        hipLaunchKernelGGL(k_weight_streams_grouped, dim3(grid_for(padded)), dim3(kGenThreads), table_bytes(g.L), s,
-                           w, streams, gp, g.c_out, g.c_in, g.w_k, g.h_k, g.n_cotile,
-                           g.mode == GEO_SC_ACC_Z ? 1 : 0, g.add_outer, g.add_inner, g.or_ch_total, g.or_ch_per_group);
-        return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
-    }
-    if (weight_rows_generator(g)) {
-        const int v_chunks = (g.h_k + 15) / 16, k_chunks = (g.k_or + 15) / 16;
-        const size_t n_blocks = (size_t)v_chunks * k_chunks * g.n_cotile;
-        const bool two_rail = !(rail_only && g.wgt_rail);
-        hipLaunchKernelGGL(k_weight_streams_rows, dim3((unsigned)(n_blocks > 256 * 16 ? 256 * 16 : n_blocks)),
-                           dim3(kGenThreads), table_bytes(g.L) + 16 * 16 * 17 * sizeof(float), s, w, streams, gp,
-                           g.c_out, g.c_in, g.w_k, g.h_k, g.n_cotile, v_chunks,
-                           g.wgt_rail ? streams + g.wgt_rail_off : nullptr,
-                           g.wgt_rail ? reinterpret_cast<uint16_t*>(streams + g.wgt_rail_idx_off) : nullptr,
-                           g.wgt_rail_lines, g.wgt_rail ? streams + g.wgt_flag_off : nullptr, two_rail ? 1 : 0);
-        return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
-    }
-    const size_t total = (size_t)g.h_k * g.k_or * g.n_cotile * kCoTile;
+    // all kernel rows in a block, up to 16, where that leaves every CU its blocks: small layers take a row each, layers long
+    // in dim 3 as many as leave eight blocks per CU (16 x 1 x 151 -> 1145: 26.9 us with 16 rows in 720 blocks)
+    const size_t columns = (size_t)((g.k_or + 15) / 16) * g.n_cotile;
+    auto blocks_of = [&](int rows) { return columns * ((g.h_k + rows - 1) / rows); };
+    int rows = std::min(g.h_k, 16);
+    while (rows >= 8 && blocks_of(rows) < 2048) rows = (rows + 1) / 2;
+    if (blocks_of(rows) < 512) rows = 1;
+    const size_t n_blocks = blocks_of(rows);
+    if (n_blocks > 0xffffffffull) return GEO_SC_ERR_UNSUPPORTED;  // (weights of more than 2^40 elements)
     const bool two_rail = !(rail_only && g.wgt_rail);
-    hipLaunchKernelGGL(k_weight_streams, dim3(grid_for(total)), dim3(kGenThreads), table_bytes(g.L), s, w, streams,
-                       gp, g.c_out, g.c_in, g.w_k, g.h_k, g.n_cotile, g.wgt_rail ? streams + g.wgt_rail_off : nullptr,
+    // (the sizes of the usual kernels without divisions by a run-time value)
+    auto kernel = rows == 1 ? k_weight_streams<1> : rows == 3 ? k_weight_streams<3> : rows == 5 ? k_weight_streams<5>
+                  : rows == 4 ? k_weight_streams<4> : rows == 8 ? k_weight_streams<8>
+                  : rows == 16 ? k_weight_streams<16> : k_weight_streams<0>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(n_blocks, (size_t)256 * 16)), dim3(kGenThreads),
+                       table_bytes(g.L) + rows * 16 * 17 * sizeof(float), s, w, streams, gp, g.c_out, g.c_in, g.w_k, g.h_k,
+                       g.n_cotile, g.mode == GEO_SC_ACC_Z ? 1 : 0, g.mode == GEO_SC_ACC_YZ ? g.z_unit : g.c_in, rows,
+                       g.wgt_rail_lines / g.packs, g.wgt_rail ? streams + g.wgt_rail_off : nullptr,
                        g.wgt_rail ? reinterpret_cast<uint16_t*>(streams + g.wgt_rail_idx_off) : nullptr,
-                       g.wgt_rail_lines, g.wgt_rail ? streams + g.wgt_flag_off : nullptr, two_rail ? 1 : 0);
+                       g.wgt_rail ? streams + g.wgt_flag_off : nullptr, two_rail ? 1 : 0);
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
 

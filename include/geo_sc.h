@@ -210,7 +210,8 @@ GEO_SC_API int geo_sc_conv2d_add_partial_forward_ex(const geo_sc_conv_desc* desc
  * A weight has at most one non-zero rail (its codes are those of clamp(w, 0, .) and
  * -clamp(w, ., 0), sc.cpp:301-304).  For 1-, 3- and 5-wide kernels the buffer continues behind these
  * lines with a second, rail-packed copy that the convolution kernel reads there (per line 16
- * words pos | neg, then per line 8 words holding 16 bits per channel: which rail);
+ * words pos | neg, zero words in front, then per line 8 words holding 16 bits per word: which channel and
+ * rail, how many zero words);
  * geo_sc_weight_stream_words is the size of the whole buffer, geo_sc_weight_streams fills all of it.
  *
  * `tables` is not used and may be NULL: the comparison tables of the six stream lengths are constant

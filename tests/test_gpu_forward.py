@@ -653,3 +653,62 @@ def test_chunked_forward_in_a_hip_graph(capi):
         other = capi.conv2d_add_partial_forward(x2, wd, L, pad, desc=d, workspace=ws, options=opt)
         torch.cuda.synchronize()
         assert not torch.equal(other, ref)
+
+
+# ------------------------------------------------------------------ weight lines with zero words
+@pytest.mark.parametrize("first,rest", [(16, 16), (14, 12), (9, 8), (0, 3), (0, 16), (16, 0), (5, 10)])
+@pytest.mark.parametrize("shape_x,shape_w,pad,L,mode", [
+    ((60, 43, 16, 16), (37, 43, 3, 3), (1, 1), 32, "y"),    # 3-wide, an odd number of channels, a partial last tile
+    ((50, 16, 10, 9), (16, 16, 3, 3), (1, 1), 64, "y"),     # an even one; shared out over waves
+    ((24, 11, 12, 13), (20, 11, 5, 5), (2, 2), 32, "y"),    # 5-wide, an odd number
+    ((64, 26, 16, 16), (64, 26, 5, 5), (2, 2), 64, "y"),    # one pair per wave
+    ((40, 2, 16, 16), (40, 2, 3, 3), (1, 1), 32, "y"),      # two channels
+    ((40, 1, 16, 16), (40, 1, 5, 5), (2, 2), 32, "y"),      # a single one
+    ((41, 20, 16, 16), (17, 20, 1, 1), (0, 0), 32, "y"),    # 1-wide
+    ((24, 9, 12, 12), (20, 9, 3, 3), (1, 1), 32, "full"),   # an OR over kernel rows as well
+    ((16, 6, 12, 12), (40, 6, 3, 3), (1, 1), 32, "z"),
+    ((60, 45, 13, 15), (83, 45, 3, 3), (1, 1), 32, "yz"),
+    ((40, 16, 1, 33), (35, 16, 1, 33), (0, 0), 32, "y"),    # item-innermost
+])
+def test_weight_lines_with_zero_words(capi, so, shape_x, shape_w, pad, L, mode, first, rest):
+    """`first` of the 16 words of the first input channel's lines are not zero and, one more or less, `rest` of the others': the
+    loops for full, thinned and mostly empty lines, entered with lines of either kind to come.  Bit for bit, twice."""
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=shape_w[0] + L + first)
+    g = torch.Generator().manual_seed(first * 17 + rest)
+    w = torch.where(w == 0, torch.full_like(w, 0.5), w.sign() * (0.75 + 0.25 * w.abs()))   # no empty word by chance
+    order = torch.rand(w.shape, generator=g)                # the channels of a line that are kept, at random
+    for c0 in range(0, w.shape[0], 16):
+        rank = order[c0:c0 + 16].argsort(0).argsort(0)
+        keep = torch.full(w.shape[1:], rest) + torch.randint(-1, 2, w.shape[1:], generator=g)
+        keep[0] = first
+        w[c0:c0 + 16] *= (rank < keep)
+    w = w.contiguous()
+    gen = "rand" if mode == "full" else "lfsr"
+    exp = (so.conv2d_general(x.numpy(), w.numpy(), L, pad, mode, 1, gen, 3) if mode == "full" else
+           so.conv2d_modes(x.numpy(), w.numpy(), L, pad, mode, 32))
+    d = capi.make_desc(x.shape, w.shape, L, pad, accumulate=mode, z_unit=32, generator=gen, seed=3)
+    y = torch.full(capi.output_shape(d), 12345, dtype=torch.int32, device="cuda")
+    act, wgt = capi.act_streams(x.cuda(), d), capi.weight_streams(w.cuda(), d)
+    for _ in range(2):
+        capi.conv2d_add_partial_from_streams(act, wgt, d, out=y)
+        assert np.array_equal(y.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("shape_x,shape_w,mode", [
+    ((2, 96, 5, 6), (500, 96, 3, 3), "y"),       # three kernel rows in a block
+    ((2, 96, 5, 6), (500, 96, 3, 3), "z"),
+    ((2, 95, 5, 6), (511, 95, 3, 3), "yz"),      # a ragged last channel block
+    ((2, 52, 6, 7), (512, 52, 5, 5), "y"),       # five
+    ((2, 96, 5, 6), (512, 96, 3, 2), "y"),       # two: a run-time number
+    ((2, 256, 2, 9), (500, 256, 1, 7), "y"),     # seven
+    ((2, 256, 1, 33), (1024, 256, 1, 31), "y"),  # sixteen, a short last run
+    ((2, 128, 1, 33), (1024, 128, 1, 32), "y"),  # eight
+    ((2, 128, 1, 33), (512, 128, 1, 29), "y"),   # four
+])
+def test_weight_generator_tiles(capi, so, shape_x, shape_w, mode):
+    """Layers large enough for more than one kernel row per block of the weight generator: bit for bit."""
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=sum(shape_w))
+    d = capi.make_desc(x.shape, w.shape, 32, (0, 0), 7, 2, 2, 2, accumulate=mode, z_unit=32)
+    exp = so.conv2d_modes(x.numpy(), w.numpy(), 32, (0, 0), mode, 32, 7, 2, 2, 2)
+    got = capi.conv2d_add_partial_from_streams(capi.act_streams(x.cuda(), d), capi.weight_streams(w.cuda(), d), d)
+    assert np.array_equal(got.cpu().numpy(), exp)
