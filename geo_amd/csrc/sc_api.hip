@@ -121,6 +121,7 @@ int make_geometry(const geo_sc_conv_desc* d, Geometry* g)
               (unsigned long long)g->act_words * 4 < 0xffffffffull;
     const size_t lines = (size_t)g->packs * d->h_k * g->k_or;
     g->wgt_words = lines * g->n_cotile * 2 * kCoTile;
+    g->right_halves = false;
     g->wgt_rail_off = g->wgt_rail_idx_off = g->wgt_flag_off = 0;
     g->wgt_rail_lines = lines;
     if (g->wgt_rail) {
@@ -205,6 +206,7 @@ int plan_forward(const geo_sc_conv_desc* d, const Options& opt, ForwardPlan* p)
     p->last = p->chunk;
     if (p->n_last && (rc = geometry_of(p->n_last, &p->last)) != GEO_SC_OK) return rc;
     p->rail_only = p->chunk.rail && p->last.rail;
+    p->chunk.right_halves = p->last.right_halves = p->rail_only && lines16_lds(p->chunk) && lines16_lds(p->last);
     p->off_wgt = 0;
     p->off_act[0] = align256(g.wgt_words * sizeof(uint32_t));
     p->off_act[1] = p->off_act[0] + (p->buffers == 2 ? align256((size_t)nc * item_bytes) : 0);

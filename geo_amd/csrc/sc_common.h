@@ -58,6 +58,10 @@ struct Geometry {
     // that rail is processed.  wgt_rail: the weight stream buffer carries the rail-packed copy (a
     // property of the weights' shape alone); rail: this geometry's launch reads it.
     bool wgt_rail, rail;
+    // The right halves of the rail-packed lines (slots 8 - 15) are written a second time, by themselves, into the two-rail lines'
+    // place (right_words / right_fields): the whole-op forward of one-wide layers with OR groups of 16 lines, none of whose
+    // launches reads two-rail lines.
+    bool right_halves;
 };
 
 // A rail-packed line holds its 16 channels with the zero words in front, in channel order on either side; live: bit c set
@@ -99,6 +103,17 @@ inline __host__ __device__ size_t table_bytes(int L)
 {
     return sizeof(uint32_t) * ((size_t)L + (size_t)L * table_words_per_code(L));
 }
+
+constexpr int kLinLines = 16, kLinTiles = 8;  // k_conv_fwd_items_rail_lds: lines of an OR group, c_out tiles of a workgroup
+// whether launch_conv_forward takes that kernel: item-innermost, two equal halves of the groups, 128 workgroups
+inline bool lines16_lds(const Geometry& g)
+{
+    const long long tiles = ((long long)(g.n + 1) / 2 * g.ho + 63) / 64;
+    return g.act_item_inner && g.w_k == 1 && g.c_in == kLinLines && g.n_cotile % kLinTiles == 0 && g.packs * g.h_k % 2 == 0 &&
+           tiles * (g.n_cotile / kLinTiles) >= 128;
+}
+// the right halves' words [n_cotile][line][8] and fields [n_cotile][line][8] of 16 bits, in the place of two-rail lines of 32 words
+inline size_t right_fields_off(const Geometry& g) { return g.wgt_rail_lines * g.n_cotile * (kCoTile / 2); }
 
 const uint32_t* stream_tables_host(int L, size_t* words);
 

@@ -221,21 +221,40 @@ __global__ __launch_bounds__(kGenThreads) void k_act_streams(const XT* __restric
 // rail_words / rail_fields: the rail-packed copy in the same pass, [c_out tile][line][slot]: the non-zero rail's word and its
 // 16-bit field, zero words in front (rail_slot, rail_field); the first block also clears the buffer's flag area.
 // two_rail = 0 leaves the two-rail lines unwritten (a caller whose convolution kernel reads the rail-packed copy only).
+// right_words / right_fields: the right halves of the packed lines once more (Geometry::right_halves).
 //
 // A block takes 16 output channels x 16 members (input channel, u) x `rows` kernel rows (ROWS, or run-time where that is 0).
 // The weights come in through LDS, read in runs along the kernel rows and, where `rows` is all of them, the members: with
 // lanes along c_out every lane read a cache line of its own.  Then a thread keeps one (channel, member) and walks the rows; the
 // lines of consecutive members are neighbours, so a block writes them in 1 KB runs, their fields in 512 bytes.
+struct WeightGen {  // (one argument: a launch of many is slower on the host)
+    const float* __restrict__ w;
+    uint32_t* __restrict__ streams;
+    uint32_t* __restrict__ rail_words;
+    uint16_t* __restrict__ rail_fields;
+    uint32_t* __restrict__ right_words;
+    uint16_t* __restrict__ right_fields;
+    uint32_t* __restrict__ flags;
+    size_t lines_per_pack;
+    GenParams gp;
+    int c_out, c_in, w_k, h_k, n_cotile, z_mode, zu, rows, two_rail;
+};
 template <int ROWS>
-__global__ __launch_bounds__(kGenThreads) void k_weight_streams(const float* __restrict__ w, uint32_t* __restrict__ streams,
-                                                               GenParams gp, int c_out, int c_in, int w_k, int h_k,
-                                                               int n_cotile, int z_mode, int zu, int rows_arg,
-                                                               size_t lines_per_pack, uint32_t* __restrict__ rail_words,
-                                                               uint16_t* __restrict__ rail_fields,
-                                                               uint32_t* __restrict__ flags, int two_rail)
+__global__ __launch_bounds__(kGenThreads) void k_weight_streams(WeightGen a)
 {
+    const GenParams& gp = a.gp;
+    const float* __restrict__ w = a.w;
+    uint32_t* __restrict__ streams = a.streams;
+    uint32_t* __restrict__ rail_words = a.rail_words;
+    uint16_t* __restrict__ rail_fields = a.rail_fields;
+    uint32_t* __restrict__ right_words = a.right_words;
+    uint16_t* __restrict__ right_fields = a.right_fields;
+    uint32_t* __restrict__ flags = a.flags;
+    const size_t lines_per_pack = a.lines_per_pack;
+    const int c_out = a.c_out, c_in = a.c_in, w_k = a.w_k, h_k = a.h_k, n_cotile = a.n_cotile;
+    const int z_mode = a.z_mode, zu = a.zu, two_rail = a.two_rail;
     extern __shared__ uint32_t lds[];
-    const int rows = ROWS ? ROWS : rows_arg;
+    const int rows = ROWS ? ROWS : a.rows;
     const uint32_t* posp1 = lds;
     const uint32_t* thr = lds + gp.L;
     float* wt = reinterpret_cast<float*>(lds + gp.L + gp.L * gp.wpc);  // [row][member][channel], rows of 17
@@ -314,8 +333,14 @@ __global__ __launch_bounds__(kGenThreads) void k_weight_streams(const float* __r
                     const uint32_t live = (uint32_t)(__ballot(word != 0u) >> (threadIdx.x & 48)) & 0xffffu;
                     const int at = rail_slot(live, co_l);
                     const size_t dst = ((size_t)cot * rail_lines + pk * lines_per_pack + line) * kCoTile + at;
+                    const uint16_t field = (uint16_t)rail_field(live, at, co_l, cn != 0);
                     rail_words[dst] = word;
-                    rail_fields[dst] = (uint16_t)rail_field(live, at, co_l, cn != 0);
+                    rail_fields[dst] = field;
+                    if (right_words && at >= kCoTile / 2) {
+                        const size_t right = ((size_t)cot * rail_lines + pk * lines_per_pack + line) * (kCoTile / 2) + at - kCoTile / 2;
+                        right_words[right] = word;
+                        right_fields[right] = field;
+                    }
                 }
             }
         }
@@ -608,17 +633,36 @@ int launch_weight_streams(const Geometry& g, const float* w, uint32_t* streams, 
     if (blocks_of(rows) < 512) rows = 1;
     const size_t n_blocks = blocks_of(rows);
     if (n_blocks > 0xffffffffull) return GEO_SC_ERR_UNSUPPORTED;  // (weights of more than 2^40 elements)
-    const bool two_rail = !(rail_only && g.wgt_rail);
+    const bool two_rail = !(rail_only && g.wgt_rail), right = g.right_halves && !two_rail;
     // (the sizes of the usual kernels without divisions by a run-time value)
     auto kernel = rows == 1 ? k_weight_streams<1> : rows == 3 ? k_weight_streams<3> : rows == 5 ? k_weight_streams<5>
                   : rows == 4 ? k_weight_streams<4> : rows == 8 ? k_weight_streams<8>
                   : rows == 16 ? k_weight_streams<16> : k_weight_streams<0>;
+    WeightGen a = {};
+    a.w = w;
+    a.streams = streams;
+    if (g.wgt_rail) {
+        a.rail_words = streams + g.wgt_rail_off;
+        a.rail_fields = reinterpret_cast<uint16_t*>(streams + g.wgt_rail_idx_off);
+        a.flags = streams + g.wgt_flag_off;
+    }
+    if (right) {
+        a.right_words = streams;
+        a.right_fields = reinterpret_cast<uint16_t*>(streams + right_fields_off(g));
+    }
+    a.lines_per_pack = g.wgt_rail_lines / g.packs;
+    a.gp = gp;
+    a.c_out = g.c_out;
+    a.c_in = g.c_in;
+    a.w_k = g.w_k;
+    a.h_k = g.h_k;
+    a.n_cotile = g.n_cotile;
+    a.z_mode = g.mode == GEO_SC_ACC_Z ? 1 : 0;
+    a.zu = g.mode == GEO_SC_ACC_YZ ? g.z_unit : g.c_in;
+    a.rows = rows;
+    a.two_rail = two_rail ? 1 : 0;
     hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(n_blocks, (size_t)256 * 16)), dim3(kGenThreads),
-                       table_bytes(g.L) + rows * 16 * 17 * sizeof(float), s, w, streams, gp, g.c_out, g.c_in, g.w_k, g.h_k,
-                       g.n_cotile, g.mode == GEO_SC_ACC_Z ? 1 : 0, g.mode == GEO_SC_ACC_YZ ? g.z_unit : g.c_in, rows,
-                       g.wgt_rail_lines / g.packs, g.wgt_rail ? streams + g.wgt_rail_off : nullptr,
-                       g.wgt_rail ? reinterpret_cast<uint16_t*>(streams + g.wgt_rail_idx_off) : nullptr,
-                       g.wgt_rail ? streams + g.wgt_flag_off : nullptr, two_rail ? 1 : 0);
+                       table_bytes(g.L) + (rows == 1 ? 0 : rows * 16 * 17 * sizeof(float)), s, a);
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
 

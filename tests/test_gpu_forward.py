@@ -669,6 +669,7 @@ def test_chunked_forward_in_a_hip_graph(capi):
     ((16, 6, 12, 12), (40, 6, 3, 3), (1, 1), 32, "z"),
     ((60, 45, 13, 15), (83, 45, 3, 3), (1, 1), 32, "yz"),
     ((40, 16, 1, 33), (35, 16, 1, 33), (0, 0), 32, "y"),    # item-innermost
+    ((1010, 16, 1, 6), (2040, 16, 1, 6), (0, 0), 32, "y"),  # the same, activation words staged through LDS
 ])
 def test_weight_lines_with_zero_words(capi, so, shape_x, shape_w, pad, L, mode, first, rest):
     """`first` of the 16 words of the first input channel's lines are not zero and, one more or less, `rest` of the others': the
@@ -685,7 +686,10 @@ def test_weight_lines_with_zero_words(capi, so, shape_x, shape_w, pad, L, mode, 
     w = w.contiguous()
     gen = "rand" if mode == "full" else "lfsr"
     exp = (so.conv2d_general(x.numpy(), w.numpy(), L, pad, mode, 1, gen, 3) if mode == "full" else
+           so.conv2d_add_partial(x.numpy(), w.numpy(), L, pad) if mode == "y" else
            so.conv2d_modes(x.numpy(), w.numpy(), L, pad, mode, 32))
+    if mode == "y":
+        assert np.array_equal(gpu_forward(capi, x, w, L, pad), exp)
     d = capi.make_desc(x.shape, w.shape, L, pad, accumulate=mode, z_unit=32, generator=gen, seed=3)
     y = torch.full(capi.output_shape(d), 12345, dtype=torch.int32, device="cuda")
     act, wgt = capi.act_streams(x.cuda(), d), capi.weight_streams(w.cuda(), d)
