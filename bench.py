@@ -14,7 +14,7 @@ duration (the backward does no bit-MACs, so the forward-only rate is reported ne
 The default workload is the configuration the headline metric is quoted on: SC conv2d
 128->128 3x3 at 16x16, batch 256, pad 1, stream length 128, activations U[0,1), weights
 U[-1,1) (with these distributions every OR rail saturates, so this input is for timing
-only; the kernels have no data-dependent early exit).  After the headline the default run also times
+only; no kernel exits early on them, and the weights have too few zero stream words to skip).  After the headline the default run also times
 the other benchmark configurations (C3 at stream lengths 32 and 256, C5, C4, the C2 training step) and
 reports them under the key ``configs``.
 """
