@@ -1308,6 +1308,9 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
 void k_conv_fwd_tile_rail(FwdParams q)
 {
     constexpr int C = kCoTile;
+    // all cache lines of the arguments in one round of loads, where the compiler's order takes four (see k_weight_streams):
+    // 9.26 -> 9.08 us in a graph, 3 -> 32 channels, 3 x 3, 32 x 32, batch 32, L 64
+    asm volatile("" ::"s"(q.act), "s"(q.wgt_rail), "s"(q.n), "s"(q.n_cotile), "s"(q.act_plane), "s"(q.or_stride), "s"(q.or_shares));
     extern __shared__ uint32_t tile_lds[];
     int* red = reinterpret_cast<int*>(tile_lds);  // [2 c + r][lane]
     uint32_t* orb = tile_lds + 2 * C * 64;        // [pair][rail][2 c + r][lane]
