@@ -72,23 +72,18 @@ __device__ __forceinline__ int rail_slot(uint32_t live, int c)
     return (live >> c) & 1u ? kCoTile - __popc(live >> c) : __popc(~live & below);
 }
 // The 16-bit field of channel c at slot `at`: bits 7:0 the register offset of its accumulators (2 c for the positive rail and
-// for zero weights, 32 + 2 c for the negative one), bits 15:12 the SRC2 and DST enables of the VGPR index mode.  But for four
-// slots, whose bits 15:8 or 11:8 say how a wave reads the line (index mode ignores bits 11:8 of M0, and the kernels set
-// the enables of slots 0 and 8 themselves):
-//   slot 0, 15:8: five times the zero words to jump over (at most 15) in the line, or in its left half where that has others;
-//   slot 1, 11:8: the line's zero words, at most 15;
-//   slot 8, 15:8: five times the zero words to jump over in the right half (at most 7);
-//   slot 9, 8   : 1 where the left half holds words that are not zero.
-// (Five: a slot's code is five words long.  A line or half without any other ORs one zero word.)
+// for zero weights, 32 + 2 c for the negative one), bits 15:12 the SRC2 and DST enables of the VGPR index mode.  Two slots say in
+// bits 11:8, which index mode ignores, how a wave reads the line:
+//   slot 0: the zero words in front, at most 15: of those before the last slot the wave may jump over as many;
+//   slot 8: bits 10:8 the zero words to jump over in the right half (at most 7), bit 11 set where the left half holds others.
+// (A line or half without any other ORs one zero word.)
 __device__ __forceinline__ uint32_t rail_field(uint32_t live, int at, int c, bool negative)
 {
     constexpr int H = kCoTile / 2;
     const int zeros = min(kCoTile - __popc(live), kCoTile - 1);
     uint32_t high = 0xC0u;
-    if (at == 0) high = 5u * (uint32_t)zeros;
-    if (at == 1) high |= (uint32_t)zeros;
-    if (at == H) high = zeros < H ? 0u : 5u * (uint32_t)(zeros - H);
-    if (at == H + 1) high |= zeros < H ? 1u : 0u;
+    if (at == 0) high |= (uint32_t)zeros;
+    if (at == H) high |= zeros < H ? (uint32_t)H : (uint32_t)(zeros - H);
     return high << 8 | ((negative ? 2u * kCoTile : 0u) + 2u * (uint32_t)c);
 }
 static_assert(kCoTile == 16, "rail-packed lines hold 16 channels");

@@ -482,8 +482,6 @@ typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 // M0 of a channel from its 16-bit field: index in bits 7:0, the SRC2 and DST enables in bits 15:12
 #define GEO_SC_RAIL_LO(I) "s_and_b32 m0, %[" I "], 0xffff\n"
 #define GEO_SC_RAIL_HI(I) "s_lshr_b32 m0, %[" I "], 16\n"
-// slots 0 and 8: bits 15:8 of their fields are not the enables (rail_field)
-#define GEO_SC_RAIL_ON(I) "s_set_gpr_idx_on %[" I "], gpr_idx(SRC2,DST)\n"
 #define GEO_SC_RAIL_OPERANDS                                                                                           \
     [w0] "s"(w[0]), [w1] "s"(w[1]), [w2] "s"(w[2]), [w3] "s"(w[3]), [w4] "s"(w[4]), [w5] "s"(w[5]), [w6] "s"(w[6]),     \
         [w7] "s"(w[7]), [w8] "s"(w[8]), [w9] "s"(w[9]), [w10] "s"(w[10]), [w11] "s"(w[11]), [w12] "s"(w[12]),           \
@@ -493,7 +491,7 @@ typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 #define GEO_SC_RAIL_16(PAIR)                                                                                           \
     PAIR("w0", "") PAIR("w1", GEO_SC_RAIL_HI("i0")) PAIR("w2", GEO_SC_RAIL_LO("i1")) PAIR("w3", GEO_SC_RAIL_HI("i1"))   \
     PAIR("w4", GEO_SC_RAIL_LO("i2")) PAIR("w5", GEO_SC_RAIL_HI("i2")) PAIR("w6", GEO_SC_RAIL_LO("i3"))                  \
-    PAIR("w7", GEO_SC_RAIL_HI("i3")) PAIR("w8", GEO_SC_RAIL_ON("i4")) PAIR("w9", GEO_SC_RAIL_HI("i4"))                  \
+    PAIR("w7", GEO_SC_RAIL_HI("i3")) PAIR("w8", GEO_SC_RAIL_LO("i4")) PAIR("w9", GEO_SC_RAIL_HI("i4"))                  \
     PAIR("w10", GEO_SC_RAIL_LO("i5")) PAIR("w11", GEO_SC_RAIL_HI("i5")) PAIR("w12", GEO_SC_RAIL_LO("i6"))               \
     PAIR("w13", GEO_SC_RAIL_HI("i6")) PAIR("w14", GEO_SC_RAIL_LO("i7")) PAIR("w15", GEO_SC_RAIL_HI("i7"))
 
@@ -549,7 +547,6 @@ GEO_SC_DEFINE_RAIL_LINES(rail_line_lo, rail_line_first_lo, "v32", "v33", "v[32:4
 #undef GEO_SC_RAIL_16
 #undef GEO_SC_RAIL_OPERANDS
 #undef GEO_SC_RAIL_LO
-#undef GEO_SC_RAIL_ON
 #undef GEO_SC_RAIL_HI
 
 // sum += popcount(pos) - popcount(neg) in three instructions (the compiler's form takes four)
@@ -831,7 +828,7 @@ struct PairLane {
 //                                           stages of lines fit the scalar registers and one is in flight while the other is
 //                                           ORed; the left half of a line with more than eight words is loaded where it is met.
 // What bounds them: DENSE the issue of v_and_or_b32; HALF the scalar instructions, one per SIMD and four cycles like
-// the vector ones, of which a line takes one per word and three for its jump.
+// the vector ones, of which a line takes one per word and four for its jump.
 // One block with its loads and waits inside, registers assigned by hand: scalar loads return out of order, so only
 // lgkmcnt(0) says that a line has arrived and the next stage's loads must be issued behind that wait, an order that the
 // compiler does not keep; and 64 pinned accumulators that live across its branches it spills.
@@ -849,59 +846,55 @@ struct PairLane {
         "s_xor_b32 m0, m0, 32\n"                                                                                       \
         "v_mov_b32 v32, 0\n"                                                                                           \
         "v_mov_b32 v33, 0\n"
-#define GEO_SC_M0_ON(F) "s_set_gpr_idx_on s[" #F "+0], gpr_idx(SRC2,DST)\n"
 #define GEO_SC_M0_LO(F, J) "s_mov_b32 m0, s[" #F "+" #J "]\n"
 #define GEO_SC_M0_HI(F, J) "s_lshr_b32 m0, s[" #F "+" #J "], 16\n"
-#define GEO_SC_EIGHT(SLOT, W, F, X0, X1)                                                                               \
-    SLOT(GEO_SC_M0_ON(F), W, 0, X0, X1) SLOT(GEO_SC_M0_HI(F, 0), W, 1, X0, X1)                                         \
+#define GEO_SC_EIGHT(SLOT, W, F, X0, X1) SLOT(GEO_SC_M0_LO(F, 0), W, 0, X0, X1) GEO_SC_SEVEN(SLOT, W, F, X0, X1)
+#define GEO_SC_SEVEN(SLOT, W, F, X0, X1) SLOT(GEO_SC_M0_HI(F, 0), W, 1, X0, X1)                                        \
     SLOT(GEO_SC_M0_LO(F, 1), W, 2, X0, X1) SLOT(GEO_SC_M0_HI(F, 1), W, 3, X0, X1)                                      \
     SLOT(GEO_SC_M0_LO(F, 2), W, 4, X0, X1) SLOT(GEO_SC_M0_HI(F, 2), W, 5, X0, X1)                                      \
     SLOT(GEO_SC_M0_LO(F, 3), W, 6, X0, X1) SLOT(GEO_SC_M0_HI(F, 3), W, 7, X0, X1)
 #define GEO_SC_INDEX_ON "s_set_gpr_idx_on 0, gpr_idx(SRC2,DST)\n"
 #define GEO_SC_INDEX_OFF "s_set_gpr_idx_off\n"
-// Over zero words: a slot is five words of code, and bits 15:8 of the first field hold five times the zero words.
-// s_getpc_b64 gives the address of the s_lshl2_add_u32, three words in front of the first slot but one for s_addk_i32.
-#define GEO_SC_JUMP(F)                                                                                                 \
-    "s_bfe_u32 s33, s[" #F "+0], 0x80008\n"                                                                            \
-    "s_addk_i32 s33, 3\n"                                                                                              \
+// Over zero words: a slot is 20 bytes of code.  A jump takes BITS bits of a field, as many as there are places behind it: whatever a
+// buffer holds, it lands on one of them.  s_getpc_b64 gives the address of the s_add_u32, three words in front of place 0.
+#define GEO_SC_JUMP(F, BITS)                                                                                           \
+    "s_bfe_u32 s33, s[" #F "+0], " #BITS "<<16|8\n"                                                                    \
+    "s_mulk_i32 s33, 20\n"                                                                                             \
+    "s_addk_i32 s33, 12\n"                                                                                             \
     "s_getpc_b64 s[34:35]\n"                                                                                           \
-    "s_lshl2_add_u32 s34, s33, s34\n"                                                                                  \
+    "s_add_u32 s34, s34, s33\n"                                                                                        \
     "s_addc_u32 s35, s35, 0\n"                                                                                         \
     "s_setpc_b64 s[34:35]\n"
-// the same with the address of the first slot in BASE and vcc_hi (GEO_SC_BASE; no carry between the slots)
+// the same over eight places with the address of place 0 in BASE and vcc_hi (GEO_SC_BASE; no carry between the places)
 #define GEO_SC_JUMP_FROM(BASE, F)                                                                                      \
-    "s_bfe_u32 s33, s[" #F "+0], 0x80008\n"                                                                            \
-    "s_lshl2_add_u32 vcc_lo, s33, " BASE "\n"                                                                          \
+    "s_bfe_u32 s33, s[" #F "+0], 3<<16|8\n"                                                                            \
+    "s_lshl4_add_u32 vcc_lo, s33, " BASE "\n"                                                                          \
+    "s_lshl2_add_u32 vcc_lo, s33, vcc_lo\n"                                                                            \
     "s_setpc_b64 vcc\n"
 #define GEO_SC_DENSE(W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W + 8, F + 4, X0, X1)
 #define GEO_SC_FIRST(W, F, X0, X1)                                                                                     \
     GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W + 8, F + 4, X0, X1)
-#define GEO_SC_SKIP(W, F, X0, X1) GEO_SC_JUMP(F) GEO_SC_DENSE(W, F, X0, X1)
-// a line's right half; LABEL marks its first slot
+#define GEO_SC_SKIP(W, F, X0, X1) GEO_SC_JUMP(F, 4) GEO_SC_DENSE(W, F, X0, X1)
+// A line's right half behind a jump, slots 9 to 15 at places 1 to 7.  Place 0, as long as a slot, leaves for a copy of the eight slots
+// (GEO_SC_LEFT, out of line) behind which the left half is loaded if it holds words.
+#define GEO_SC_RIGHT(LABEL, SEVEN)                                                                                     \
+    ".Lsc_" LABEL "_%=:\n"                                                                                             \
+    "s_branch .Lsc_" LABEL "_left_%=\n"                                                                                \
+    "s_nop 0\ns_nop 0\ns_nop 0\ns_nop 0\n" SEVEN ".Lsc_" LABEL "_done_%=:\n"
 #define GEO_SC_HALF(LABEL, BASE, W, F, X0, X1)                                                                         \
-    GEO_SC_JUMP_FROM(BASE, F) ".Lsc_" LABEL "_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)
+    GEO_SC_JUMP_FROM(BASE, F) GEO_SC_RIGHT(LABEL, GEO_SC_SEVEN(GEO_SC_SLOT, W, F, X0, X1))
 #define GEO_SC_BASE(LABEL, BASE) "s_add_u32 " BASE ", vcc_lo, .Lsc_" LABEL "_%=-.Lsc_pc_%=\n"
-// Bit 24 of a line's fifth field word: its left half holds words too.  Lines of a stage with the flag, out of line:
-#define GEO_SC_ANY_LEFT2(LABEL, F0, F1)                                                                                \
-    "s_or_b32 s33, s[" #F0 "+0], s[" #F1 "+0]\n"                                                                       \
-    "s_bitcmp1_b32 s33, 24\n"                                                                                          \
-    "s_cbranch_scc1 .Lsc_" LABEL "_%=\n"                                                                               \
-    ".Lsc_" LABEL "_back_%=:\n"
-#define GEO_SC_ANY_LEFT3(LABEL, F0, F1, F2)                                                                            \
-    "s_or_b32 s33, s[" #F0 "+0], s[" #F1 "+0]\n"                                                                       \
-    "s_or_b32 s33, s33, s[" #F2 "+0]\n"                                                                                \
-    "s_bitcmp1_b32 s33, 24\n"                                                                                          \
-    "s_cbranch_scc1 .Lsc_" LABEL "_%=\n"                                                                               \
-    ".Lsc_" LABEL "_back_%=:\n"
-#define GEO_SC_LEFT(W, F, X0, X1, L)                                                                                   \
-    "s_bitcmp1_b32 s[" #F "+0], 24\n"                                                                                  \
-    "s_cbranch_scc0 2f\n"                                                                                              \
+// line L of its channel, of eight words or more
+#define GEO_SC_LEFT(LABEL, W, F, X0, X1, L)                                                                            \
+    ".Lsc_" LABEL "_left_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                \
+    "s_bitcmp1_b32 s[" #F "+0], 11\n"                                                                                  \
+    "s_cbranch_scc0 .Lsc_" LABEL "_done_%=\n"                                                                          \
     "s_lshr_b32 s33, %[wo], 1\n"                                                                                       \
     "s_load_dwordx8 s[" #W ":" #W "+7], %[wp], %[wo] offset:64*" #L "\n"                                               \
     "s_load_dwordx4 s[" #F ":" #F "+3], %[ip], s33 offset:32*" #L "\n"                                                 \
     "s_waitcnt lgkmcnt(0)\n"                                                                                           \
-    GEO_SC_JUMP(F) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                             \
-    "2:\n"
+    GEO_SC_JUMP(F, 3) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                          \
+    "s_branch .Lsc_" LABEL "_done_%=\n"
 // loads of line L of the channel AT bytes behind %[wo] (in the words; half of it in the fields, s33)
 #define GEO_SC_FIELD_OFFSET "s_lshr_b32 s33, %[wo], 1\n"
 #define GEO_SC_LOAD(W, F, L)                                                                                           \
@@ -972,12 +965,12 @@ struct PairLane {
     GEO_SC_DENSE(36, 84, "x3", "x4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                       \
     GEO_SC_DENSE(52, 92, "x4", "x5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
     GEO_SC_NEXT_OR_END
-// the first lines' zero words (bits 27:24 of the first field word) pick the loop for the channels behind the first
+// the first lines' zero words (bits 11:8 of the first field word) pick the loop for the channels behind the first
 #define GEO_SC_COUNT_ZEROS                                                                                             \
-    "s_bfe_u32 s35, s84, 0x40018\n"                                                                                    \
-    "s_bfe_u32 s33, s92, 0x40018\n"                                                                                    \
+    "s_bfe_u32 s35, s84, 0x40008\n"                                                                                    \
+    "s_bfe_u32 s33, s92, 0x40008\n"                                                                                    \
     "s_add_u32 s35, s35, s33\n"                                                                                        \
-    "s_bfe_u32 s33, s24, 0x40018\n"                                                                                    \
+    "s_bfe_u32 s33, s24, 0x40008\n"                                                                                    \
     "s_add_u32 s35, s35, s33\n"
 #define GEO_SC_LOADS_FULL GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 0) GEO_SC_LOAD(52, 92, 1) GEO_SC_LOAD(68, 24, 2)
 #define GEO_SC_LOADS_HALF_A(AT)                                                                                        \
@@ -1053,19 +1046,16 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_HALF_CHANNEL3(GEO_SC_LOAD_HALF(60, 96, 0, 192) GEO_SC_LOAD_HALF(68, 24, 1, 192)
                                  GEO_SC_LOAD_HALF(76, 28, 2, 192), GEO_SC_FETCH4("y"))
             GEO_SC_HALF("a0", "s18", 36, 84, "x0", "x1") GEO_SC_HALF("a1", "s19", 44, 88, "x1", "x2")
-            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3") GEO_SC_ANY_LEFT3("left_a", 84, 88, 92)
+            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3")
             "s_addk_i32 %[wo], 192\n" GEO_SC_NEXT_OR_END
             GEO_SC_HALF_CHANNEL3(GEO_SC_LOADS_HALF_A(192), GEO_SC_FETCH4("x"))
             GEO_SC_HALF("b0", "s21", 60, 96, "y0", "y1") GEO_SC_HALF("b1", "s22", 68, 24, "y1", "y2")
-            GEO_SC_HALF("b2", "s23", 76, 28, "y2", "y3") GEO_SC_ANY_LEFT3("left_b", 96, 24, 28)
+            GEO_SC_HALF("b2", "s23", 76, 28, "y2", "y3")
             "s_addk_i32 %[wo], 192\n" GEO_SC_NEXT_OR_END
             "s_branch 31b\n",
-            ".Lsc_left_a_%=:\n"
-            GEO_SC_LEFT(36, 84, "x0", "x1", 0) GEO_SC_LEFT(44, 88, "x1", "x2", 1) GEO_SC_LEFT(52, 92, "x2", "x3", 2)
-            "s_branch .Lsc_left_a_back_%=\n"
-            ".Lsc_left_b_%=:\n"
-            GEO_SC_LEFT(60, 96, "y0", "y1", 0) GEO_SC_LEFT(68, 24, "y1", "y2", 1) GEO_SC_LEFT(76, 28, "y2", "y3", 2)
-            "s_branch .Lsc_left_b_back_%=\n")
+            GEO_SC_LEFT("a0", 36, 84, "x0", "x1", 0) GEO_SC_LEFT("a1", 44, 88, "x1", "x2", 1)
+            GEO_SC_LEFT("a2", 52, 92, "x2", "x3", 2) GEO_SC_LEFT("b0", 60, 96, "y0", "y1", 0)
+            GEO_SC_LEFT("b1", 68, 24, "y1", "y2", 1) GEO_SC_LEFT("b2", 76, 28, "y2", "y3", 2))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2), [y3] "=&v"(y3),
           [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
@@ -1095,14 +1085,13 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_FETCH6("y")
             "1:\n" GEO_SC_INDEX_ON
             GEO_SC_HALF("a0", "s18", 36, 84, "x0", "x1") GEO_SC_HALF("a1", "s19", 44, 88, "x1", "x2")
-            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3") GEO_SC_ANY_LEFT3("left_a", 84, 88, 92)
+            GEO_SC_HALF("a2", "s20", 52, 92, "x2", "x3")
             GEO_SC_WAIT_LINES
             "s_cmp_lt_u32 %[left], 2\n"
             "s_cbranch_scc1 1f\n"
             GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(320)
             "1:\n"
             GEO_SC_HALF("b0", "s21", 60, 96, "x3", "x4") GEO_SC_HALF("b1", "s22", 68, 24, "x4", "x5")
-            GEO_SC_ANY_LEFT2("left_b", 96, 24)
             "s_addk_i32 %[wo], 320\n" GEO_SC_NEXT_OR_END
             GEO_SC_INDEX_OFF
             "s_waitcnt vmcnt(0)\n"
@@ -1113,12 +1102,9 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             "v_mov_b32 %[x4], %[y4]\n"
             "v_mov_b32 %[x5], %[y5]\n"
             "s_branch 31b\n",
-            ".Lsc_left_a_%=:\n"
-            GEO_SC_LEFT(36, 84, "x0", "x1", 0) GEO_SC_LEFT(44, 88, "x1", "x2", 1) GEO_SC_LEFT(52, 92, "x2", "x3", 2)
-            "s_branch .Lsc_left_a_back_%=\n"
-            ".Lsc_left_b_%=:\n"
-            GEO_SC_LEFT(60, 96, "x3", "x4", 3) GEO_SC_LEFT(68, 24, "x4", "x5", 4)
-            "s_branch .Lsc_left_b_back_%=\n")
+            GEO_SC_LEFT("a0", 36, 84, "x0", "x1", 0) GEO_SC_LEFT("a1", 44, 88, "x1", "x2", 1)
+            GEO_SC_LEFT("a2", 52, 92, "x2", "x3", 2) GEO_SC_LEFT("b0", 60, 96, "x3", "x4", 3)
+            GEO_SC_LEFT("b1", 68, 24, "x4", "x5", 4))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [x4] "=&v"(x4), [x5] "=&v"(x5), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2),
           [y3] "=&v"(y3), [y4] "=&v"(y4), [y5] "=&v"(y5), [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
@@ -1143,29 +1129,30 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
     GEO_SC_X16(36, "wp", 32*L) GEO_SC_X8(52, "wp", 32*L+64) GEO_SC_X8(84, "ip", 16*L) GEO_SC_X4(92, "ip", 16*L+32)
 #define GEO_SC_HALVES_B(L)                                                                                             \
     GEO_SC_X16(60, "wp", 32*L) GEO_SC_X8(76, "wp", 32*L+64) GEO_SC_X4(96, "ip", 16*L) GEO_SC_X8(24, "ip", 16*L+16)
-#define GEO_SC_HALF16(W, F, X0, X1) GEO_SC_JUMP(F) GEO_SC_EIGHT(GEO_SC_SLOT64, W, F, X0, X1)
-#define GEO_SC_LEFT16(W, F, X0, X1, L)                                                                                 \
-    "s_bitcmp1_b32 s[" #F "+0], 24\n"                                                                                  \
-    "s_cbranch_scc0 2f\n"                                                                                              \
+#define GEO_SC_HALF16(LABEL, W, F, X0, X1)                                                                             \
+    GEO_SC_JUMP(F, 3) GEO_SC_RIGHT(LABEL, GEO_SC_SEVEN(GEO_SC_SLOT64, W, F, X0, X1))
+#define GEO_SC_LEFT16(LABEL, W, F, X0, X1, L)                                                                          \
+    ".Lsc_" LABEL "_left_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT64, W, F, X0, X1)                                              \
+    "s_bitcmp1_b32 s[" #F "+0], 11\n"                                                                                  \
+    "s_cbranch_scc0 .Lsc_" LABEL "_done_%=\n"                                                                          \
     "s_load_dwordx8 s[" #W ":" #W "+7], %[wl], 64*" #L "\n"                                                            \
     "s_load_dwordx4 s[" #F ":" #F "+3], %[il], 32*" #L "\n"                                                            \
     "s_waitcnt lgkmcnt(0)\n"                                                                                           \
-    GEO_SC_JUMP(F) GEO_SC_EIGHT(GEO_SC_SLOT64, W, F, X0, X1)                                                           \
-    "2:\n"
+    GEO_SC_JUMP(F, 3) GEO_SC_EIGHT(GEO_SC_SLOT64, W, F, X0, X1)                                                        \
+    "s_branch .Lsc_" LABEL "_done_%=\n"
+// N + 0, N + 1, N + 2 name the lines' labels
 #define GEO_SC_LINES16_A(N)                                                                                            \
-    GEO_SC_INDEX_ON GEO_SC_HALF16(36, 84, "x0", "x1") GEO_SC_HALF16(44, 88, "x2", "x3") GEO_SC_HALF16(52, 92, "x4", "x5") \
-    GEO_SC_ANY_LEFT3("left" #N, 84, 88, 92) GEO_SC_INDEX_OFF
+    GEO_SC_INDEX_ON GEO_SC_HALF16(#N "p0", 36, 84, "x0", "x1") GEO_SC_HALF16(#N "p1", 44, 88, "x2", "x3")              \
+    GEO_SC_HALF16(#N "p2", 52, 92, "x4", "x5") GEO_SC_INDEX_OFF
 #define GEO_SC_LINES16_B(N)                                                                                            \
-    GEO_SC_INDEX_ON GEO_SC_HALF16(60, 96, "y0", "y1") GEO_SC_HALF16(68, 24, "y2", "y3") GEO_SC_HALF16(76, 28, "y4", "y5") \
-    GEO_SC_ANY_LEFT3("left" #N, 96, 24, 28) GEO_SC_INDEX_OFF
+    GEO_SC_INDEX_ON GEO_SC_HALF16(#N "p0", 60, 96, "y0", "y1") GEO_SC_HALF16(#N "p1", 68, 24, "y2", "y3")              \
+    GEO_SC_HALF16(#N "p2", 76, 28, "y4", "y5") GEO_SC_INDEX_OFF
 #define GEO_SC_LEFT16_A(N)                                                                                             \
-    ".Lsc_left" #N "_%=:\n"                                                                                             \
-    GEO_SC_LEFT16(36, 84, "x0", "x1", N) GEO_SC_LEFT16(44, 88, "x2", "x3", (N + 1)) GEO_SC_LEFT16(52, 92, "x4", "x5", (N + 2)) \
-    "s_branch .Lsc_left" #N "_back_%=\n"
+    GEO_SC_LEFT16(#N "p0", 36, 84, "x0", "x1", N) GEO_SC_LEFT16(#N "p1", 44, 88, "x2", "x3", (N + 1))                  \
+    GEO_SC_LEFT16(#N "p2", 52, 92, "x4", "x5", (N + 2))
 #define GEO_SC_LEFT16_B(N)                                                                                             \
-    ".Lsc_left" #N "_%=:\n"                                                                                             \
-    GEO_SC_LEFT16(60, 96, "y0", "y1", N) GEO_SC_LEFT16(68, 24, "y2", "y3", (N + 1)) GEO_SC_LEFT16(76, 28, "y4", "y5", (N + 2)) \
-    "s_branch .Lsc_left" #N "_back_%=\n"
+    GEO_SC_LEFT16(#N "p0", 60, 96, "y0", "y1", N) GEO_SC_LEFT16(#N "p1", 68, 24, "y2", "y3", (N + 1))                  \
+    GEO_SC_LEFT16(#N "p2", 76, 28, "y4", "y5", (N + 2))
 // FX(N), FY(N): the activation words of lines N, N + 1, N + 2 to x and y; FY1(N): of line N
 #define GEO_SC_LINES16(WAIT, FX, FY, FY1)                                                                              \
     "s_nop 4\n" GEO_SC_HALVES_A(0) FX(0)                                                                               \
@@ -1174,9 +1161,10 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
     WAIT GEO_SC_HALVES_B(9) FY(9) GEO_SC_LINES16_A(6)                                                                 \
     WAIT GEO_SC_HALVES_A(12) FX(12) GEO_SC_LINES16_B(9)                                                               \
     WAIT GEO_SC_X8(60, "wp", 480) GEO_SC_X4(96, "ip", 240) FY1(15) GEO_SC_LINES16_A(12)                             \
-    WAIT GEO_SC_INDEX_ON GEO_SC_HALF16(60, 96, "y0", "y1") GEO_SC_LEFT16(60, 96, "y0", "y1", 15)                       \
+    WAIT GEO_SC_INDEX_ON GEO_SC_HALF16("15p0", 60, 96, "y0", "y1")                                                     \
     "s_branch 99f\n"                                                                                                   \
     GEO_SC_LEFT16_A(0) GEO_SC_LEFT16_B(3) GEO_SC_LEFT16_A(6) GEO_SC_LEFT16_B(9) GEO_SC_LEFT16_A(12)                    \
+    GEO_SC_LEFT16("15p0", 60, 96, "y0", "y1", 15)                                                                      \
     "99:\n" GEO_SC_INDEX_OFF
 
 // OR of one (pack, add group) pair over share `share` of `shares` of the group's channels, assigned to the
@@ -1649,7 +1637,7 @@ void k_conv_fwd_items_rail_lds(FwdParams q)
 #pragma unroll 8
         for (int i = 0; i < 8 * NWV; i++) {
             const RailLines at(q, first_tile + i % NWV, (size_t)(i / NWV) * (q.rail_lines / 8));
-            zeros += (at.f[0] >> 24) & 15u;
+            zeros += (at.f[0] >> 8) & 15u;
         }
     }
     fetch(group_off, 0);

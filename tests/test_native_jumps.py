@@ -1,0 +1,101 @@
+"""The forward kernels jump over the zero words of a weight line by a number that they read from the line, and a caller may hand
+them any buffer.  Here the built code is disassembled, and every computed jump is followed for every value of the 16 bits that it
+reads: it has to land on a slot (an instruction that sets M0) or on a branch, never inside an instruction."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+def code_objects(path):
+    with open(path, "rb") as f:
+        data = f.read()
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        (entries,), p = struct.unpack_from("<Q", data, at + 24), at + 32
+        for _ in range(entries):
+            offset, size, name_len = struct.unpack_from("<QQQ", data, p)
+            if b"gfx950" in data[p + 24:p + 24 + name_len]:
+                yield data[at + offset:at + offset + size]
+            p += 24 + name_len
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+
+
+def kernels(path, tmp_path):
+    """name -> [(address, mnemonic, operands)]"""
+    out = {}
+    for i, obj in enumerate(code_objects(path)):
+        f = tmp_path / f"{i}.co"
+        f.write_bytes(obj)
+        text = subprocess.run([OBJDUMP, "-d", str(f)], check=True, capture_output=True, text=True).stdout
+        name = None
+        for line in text.splitlines():
+            m = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            if m:
+                name = m.group(1)
+            m = re.match(r"\s+(\S+)\s*(.*?)\s*// ([0-9A-F]+):", line)
+            if m and name:
+                out.setdefault(name, []).append((int(m.group(3), 16), m.group(1), [o.strip() for o in m.group(2).split(",")]))
+    return out
+
+
+def low(reg):
+    return "vcc_lo" if reg == "vcc" else re.sub(r"s\[(\d+):\d+\]", r"s\1", reg)
+
+
+def targets(code, i, bases):
+    """where the s_setpc_b64 at index i goes, for every value of the bits that the s_bfe_u32 in front of it takes"""
+    start = next(j for j in range(i, max(-1, i - 10), -1) if code[j][1] == "s_bfe_u32")
+    field, spec = code[start][2][1], int(code[start][2][2], 0)
+    assert re.match(r"s\d+$", field)
+    reach = set()
+    for bits in range(1 << 16):
+        reach.add(bits >> (spec & 31) & ((1 << (spec >> 16)) - 1))
+    for number in reach:
+        regs = dict(bases)
+        regs[code[start][2][0]] = number
+
+        def value(o):
+            return regs[o] if o in regs else int(o, 0)
+        for addr, op, args in code[start + 1:i]:
+            if op == "s_getpc_b64":
+                regs[low(args[0])] = addr + 4
+            elif op == "s_mulk_i32":
+                regs[args[0]] *= int(args[1], 0)
+            elif op == "s_addk_i32":
+                regs[args[0]] += int(args[1], 0)
+            elif op == "s_add_u32":
+                regs[args[0]] = value(args[1]) + value(args[2])
+            elif re.match(r"s_lshl[1-4]_add_u32$", op):
+                regs[args[0]] = (value(args[1]) << int(op[6])) + value(args[2])
+            elif op != "s_addc_u32":  # (the upper halves: the code lies in one 4 GB here)
+                raise AssertionError(f"{op} in front of a jump")
+        yield number, regs[low(code[i][2][0])]
+
+
+def test_computed_jumps_land_on_slots(tmp_path):
+    from geo_amd import _native
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no disassembler here")
+    jumps = 0
+    for name, code in kernels(_native.lib_path(), tmp_path).items():
+        at = {addr: i for i, (addr, _, _) in enumerate(code)}
+        bases, pc = {}, None
+        for i, (addr, op, args) in enumerate(code):
+            if op == "s_getpc_b64" and args[0] == "vcc":
+                pc = addr + 4
+            if op == "s_add_u32" and args[1] == "vcc_lo" and pc is not None:
+                offset = int(args[2], 0)
+                bases[args[0]] = pc + (offset - (1 << 32) if offset >> 31 else offset)
+            if op != "s_setpc_b64":
+                continue
+            jumps += 1
+            for number, target in targets(code, i, bases):
+                assert target in at, f"{name}: {number} words at {addr:#x} lead into an instruction"
+                t_op, t_args = code[at[target]][1], code[at[target]][2]
+                assert t_op in ("s_branch", "s_set_gpr_idx_on") or t_args[0] == "m0", f"{name}: {number} words at {addr:#x} lead to {t_op}"
+    assert jumps > 0
