@@ -827,6 +827,7 @@ struct PairLane {
 //   HALF  (kHalfZeros or more)              only the right halves of the lines (slots 8 - 15) are loaded, so that two
 //                                           stages of lines fit the scalar registers and one is in flight while the other is
 //                                           ORed; the left half of a line with more than eight words is loaded where it is met.
+//                                           Where many of them need it the rest of the group changes loops (GEO_SC_FALL_IF).
 // What bounds them: DENSE the issue of v_and_or_b32; HALF the scalar instructions, one per SIMD and four cycles like
 // the vector ones, of which a line takes one per word and four for its jump.
 // One block with its loads and waits inside, registers assigned by hand: scalar loads return out of order, so only
@@ -881,11 +882,12 @@ struct PairLane {
     ".Lsc_" LABEL "_%=:\n"                                                                                             \
     "s_branch .Lsc_" LABEL "_left_%=\n"                                                                                \
     "s_nop 0\ns_nop 0\ns_nop 0\ns_nop 0\n" SEVEN ".Lsc_" LABEL "_done_%=:\n"
+// (three words that no wave comes to: a line's code is 192 bytes, and the loop begins at a multiple of 32; without, 0.5 % more)
 #define GEO_SC_HALF(LABEL, BASE, W, F, X0, X1)                                                                         \
-    GEO_SC_JUMP_FROM(BASE, F) GEO_SC_RIGHT(LABEL, GEO_SC_SEVEN(GEO_SC_SLOT, W, F, X0, X1))
+    GEO_SC_JUMP_FROM(BASE, F) "s_nop 0\ns_nop 0\ns_nop 0\n" GEO_SC_RIGHT(LABEL, GEO_SC_SEVEN(GEO_SC_SLOT, W, F, X0, X1))
 #define GEO_SC_BASE(LABEL, BASE) "s_add_u32 " BASE ", vcc_lo, .Lsc_" LABEL "_%=-.Lsc_pc_%=\n"
-// line L of its channel, of eight words or more
-#define GEO_SC_LEFT(LABEL, W, F, X0, X1, L)                                                                            \
+// line L of its channel, of eight words or more; AFTER: behind its left half
+#define GEO_SC_LEFT(LABEL, BASE, W, F, X0, X1, L, AFTER)                                                               \
     ".Lsc_" LABEL "_left_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                \
     "s_bitcmp1_b32 s[" #F "+0], 11\n"                                                                                  \
     "s_cbranch_scc0 .Lsc_" LABEL "_done_%=\n"                                                                          \
@@ -893,8 +895,41 @@ struct PairLane {
     "s_load_dwordx8 s[" #W ":" #W "+7], %[wp], %[wo] offset:64*" #L "\n"                                               \
     "s_load_dwordx4 s[" #F ":" #F "+3], %[ip], s33 offset:32*" #L "\n"                                                 \
     "s_waitcnt lgkmcnt(0)\n"                                                                                           \
-    GEO_SC_JUMP(F, 3) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                          \
+    "s_bfe_u32 s33, s[" #F "+0], 3<<16|8\n"                                                                            \
+    "s_lshl4_add_u32 vcc_lo, s33, " BASE "\n"                                                                          \
+    "s_lshl2_add_u32 vcc_lo, s33, vcc_lo\n"                                                                            \
+    "s_add_u32 vcc_lo, vcc_lo, .Lsc_" LABEL "_half_%=-.Lsc_" LABEL "_%=\n"                                             \
+    "s_setpc_b64 vcc\n"                                                                                                \
+    ".Lsc_" LABEL "_half_%=:\n" GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1)                                                \
+    AFTER                                                                                                              \
     "s_branch .Lsc_" LABEL "_done_%=\n"
+// The first lines can be emptier than the rest of the group.  A level rises by 4 with each line of stage B that needs its left half,
+// falls by DECAY with each channel (by two for each line of stage B) and not below 0; above 10 the next channels go through another
+// loop, DENSE where the stage's last line has fewer than kSkipZeros zero words.  %[cnt]: the level, less DECAY for each channel
+// that is left.  A first channel without words in front of full ones, 64 -> 64 at 28 x 28, batch 64, L 128: 289 us, 370 in HALF to
+// the end, 294 before any words were skipped.
+#define GEO_SC_RISE "s_addk_i32 %[cnt], 4\n"
+#define GEO_SC_FALL_IF(DECAY)                                                                                          \
+    "s_mul_i32 s33, %[left], " #DECAY "\n"                                                                             \
+    "s_add_i32 %[cnt], %[cnt], s33\n"                                                                                  \
+    "s_max_i32 %[cnt], %[cnt], 0\n"                                                                                    \
+    "s_addk_i32 %[cnt], 4\n"                                                                                           \
+    "s_cmp_gt_i32 %[cnt], 10\n"                                                                                         \
+    "s_cbranch_scc1 .Lsc_fall_%=\n"                                                                                    \
+    "s_sub_i32 %[cnt], %[cnt], s33\n"
+// 0 at the first channel of stage B
+#define GEO_SC_FALL_COUNT(DECAY, CHANNELS)                                                                             \
+    "s_sub_u32 %[cnt], " #CHANNELS ", %[left]\n"                                                                       \
+    "s_mul_i32 %[cnt], %[cnt], " #DECAY "\n"
+// B: bytes of a channel's lines; F: the first field of the last line's left half; the next channel's words are on their way
+#define GEO_SC_FALL(B, F, TO_DENSE, TO_SKIP)                                                                           \
+    ".Lsc_fall_%=:\n"                                                                                                  \
+    "s_addk_i32 %[wo], " #B "\n" GEO_SC_NEXT_OR_END                                                                    \
+    "s_waitcnt lgkmcnt(0)\n"                                                                                           \
+    "s_bfe_u32 s34, s[" #F "+0], 3<<16|8\n" GEO_SC_LOADS_FULL                                                          \
+    "s_cmp_lt_u32 s34, %[zskip]/3\n"                                                                                   \
+    "s_cbranch_scc1 " TO_DENSE "\n"                                                                                    \
+    "s_branch " TO_SKIP "\n"
 // loads of line L of the channel AT bytes behind %[wo] (in the words; half of it in the fields, s33)
 #define GEO_SC_FIELD_OFFSET "s_lshr_b32 s33, %[wo], 1\n"
 #define GEO_SC_LOAD(W, F, L)                                                                                           \
@@ -944,7 +979,7 @@ struct PairLane {
     GEO_SC_NEXT_OR_END
 // the first channel's first line
 #define GEO_SC_LINE0                                                                                                   \
-    "s_cmp_lg_u32 %[row], 0\n"                                                                                         \
+    "s_cmp_lg_u32 %[cnt], 0\n"                                                                                         \
     "s_cbranch_scc1 3f\n"                                                                                              \
     GEO_SC_FIRST(36, 84, "x0", "x1")                                                                                   \
     "s_branch 4f\n"                                                                                                    \
@@ -978,7 +1013,7 @@ struct PairLane {
 // The first channel (its first line assigns where `row` is 0), then a loop; each has the channel's words in x or y in turn.
 // The order of the code keeps a short DENSE group to one jump, which is under way with its first loads: an instruction fetch
 // from a place that no wave of the CU has been to takes longer than a line.
-#define GEO_SC_OR_CHANNELS(B, FETCHES, FIRST_CHANNEL, REST_OF_FIRST, CHANNEL, BASES, HALF_LOOP, LEFT_HALVES)           \
+#define GEO_SC_OR_CHANNELS(B, FETCHES, FIRST_CHANNEL, REST_OF_FIRST, CHANNEL, BASES, FALL_COUNT, HALF_LOOP, LEFT_HALVES) \
     "s_nop 4\n" /* the compiler may have written an operand of the loads with a vector instruction just before */      \
     GEO_SC_LOADS_FULL FETCHES                                                                                          \
     "s_branch 7f\n"                                                                                                    \
@@ -997,18 +1032,18 @@ struct PairLane {
     /* all slots between here and 99 in one 4 GB: a carry takes the other loop */                                      \
     "s_add_u32 s33, vcc_lo, 99f-.Lsc_pc_%=\n"                                                                          \
     "s_cbranch_scc1 20b\n"                                                                                             \
-    GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(0) BASES                                                                   \
-    "31:\n" HALF_LOOP LEFT_HALVES                                                                                      \
+    GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(0) BASES FALL_COUNT                                                        \
+    ".p2align 5\n31:\n" HALF_LOOP LEFT_HALVES                                                                                      \
     "7:\n" GEO_SC_WAIT_ALL GEO_SC_COUNT_ZEROS                                                                          \
     "s_cmp_ge_u32 s35, %[zhalf]\n"                                                                                     \
     "s_cbranch_scc1 5b\n"                                                                                              \
     FIRST_CHANNEL                                                                                                      \
     "s_cmp_ge_u32 s35, %[zskip]\n"                                                                                     \
     "s_cbranch_scc1 22b\n"                                                                                             \
-    "12:\n" CHANNEL(GEO_SC_DENSE, "y", "x") CHANNEL(GEO_SC_DENSE, "x", "y") "s_branch 12b\n"                           \
+    "12:\n" CHANNEL(GEO_SC_DENSE, "y", "x") "13:\n" CHANNEL(GEO_SC_DENSE, "x", "y") "s_branch 12b\n"                  \
     "99:\n" GEO_SC_INDEX_OFF
 #define GEO_SC_OR_OPERANDS                                                                                             \
-    [wp] "s"(wp), [ip] "s"(ip), [act] "s"(act), [orb] "s"(or_b), [row] "s"(row), [zskip] "n"(3 * kSkipZeros),          \
+    [wp] "s"(wp), [ip] "s"(ip), [act] "s"(act), [orb] "s"(or_b), [zskip] "n"(3 * kSkipZeros), \
         [zhalf] "n"(3 * kHalfZeros), [v0] "v"(voff[0]), [v1] "v"(voff[1]), [v2] "v"(voff[2]), [v3] "v"(voff[3])
 #define GEO_SC_OR_CLOBBERS                                                                                            \
     "m0", "scc", "vcc", "memory", "s18", "s19", "s20", "s21", "s22", "s23", "s24", "s25", "s26", "s27", "s28",         \
@@ -1042,7 +1077,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
     asm volatile(
         GEO_SC_OR_CHANNELS(192, GEO_SC_FETCH4("x"), GEO_SC_FIRST_CHANNEL3, "", GEO_SC_CHANNEL3,
             GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
-            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22") GEO_SC_BASE("b2", "s23"),
+            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22") GEO_SC_BASE("b2", "s23"), GEO_SC_FALL_COUNT(3, 1),
             GEO_SC_HALF_CHANNEL3(GEO_SC_LOAD_HALF(60, 96, 0, 192) GEO_SC_LOAD_HALF(68, 24, 1, 192)
                                  GEO_SC_LOAD_HALF(76, 28, 2, 192), GEO_SC_FETCH4("y"))
             GEO_SC_HALF("a0", "s18", 36, 84, "x0", "x1") GEO_SC_HALF("a1", "s19", 44, 88, "x1", "x2")
@@ -1053,12 +1088,13 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_HALF("b2", "s23", 76, 28, "y2", "y3")
             "s_addk_i32 %[wo], 192\n" GEO_SC_NEXT_OR_END
             "s_branch 31b\n",
-            GEO_SC_LEFT("a0", 36, 84, "x0", "x1", 0) GEO_SC_LEFT("a1", 44, 88, "x1", "x2", 1)
-            GEO_SC_LEFT("a2", 52, 92, "x2", "x3", 2) GEO_SC_LEFT("b0", 60, 96, "y0", "y1", 0)
-            GEO_SC_LEFT("b1", 68, 24, "y1", "y2", 1) GEO_SC_LEFT("b2", 76, 28, "y2", "y3", 2))
+            GEO_SC_LEFT("a0", "s18", 36, 84, "x0", "x1", 0, "") GEO_SC_LEFT("a1", "s19", 44, 88, "x1", "x2", 1, "")
+            GEO_SC_LEFT("a2", "s20", 52, 92, "x2", "x3", 2, "") GEO_SC_LEFT("b0", "s21", 60, 96, "y0", "y1", 0, GEO_SC_RISE)
+            GEO_SC_LEFT("b1", "s22", 68, 24, "y1", "y2", 1, GEO_SC_RISE) GEO_SC_LEFT("b2", "s23", 76, 28, "y2", "y3", 2, GEO_SC_FALL_IF(3))
+            GEO_SC_FALL(192, 28, "13f", "21b"))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2), [y3] "=&v"(y3),
-          [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
+          [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left), [cnt] "+&s"(row)
         : GEO_SC_OR_OPERANDS
         : GEO_SC_OR_CLOBBERS);
 }
@@ -1076,7 +1112,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_DENSE(36, 84, "x3", "x4") GEO_SC_DENSE(52, 92, "x4", "x5"),
             GEO_SC_CHANNEL5,
             GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
-            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22"),
+            GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22"), GEO_SC_FALL_COUNT(4, 0),
             GEO_SC_WAIT_ALL
             GEO_SC_FIELD_OFFSET GEO_SC_LOAD_HALF(60, 96, 3, 0) GEO_SC_LOAD_HALF(68, 24, 4, 0)
             "s_cmp_lt_u32 %[left], 2\n"
@@ -1102,12 +1138,13 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             "v_mov_b32 %[x4], %[y4]\n"
             "v_mov_b32 %[x5], %[y5]\n"
             "s_branch 31b\n",
-            GEO_SC_LEFT("a0", 36, 84, "x0", "x1", 0) GEO_SC_LEFT("a1", 44, 88, "x1", "x2", 1)
-            GEO_SC_LEFT("a2", 52, 92, "x2", "x3", 2) GEO_SC_LEFT("b0", 60, 96, "x3", "x4", 3)
-            GEO_SC_LEFT("b1", 68, 24, "x4", "x5", 4))
+            GEO_SC_LEFT("a0", "s18", 36, 84, "x0", "x1", 0, "") GEO_SC_LEFT("a1", "s19", 44, 88, "x1", "x2", 1, "")
+            GEO_SC_LEFT("a2", "s20", 52, 92, "x2", "x3", 2, "") GEO_SC_LEFT("b0", "s21", 60, 96, "x3", "x4", 3, GEO_SC_RISE)
+            GEO_SC_LEFT("b1", "s22", 68, 24, "x4", "x5", 4, GEO_SC_FALL_IF(4))
+            GEO_SC_FALL(320, 24, "12f", "22b"))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [x4] "=&v"(x4), [x5] "=&v"(x5), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2),
-          [y3] "=&v"(y3), [y4] "=&v"(y4), [y5] "=&v"(y5), [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left)
+          [y3] "=&v"(y3), [y4] "=&v"(y4), [y5] "=&v"(y5), [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left), [cnt] "+&s"(row)
         : GEO_SC_OR_OPERANDS, [v4] "v"(voff[4]), [v5] "v"(voff[5])
         : GEO_SC_OR_CLOBBERS);
 }

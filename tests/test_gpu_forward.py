@@ -716,3 +716,56 @@ def test_weight_generator_tiles(capi, so, shape_x, shape_w, mode):
     exp = so.conv2d_modes(x.numpy(), w.numpy(), 32, (0, 0), mode, 32, 7, 2, 2, 2)
     got = capi.conv2d_add_partial_from_streams(capi.act_streams(x.cuda(), d), capi.weight_streams(w.cuda(), d), d)
     assert np.array_equal(got.cpu().numpy(), exp)
+
+
+def thinned(w, keep, seed):
+    """w with `keep` (of w.shape[1:]) channels of every 16 at random, none of their words empty"""
+    w = torch.where(w == 0, torch.full_like(w, 0.5), w.sign() * (0.75 + 0.25 * w.abs()))
+    order = torch.rand(w.shape, generator=torch.Generator().manual_seed(seed))
+    for c0 in range(0, w.shape[0], 16):
+        w[c0:c0 + 16] *= order[c0:c0 + 16].argsort(0).argsort(0) < keep
+    return w.contiguous()
+
+
+@pytest.mark.parametrize("sparse", [1, 2, 3, 4])
+@pytest.mark.parametrize("full,column", [(16, 16), (12, 12), (15, 0), (9, 6)])
+@pytest.mark.parametrize("shape_x,shape_w,pad", [
+    ((30, 9, 16, 16), (20, 9, 3, 3), 1), ((30, 6, 16, 16), (20, 6, 3, 3), 1), ((20, 24, 12, 13), (48, 24, 3, 3), 1),
+    ((24, 8, 12, 13), (20, 8, 5, 5), 2), ((24, 17, 12, 13), (40, 17, 5, 5), 2), ((24, 3, 12, 13), (20, 3, 5, 5), 2)])
+def test_full_weight_lines_behind_empty_ones(capi, so, shape_x, shape_w, pad, full, column, sparse):
+    """The first `sparse` channels' lines hold three words, the others' `full`, of their first kernel column `column`: the change from the
+    loop for mostly empty lines to the others behind either of its channels, and behind the last.  Bit for bit."""
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=shape_w[0] + sparse + full)
+    keep = torch.full(w.shape[1:], full)
+    keep[:, 0] = column
+    keep[:sparse] = 3
+    w = thinned(w, keep, sparse)
+    assert np.array_equal(gpu_forward(capi, x, w, 32, (pad, pad)), so.conv2d_add_partial(x.numpy(), w.numpy(), 32, (pad, pad)))
+
+
+def launch_time(capi, shape_x, shape_w, pad, L, keep):
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=3)
+    d = capi.make_desc(shape_x, shape_w, L, (pad, pad))
+    act, wgt = capi.act_streams(x.cuda(), d), capi.weight_streams(thinned(w, keep, 5).cuda(), d)
+    y = capi.conv2d_add_partial_from_streams(act, wgt, d)
+    best = 1e9
+    for _ in range(8):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(10):
+            capi.conv2d_add_partial_from_streams(act, wgt, d, out=y)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+@pytest.mark.parametrize("first", [0, 8])
+def test_full_weight_lines_behind_empty_ones_take_their_time(capi, first):
+    """A group whose first channel is nearly empty is no slower than one of full lines (1.24 times that if it stays in the loop for
+    mostly empty lines; 1.00 - 1.01 measured)."""
+    shape_x, shape_w = (64, 64, 28, 28), (64, 64, 3, 3)
+    keep = torch.full(shape_w[1:], 16)
+    full = launch_time(capi, shape_x, shape_w, 1, 128, keep)
+    keep[0] = first
+    assert launch_time(capi, shape_x, shape_w, 1, 128, keep) < 1.12 * full
