@@ -839,11 +839,11 @@ struct PairLane {
 // s[34:35]: temporary, and the zero words of the first lines.
 // Index mode stays on between the loads of a channel and the next one's: nothing but the slots' vector instructions is issued.
 #define GEO_SC_SLOT(SET, W, I, X0, X1)                                                                                 \
-    SET "v_and_or_b32 v32, s[" #W "+" #I "], %[" X0 "], v32\n"                                                          \
+    SET "v_and_or_b32 v32, s[" #W "+" #I "], %[" X0 "], v32\n"                                                         \
         "v_and_or_b32 v33, s[" #W "+" #I "], %[" X1 "], v33\n"
 #define GEO_SC_SLOT_FIRST(SET, W, I, X0, X1)                                                                           \
-    SET "v_and_b32 v32, s[" #W "+" #I "], %[" X0 "]\n"                                                                  \
-        "v_and_b32 v33, s[" #W "+" #I "], %[" X1 "]\n"                                                                  \
+    SET "v_and_b32 v32, s[" #W "+" #I "], %[" X0 "]\n"                                                                 \
+        "v_and_b32 v33, s[" #W "+" #I "], %[" X1 "]\n"                                                                 \
         "s_xor_b32 m0, m0, 32\n"                                                                                       \
         "v_mov_b32 v32, 0\n"                                                                                           \
         "v_mov_b32 v33, 0\n"
@@ -872,10 +872,23 @@ struct PairLane {
     "s_lshl4_add_u32 vcc_lo, s33, " BASE "\n"                                                                          \
     "s_lshl2_add_u32 vcc_lo, s33, vcc_lo\n"                                                                            \
     "s_setpc_b64 vcc\n"
-#define GEO_SC_DENSE(W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W + 8, F + 4, X0, X1)
+#define GEO_SC_WHOLE(W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT, W + 8, F + 4, X0, X1)
 #define GEO_SC_FIRST(W, F, X0, X1)                                                                                     \
     GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W, F, X0, X1) GEO_SC_EIGHT(GEO_SC_SLOT_FIRST, W + 8, F + 4, X0, X1)
-#define GEO_SC_SKIP(W, F, X0, X1) GEO_SC_JUMP(F, 4) GEO_SC_DENSE(W, F, X0, X1)
+// A line of the loops DENSE and SKIP, the I-th of its channel; X: "x" or "y", the channel's words.  SKIP: past the jump where no word
+// is zero (64 -> 64 at 28 x 28, batch 64, L 128, 12 words in the first channel's lines and 16 in the others': 296 us, 323 with a jump
+// at every line); s18 + I and vcc_hi hold the address of the line's first slot in the loop's copy for x (GEO_SC_SKIP_BASES).
+#define GEO_SC_DENSE(X, I, W, F, X0, X1) GEO_SC_WHOLE(W, F, X0, X1)
+#define GEO_SC_SKIP(X, I, W, F, X0, X1)                                                                                \
+    "s_bfe_u32 s33, s[" #F "+0], 4<<16|8\n"                                                                            \
+    "s_cbranch_scc0 .Lsc_s" X #I "_%=\n"                                                                               \
+    "s_lshl4_add_u32 vcc_lo, s33, s[18+" #I "]\n"                                                                      \
+    "s_lshl2_add_u32 vcc_lo, s33, vcc_lo\n"                                                                            \
+    ".ifnc " X ",x\n"                                                                                                  \
+    "s_add_u32 vcc_lo, vcc_lo, .Lsc_sy" #I "_%=-.Lsc_sx" #I "_%=\n"                                                    \
+    ".endif\n"                                                                                                         \
+    "s_setpc_b64 vcc\n"                                                                                                \
+    ".Lsc_s" X #I "_%=:\n" GEO_SC_WHOLE(W, F, X0, X1)
 // A line's right half behind a jump, slots 9 to 15 at places 1 to 7.  Place 0, as long as a slot, leaves for a copy of the eight slots
 // (GEO_SC_LEFT, out of line) behind which the left half is loaded if it holds words.
 #define GEO_SC_RIGHT(LABEL, SEVEN)                                                                                     \
@@ -914,7 +927,7 @@ struct PairLane {
     "s_add_i32 %[cnt], %[cnt], s33\n"                                                                                  \
     "s_max_i32 %[cnt], %[cnt], 0\n"                                                                                    \
     "s_addk_i32 %[cnt], 4\n"                                                                                           \
-    "s_cmp_gt_i32 %[cnt], 10\n"                                                                                         \
+    "s_cmp_gt_i32 %[cnt], 10\n"                                                                                        \
     "s_cbranch_scc1 .Lsc_fall_%=\n"                                                                                    \
     "s_sub_i32 %[cnt], %[cnt], s33\n"
 // 0 at the first channel of stage B
@@ -962,20 +975,20 @@ struct PairLane {
 // One channel with its words in X, the next one's to Y.
 #define GEO_SC_CHANNEL3(LINE, X, Y)                                                                                    \
     GEO_SC_WAIT_ALL GEO_SC_INDEX_OFF GEO_SC_AHEAD(192, GEO_SC_FETCH4(Y)) GEO_SC_INDEX_ON                               \
-    LINE(36, 84, X "0", X "1") GEO_SC_LOAD_NEXT(36, 84, 0)                                                             \
-    LINE(52, 92, X "1", X "2") GEO_SC_LOAD_NEXT(52, 92, 1)                                                             \
-    LINE(68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                             \
+    LINE(X, 0, 36, 84, X "0", X "1") GEO_SC_LOAD_NEXT(36, 84, 0)                                                       \
+    LINE(X, 1, 52, 92, X "1", X "2") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
+    LINE(X, 2, 68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
     GEO_SC_NEXT_OR_END
 // (lines 3 and 4 take the place of lines 0 and 1)
 #define GEO_SC_CHANNEL5(LINE, X, Y)                                                                                    \
     GEO_SC_WAIT_ALL GEO_SC_INDEX_ON                                                                                    \
-    LINE(36, 84, X "0", X "1") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3)                                              \
-    LINE(52, 92, X "1", X "2") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(52, 92, 4)                                              \
+    LINE(X, 0, 36, 84, X "0", X "1") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3)                                        \
+    LINE(X, 1, 52, 92, X "1", X "2") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(52, 92, 4)                                        \
     GEO_SC_INDEX_OFF GEO_SC_AHEAD(320, GEO_SC_FETCH6(Y)) GEO_SC_INDEX_ON                                               \
-    LINE(68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                             \
+    LINE(X, 2, 68, 24, X "2", X "3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
     GEO_SC_WAIT_LINES                                                                                                  \
-    LINE(36, 84, X "3", X "4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                             \
-    LINE(52, 92, X "4", X "5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                             \
+    LINE(X, 3, 36, 84, X "3", X "4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                       \
+    LINE(X, 4, 52, 92, X "4", X "5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
     GEO_SC_NEXT_OR_END
 // the first channel's first line
 #define GEO_SC_LINE0                                                                                                   \
@@ -983,22 +996,22 @@ struct PairLane {
     "s_cbranch_scc1 3f\n"                                                                                              \
     GEO_SC_FIRST(36, 84, "x0", "x1")                                                                                   \
     "s_branch 4f\n"                                                                                                    \
-    "3:\n" GEO_SC_DENSE(36, 84, "x0", "x1") "4:\n"
+    "3:\n" GEO_SC_WHOLE(36, 84, "x0", "x1") "4:\n"
 // the first channel in front of DENSE and SKIP: the next one's loads go out as in the loops
 #define GEO_SC_FIRST_CHANNEL3                                                                                          \
     GEO_SC_AHEAD(192, GEO_SC_FETCH4("y")) GEO_SC_INDEX_ON                                                              \
     GEO_SC_LINE0 GEO_SC_LOAD_NEXT(36, 84, 0)                                                                           \
-    GEO_SC_DENSE(52, 92, "x1", "x2") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
-    GEO_SC_DENSE(68, 24, "x2", "x3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
+    GEO_SC_WHOLE(52, 92, "x1", "x2") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
+    GEO_SC_WHOLE(68, 24, "x2", "x3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
     GEO_SC_NEXT_OR_END
 #define GEO_SC_FIRST_CHANNEL5                                                                                          \
     GEO_SC_INDEX_ON GEO_SC_LINE0 GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3)                                            \
-    GEO_SC_DENSE(52, 92, "x1", "x2") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(52, 92, 4)                                        \
+    GEO_SC_WHOLE(52, 92, "x1", "x2") GEO_SC_FIELD_OFFSET GEO_SC_LOAD(52, 92, 4)                                        \
     GEO_SC_INDEX_OFF GEO_SC_AHEAD(320, GEO_SC_FETCH6("y")) GEO_SC_INDEX_ON                                             \
-    GEO_SC_DENSE(68, 24, "x2", "x3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
+    GEO_SC_WHOLE(68, 24, "x2", "x3") GEO_SC_LOAD_NEXT(68, 24, 2)                                                       \
     GEO_SC_WAIT_LINES                                                                                                  \
-    GEO_SC_DENSE(36, 84, "x3", "x4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                       \
-    GEO_SC_DENSE(52, 92, "x4", "x5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
+    GEO_SC_WHOLE(36, 84, "x3", "x4") GEO_SC_LOAD_NEXT(36, 84, 0)                                                       \
+    GEO_SC_WHOLE(52, 92, "x4", "x5") GEO_SC_LOAD_NEXT(52, 92, 1)                                                       \
     GEO_SC_NEXT_OR_END
 // the first lines' zero words (bits 11:8 of the first field word) pick the loop for the channels behind the first
 #define GEO_SC_COUNT_ZEROS                                                                                             \
@@ -1010,19 +1023,33 @@ struct PairLane {
 #define GEO_SC_LOADS_FULL GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 0) GEO_SC_LOAD(52, 92, 1) GEO_SC_LOAD(68, 24, 2)
 #define GEO_SC_LOADS_HALF_A(AT)                                                                                        \
     GEO_SC_LOAD_HALF(36, 84, 0, AT) GEO_SC_LOAD_HALF(44, 88, 1, AT) GEO_SC_LOAD_HALF(52, 92, 2, AT)
+// The addresses that SKIP's jumps start from, where the code from here to 99 lies in one 4 GB, otherwise to DENSE; AT: a label's name.
+#define GEO_SC_SKIP_BASES(AT, DENSE, BASES)                                                                            \
+    "s_getpc_b64 vcc\n"                                                                                                \
+    ".Lsc_pc" AT "_%=:\n"                                                                                              \
+    "s_add_u32 s33, vcc_lo, 99f-.Lsc_pc" AT "_%=\n"                                                                    \
+    "s_cbranch_scc1 " DENSE "\n" BASES
+#define GEO_SC_SKIP_BASE(AT, I) "s_add_u32 s[18+" #I "], vcc_lo, .Lsc_sx" #I "_%=-.Lsc_pc" AT "_%=\n"
+#define GEO_SC_SKIP_BASES3(AT, DENSE)                                                                                  \
+    GEO_SC_SKIP_BASES(AT, DENSE, GEO_SC_SKIP_BASE(AT, 0) GEO_SC_SKIP_BASE(AT, 1) GEO_SC_SKIP_BASE(AT, 2))
+#define GEO_SC_SKIP_BASES5(AT, DENSE)                                                                                  \
+    GEO_SC_SKIP_BASES(AT, DENSE, GEO_SC_SKIP_BASE(AT, 0) GEO_SC_SKIP_BASE(AT, 1) GEO_SC_SKIP_BASE(AT, 2)               \
+                      GEO_SC_SKIP_BASE(AT, 3) GEO_SC_SKIP_BASE(AT, 4))
 // The first channel (its first line assigns where `row` is 0), then a loop; each has the channel's words in x or y in turn.
 // The order of the code keeps a short DENSE group to one jump, which is under way with its first loads: an instruction fetch
 // from a place that no wave of the CU has been to takes longer than a line.
-#define GEO_SC_OR_CHANNELS(B, FETCHES, FIRST_CHANNEL, REST_OF_FIRST, CHANNEL, BASES, FALL_COUNT, HALF_LOOP, LEFT_HALVES) \
+#define GEO_SC_OR_CHANNELS(B, FETCHES, FIRST_CHANNEL, REST_OF_FIRST, CHANNEL, SKIP_BASES, BASES, FALL_COUNT, HALF_LOOP, LEFT_HALVES) \
     "s_nop 4\n" /* the compiler may have written an operand of the loads with a vector instruction just before */      \
     GEO_SC_LOADS_FULL FETCHES                                                                                          \
     "s_branch 7f\n"                                                                                                    \
-    /* SKIP, entered at 20 with nothing loaded but the words on their way to x, at 22 with all on its way, words to y */ \
+    /* SKIP, entered at 20 with nothing loaded but the words on their way to x, at 23 and 24 with all on its way, words to x or y */ \
+    "24:\n" SKIP_BASES("y", "12f") "s_branch 22f\n"                                                                    \
     "20:\n" GEO_SC_LOADS_FULL                                                                                          \
-    "21:\n" CHANNEL(GEO_SC_SKIP, "x", "y") "22:\n" CHANNEL(GEO_SC_SKIP, "y", "x") "s_branch 21b\n"                    \
+    "23:\n" SKIP_BASES("x", "13f")                                                                                     \
+    "21:\n" CHANNEL(GEO_SC_SKIP, "x", "y") "22:\n" CHANNEL(GEO_SC_SKIP, "y", "x") "s_branch 21b\n"                     \
     /* HALF: its first channel, too, takes whole lines */                                                              \
     "5:\n" GEO_SC_INDEX_ON GEO_SC_LINE0                                                                                \
-    GEO_SC_DENSE(52, 92, "x1", "x2") GEO_SC_DENSE(68, 24, "x2", "x3") REST_OF_FIRST                                    \
+    GEO_SC_WHOLE(52, 92, "x1", "x2") GEO_SC_WHOLE(68, 24, "x2", "x3") REST_OF_FIRST                                    \
     GEO_SC_NEXT_OR_END GEO_SC_INDEX_OFF                                                                                \
     "s_add_u32 %[co], %[co], %[orb]\n"                                                                                 \
     "s_addk_i32 %[wo], " #B "\n"                                                                                       \
@@ -1033,28 +1060,29 @@ struct PairLane {
     "s_add_u32 s33, vcc_lo, 99f-.Lsc_pc_%=\n"                                                                          \
     "s_cbranch_scc1 20b\n"                                                                                             \
     GEO_SC_FIELD_OFFSET GEO_SC_LOADS_HALF_A(0) BASES FALL_COUNT                                                        \
-    ".p2align 5\n31:\n" HALF_LOOP LEFT_HALVES                                                                                      \
+    ".p2align 5\n31:\n" HALF_LOOP LEFT_HALVES                                                                          \
     "7:\n" GEO_SC_WAIT_ALL GEO_SC_COUNT_ZEROS                                                                          \
     "s_cmp_ge_u32 s35, %[zhalf]\n"                                                                                     \
     "s_cbranch_scc1 5b\n"                                                                                              \
     FIRST_CHANNEL                                                                                                      \
     "s_cmp_ge_u32 s35, %[zskip]\n"                                                                                     \
-    "s_cbranch_scc1 22b\n"                                                                                             \
-    "12:\n" CHANNEL(GEO_SC_DENSE, "y", "x") "13:\n" CHANNEL(GEO_SC_DENSE, "x", "y") "s_branch 12b\n"                  \
+    "s_cbranch_scc1 24b\n"                                                                                             \
+    "12:\n" CHANNEL(GEO_SC_DENSE, "y", "x") "13:\n" CHANNEL(GEO_SC_DENSE, "x", "y") "s_branch 12b\n"                   \
     "99:\n" GEO_SC_INDEX_OFF
 #define GEO_SC_OR_OPERANDS                                                                                             \
-    [wp] "s"(wp), [ip] "s"(ip), [act] "s"(act), [orb] "s"(or_b), [zskip] "n"(3 * kSkipZeros), \
+    [wp] "s"(wp), [ip] "s"(ip), [act] "s"(act), [orb] "s"(or_b), [zskip] "n"(3 * kSkipZeros),                          \
         [zhalf] "n"(3 * kHalfZeros), [v0] "v"(voff[0]), [v1] "v"(voff[1]), [v2] "v"(voff[2]), [v3] "v"(voff[3])
-#define GEO_SC_OR_CLOBBERS                                                                                            \
+#define GEO_SC_OR_CLOBBERS                                                                                             \
     "m0", "scc", "vcc", "memory", "s18", "s19", "s20", "s21", "s22", "s23", "s24", "s25", "s26", "s27", "s28",         \
     "s29", "s30", "s31", "s33", "s34", "s35", "s36", "s37", "s38", "s39", "s40", "s41", "s42", "s43", "s44",           \
     "s45", "s46", "s47", "s48", "s49", "s50", "s51", "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59",           \
     "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74",           \
     "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89",           \
     "s90", "s91", "s92", "s93", "s94", "s95", "s96", "s97", "s98", "s99"
-// Mean zero words per line from which the loops are taken.  Below two the jump costs what it saves (uniform weights: one
-// line in three has a zero word, and jumping over it took the 128 -> 128 layer at L 128 from 1.154 to 1.197 ms).  HALF from 7,
-// 9 or 11 zero words on: the 4-layer CNN at batch 256 562 / 566 / 583 us, 64 -> 64 at 56 x 56 (step, L 256) 4.36 / 4.37 / 4.42 ms.
+// Mean zero words per line from which the loops are taken.  SKIP from 1, 2 or 3 on: uniform weights (one line in three has a zero
+// word), 128 -> 128 at 16 x 16, batch 256, L 128 1.135 / 1.129 / 1.127 ms; initial weights widened threefold, 64 -> 64 at 32 x 32, batch
+// 128, L 128 478 / 486 / 508 us.  HALF from 6, 7 or 8 on: 64 -> 64 at 56 x 56, 30 items, L 256, initial weights 509 / 510 / 511 us, widened
+// twofold 674 / 664 / 659.
 constexpr int kSkipZeros = 2, kHalfZeros = 7;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1075,7 +1103,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
     GEO_SC_FIELD_OFFSET LOADS FETCHES                                                                                  \
     "1:\n" GEO_SC_INDEX_ON
     asm volatile(
-        GEO_SC_OR_CHANNELS(192, GEO_SC_FETCH4("x"), GEO_SC_FIRST_CHANNEL3, "", GEO_SC_CHANNEL3,
+        GEO_SC_OR_CHANNELS(192, GEO_SC_FETCH4("x"), GEO_SC_FIRST_CHANNEL3, "", GEO_SC_CHANNEL3, GEO_SC_SKIP_BASES3,
             GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
             GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22") GEO_SC_BASE("b2", "s23"), GEO_SC_FALL_COUNT(3, 1),
             GEO_SC_HALF_CHANNEL3(GEO_SC_LOAD_HALF(60, 96, 0, 192) GEO_SC_LOAD_HALF(68, 24, 1, 192)
@@ -1091,7 +1119,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_LEFT("a0", "s18", 36, 84, "x0", "x1", 0, "") GEO_SC_LEFT("a1", "s19", 44, 88, "x1", "x2", 1, "")
             GEO_SC_LEFT("a2", "s20", 52, 92, "x2", "x3", 2, "") GEO_SC_LEFT("b0", "s21", 60, 96, "y0", "y1", 0, GEO_SC_RISE)
             GEO_SC_LEFT("b1", "s22", 68, 24, "y1", "y2", 1, GEO_SC_RISE) GEO_SC_LEFT("b2", "s23", 76, 28, "y2", "y3", 2, GEO_SC_FALL_IF(3))
-            GEO_SC_FALL(192, 28, "13f", "21b"))
+            GEO_SC_FALL(192, 28, "13f", "23b"))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2), [y3] "=&v"(y3),
           [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left), [cnt] "+&s"(row)
@@ -1109,8 +1137,8 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
     asm volatile(
         GEO_SC_OR_CHANNELS(320, GEO_SC_FETCH6("x"), GEO_SC_FIRST_CHANNEL5,
             GEO_SC_FIELD_OFFSET GEO_SC_LOAD(36, 84, 3) GEO_SC_LOAD(52, 92, 4) GEO_SC_WAIT_LINES
-            GEO_SC_DENSE(36, 84, "x3", "x4") GEO_SC_DENSE(52, 92, "x4", "x5"),
-            GEO_SC_CHANNEL5,
+            GEO_SC_WHOLE(36, 84, "x3", "x4") GEO_SC_WHOLE(52, 92, "x4", "x5"),
+            GEO_SC_CHANNEL5, GEO_SC_SKIP_BASES5,
             GEO_SC_BASE("a0", "s18") GEO_SC_BASE("a1", "s19") GEO_SC_BASE("a2", "s20")
             GEO_SC_BASE("b0", "s21") GEO_SC_BASE("b1", "s22"), GEO_SC_FALL_COUNT(4, 0),
             GEO_SC_WAIT_ALL
@@ -1141,7 +1169,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
             GEO_SC_LEFT("a0", "s18", 36, 84, "x0", "x1", 0, "") GEO_SC_LEFT("a1", "s19", 44, 88, "x1", "x2", 1, "")
             GEO_SC_LEFT("a2", "s20", 52, 92, "x2", "x3", 2, "") GEO_SC_LEFT("b0", "s21", 60, 96, "x3", "x4", 3, GEO_SC_RISE)
             GEO_SC_LEFT("b1", "s22", 68, 24, "x4", "x5", 4, GEO_SC_FALL_IF(4))
-            GEO_SC_FALL(320, 24, "12f", "22b"))
+            GEO_SC_FALL(320, 24, "12f", "24b"))
         : "+{v[32:47]}"(p0), "+{v[48:63]}"(p1), "+{v[64:79]}"(n0), "+{v[80:95]}"(n1), [x0] "=&v"(x0), [x1] "=&v"(x1),
           [x2] "=&v"(x2), [x3] "=&v"(x3), [x4] "=&v"(x4), [x5] "=&v"(x5), [y0] "=&v"(y0), [y1] "=&v"(y1), [y2] "=&v"(y2),
           [y3] "=&v"(y3), [y4] "=&v"(y4), [y5] "=&v"(y5), [co] "+&s"(ch_off), [wo] "+&s"(wo), [left] "+&s"(left), [cnt] "+&s"(row)

@@ -760,12 +760,12 @@ def launch_time(capi, shape_x, shape_w, pad, L, keep):
     return best
 
 
-@pytest.mark.parametrize("first", [0, 8])
-def test_full_weight_lines_behind_empty_ones_take_their_time(capi, first):
-    """A group whose first channel is nearly empty is no slower than one of full lines (1.24 times that if it stays in the loop for
-    mostly empty lines; 1.00 - 1.01 measured)."""
+@pytest.mark.parametrize("first,bound", [(0, 1.12), (8, 1.12), (12, 1.06)])
+def test_full_weight_lines_behind_emptier_ones_take_their_time(capi, first, bound):
+    """A group whose first channel is emptier than the others is hardly slower than one of full lines (1.00 - 1.02 measured; 1.24 times
+    that if it stays in the loop for mostly empty lines, 1.09 if full lines take the jump of the loop for thinned ones)."""
     shape_x, shape_w = (64, 64, 28, 28), (64, 64, 3, 3)
     keep = torch.full(shape_w[1:], 16)
     full = launch_time(capi, shape_x, shape_w, 1, 128, keep)
     keep[0] = first
-    assert launch_time(capi, shape_x, shape_w, 1, 128, keep) < 1.12 * full
+    assert launch_time(capi, shape_x, shape_w, 1, 128, keep) < bound * full

@@ -56,7 +56,7 @@ def targets(code, i, bases):
     for bits in range(1 << 16):
         reach.add(bits >> (spec & 31) & ((1 << (spec >> 16)) - 1))
     for number in reach:
-        regs = dict(bases)
+        regs, there = dict(bases), None
         regs[code[start][2][0]] = number
 
         def value(o):
@@ -72,9 +72,12 @@ def targets(code, i, bases):
                 regs[args[0]] = value(args[1]) + value(args[2])
             elif re.match(r"s_lshl[1-4]_add_u32$", op):
                 regs[args[0]] = (value(args[1]) << int(op[6])) + value(args[2])
+            elif op == "s_cbranch_scc0":  # s_bfe_u32 says whether its result is zero
+                if number == 0:
+                    there = addr + 4 + 4 * (int(args[0], 0) ^ 0x8000) - 4 * 0x8000
             elif op != "s_addc_u32":  # (the upper halves: the code lies in one 4 GB here)
                 raise AssertionError(f"{op} in front of a jump")
-        yield number, regs[low(code[i][2][0])]
+        yield number, regs[low(code[i][2][0])] if there is None else there
 
 
 def test_computed_jumps_land_on_slots(tmp_path):
