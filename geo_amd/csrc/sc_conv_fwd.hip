@@ -1185,7 +1185,7 @@ __device__ __forceinline__ void or_channels_rail(const u32x4& act, const unsigne
         "v_and_or_b32 v65, s[" #W "+" #I "], %[" X1 "], v65\n"
 // Loads.  %[wp], %[ip]: the group's right halves by themselves, 32 bytes per line of the words and 16 of the fields; %[wl],
 // %[il]: its whole lines.  The scalar cache's misses bound this loop (four waves of a SIMD with a line sequence of their own
-// each): of whole lines, half of every 64 bytes unused, the 4096 x 4096 layer at batch 1024 takes 2.33 ms, of these 1.45.
+// each): of whole lines, half of every 64 bytes unused, the 4096 x 4096 layer at batch 1024 takes 2.33 ms, of these 1.4.
 #define GEO_SC_X16(W, BASE, AT) "s_load_dwordx16 s[" #W ":" #W "+15], %[" BASE "], " #AT "\n"
 #define GEO_SC_X8(W, BASE, AT) "s_load_dwordx8 s[" #W ":" #W "+7], %[" BASE "], " #AT "\n"
 #define GEO_SC_X4(W, BASE, AT) "s_load_dwordx4 s[" #W ":" #W "+3], %[" BASE "], " #AT "\n"
@@ -1589,20 +1589,20 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 
 // The item-innermost kernel for OR groups of LPG = 16 one-wide lines (the SC-linear mapping with groups of
 // 16 inputs), as one workgroup of 16 waves per (128 items, 8 c_out tiles): wave = (c_out tile, half of
-// the (pack, kernel row) groups).  The eight waves of a half read the same activation words; per group
-// every wave fetches two of the 16 lines (buffer loads, 4 dwords per lane) and leaves them in LDS, and
-// all read a line back with one ds_read_b64: an eighth of the vector loads, and what a wave waits for in
-// front of a line's 32 vector instructions is LDS and the scalar cache.  Groups are double-buffered
-// (the loads of group t + 1 are issued before group t is computed and written to LDS after it), one
-// barrier per group.  The two halves add their sums in LDS and the workgroup stores 128 items x 128
+// the (pack, kernel row) groups).  The eight waves of a half read the same activation words: per group
+// every wave sends two of the 16 lines straight to LDS (one dword per lane and transfer, in the order of the lanes),
+// and all read a line back with one ds_read2st64_b32: an eighth of the vector loads, and what a wave waits for in
+// front of a line's 32 vector instructions is LDS and the scalar cache.  Groups are double-buffered: the transfers
+// of group t + 1 are under way while group t is computed, and one barrier per group stands behind both.  The
+// two halves add their sums in LDS and the workgroup stores 128 items x 128
 // channels, 512-byte runs per item.  With 8 position tiles x 32 tile groups (4096 x 4096 at batch 1024)
 // that is 256 workgroups, one per CU, in a single round.
-// The 256 workgroups walk their weight streams in step (768 KB of lines per group and L2): a touch two
-// groups ahead is still in L2 when its lines are read (1 or 2 groups ahead 3.06 ms, 4: 3.19, 8: 4.43, none: 5.2).
+// The 256 workgroups walk their weight streams in step (768 KB of lines per group and L2, 384 KB of right halves): a touch two
+// groups ahead is still in L2 when its lines are read (every word: 1, 2 or 4 groups ahead 2.99 / 2.92 / 3.26 ms; right halves, with the
+// generators: 1.65 / 1.60 / 1.79).
 // Mostly empty lines (kHalfZeros, sampled over the workgroup's tiles) take their right halves only, ahead of their use, from the
-// copy that the whole-op forward keeps of them: 4096 x 4096 at batch 1024, initial weights, 0.77 of the words zero: 3.09 ms with
-// every word, 2.33 with halves of whole lines, 1.4 with the copy.  With every word 3.02 (3.09 before the activation words went to
-// LDS without registers).
+// copy that the whole-op forward keeps of them: 4096 x 4096 at batch 1024, initial weights, 0.77 of the words zero: 1.4 ms, 2.33 with halves
+// of whole lines, 2.92 with every word.
 constexpr int kLinHalves = 2, kLinTouchGroups = 2;
 // The lane's number, formed anew where it is used: the kernel below fills its 128 registers, and a value that is kept across its
 // loops goes to scratch memory, whose loads wait for every load in flight.
@@ -1630,6 +1630,27 @@ __device__ __forceinline__ void or_lines16_lds(uint32_t lds, ConstWords wp, Cons
                    [y5] "=&{v63}"(y5)
                  : [wp] "s"(wp), [ip] "s"(ip), [wl] "s"(wl), [il] "s"(il), [lds] "v"(lds)
                  : GEO_SC_OR_CLOBBERS);
+}
+// The lane's two words of consecutive lines from byte address `lds` on.  In front of a plain read the compiler waits for every
+// transfer to LDS that is under way, the next group's among them, as it cannot tell the two buffers apart: 4096 x 4096 at batch
+// 1024 with every word 3.02 ms instead of 2.92.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void lds_lines(uint32_t (&aw)[3][2], uint32_t lds)
+{
+    u32x2 a, b, c;
+    asm volatile("ds_read2st64_b32 %0, %3 offset1:1\n"
+                 "ds_read2st64_b32 %1, %3 offset0:2 offset1:3\n"
+                 "ds_read2st64_b32 %2, %3 offset0:4 offset1:5\n"
+                 "s_waitcnt lgkmcnt(0)" : "=&v"(a), "=&v"(b), "=&v"(c) : "v"(lds) : "memory");
+    aw[0][0] = a.x, aw[0][1] = a.y, aw[1][0] = b.x, aw[1][1] = b.y, aw[2][0] = c.x, aw[2][1] = c.y;
+}
+__device__ __forceinline__ void lds_lines(uint32_t (&aw)[2][2], uint32_t lds)
+{
+    u32x2 a, b;
+    asm volatile("ds_read2st64_b32 %0, %2 offset1:1\n"
+                 "ds_read2st64_b32 %1, %2 offset0:2 offset1:3\n"
+                 "s_waitcnt lgkmcnt(0)" : "=&v"(a), "=&v"(b) : "v"(lds) : "memory");
+    aw[0][0] = a.x, aw[0][1] = a.y, aw[1][0] = b.x, aw[1][1] = b.y;
 }
 __global__ __launch_bounds__(64 * kLinTiles * kLinHalves) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_conv_fwd_items_rail_lds(FwdParams q)
@@ -1730,13 +1751,10 @@ void k_conv_fwd_items_rail_lds(FwdParams q)
         auto lines = [&](auto n_tag, auto first_tag, int l0) {
             constexpr int N = decltype(n_tag)::value;
             constexpr bool FIRST = decltype(first_tag)::value;
-            uint32_t aw[N][R];
-#pragma unroll
-            for (int l = 0; l < N; l++)
-#pragma unroll
-                for (int r = 0; r < R; r++) aw[l][r] = ((LdsWords)(uintptr_t)lane_lds)[((l0 + l) * R + r) * 64];
             uint32_t wv[N][C], iv[N][C / 2];
             rl.load(wv, iv);
+            uint32_t aw[N][R];
+            lds_lines(aw, lane_lds + l0 * 512u);
 #pragma unroll
             for (int l = 0; l < N; l++) {
                 if (FIRST && l == 0)

@@ -102,3 +102,22 @@ def test_computed_jumps_land_on_slots(tmp_path):
                 t_op, t_args = code[at[target]][1], code[at[target]][2]
                 assert t_op in ("s_branch", "s_set_gpr_idx_on") or t_args[0] == "m0", f"{name}: {number} words at {addr:#x} lead to {t_op}"
     assert jumps > 0
+
+
+def test_linear_kernel_computes_behind_its_prefetch(tmp_path):
+    """k_conv_fwd_items_rail_lds sends the next group's activation words to LDS and then ORs the present one: neither of its loops may
+    wait for the transfers (vmcnt) before that work."""
+    from geo_amd import _native
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no disassembler here")
+    [code] = [c for n, c in kernels(_native.lib_path(), tmp_path).items() if "k_conv_fwd_items_rail_lds" in n]
+    behind, ors = [], None  # ORs between the last transfer of a run of them and the first wait
+    for _, op, args in code:
+        if op == "buffer_load_dword" and args[-1].endswith("lds"):
+            ors = 0
+        elif op == "v_and_or_b32" and ors is not None:
+            ors += 1
+        elif op == "s_waitcnt" and "vmcnt(0)" in args[0] and ors is not None:
+            behind.append(ors)
+            ors = None
+    assert sum(n >= 400 for n in behind) == 2, behind   # (16 lines of 32; the transfers in front of the loops are waited for at once)
