@@ -68,8 +68,8 @@ struct Geometry {
 // where channel c's word is not zero.  A wave that accumulates the line jumps over the zero words.
 __device__ __forceinline__ int rail_slot(uint32_t live, int c)
 {
-    const uint32_t below = (1u << c) - 1u;
-    return (live >> c) & 1u ? kCoTile - __popc(live >> c) : __popc(~live & below);
+    const int from = (int)__popc(live >> c), below = (int)__popc(~live & ((1u << c) - 1u));
+    return (live >> c) & 1u ? kCoTile - from : below;
 }
 // The 16-bit field of channel c at slot `at`: bits 7:0 the register offset of its accumulators (2 c for the positive rail and
 // for zero weights, 32 + 2 c for the negative one), bits 15:12 the SRC2 and DST enables of the VGPR index mode.  Two slots say in
@@ -80,7 +80,7 @@ __device__ __forceinline__ int rail_slot(uint32_t live, int c)
 __device__ __forceinline__ uint32_t rail_field(uint32_t live, int at, int c, bool negative)
 {
     constexpr int H = kCoTile / 2;
-    const int zeros = min(kCoTile - __popc(live), kCoTile - 1);
+    const int zeros = min(kCoTile - (int)__popc(live), kCoTile - 1);  // (of unsigned and int, min is the one of doubles)
     uint32_t high = 0xC0u;
     if (at == 0) high |= (uint32_t)zeros;
     if (at == H) high |= zeros < H ? (uint32_t)H : (uint32_t)(zeros - H);

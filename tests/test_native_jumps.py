@@ -121,3 +121,16 @@ def test_linear_kernel_computes_behind_its_prefetch(tmp_path):
             behind.append(ors)
             ors = None
     assert sum(n >= 400 for n in behind) == 2, behind   # (16 lines of 32; the transfers in front of the loops are waited for at once)
+
+
+def test_weight_packing_counts_in_integers(tmp_path):
+    """The number of a line's zero words is an integer; taken through the minimum of doubles it costs conversions per word."""
+    from geo_amd import _native
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no disassembler here")
+    seen = 0
+    for name, code in kernels(_native.lib_path(), tmp_path).items():
+        if "k_weight_streams" in name or "k_rail_pack" in name:
+            seen += 1
+            assert not [op for _, op, _ in code if "_f64" in op], name
+    assert seen >= 2
