@@ -1600,7 +1600,7 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // The 256 workgroups walk their weight streams in step (768 KB of lines per group and L2, 384 KB of right halves): a touch two
 // groups ahead is still in L2 when its lines are read (every word: 1, 2 or 4 groups ahead 2.99 / 2.92 / 3.26 ms; right halves, with the
 // generators: 1.65 / 1.60 / 1.79).
-// Mostly empty lines (kHalfZeros, sampled over the workgroup's tiles) take their right halves only, ahead of their use, from the
+// Mostly empty lines (sampled over the workgroup's tiles) take their right halves only, ahead of their use, from the
 // copy that the whole-op forward keeps of them: 4096 x 4096 at batch 1024, initial weights, 0.77 of the words zero: 1.4 ms, 2.33 with halves
 // of whole lines, 2.92 with every word.
 constexpr int kLinHalves = 2, kLinTouchGroups = 2;
@@ -1716,16 +1716,29 @@ void k_conv_fwd_items_rail_lds(FwdParams q)
             group_off += pack_b - (unsigned)q.h_k * row_b;
         }
     };
-    // The mean zero words of 64 lines, eight of each of the workgroup's tiles: one choice for all waves, which meet at barriers
-    unsigned zeros = 0;
+    // Right halves only where few of 128 lines, sixteen of each of the workgroup's tiles, spread over members, rows and packs, need
+    // their left half, and no tile's: the waves meet at barriers, so that they take one choice, and a tile of full lines holds up the
+    // others.  1024 items, 4096 outputs, 64 groups of 16, against every word's loop: a fifth of all lines full 0.89 of its time, two in
+    // five 1.04, all 1.44; all lines of one tile in eight 1.27.
+    bool half_lines = false;
     if (q.wgt_right) {
         const int first_tile = (blockIdx.x % cot_groups) * NWV;
-#pragma unroll 8
-        for (int i = 0; i < 8 * NWV; i++) {
-            const RailLines at(q, first_tile + i % NWV, (size_t)(i / NWV) * (q.rail_lines / 8));
-            zeros += (at.f[0] >> 8) & 15u;
+        unsigned long long full[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const unsigned i = (unsigned)(64 * k + lane);
+            const size_t line = min((size_t)i * q.rail_lines / 128 + (2 * (i / NWV) + i) % LPG, q.rail_lines - 1);
+            const size_t at = (size_t)(first_tile + i % NWV) * q.rail_lines + line;
+            full[k] = __ballot((q.wgt_rail_idx[at * (C / 2)] >> 11 & 1u) == 0);  // bits 11:8: the line's zero words
+        }
+        half_lines = __popcll(full[0]) + __popcll(full[1]) <= 48;
+#pragma unroll
+        for (int t = 0; t < NWV; t++) {
+            const unsigned long long tile = 0x0101010101010101ull << t;
+            half_lines &= __popcll(full[0] & tile) + __popcll(full[1] & tile) < 11;
         }
     }
+    static_assert(NWV == 8, "every eighth sample is of the same tile");
     fetch(group_off, 0);
     arrive();
     auto walk = [&](auto half_tag) {
@@ -1789,7 +1802,7 @@ void k_conv_fwd_items_rail_lds(FwdParams q)
         arrive();
     }
     };
-    if (zeros >= (unsigned)(kHalfZeros * 8 * NWV))
+    if (half_lines)
         walk(std::true_type());
     else
         walk(std::false_type());

@@ -769,3 +769,33 @@ def test_full_weight_lines_behind_emptier_ones_take_their_time(capi, first, boun
     full = launch_time(capi, shape_x, shape_w, 1, 128, keep)
     keep[0] = first
     assert launch_time(capi, shape_x, shape_w, 1, 128, keep) < bound * full
+
+
+def linear_time(capi, keep, n=1024, c_out=4096, rows=16):
+    """The 16-line linear layer as one call (its generator included), keep[c_out tile, line, row] channels of a line not empty."""
+    x, w = wl.make_inputs((n, 16, 1, rows), (c_out, 16, 1, rows), "q7", seed=4)
+    w = torch.cat([thinned(w[16 * t:16 * t + 16], keep[t][:, None], t) for t in range(c_out // 16)]).cuda()
+    x, d = x.cuda(), capi.make_desc((n, 16, 1, rows), (c_out, 16, 1, rows), 128, (0, 0))
+    best = 1e9
+    for _ in range(8):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            capi.conv2d_add_partial_forward(x, w, 128, (0, 0), desc=d)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+def test_linear_lines_with_words_in_the_left_half_take_their_time(capi):
+    """Few words on average, but full lines that hold up the workgroup: no slower than every line full (1.0 measured; in the loop of right
+    halves 1.4 with nine words in every line, 1.5 where every other tile is full, 1.5 where only the first line of a group is empty)."""
+    full = linear_time(capi, torch.full((256, 16, 16), 16))
+    nine = torch.full((256, 16, 16), 9)
+    tiles = torch.full((256, 16, 16), 16)
+    tiles[::2] = 0
+    first = torch.full((256, 16, 16), 16)
+    first[:, 0] = 0
+    for keep in (nine, tiles, first):
+        assert linear_time(capi, keep) < 1.12 * full
