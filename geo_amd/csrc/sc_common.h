@@ -99,13 +99,14 @@ inline __host__ __device__ size_t table_bytes(int L)
     return sizeof(uint32_t) * ((size_t)L + (size_t)L * table_words_per_code(L));
 }
 
-constexpr int kLinLines = 16, kLinTiles = 8;  // k_conv_fwd_items_rail_lds: lines of an OR group, c_out tiles of a workgroup
-// whether launch_conv_forward takes that kernel: item-innermost, two equal halves of the groups, 128 workgroups
+// k_conv_fwd_items_rail_lds: lines of an OR group, c_out tiles of a workgroup, shares that it cuts the groups into
+constexpr int kLinLines = 16, kLinTiles = 8, kLinHalves = 2;
+// whether launch_conv_forward takes that kernel: item-innermost, equal shares of the groups, 128 workgroups
 inline bool lines16_lds(const Geometry& g)
 {
     const long long tiles = ((long long)(g.n + 1) / 2 * g.ho + 63) / 64;
-    return g.act_item_inner && g.w_k == 1 && g.c_in == kLinLines && g.n_cotile % kLinTiles == 0 && g.packs * g.h_k % 2 == 0 &&
-           tiles * (g.n_cotile / kLinTiles) >= 128;
+    return g.act_item_inner && g.w_k == 1 && g.c_in == kLinLines && g.n_cotile % kLinTiles == 0 &&
+           g.packs * g.h_k % kLinHalves == 0 && tiles * (g.n_cotile / kLinTiles) >= 128;
 }
 // the right halves' words [n_cotile][line][8] and fields [n_cotile][line][8] of 16 bits, in the place of two-rail lines of 32 words
 inline size_t right_fields_off(const Geometry& g) { return g.wgt_rail_lines * g.n_cotile * (kCoTile / 2); }

@@ -1603,7 +1603,7 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // Mostly empty lines (sampled over the workgroup's tiles) take their right halves only, ahead of their use, from the
 // copy that the whole-op forward keeps of them: 4096 x 4096 at batch 1024, initial weights, 0.77 of the words zero: 1.4 ms, 2.33 with halves
 // of whole lines, 2.92 with every word.
-constexpr int kLinHalves = 2, kLinTouchGroups = 2;
+constexpr int kLinTouchGroups = 2;
 // The lane's number, formed anew where it is used: the kernel below fills its 128 registers, and a value that is kept across its
 // loops goes to scratch memory, whose loads wait for every load in flight.
 __device__ __forceinline__ int fresh_lane()
@@ -2016,8 +2016,7 @@ int launch(const Geometry& g, FwdParams q, hipStream_t s)
         if (!g.rail || g.mode != GEO_SC_ACC_Y) return GEO_SC_ERR_INVALID_ARGUMENT;  // make_geometry sets both with act_item_inner
         // OR groups of 16 one-wide lines with whole sets of 8 c_out tiles and enough of them to fill the
         // GPU: the workgroup that stages the activation words of its 8 tiles through LDS
-        if (WK == 1 && g.c_in == kLinLines && g.n_cotile % kLinTiles == 0 && pv % kLinHalves == 0 &&
-            tiles * (g.n_cotile / kLinTiles) >= 128) {
+        if (WK == 1 && lines16_lds(g)) {
             q.pv_per_block = pv / kLinHalves;
             hipLaunchKernelGGL(k_conv_fwd_items_rail_lds, dim3((unsigned)(tiles * (g.n_cotile / kLinTiles))),
                                dim3(64 * kLinTiles * kLinHalves), 0, s, q);
