@@ -799,3 +799,24 @@ def test_linear_lines_with_words_in_the_left_half_take_their_time(capi):
     first[:, 0] = 0
     for keep in (nine, tiles, first):
         assert linear_time(capi, keep) < 1.12 * full
+
+
+@pytest.mark.parametrize("words", [3, 7, 16])
+@pytest.mark.parametrize("n,rows,L,budget,chunk", [
+    (400, 6, 32, None, 400), (387, 5, 64, None, 387), (390, 3, 128, None, 390),  # one, two and four packs of the stream
+    (1190, 5, 64, 800, 400),                                                     # chunks of 400, 400 and 390 items on two streams
+    (900, 5, 64, 850, 425),                                                      # the last one, of 50, without right halves: none has them
+])
+def test_linear_right_halves(capi, so, n, rows, L, budget, chunk, words):
+    """16-line linear layers as one call, whose generator leaves the right halves of the weight lines where the kernel reads them: lines of
+    `words` channels, one more or less, and some full ones.  Bit for bit."""
+    shape_x, shape_w = (n, 16, 1, rows), (4096, 16, 1, rows)
+    x, w = wl.make_inputs(shape_x, shape_w, "q7", seed=n + words)
+    keep = torch.full(shape_w[1:], words) + torch.randint(-1, 2, shape_w[1:], generator=torch.Generator().manual_seed(n))
+    keep[5, 0, rows // 2] = 16
+    w = thinned(w, keep, words)
+    d = capi.make_desc(shape_x, shape_w, L, (0, 0))
+    opt = None if budget is None else capi.make_options(forward_stream_bytes=4 * (L // 32) * 16 * rows * budget)
+    assert capi.forward_chunk(d, opt) == chunk
+    got = capi.conv2d_add_partial_forward(x.cuda(), w.cuda(), L, (0, 0), desc=d, options=opt)
+    assert np.array_equal(got.cpu().numpy(), so.conv2d_add_partial(x.numpy(), w.numpy(), L, (0, 0)))
