@@ -14,8 +14,9 @@ duration (the backward does no bit-MACs, so the forward-only rate is reported ne
 The default workload is the configuration the headline metric is quoted on: SC conv2d
 128->128 3x3 at 16x16, batch 256, pad 1, stream length 128, activations U[0,1), weights
 U[-1,1) (with these distributions every OR rail saturates, so this input is for timing
-only; no kernel exits early on them, and the weights have too few zero stream words to skip).  After the headline the default run also times
-the other benchmark configurations (C3 at stream lengths 32 and 256, C5, C4, the C2 training step) and
+only; no kernel exits early on them, and the weights have too few zero stream words to skip).  Rates and fractions of
+word operations count the and-ors of weight words that are not zero; the kernels may execute more.  After the headline the default
+run also times the other benchmark configurations (C3 at stream lengths 32 and 256, C5, C4, the C2 training step) and
 reports them under the key ``configs``.
 """
 from __future__ import annotations
@@ -193,7 +194,7 @@ def network_step_result(args, torch):
 
     layers = {}
     B_total = 0
-    word_ops_total = 0.0
+    word_ops_total = dense_total = 0.0
     k_total = 0.0
     for name, sx, sw, pad in C2_LAYERS:
         xa, wa = wl.make_inputs(sx, sw, "q7", 0)
@@ -212,11 +213,14 @@ def network_step_result(args, torch):
         k = time_events(lambda: capi.conv2d_add_partial_from_streams(act, wgt, d, out=out), args.steps, 2, torch)
         B = wl.bit_macs(sx, sw, pad, L)
         B_total += B
-        ops = min_word_ops(sx, sw, pad, L)
+        live = live_share(wgt, sw, L)
+        ops = min_word_ops(sx, sw, pad, L, live)
         word_ops_total += ops
+        dense_total += B / 32
         k_total += sum(k) / len(k)
         layers[name] = {"fwd_ms": sum(f) / len(f), "bwd_ms": sum(b) / len(b), "conv_kernel_ms": sum(k) / len(k),
-                        "bit_macs": B, "valu_frac": ops / (sum(k) / len(k) * 1e-3) / PEAK_VALU_WORD_OPS}
+                        "bit_macs": B, "live_share": live,
+                        "valu_frac": ops / (sum(k) / len(k) * 1e-3) / PEAK_VALU_WORD_OPS}
     achieved = word_ops_total / (k_total * 1e-3)
     result = {
         "metric": f"SC bit-MACs/sec over one training step of the 4-layer SC CNN at stream len {L}",
@@ -237,7 +241,9 @@ def network_step_result(args, torch):
         "layers": layers,
         "roofline": {"bound": "valu", "kernel": "the four layers' convolution launches together",
                      "achieved": achieved / 1e12, "peak": PEAK_VALU_WORD_OPS / 1e12, "unit": "T word-op/s",
-                     "frac": achieved / PEAK_VALU_WORD_OPS, "kernel_ms_sum": k_total, "traffic": None},
+                     "frac": achieved / PEAK_VALU_WORD_OPS, "kernel_ms_sum": k_total,
+                     # priced as if every weight word were ORed (not a roofline fraction)
+                     "dense_equivalent_rate": dense_total / (k_total * 1e-3) / 1e12, "traffic": None},
     }
     return result
 
@@ -319,15 +325,24 @@ DTYPE_FWD_BWD = (DTYPE_FWD + " (forward); fp32 gradients: each fp32 product from
                  "operand split, fp32 accumulate (backward)")
 
 
-def min_word_ops(x_shape, w_shape, pad, L):
+def live_share(wgt, w_shape, L):
+    """Share of the weight stream words that are not zero: the two-rail lines at the head of a weight stream buffer, of which a
+    weight has one word of two (sc.cpp:301-304)."""
+    Cout, Cin, W, H = w_shape
+    lines = (L + 31) // 32 * H * Cin * W
+    return wgt.view(-1)[:lines * (Cout + 15) // 16 * 32].ne(0).sum().item() / (lines * Cout)
+
+
+def min_word_ops(x_shape, w_shape, pad, L, live=1.0):
     """32-bit VALU lane operations no kernel for this problem can do without: one and-or per (activation
     word, weight) - a weight has a single non-zero rail (sc.cpp:301-304), so B/32 of them, not the 2*B/32
-    of a kernel that processes both rails - plus one popcount-add per (output, rail, add group, pack)."""
+    of a kernel that processes both rails - where the weight's word is not zero (a share `live` of them),
+    plus one popcount-add per (output, rail, add group, pack)."""
     N, Cin, Wx, Hx = x_shape
     Cout, _, W, H = w_shape
     Wo, Ho = Wx + 2 * pad - W + 1, Hx + 2 * pad - H + 1
     B = N * Cout * Wo * Ho * Cin * W * H * L
-    return B / 32 + 2 * N * Cout * Wo * Ho * H * ((L + 31) // 32)
+    return live * B / 32 + 2 * N * Cout * Wo * Ho * H * ((L + 31) // 32)
 
 
 def measure_layer(torch, workload, L, steps, warmup, with_bwd=True, accumulate="y", z_unit=32, generator="lfsr"):
@@ -378,7 +393,8 @@ def measure_layer(torch, workload, L, steps, warmup, with_bwd=True, accumulate="
                               2, torch)
     m["rail"] = capi.skips_zero_rail(desc)
     m["B"] = wl.bit_macs(xd.shape, wd.shape, pad, L)
-    m["min_word_ops"] = min_word_ops(xd.shape, wd.shape, pad, L)
+    m["live"] = live_share(wgt, wd.shape, L)
+    m["min_word_ops"] = min_word_ops(xd.shape, wd.shape, pad, L, m["live"])
     N, Cin, _, _ = xd.shape
     Cout, _, W, H = wd.shape
     m["bwd_flops"] = 12 * N * Cout * out.shape[2] * out.shape[3] * Cin * W * H
@@ -399,7 +415,7 @@ def config_summary(m):
          "bwd_ms": avg(m["bwd_ms"]) if m["bwd_ms"] else None, "kernel_ms": k,
          "bit_macs_per_s": m["B"] / (m["ms_per_step"] * 1e-3),
          "fwd_bit_macs_per_s": m["B"] / (avg(m["fwd_ms"]) * 1e-3),
-         "executed_frac": m["min_word_ops"] / (k * 1e-3) / PEAK_VALU_WORD_OPS,
+         "live_share": m["live"], "live_word_frac": m["min_word_ops"] / (k * 1e-3) / PEAK_VALU_WORD_OPS,
          "bwd_tflops": m["bwd_flops"] / (avg(m["bwd_ms"]) * 1e-3) / 1e12 if m["bwd_ms"] else None}
     return e
 
@@ -418,7 +434,7 @@ def other_configs(args, torch):
         "torch_statistics_ms_per_step": r["torch_statistics_ms_per_step"],
         "module_chain_ms_per_step": r["module_chain_ms_per_step"], "workload": r["config"]["workload"],
         "bit_macs_per_s": r["value"], "kernel_ms": r["roofline"]["kernel_ms_sum"],
-        "executed_frac": r["roofline"]["frac"],
+        "live_word_frac": r["roofline"]["frac"],
         "fwd_ms": sum(l["fwd_ms"] for l in r["layers"].values()),
         "bwd_ms": sum(l["bwd_ms"] for l in r["layers"].values()), "bwd_tflops": None}
     torch.cuda.empty_cache()
@@ -460,7 +476,7 @@ def probe_mfma_forward(torch):
             "slices_per_cu": slices, "tile": "128 positions x 256 rail-columns x 384 members", "times": t,
             "fp4_tflops_mfma_only": 2 * macs / (t["mfma_only_ms"] * 1e-3) / 1e12,
             "fp4_tflops_with_threshold": 2 * macs / (t["with_threshold_and_count_ms"] * 1e-3) / 1e12,
-            "note": "operands arrive expanded to one fp4 value per stream bit; the vector-ALU kernel takes 1.155 ms for "
+            "note": "operands arrive expanded to one fp4 value per stream bit; the vector-ALU kernel takes 1.13 ms for "
                     "the same layer from bit-packed streams"}
 
 
@@ -510,7 +526,6 @@ def main():
     rail = m["rail"]
     ops = m["min_word_ops"]
     achieved = ops / (k_avg * 1e-3)
-    issued = (B / 32 if rail else 2 * B / 32)
     probe_rate = capi.probe_and_or_rate()
     traffic, traffic_kernel = (None, None) if variant else profiled_traffic(args.workload, L)
 
@@ -541,22 +556,24 @@ def main():
                      "bwd_min": min(bwd_ms) if with_bwd else None},
         "roofline": {
             "bound": "valu",
-            "kernel": ("the rail-skipping convolution kernel (v_and_or_b32 on register-indexed accumulators: one "
+            "kernel": ("the rail-skipping convolution kernel (v_and_or_b32 on register-indexed accumulators: at most one "
                        "and-or per activation word and weight; k_conv_fwd_tile_rail at the headline)"
                        if rail else "k_conv_fwd (v_and_or_b32 / v_bcnt_u32_b32, both rails)"),
-            # work no kernel can avoid (one and-or per activation word and weight, plus the popcount-adds) per
-            # second of the kernel's average launch duration, against lanes x clock
+            # work no kernel can avoid (one and-or per activation word and weight whose word is not zero, plus the
+            # popcount-adds) per second of the kernel's average launch duration, against lanes x clock
             "achieved": achieved / 1e12,
             "peak": PEAK_VALU_WORD_OPS / 1e12,
             "unit": "T word-op/s",
             "frac": achieved / PEAK_VALU_WORD_OPS,
             "min_word_ops": ops,
+            "live_share": m["live"],
             "kernel_ms_avg": k_avg,
             "kernel_ms_min": min(k_ms),
             "measured_issue_rate": probe_rate / 1e12,
             "frac_of_measured_issue_rate": achieved / probe_rate,
-            # and-or instructions this kernel issues (lane operations): B/32 when it skips the zero rail, else 2B/32
-            "issued_and_or_word_ops": issued,
+            # one and-or per activation word and weight, zero words included: what the kernel issues where it skips none
+            "dense_word_ops": B / 32,
+            "dense_equivalent_rate": B / 32 / (k_avg * 1e-3) / 1e12,
             # the same time priced with the two-rail count 2*B/32 that a kernel processing both rails would
             # execute (can pass the peak; not a roofline fraction)
             "two_rail_word_ops": 2 * B / 32,
