@@ -266,6 +266,7 @@ __global__ __launch_bounds__(kGenThreads) void k_weight_streams(WeightGen a)
     const float Lf = (float)gp.L, top = (float)(gp.L - 1);
     const unsigned n_blocks = (unsigned)v_chunks * k_chunks * n_cotile;
     const size_t rail_lines = lines_per_pack * gp.packs;
+    const size_t two_step = lines_per_pack * n_cotile * (2 * kCoTile), packed_step = lines_per_pack * kCoTile;
     const int co_l = threadIdx.x & 15, k_l = threadIdx.x >> 4;
     int cot, k0, v0;
     auto tile_of = [&](unsigned blk) {
@@ -324,26 +325,25 @@ __global__ __launch_bounds__(kGenThreads) void k_weight_streams(WeightGen a)
             const int code = cp | cn;
             const int o = (int)posp1[((cn ? 37 : 67) + seed0 + v * seed_step) % (gp.L - 1)];
             const size_t line = line0 + (size_t)v * line_step;
-            const size_t base = (line * n_cotile + cot) * (2 * kCoTile) + co_l;
-            for (int pk = 0; pk < gp.packs; pk++) {
+            // both lines of the first pack, then from pack to pack
+            uint32_t* two = streams + (line * n_cotile + cot) * (2 * kCoTile) + co_l;
+            size_t packed = ((size_t)cot * rail_lines + line) * kCoTile;
+            for (int pk = 0; pk < gp.packs; pk++, two += two_step, packed += packed_step) {
                 const uint32_t word = code ? stream_word(thr, code, o, pk, gp) : 0u;
                 if (two_rail) {
-                    uint32_t* dst = streams + pk * lines_per_pack * n_cotile * (2 * kCoTile) + base;
-                    dst[0] = cp ? word : 0u;
-                    dst[kCoTile] = cn ? word : 0u;
+                    two[0] = cp ? word : 0u;
+                    two[kCoTile] = cn ? word : 0u;
                 }
                 if (rail_words) {
                     // the line's 16 channels are 16 consecutive lanes
                     const uint32_t live = (uint32_t)(__ballot(word != 0u) >> (threadIdx.x & 48)) & 0xffffu;
                     const int at = rail_slot(live, co_l);
-                    const size_t dst = ((size_t)cot * rail_lines + pk * lines_per_pack + line) * kCoTile + at;
                     const uint16_t field = (uint16_t)rail_field(live, at, co_l, cn != 0);
-                    rail_words[dst] = word;
-                    rail_fields[dst] = field;
+                    rail_words[packed + at] = word;
+                    rail_fields[packed + at] = field;
                     if (right_words && at >= kCoTile / 2) {
-                        const size_t right = ((size_t)cot * rail_lines + pk * lines_per_pack + line) * (kCoTile / 2) + at - kCoTile / 2;
-                        right_words[right] = word;
-                        right_fields[right] = field;
+                        right_words[packed / 2 + at - kCoTile / 2] = word;
+                        right_fields[packed / 2 + at - kCoTile / 2] = field;
                     }
                 }
             }
