@@ -834,8 +834,8 @@ struct PairLane {
 // compiler does not keep; and 64 pinned accumulators that live across its branches it spills.
 // Scalar registers (s32 is the compiler's): DENSE and SKIP: words of three lines in s[36:51], s[52:67], s[68:83], their fields
 // in s[84:91], s[92:99], s[24:31].  HALF: words of stage A's three lines in s[36:59], of stage B's in s[60:83], fields in
-// s[84:95] and s[96:99], s[24:31]; addresses of the lines' first slots in s[18:23] (low) and vcc_hi (high).  s33: temporary;
-// s[34:35]: temporary, and the zero words of the first lines.
+// s[84:95] and s[96:99], s[24:31].  SKIP and HALF: the addresses that the lines' jumps start from in s[18:23] (low) and vcc_hi (high).
+// s33, s34: temporary; s35: the zero words of the first lines.
 // Index mode stays on between the loads of a channel and the next one's: nothing but the slots' vector instructions is issued.
 #define GEO_SC_SLOT(SET, W, I, X0, X1)                                                                                 \
     SET "v_and_or_b32 v32, s[" #W "+" #I "], %[" X0 "], v32\n"                                                         \
@@ -1344,7 +1344,7 @@ void k_conv_fwd_pair_rail(FwdParams q, unsigned n_tiles)
 // Bound by the issue rate of v_and_or_b32 where the launch fills the GPU; what decides then is the number of
 // waves a SIMD can choose from, as every wave waits for its channel's words and weight lines before it can issue
 // their 96 and-ors (3 lines): the counts are summed in LDS (ds_add_u32) instead of in 32 registers, so
-// that five waves fit a SIMD.  128 -> 128 channels, 3 x 3, 16 x 16, batch 256, L 128: 1.155 ms; with the sums in
+// that five waves fit a SIMD.  128 -> 128 channels, 3 x 3, 16 x 16, batch 256, L 128: 1.13 ms; with the sums in
 // registers (four waves) 1.38, and 1.29 with the activation words of four c_out tiles staged through LDS besides,
 // which this kernel replaced; 64 -> 64 at 56 x 56, L 256, batch 30: 0.95 -> 0.87.
 // or_shares > 1, for launches with too few (tile, pair) waves: an OR can be cut anywhere, so every wave of a pair
@@ -1921,8 +1921,8 @@ RailPlan plan_rail_unbounded(const Geometry& g, const SplitPlan& sp)
     const int pv = sp.pv;
     RailPlan p = {kRailTile, 1, 4, 1, 1};
     // The lines between the forms were set on 2800 launches of random sizes (streams of 32 to 256 bits, kernels of 1, 3 and
-    // 5, every accumulation), each timed in some forty forms: what this rule takes is 5.4 % over the best form of each on
-    // the (geometric) average.
+    // 5, every accumulation), each timed in some forty forms with every word of a line ORed: what this rule took was 5.4 %
+    // over the best form of each on the (geometric) average.  (Only the tile and pair kernels skip zero words.)
     // Short groups, where the 32 LDS additions at the end of a group weigh most, keep their sums in registers
     // once four waves per SIMD exist without splitting a tile (3 -> 32, 5 x 5, 32 x 32, batch 256, L 64: 64 us
     // against 72), where a tile has a single pair (4 -> 11 channels, 1 x 1, 13 x 31, batch 86: 5.3 against 7.1), with a dozen
