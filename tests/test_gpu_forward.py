@@ -760,7 +760,7 @@ def launch_time(capi, shape_x, shape_w, pad, L, keep):
     return best
 
 
-@pytest.mark.parametrize("first,bound", [(0, 1.12), (8, 1.12), (12, 1.06)])
+@pytest.mark.parametrize("first,bound", [(0, 1.12), (8, 1.12), (12, 1.07)])
 def test_full_weight_lines_behind_emptier_ones_take_their_time(capi, first, bound):
     """A group whose first channel is emptier than the others is hardly slower than one of full lines (1.00 - 1.02 measured; 1.24 times
     that if it stays in the loop for mostly empty lines, 1.09 if full lines take the jump of the loop for thinned ones)."""
