@@ -22,7 +22,10 @@
 // these kernels too (77 items of 45 x 27 x 19 -> 83 channels, z_unit 32: weight gradient 216 us on
 // fp32 MFMAs with element-wise loads, 97 here; input gradient 136, 83);
 // exp and the product with g are fused into the first GEMM's epilogue; the second is split over m
-// and reduced deterministically.
+// and reduced deterministically.  Where every x and w is a bf16 number, as the 7-bit operands of the layers are
+// (k / 128), eleven of the eighteen term products would multiply by zeros: a scan finds that out on the device and the
+// products are left out (GemmParams::one_term), the same results bit for bit.  Three products of 64 -> 64 at 56 x 56,
+// batch 128: 438 + 411 + 426 -> 349 + 303 + 349 us; 512 -> 512 at 4 x 4, batch 128, first product: 126 -> 61.
 //
 // The other accumulation modes have the same surrogate with other add groups
 // (utils_functional.py:254-299): one exponential per add group, whose argument sums the OR
@@ -54,6 +57,10 @@ __device__ __forceinline__ float exp_neg(float z) { return __expf(-z); }
 
 constexpr int kTile = 128;   // block tile in I and J
 constexpr int kChunk = 16;   // K per LDS stage
+
+// the three products of the backward: E from col and wcat, the weight gradient from col and E, the input gradient from the
+// weights and E
+enum Product { PRODUCT_E = 0, PRODUCT_DW = 1, PRODUCT_DX = 2 };
 
 enum Epilogue { EPI_STORE = 0, EPI_EXP_TIMES_G = 1, EPI_EXP_TIMES_G_PLANES = 2, EPI_STORE_ITEMS = 3 };
 
@@ -90,6 +97,10 @@ struct GemmParams {
     // exists, zero elsewhere (read from sh_zero).
     const float* __restrict__ sh_zero;
     int sh_j, sh_wo, sh_ho, sh_win, sh_hin, sh_pad, sh_padh, sh_wk, sh_hk;
+    // not null: a word that says whether every x and w is a bf16 number (k_bwd_prep).  Where it is not zero, the
+    // operands made from them are one term of the split instead of three, and the rows that `a` of the first two products
+    // points to hold bf16 numbers (the same elements at the same indexes).
+    const int* __restrict__ one_term;
     // EPI_STORE_ITEMS: column j = (n, rest) of the result goes to c[(n * I + i) * c_plane + rest] (c_plane
     // columns per item): the input gradient in the caller's layout (n, c_in, w_in, h_in)
     int c_plane;
@@ -249,23 +260,105 @@ __device__ __forceinline__ void split3(float a, float b, unsigned& hi, unsigned&
     lo = pack_bf16(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
 }
 
+// What a thread holds of eight staged elements: fp32 values; bf16 bits, one element per register where the operand
+// is K-major (eight loads), two where it is I-major (in the first four registers).
+typedef unsigned short bf16_bits;
+template <typename T>
+using raw_of = typename std::conditional<std::is_same<T, float>::value, float, unsigned>::type;
+
+// eight elements along k of an I-major row whose first element lies on an 8-byte (bf16) or 16-byte (fp32) boundary
+__device__ __forceinline__ void load_row(const float* p, float (&r)[8])
+{
+    const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
+    r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
+    r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
+}
+__device__ __forceinline__ void load_row(const bf16_bits* p, unsigned (&r)[8])
+{
+    const uint2 v0 = *(const uint2*)p, v1 = *(const uint2*)(p + 4);
+    r[0] = v0.x; r[1] = v0.y; r[2] = v1.x; r[3] = v1.y;
+}
+// the same of a partial chunk: elements from k_left on (counted from the chunk, this thread's start at k0) are read from
+// the chunk's first element instead
+__device__ __forceinline__ void load_row_part(const float* p, int k0, int k_left, float (&r)[8])
+{
+#pragma unroll
+    for (int c = 0; c < 8; c++) r[c] = p[k0 + c < k_left ? c : -k0];
+}
+__device__ __forceinline__ void load_row_part(const bf16_bits* p, int k0, int k_left, unsigned (&r)[8])
+{
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        r[c] = (unsigned)p[k0 + 2 * c < k_left ? 2 * c : -k0] | (unsigned)p[k0 + 2 * c + 1 < k_left ? 2 * c + 1 : -k0] << 16;
+}
+// zeroes the elements from k_left on
+template <typename T, bool KMAJOR>
+__device__ __forceinline__ void zero_past(raw_of<T> (&r)[8], int k0, int k_left)
+{
+    if constexpr (std::is_same<T, float>::value || KMAJOR) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) r[c] = k0 + c < k_left ? r[c] : (raw_of<T>)0;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            r[c] &= (k0 + 2 * c < k_left ? 0x0000ffffu : 0u) | (k0 + 2 * c + 1 < k_left ? 0xffff0000u : 0u);
+    }
+}
+// pair c of eight staged elements as one term
+template <typename T, bool KMAJOR>
+__device__ __forceinline__ unsigned one_term_pair(const raw_of<T> (&r)[8], int c)
+{
+    if constexpr (std::is_same<T, float>::value)
+        return pack_bf16(r[2 * c], r[2 * c + 1]);
+    else
+        return KMAJOR ? r[2 * c] | r[2 * c + 1] << 16 : r[c];
+}
+// eight staged elements as TERMS terms into LDS
+template <int TERMS, typename T, bool KMAJOR>
+__device__ __forceinline__ void commit_terms(uint4 (*s)[2][kLdx], int half, int ii, const raw_of<T> (&r)[8])
+{
+    unsigned hi[4], mid[4], lo[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        if constexpr (TERMS == 1)
+            hi[c] = one_term_pair<T, KMAJOR>(r, c);
+        else
+            split3(r[2 * c], r[2 * c + 1], hi[c], mid[c], lo[c]);
+    }
+    s[0][half][ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    if constexpr (TERMS == 3) {
+        s[1][half][ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+        s[2][half][ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+}
+
+// The term products of a product of operands with TA and TB terms, smallest first; 0 = hi, 1 = mid, 2 = lo.  An operand
+// of one term leaves the products out that would multiply by its zero terms: the sums are the same bit for bit.
+template <int TA, int TB>
+struct TermProducts {
+    static_assert((TA == 1 || TA == 3) && (TB == 1 || TB == 3), "one term or three");
+    static constexpr int N = TA == 3 && TB == 3 ? 6 : TA == 3 || TB == 3 ? 3 : 1;
+    static constexpr int a(int t) { constexpr int v[6] = {2, 0, 1, 1, 0, 0}; return TA == 1 ? 0 : TB == 1 ? 2 - t : v[t]; }
+    static constexpr int b(int t) { constexpr int v[6] = {0, 2, 1, 0, 1, 0}; return TB == 1 ? 0 : TA == 1 ? 2 - t : v[t]; }
+};
+
 // Staging for the split kernel: a thread owns eight consecutive k (one half of the chunk) of one i,
 // which is what one lane feeds to the MFMA, and commit() writes them as s[term][k half][i], 16 bytes
 // (four words of two bf16) per term.
-//   K-major operand (element (k, i) at p[k*ld + i]): eight dword loads from a wave-uniform row pointer
+//   K-major operand (element (k, i) at p[k*ld + i]): eight element loads from a wave-uniform row pointer
 //     each, lanes along i; the k half is the wave's (uniform)
-//   I-major operand (element (k, i) at p[i*ld + k]): two float4 along k
+//   I-major operand (element (k, i) at p[i*ld + k]): load_row along k
 // Rows i outside the operand are clamped to its last row: what they produce is never stored.  Only a
 // partial last chunk is zeroed beyond its k range.
-template <bool KMAJOR>
+template <bool KMAJOR, typename T = float>
 struct SplitStager {
-    const float* p;   // K-major: row k_begin + 8 * half of the operand (uniform); I-major: this thread's first element
+    const T* p;       // K-major: row k_begin + 8 * half of the operand (uniform); I-major: this thread's first element
     long long ld;
     int off;          // K-major: this thread's i (clamped)
     int half, ii;
 
     // (ii_, half_): the row of the tile and the k half this thread stages (stage_slot)
-    __device__ __forceinline__ void init(const float* base, long long ld_, int i0, int k_begin, int I, int ii_, int half_)
+    __device__ __forceinline__ void init(const T* base, long long ld_, int i0, int k_begin, int I, int ii_, int half_)
     {
         ld = ld_;
         ii = ii_;
@@ -280,21 +373,18 @@ struct SplitStager {
     // past a chunk that another thread stages
     __device__ __forceinline__ void skip_chunk() { p += KMAJOR ? (long long)kChunk * ld : (long long)kChunk; }
     // a whole chunk, no branches
-    __device__ __forceinline__ void fetch_whole(float (&r)[8])
+    __device__ __forceinline__ void fetch_whole(raw_of<T> (&r)[8])
     {
         if (KMAJOR) {
 #pragma unroll
             for (int c = 0; c < 8; c++) r[c] = (p + (long long)c * ld)[off];
-            p += (long long)kChunk * ld;
         } else {
-            const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
-            r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-            r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
-            p += kChunk;
+            load_row(p, r);
         }
+        skip_chunk();
     }
     // k_left: what is left of the k range from this chunk's start (a partial last chunk has < kChunk)
-    __device__ __forceinline__ void fetch(float (&r)[8], int k_left)
+    __device__ __forceinline__ void fetch(raw_of<T> (&r)[8], int k_left)
     {
         const bool tail = k_left < kChunk;
         if (KMAJOR) {
@@ -304,35 +394,19 @@ struct SplitStager {
                 const long long row = (tail && 8 * half + c >= k_left) ? -8 * half : c;
                 r[c] = (p + row * ld)[off];
             }
-            p += (long long)kChunk * ld;
         } else {
-            if (!tail) {
-                const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
-                r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-                r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 8; c++) r[c] = p[8 * half + c < k_left ? c : -8 * half];
-            }
-            p += kChunk;
+            if (!tail)
+                load_row(p, r);
+            else
+                load_row_part(p, 8 * half, k_left, r);
         }
+        skip_chunk();
     }
-    __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], float (&r)[8], int k_left) const
+    template <int TERMS>
+    __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], raw_of<T> (&r)[8], int k_left) const
     {
-        if (k_left < kChunk) {
-#pragma unroll
-            for (int c = 0; c < 8; c++) r[c] = 8 * half + c < k_left ? r[c] : 0.0f;
-        }
-        commit_whole(s, r);
-    }
-    __device__ __forceinline__ void commit_whole(uint4 (*s)[2][kLdx], const float (&r)[8]) const
-    {
-        unsigned hi[4], mid[4], lo[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) split3(r[2 * c], r[2 * c + 1], hi[c], mid[c], lo[c]);
-        s[0][half][ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        s[1][half][ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
-        s[2][half][ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        if (k_left < kChunk) zero_past<T, KMAJOR>(r, 8 * half, k_left);
+        commit_terms<TERMS, T, KMAJOR>(s, half, ii, r);
     }
 };
 
@@ -345,11 +419,11 @@ struct SplitStager {
 // AHEAD (K-major only): the table entries of a chunk are read when the chunk before it is fetched, so that a
 // fetch issues its loads without waiting for the table first; the entries read for the chunk behind the last
 // one (up to 2 * kChunk + 8 entries behind the member's part of the table) are never used.
-template <bool KMAJOR, bool AHEAD = false>
+template <bool KMAJOR, typename T = float, bool AHEAD = false>
 struct ViewStager {
-    const float* base;
+    const T* base;
     const long long* rows;  // K-major: the table of this batch member (uniform)
-    const float* p;         // I-major: this thread's first element
+    const T* p;             // I-major: this thread's first element
     int off;                // K-major: this thread's element of every row
     int kr;                 // K-major: first row of this thread's half of the current chunk
     int in_item, item, skip;
@@ -366,7 +440,7 @@ struct ViewStager {
 
     __device__ __forceinline__ void init(const GemmParams& q, int batch, int i0, int k_begin, int I, int ii_, int half_)
     {
-        base = q.a;
+        base = (const T*)q.a;
         rows = q.a_rows + batch * q.a_rows_batch;
         item = q.a_item;
         skip = q.a_skip;
@@ -407,7 +481,7 @@ struct ViewStager {
         advance();
         read_ahead();
     }
-    __device__ __forceinline__ void fetch_whole(float (&r)[8])
+    __device__ __forceinline__ void fetch_whole(raw_of<T> (&r)[8])
     {
         if constexpr (KMAJOR && AHEAD) {
 #pragma unroll
@@ -420,13 +494,11 @@ struct ViewStager {
 #pragma unroll
             for (int c = 0; c < 8; c++) r[c] = (base + rows[kr + c])[off];
         } else {
-            const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
-            r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-            r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
+            load_row(p, r);
         }
         advance();
     }
-    __device__ __forceinline__ void fetch(float (&r)[8], int k_left)
+    __device__ __forceinline__ void fetch(raw_of<T> (&r)[8], int k_left)
     {
         const bool tail = k_left < kChunk;
         if (KMAJOR) {
@@ -437,29 +509,18 @@ struct ViewStager {
                 r[c] = (base + rows[row])[off];
             }
         } else {
-            if (!tail) {
-                const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
-                r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-                r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 8; c++) r[c] = p[8 * half + c < k_left ? c : -8 * half];
-            }
+            if (!tail)
+                load_row(p, r);
+            else
+                load_row_part(p, 8 * half, k_left, r);
         }
         advance();
     }
-    __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], float (&r)[8], int k_left) const
+    template <int TERMS>
+    __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], raw_of<T> (&r)[8], int k_left) const
     {
-        if (k_left < kChunk) {
-#pragma unroll
-            for (int c = 0; c < 8; c++) r[c] = 8 * half + c < k_left ? r[c] : 0.0f;
-        }
-        unsigned hi[4], mid[4], lo[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) split3(r[2 * c], r[2 * c + 1], hi[c], mid[c], lo[c]);
-        s[0][half][ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        s[1][half][ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
-        s[2][half][ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        if (k_left < kChunk) zero_past<T, KMAJOR>(r, 8 * half, k_left);
+        commit_terms<TERMS, T, KMAJOR>(s, half, ii, r);
     }
 };
 
@@ -528,26 +589,21 @@ struct ShiftStager {
     }
     __device__ __forceinline__ void fetch_whole(float (&r)[8])
     {
-        const float4 v0 = *(const float4*)p, v1 = *(const float4*)(p + 4);
-        r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-        r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
+        load_row(p, r);
         advance();
     }
     __device__ __forceinline__ void fetch(float (&r)[8], int) { fetch_whole(r); }
+    template <int TERMS>
     __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], float (&r)[8], int) const
     {
-        unsigned hi[4], mid[4], lo[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) split3(r[2 * c], r[2 * c + 1], hi[c], mid[c], lo[c]);
-        s[0][half][ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        s[1][half][ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
-        s[2][half][ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        commit_terms<TERMS, float, false>(s, half, ii, r);
     }
 };
 
 // v_mfma_f32_32x32x16_bf16: lane l feeds A[i = l%32][k = 8 (l/32) .. + 7] and B[those k][j = l%32]:
 // the 16 bytes at s[term][l/32][i]; results as in the fp32 instruction.
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int NX, int NY, bool VA, bool VB>
+// TA, TB: terms of the operands; A: type of A's elements in memory (B's are fp32).
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int NX, int NY, bool VA, bool VB, int TA, int TB, typename A>
 __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)[3][2][kLdx], uint4 (*bs)[3][2][kLdx],
                                                 int i0, int j0, int batch, int split, int k_begin, int k_end, int wi,
                                                 int wj, int l32, int lk, int wave)
@@ -560,24 +616,26 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[x][y][r] = 0.0f;
 
-    typename std::conditional<VA, ViewStager<A_KMAJOR>, SplitStager<A_KMAJOR>>::type sa;
+    constexpr bool BK = B_KMAJOR && !VB;
+    typename std::conditional<VA, ViewStager<A_KMAJOR, A>, SplitStager<A_KMAJOR, A>>::type sa;
     typename std::conditional<VB, ShiftStager, SplitStager<B_KMAJOR>>::type sb;
     // K-major operand: waves 0, 1 stage the first k half of the 128 rows, waves 2, 3 the second;
     // I-major operand: two threads per row, one k half each
     const int t = threadIdx.x;
     const int a_ii = A_KMAJOR ? (t & 127) : (t >> 1), a_half = A_KMAJOR ? (wave >> 1) : (t & 1);
-    const int b_ii = (B_KMAJOR && !VB) ? (t & 127) : (t >> 1), b_half = (B_KMAJOR && !VB) ? (wave >> 1) : (t & 1);
+    const int b_ii = BK ? (t & 127) : (t >> 1), b_half = BK ? (wave >> 1) : (t & 1);
     if constexpr (VA)
         sa.init(q, batch, i0, k_begin, min(q.I, i0 + q.tile_i), a_ii, a_half);
     else
-        sa.init(q.a + batch * q.a_batch_stride, q.lda, i0, k_begin, min(q.I, i0 + q.tile_i), a_ii, a_half);
+        sa.init((const A*)q.a + batch * q.a_batch_stride, q.lda, i0, k_begin, min(q.I, i0 + q.tile_i), a_ii, a_half);
     if constexpr (VB)
         sb.init(q, batch, j0, k_begin, min(q.J, j0 + q.tile_j), b_ii, b_half);
     else
         sb.init(q.b + batch * q.b_batch_stride, q.ldb, j0, k_begin, min(q.J, j0 + q.tile_j), b_ii, b_half);
     // Two chunks ahead: while chunk c is multiplied out of LDS, chunk c + 1 sits in one register set
     // (its loads issued a whole trip ago) and the loads of chunk c + 2 go out into the other.
-    float ra[2][8], rb[2][8];
+    raw_of<A> ra[2][8];
+    float rb[2][8];
     const int k_len = k_end - k_begin;
     const int n_chunks = k_len > 0 ? (k_len + kChunk - 1) / kChunk : 0;
     if (n_chunks > 0) {
@@ -589,57 +647,56 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
         sb.fetch(rb[1], k_len - kChunk);
     }
     if (n_chunks > 0) {
-        sa.commit(as[0], ra[0], k_len);
-        sb.commit(bs[0], rb[0], k_len);
+        sa.template commit<TA>(as[0], ra[0], k_len);
+        sb.template commit<TB>(bs[0], rb[0], k_len);
     }
     __syncthreads();
+    using Products = TermProducts<TA, TB>;
     auto multiply = [&](int buf) {
-        bf16x8 a[NX ? NX : 1][3], b[NY ? NY : 1][3];
+        bf16x8 a[NX ? NX : 1][TA], b[NY ? NY : 1][TB];
 #pragma unroll
-        for (int t = 0; t < 3; t++) {
+        for (int t = 0; t < TA; t++)
 #pragma unroll
             for (int x = 0; x < NX; x++) a[x][t] = __builtin_bit_cast(bf16x8, as[buf][t][lk][wi + 32 * x + l32]);
 #pragma unroll
-            for (int y = 0; y < NY; y++) b[y][t] = __builtin_bit_cast(bf16x8, bs[buf][t][lk][wj + 32 * y + l32]);
-        }
-        // smallest terms first; 0 = hi, 1 = mid, 2 = lo
-        constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+        for (int t = 0; t < TB; t++)
 #pragma unroll
-        for (int t = 0; t < 6; t++)
+            for (int y = 0; y < NY; y++) b[y][t] = __builtin_bit_cast(bf16x8, bs[buf][t][lk][wj + 32 * y + l32]);
+#pragma unroll
+        for (int t = 0; t < Products::N; t++)
 #pragma unroll
             for (int x = 0; x < NX; x++)
 #pragma unroll
                 for (int y = 0; y < NY; y++)
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][ta[t]], b[y][tb[t]], acc[x][y], 0, 0, 0);
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][Products::a(t)], b[y][Products::b(t)], acc[x][y], 0, 0, 0);
     };
     int c = 0;
-    // Whole chunks, no branches in the trip.  The split of chunk c + 1 (vector ALU, 24 steps: three per
+    // Whole chunks, no branches in the trip.  The split of chunk c + 1 (vector ALU, 24 steps of three terms: three per
     // pair of elements) is written between the MFMAs of chunk c, one step per MFMA with four blocks, so
     // that it issues while the matrix pipe is busy.  (Scheduling barriers that spelled this order out held in
     // the first of the loop's two trips only: in the second the compiler chained the six MFMAs of each
     // block back to back.  Without them both trips keep the written order.)
     const int n_whole = k_len > 0 ? k_len / kChunk : 0;
-    constexpr int kMfmas = NX * NY > 0 ? 6 * NX * NY : 1;  // per trip
-    constexpr int kStepsPerMfma = (24 + kMfmas - 1) / kMfmas;
+    constexpr int kMfmas = NX * NY > 0 ? Products::N * NX * NY : 1;  // per trip
+    constexpr int kStepsA = 4 * TA, kSteps = kStepsA + 4 * TB;
+    constexpr int kStepsPerMfma = (kSteps + kMfmas - 1) / kMfmas;
     auto multiply_and_split = [&](auto set) {
         constexpr int S = decltype(set)::value;
         sa.fetch_whole(ra[S]);
         sb.fetch_whole(rb[S]);
-        bf16x8 a[NX ? NX : 1][3], b[NY ? NY : 1][3];
+        bf16x8 a[NX ? NX : 1][TA], b[NY ? NY : 1][TB];
 #pragma unroll
-        for (int t = 0; t < 3; t++) {
+        for (int t = 0; t < TA; t++)
 #pragma unroll
             for (int x = 0; x < NX; x++) a[x][t] = __builtin_bit_cast(bf16x8, as[S][t][lk][wi + 32 * x + l32]);
 #pragma unroll
+        for (int t = 0; t < TB; t++)
+#pragma unroll
             for (int y = 0; y < NY; y++) b[y][t] = __builtin_bit_cast(bf16x8, bs[S][t][lk][wj + 32 * y + l32]);
-        }
-        constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
         // pairs 0..3: this thread's elements of A, 4..7: of B
         unsigned hi[8], mid[8], lo[8];
         float r0[8], r1[8];
-        auto step = [&](int n) {
-            const int pr = n / 3, st = n % 3;
-            const float* src = pr < 4 ? ra[S ^ 1] : rb[S ^ 1];
+        auto split_step = [&](int pr, int st, const float (&src)[8]) {
             const int e = 2 * (pr & 3);
             if (st == 0) {
                 hi[pr] = pack_bf16(src[e], src[e + 1]);
@@ -653,20 +710,37 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
                 lo[pr] = pack_bf16(r0[pr], r1[pr]);
             }
         };
+        auto step = [&](int n) {
+            if (n < kStepsA) {
+                if constexpr (TA == 1)
+                    hi[n] = one_term_pair<A, A_KMAJOR>(ra[S ^ 1], n);
+                else
+                    split_step(n / 3, n % 3, ra[S ^ 1]);
+            } else {
+                const int m = n - kStepsA;
+                if constexpr (TB == 1)
+                    hi[4 + m] = one_term_pair<float, BK>(rb[S ^ 1], m);
+                else
+                    split_step(4 + m / 3, m % 3, rb[S ^ 1]);
+            }
+        };
 #pragma unroll
         for (int m = 0; m < kMfmas; m++) {
             constexpr int kBlocks = NX * NY > 0 ? NX * NY : 1, kNy = NY > 0 ? NY : 1;
             const int t = m / kBlocks, x = (m % kBlocks) / kNy, y = m % kNy;
-            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][ta[t]], b[y][tb[t]], acc[x][y], 0, 0, 0);
+            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][Products::a(t)], b[y][Products::b(t)], acc[x][y], 0, 0, 0);
 #pragma unroll
-            for (int n = m * kStepsPerMfma; n < (m + 1) * kStepsPerMfma && n < 24; n++) step(n);
+            for (int n = m * kStepsPerMfma; n < (m + 1) * kStepsPerMfma && n < kSteps; n++) step(n);
         }
-        as[S ^ 1][0][sa.half][sa.ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        as[S ^ 1][1][sa.half][sa.ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
-        as[S ^ 1][2][sa.half][sa.ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-        bs[S ^ 1][0][sb.half][sb.ii] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-        bs[S ^ 1][1][sb.half][sb.ii] = make_uint4(mid[4], mid[5], mid[6], mid[7]);
-        bs[S ^ 1][2][sb.half][sb.ii] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
+        auto write = [&](uint4 (*to)[2][kLdx], int half, int ii, int o, int terms) {
+            to[0][half][ii] = make_uint4(hi[o], hi[o + 1], hi[o + 2], hi[o + 3]);
+            if (terms == 3) {
+                to[1][half][ii] = make_uint4(mid[o], mid[o + 1], mid[o + 2], mid[o + 3]);
+                to[2][half][ii] = make_uint4(lo[o], lo[o + 1], lo[o + 2], lo[o + 3]);
+            }
+        };
+        write(as[S ^ 1], sa.half, sa.ii, 0, TA);
+        write(bs[S ^ 1], sb.half, sb.ii, 4, TB);
         __syncthreads();
     };
     if (NX * NY > 0) {
@@ -682,8 +756,8 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
             sb.fetch(rb[0], k_len - (c + 2) * kChunk);
         }
         multiply(0);
-        sa.commit(as[1], ra[1], k_len - (c + 1) * kChunk);
-        sb.commit(bs[1], rb[1], k_len - (c + 1) * kChunk);
+        sa.template commit<TA>(as[1], ra[1], k_len - (c + 1) * kChunk);
+        sb.template commit<TB>(bs[1], rb[1], k_len - (c + 1) * kChunk);
         __syncthreads();
         // chunk c + 1 from LDS buffer 1; register set 0 holds chunk c + 2
         if (c + 3 < n_chunks) {
@@ -692,8 +766,8 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
         }
         multiply(1);
         if (c + 2 < n_chunks) {
-            sa.commit(as[0], ra[0], k_len - (c + 2) * kChunk);
-            sb.commit(bs[0], rb[0], k_len - (c + 2) * kChunk);
+            sa.template commit<TA>(as[0], ra[0], k_len - (c + 2) * kChunk);
+            sb.template commit<TB>(bs[0], rb[0], k_len - (c + 2) * kChunk);
         }
         __syncthreads();
     }
@@ -703,7 +777,7 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
 }
 
 // Operands with 16-byte aligned rows and chunks (launch_gemm checks).
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool VA = false, bool VB = false>
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA = false, bool VB = false>
 // three waves per SIMD (at most 168 registers; three workgroups' LDS fit a CU)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_gemm_split(GemmParams q)
 {
@@ -723,16 +797,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const bool x0 = i0 + wi < q.I, x1 = !narrow_j && i0 + wi + 32 < q.I;
     const bool y0 = j0 + wj < q.J, y1 = !narrow_i && j0 + wj + 32 < q.J;
     const int blocks_xy = (x0 && y0) ? 2 * (int)x1 + (int)y1 : -1;
+    auto tile = [&](auto ta, auto tb, auto element) {
+        constexpr int TA = decltype(ta)::value, TB = decltype(tb)::value;
+        using A = decltype(element);
 #define GEO_SC_GEMM_WAVE(NX, NY)                                                                                        \
-    gemm_wave_split<A_KMAJOR, B_KMAJOR, EPI, NX, NY, VA, VB>(q, as, bs, i0, j0, batch, split, k_begin, k_end, wi, wj, l32, lk, wave)
-    switch (blocks_xy) {
-    case 3: GEO_SC_GEMM_WAVE(2, 2); break;
-    case 2: GEO_SC_GEMM_WAVE(2, 1); break;
-    case 1: GEO_SC_GEMM_WAVE(1, 2); break;
-    case 0: GEO_SC_GEMM_WAVE(1, 1); break;
-    default: GEO_SC_GEMM_WAVE(0, 0); break;
-    }
+    gemm_wave_split<A_KMAJOR, B_KMAJOR, EPI, NX, NY, VA, VB, TA, TB, A>(q, as, bs, i0, j0, batch, split, k_begin, k_end, wi, wj, l32, lk, wave)
+        switch (blocks_xy) {
+        case 3: GEO_SC_GEMM_WAVE(2, 2); break;
+        case 2: GEO_SC_GEMM_WAVE(2, 1); break;
+        case 1: GEO_SC_GEMM_WAVE(1, 2); break;
+        case 0: GEO_SC_GEMM_WAVE(1, 1); break;
+        default: GEO_SC_GEMM_WAVE(0, 0); break;
+        }
 #undef GEO_SC_GEMM_WAVE
+    };
+    using One = std::integral_constant<int, 1>;
+    using Three = std::integral_constant<int, 3>;
+    if (!(q.one_term && *q.one_term))
+        tile(Three(), Three(), 0.0f);
+    else if constexpr (PRODUCT == PRODUCT_E)
+        tile(One(), One(), bf16_bits());
+    else if constexpr (PRODUCT == PRODUCT_DW)
+        tile(One(), Three(), bf16_bits());
+    else
+        tile(One(), Three(), 0.0f);
 }
 
 // ---- the split kernel with eight waves per workgroup and a tile of 64 NX x 256 ----
@@ -757,13 +845,12 @@ inline int big_rows(int I) { return I % 256 == 0 ? 256 : I % 192 == 0 ? 192 : I 
 // KC: chunks per trip.  With NX = 2 a trip of one chunk holds 24 MFMAs per wave, too few for what every trip
 // costs besides (barrier, the latency of the first LDS reads, the loads' address arithmetic); two chunks per
 // trip (KC = 2, 150 KB of LDS) halve that share.
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool VA, bool VB, int NX, int KC = 1>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_big(GemmParams q)
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool VA, bool VB, int NX, int KC, int TA, int TB, typename A>
+__device__ __forceinline__ void gemm_big_tiles(const GemmParams& q, uint4 (*as)[3][2 * KC][64 * NX + 4],
+                                               uint4 (*bs)[3][2 * KC][kBigJ + 4])
 {
-    constexpr int RA = 64 * NX, LA = RA + 4, LB = kBigJ + 4;
+    constexpr int RA = 64 * NX;
     constexpr int kUnit = KC * kChunk;  // k per trip
-    __shared__ uint4 as[2][3][2 * KC][LA];
-    __shared__ uint4 bs[2][3][2 * KC][LB];
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
     const int wi = (wave >> 2) * (32 * NX), wj = (wave & 3) * 64;
     const int l32 = lane & 31, lk = lane >> 5;
@@ -777,7 +864,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int a_ii = A_KMAJOR ? (wa % NX) * 64 + lane : ta / (2 * KC);
     const int a_q = A_KMAJOR ? wa / NX : ta % (2 * KC);  // which eight k of the trip
     const int b_ii = BK ? (t & 255) : (t >> 1), b_half = BK ? (wave >> 2) : (t & 1);
-    typename std::conditional<VA, ViewStager<A_KMAJOR, true>, SplitStager<A_KMAJOR>>::type sa;
+    typename std::conditional<VA, ViewStager<A_KMAJOR, A, true>, SplitStager<A_KMAJOR, A>>::type sa;
     typename std::conditional<VB, ShiftStager, SplitStager<B_KMAJOR>>::type sb;
 
     const int n_tiles = q.ni * q.nj * q.nz;
@@ -793,7 +880,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if constexpr (VA)
             sa.init(q, batch, it * RA, ka, q.I, a_ii, a_q & 1);
         else
-            sa.init(q.a + batch * q.a_batch_stride, q.lda, it * RA, ka, q.I, a_ii, a_q & 1);
+            sa.init((const A*)q.a + batch * q.a_batch_stride, q.lda, it * RA, ka, q.I, a_ii, a_q & 1);
         if constexpr (VB)
             sb.init(q, batch, jt * kBigJ, k_begin, q.J, b_ii, b_half);
         else
@@ -803,7 +890,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // round that tile again (loads of valid addresses that nobody uses): every path through here issues the
     // same loads, so the waits that the compiler places in front of the split count only the loads of the
     // set they need - with a path that issues none, they would wait for the newest loads as well.
-    auto fetch_next = [&](float (&ra)[8], float (&rb)[KC][8]) {
+    auto fetch_next = [&](raw_of<A> (&ra)[8], float (&rb)[KC][8]) {
         if (left_f == 0) {
             if (w_f + (int)gridDim.x < n_tiles) w_f += gridDim.x;
             open_tile();
@@ -845,30 +932,62 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Register set c % 2 holds trip c of the stream until it is split and written to LDS buffer c % 2, one
     // trip before it is multiplied; its loads go out two trips before that.
     constexpr int kPairs = 4 + 4 * KC;  // pairs of elements per thread and trip: A, then B chunk by chunk
-    float ra[2][8], rb[2][KC][8];
+    raw_of<A> ra[2][8];
+    float rb[2][KC][8];
     auto write_split = [&](int buf, const unsigned (&hi)[kPairs], const unsigned (&mid)[kPairs], const unsigned (&lo)[kPairs]) {
         as[buf][0][a_q][a_ii] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        as[buf][1][a_q][a_ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
-        as[buf][2][a_q][a_ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        if (TA == 3) {
+            as[buf][1][a_q][a_ii] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+            as[buf][2][a_q][a_ii] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        }
 #pragma unroll
         for (int kc = 0; kc < KC; kc++) {
             const int o = 4 + 4 * kc;
             bs[buf][0][2 * kc + b_half][b_ii] = make_uint4(hi[o], hi[o + 1], hi[o + 2], hi[o + 3]);
-            bs[buf][1][2 * kc + b_half][b_ii] = make_uint4(mid[o], mid[o + 1], mid[o + 2], mid[o + 3]);
-            bs[buf][2][2 * kc + b_half][b_ii] = make_uint4(lo[o], lo[o + 1], lo[o + 2], lo[o + 3]);
+            if (TB == 3) {
+                bs[buf][1][2 * kc + b_half][b_ii] = make_uint4(mid[o], mid[o + 1], mid[o + 2], mid[o + 3]);
+                bs[buf][2][2 * kc + b_half][b_ii] = make_uint4(lo[o], lo[o + 1], lo[o + 2], lo[o + 3]);
+            }
+        }
+    };
+    // The split of a trip's elements: step n of kSteps, three per pair of an operand with three terms, one per pair else.
+    constexpr int kStepsA = 4 * TA, kSteps = kStepsA + 4 * KC * TB;
+    auto split_step = [](int pr, int st, float e0, float e1, unsigned (&hi)[kPairs], unsigned (&mid)[kPairs],
+                         unsigned (&lo)[kPairs], float (&r0)[kPairs], float (&r1)[kPairs]) {
+        if (st == 0) {
+            hi[pr] = pack_bf16(e0, e1);
+            r0[pr] = e0 - __uint_as_float(hi[pr] << 16);
+            r1[pr] = e1 - __uint_as_float(hi[pr] & 0xffff0000u);
+        } else if (st == 1) {
+            mid[pr] = pack_bf16(r0[pr], r1[pr]);
+            r0[pr] -= __uint_as_float(mid[pr] << 16);
+            r1[pr] -= __uint_as_float(mid[pr] & 0xffff0000u);
+        } else {
+            lo[pr] = pack_bf16(r0[pr], r1[pr]);
+        }
+    };
+    auto step = [&](int n, const raw_of<A> (&a)[8], const float (&b)[KC][8], unsigned (&hi)[kPairs], unsigned (&mid)[kPairs],
+                    unsigned (&lo)[kPairs], float (&r0)[kPairs], float (&r1)[kPairs]) {
+        if (n < kStepsA) {
+            if constexpr (TA == 1)
+                hi[n] = one_term_pair<A, A_KMAJOR>(a, n);
+            else
+                split_step(n / 3, n % 3, a[2 * (n / 3)], a[2 * (n / 3) + 1], hi, mid, lo, r0, r1);
+        } else {
+            const int m = (n - kStepsA) / TB, st = (n - kStepsA) % TB;  // pair of B, chunk m / 4
+            if constexpr (TB == 1)
+                hi[4 + m] = one_term_pair<float, BK>(b[m >> 2], m & 3);
+            else
+                split_step(4 + m, st, b[m >> 2][2 * (m & 3)], b[m >> 2][2 * (m & 3) + 1], hi, mid, lo, r0, r1);
         }
     };
     fetch_next(ra[0], rb[0]);
     fetch_next(ra[1], rb[1]);
     {
         unsigned hi[kPairs], mid[kPairs], lo[kPairs];
+        float r0[kPairs], r1[kPairs];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            split3(ra[0][2 * c], ra[0][2 * c + 1], hi[c], mid[c], lo[c]);
-#pragma unroll
-            for (int kc = 0; kc < KC; kc++)
-                split3(rb[0][kc][2 * c], rb[0][kc][2 * c + 1], hi[4 + 4 * kc + c], mid[4 + 4 * kc + c], lo[4 + 4 * kc + c]);
-        }
+        for (int n = 0; n < kSteps; n++) step(n, ra[0], rb[0], hi, mid, lo, r0, r1);
         write_split(0, hi, mid, lo);
     }
     fetch_next(ra[0], rb[0]);
@@ -879,45 +998,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // split works on stale registers and its result is never read.
     auto trip = [&](auto set) {
         constexpr int S = decltype(set)::value, R = S ^ 1;
-        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};  // smallest terms first; 0 = hi
-        constexpr int kSteps = 3 * kPairs, kMfmas = 12 * NX * KC;
+        using Products = TermProducts<TA, TB>;
+        constexpr int kMfmas = 2 * Products::N * NX * KC;
         unsigned hi[kPairs], mid[kPairs], lo[kPairs];
         float r0[kPairs], r1[kPairs];
-        auto step = [&](int n) {
-            const int pr = n / 3, st = n % 3;
-            const float* src = pr < 4 ? ra[R] : rb[R][(pr - 4) >> 2];
-            const int e = 2 * (pr & 3);
-            if (st == 0) {
-                hi[pr] = pack_bf16(src[e], src[e + 1]);
-                r0[pr] = src[e] - __uint_as_float(hi[pr] << 16);
-                r1[pr] = src[e + 1] - __uint_as_float(hi[pr] & 0xffff0000u);
-            } else if (st == 1) {
-                mid[pr] = pack_bf16(r0[pr], r1[pr]);
-                r0[pr] -= __uint_as_float(mid[pr] << 16);
-                r1[pr] -= __uint_as_float(mid[pr] & 0xffff0000u);
-            } else {
-                lo[pr] = pack_bf16(r0[pr], r1[pr]);
-            }
-        };
 #pragma unroll
         for (int kc = 0; kc < KC; kc++)
 #pragma unroll
-            for (int p6 = 0; p6 < 6; p6++) {
+            for (int p6 = 0; p6 < Products::N; p6++) {
                 bf16x8 a[NX], b[2];
 #pragma unroll
                 for (int x = 0; x < NX; x++)
-                    a[x] = __builtin_bit_cast(bf16x8, as[S][pa[p6]][2 * kc + lk][wi + 32 * x + l32]);
+                    a[x] = __builtin_bit_cast(bf16x8, as[S][Products::a(p6)][2 * kc + lk][wi + 32 * x + l32]);
 #pragma unroll
                 for (int y = 0; y < 2; y++)
-                    b[y] = __builtin_bit_cast(bf16x8, bs[S][pb[p6]][2 * kc + lk][wj + 32 * y + l32]);
+                    b[y] = __builtin_bit_cast(bf16x8, bs[S][Products::b(p6)][2 * kc + lk][wj + 32 * y + l32]);
 #pragma unroll
                 for (int m = 0; m < 2 * NX; m++) {
                     acc[m >> 1][m & 1] =
                         __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m >> 1], b[m & 1], acc[m >> 1][m & 1], 0, 0, 0);
                     // the split's steps spread over the trip's MFMAs
-                    const int gm = (kc * 6 + p6) * 2 * NX + m;
+                    const int gm = (kc * Products::N + p6) * 2 * NX + m;
 #pragma unroll
-                    for (int n = kSteps * gm / kMfmas; n < kSteps * (gm + 1) / kMfmas; n++) step(n);
+                    for (int n = kSteps * gm / kMfmas; n < kSteps * (gm + 1) / kMfmas; n++)
+                        step(n, ra[R], rb[R], hi, mid, lo, r0, r1);
                 }
             }
         write_split(R, hi, mid, lo);
@@ -957,6 +1061,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA, bool VB, int NX, int KC = 1>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_big(GemmParams q)
+{
+    __shared__ uint4 as[2][3][2 * KC][64 * NX + 4];
+    __shared__ uint4 bs[2][3][2 * KC][kBigJ + 4];
+    if (!(q.one_term && *q.one_term))
+        gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 3, 3, float>(q, as, bs);
+    else if constexpr (PRODUCT == PRODUCT_E)
+        gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 1, bf16_bits>(q, as, bs);
+    else if constexpr (PRODUCT == PRODUCT_DW)
+        gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 3, bf16_bits>(q, as, bs);
+    else
+        gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 3, float>(q, as, bs);
+}
+
 // gt[n*npos + pos][co] = g[n][co][pos]: the upstream gradient with the channel innermost, so that the
 // first GEMM's epilogue (lanes along the channel) reads it in contiguous runs instead of one
 // cache line per lane.  32 x 32 tiles through LDS; blockIdx.z = n.
@@ -975,25 +1094,6 @@ __global__ __launch_bounds__(256) void k_transpose_grad(const float* __restrict_
     for (int r = ty; r < 32; r += 8) {
         const int p = p0 + r, c = c0 + tx;
         if (p < npos && c < c_out) gt[item + (size_t)p * c_out + c] = tile[tx][r];
-    }
-}
-
-// Per output position m = (n, a, b): where its receptive field starts in the unpadded input.
-//   base[m] = ((n*c_in)*w_in + (a - pad_w))*h_in + (b - pad_h),  arow[m] = a - pad_w,  bcol[m] = b - pad_h
-// Built once per call; it keeps integer divisions out of the per-element kernels.
-__global__ __launch_bounds__(256) void k_position_table(int* __restrict__ base, int* __restrict__ arow,
-                                                        int* __restrict__ bcol, int m_total,
-                                                        int c_in, int c_out, int w_in, int h_in, int pad_w, int pad_h,
-                                                        int wo, int ho)
-{
-    for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
-        const int b = m % ho;
-        const int t = m / ho;
-        const int a = t % wo;
-        const int n = t / wo;
-        base[m] = ((n * c_in) * w_in + (a - pad_w)) * h_in + (b - pad_h);
-        arow[m] = a - pad_w;
-        bcol[m] = b - pad_h;
     }
 }
 
@@ -1080,12 +1180,101 @@ __host__ __device__ inline void group_of(const Groups& G, int ci, int u, int v, 
     }
 }
 
+// The bf16 numbers that floats known to be such stand for, and whether a float is one: its low half is zero.  Infinities
+// and NaN are left to three terms.
+__device__ __forceinline__ bf16_bits exact_bf16(float v) { return (bf16_bits)(__float_as_uint(v) >> 16); }
+__device__ __forceinline__ uint2 exact_bf16(const float4& v)
+{
+    return make_uint2(__float_as_uint(v.x) >> 16 | (__float_as_uint(v.y) & 0xffff0000u),
+                      __float_as_uint(v.z) >> 16 | (__float_as_uint(v.w) & 0xffff0000u));
+}
+__device__ __forceinline__ bool takes_three_terms(float v)
+{
+    const unsigned u = __float_as_uint(v);
+    return (u & 0xffffu) != 0 || (u & 0x7f800000u) == 0x7f800000u;
+}
+
+// Whether x and w are bf16 numbers throughout, which 7-bit operands (k / 128) are: the scan's blocks leave what they found
+// (scan_operands), the launch behind them agrees on it (operands_are_bf16) and keeps it for those that follow, which
+// read one word.  A thread stops at its first element that is none, so that the scan of other operands costs next to
+// nothing; 25.7 M floats of x take 20 us (64 -> 64 at 56 x 56, batch 128), of which bf16 planes alone give 16 back.
+// One row of kScanBlocks blocks, kScanRows from kScanFew elements on (36 us with 256 blocks).
+constexpr int kScanRows = 4;
+constexpr long long kScanFew = 1 << 21;
+inline int scan_rows(long long elements) { return elements < kScanFew ? 1 : kScanRows; }
+constexpr int kScanBlocks = 256;
+__device__ __forceinline__ void scan_operands(const float* __restrict__ x, long long nx, const float* __restrict__ w,
+                                              long long nw, int block, int blocks, int* __restrict__ found)
+{
+    bool three = false;
+    auto scan = [&](const float* __restrict__ p, long long n) {
+        const long long lead = min(n, (long long)((4 - (((uintptr_t)p >> 2) & 3)) & 3));  // floats in front of a quad
+        const long long quads = (n - lead) >> 2;
+        const float4* p4 = (const float4*)(p + lead);
+        if (block == 0 && threadIdx.x < 8) {
+            // the ends: what lies in front of the first quad and behind the last one
+            const long long e = threadIdx.x < 4 ? (long long)threadIdx.x : lead + 4 * quads + (threadIdx.x - 4);
+            if (threadIdx.x < 4 ? e < lead : e < n) three |= takes_three_terms(p[e]);
+        }
+        constexpr int kStep = 4;
+        const long long stride = (long long)blocks * 256;
+        for (long long i = (long long)block * 256 + threadIdx.x; i < quads && !three; i += kStep * stride) {
+            float4 v[kStep];
+#pragma unroll
+            for (int q = 0; q < kStep; q++) v[q] = p4[i + q * stride < quads ? i + q * stride : i];
+#pragma unroll
+            for (int q = 0; q < kStep; q++)
+                three |= takes_three_terms(v[q].x) || takes_three_terms(v[q].y) || takes_three_terms(v[q].z) ||
+                         takes_three_terms(v[q].w);
+        }
+    };
+    scan(w, nw);
+    scan(x, nx);
+    const int any = __syncthreads_or(three);
+    if (threadIdx.x == 0) found[block] = any;
+}
+// every thread of a block of 256; rows of the scan
+__device__ __forceinline__ bool operands_are_bf16(const int* __restrict__ found, int rows)
+{
+    static_assert(kScanBlocks == 256, "one word per thread and row");
+    int any = 0;
+    for (int r = 0; r < rows; r++) any |= found[r * 256 + threadIdx.x];
+    return !__syncthreads_or(any);
+}
+
+// Per output position m = (n, a, b): where its receptive field starts in the unpadded input.
+//   base[m] = ((n*c_in)*w_in + (a - pad_w))*h_in + (b - pad_h),  arow[m] = a - pad_w,  bcol[m] = b - pad_h
+// Built once per call; it keeps integer divisions out of the per-element kernels.
+// With `found`, the first block also turns what scan_operands found into *one_term.
+__global__ __launch_bounds__(256) void k_position_table(int* __restrict__ base, int* __restrict__ arow,
+                                                        int* __restrict__ bcol, const int* __restrict__ found, int found_rows,
+                                                        int* __restrict__ one_term, int m_total,
+                                                        int c_in, int c_out, int w_in, int h_in, int pad_w, int pad_h,
+                                                        int wo, int ho)
+{
+    if (found && blockIdx.x == 0) {
+        const bool one = operands_are_bf16(found, found_rows);
+        if (threadIdx.x == 0) *one_term = one;
+    }
+    for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
+        const int b = m % ho;
+        const int t = m / ho;
+        const int a = t % wo;
+        const int n = t / wo;
+        base[m] = ((n * c_in) * w_in + (a - pad_w)) * h_in + (b - pad_h);
+        arow[m] = a - pad_w;
+        bcol[m] = b - pad_h;
+    }
+}
+
 // col[g][k][m] = x~[n, ci, a+u, b+v] for groups g0 + blockIdx.z, (ci, u, v) = member k of the
 // group, m = (n, a, b); x~ is the zero-padded activation, read straight from the unpadded
 // tensor.  blockIdx.y selects kIm2colMembers consecutive members; a thread reads its position's
-// table entry once and moves those members.  Reads and writes run along m; rows are ld elements apart.
+// table entry once and moves those members.  Reads and writes run along m; rows are ld elements apart.  Where *one_term
+// says that x holds bf16 numbers, so does col.
 constexpr int kIm2colMembers = 12;
 __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x, float* __restrict__ col,
+                                                     const int* __restrict__ one_term,
                                                      const int* __restrict__ base, const int* __restrict__ arow,
                                                      const int* __restrict__ bcol, int g0, int m_total, int ld,
                                                      Groups G, int w_in, int h_in, size_t g_stride)
@@ -1094,6 +1283,7 @@ __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x
     const int k0 = blockIdx.y * kIm2colMembers;
     const int k1 = min(G.n_members, k0 + kIm2colMembers);
     float* colg = col + (size_t)blockIdx.z * g_stride;
+    const bool bf16_col = *one_term != 0;
     for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
         // all loads first, from x[0] where the member lies in the padding (a load inside a branch is
@@ -1107,6 +1297,12 @@ __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x
             const float val = x[ok ? b0 + (e.ci * w_in + e.u) * h_in + e.v : 0];
             vals[q] = ok ? val : 0.0f;
             next_member(G, e);
+        }
+        if (bf16_col) {
+#pragma unroll
+            for (int q = 0; q < kIm2colMembers; q++)
+                if (k0 + q < k1) ((bf16_bits*)col)[blockIdx.z * g_stride + (size_t)(k0 + q) * ld + m] = exact_bf16(vals[q]);
+            continue;
         }
 #pragma unroll
         for (int q = 0; q < kIm2colMembers; q++)
@@ -1132,6 +1328,7 @@ __device__ __forceinline__ float4 shifted_quad(const float4& a, const float4& b,
 // quads (the kernel tap shifts them by v - pad_h) and stored as one quad: a quarter of the loads,
 // stores and table reads of the one-position kernel.
 __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict__ x, float* __restrict__ col,
+                                                        const int* __restrict__ one_term,
                                                         const int* __restrict__ base, const int* __restrict__ arow,
                                                         const int* __restrict__ bcol, int g0, int m_total, Groups G,
                                                         int w_in, int h_in, size_t g_stride)
@@ -1142,6 +1339,7 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
     float* colg = col + (size_t)blockIdx.z * g_stride;
     const float4* x4 = (const float4*)x;
     const int quads = m_total >> 2;
+    const bool bf16_col = *one_term != 0;
     for (int mq = blockIdx.x * 256 + threadIdx.x; mq < quads; mq += gridDim.x * 256) {
         const int m = mq << 2;
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
@@ -1161,6 +1359,13 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
             vals[q] = shifted_quad(a, b, sh);
             next_member(G, e);
         }
+        if (bf16_col) {
+#pragma unroll
+            for (int q = 0; q < kIm2colMembers; q++)
+                if (k0 + q < k1)
+                    *(uint2*)((bf16_bits*)col + blockIdx.z * g_stride + (size_t)(k0 + q) * m_total + m) = exact_bf16(vals[q]);
+            continue;
+        }
 #pragma unroll
         for (int q = 0; q < kIm2colMembers; q++)
             if (k0 + q < k1) *(float4*)(colg + (size_t)(k0 + q) * m_total + m) = vals[q];
@@ -1173,32 +1378,58 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
 // the plane (v, ci) read from u * ho elements in, with the positions of item n shifted by
 // n * (w_k - 1) * ho -- a third of col's bytes for a 3-wide kernel, and the rows of one channel share
 // their cache lines.  Four columns per thread (ho and h_in multiples of four, 16-byte aligned x), as in
-// k_im2col_rows_v4.  `total` quads; the (w_k - 1) * ho elements behind the last plane are never read.
-__global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ x, float* __restrict__ xs, long long total,
-                                                      int n_items, int c_in, int w_in, int h_in, int pad_w, int pad_h,
+// k_im2col_rows_v4.  `total` quads; the (w_k - 1) * ho elements behind the last plane are never read.  Planes of bf16
+// numbers where x and w are such throughout, which the first block tells the products.
+constexpr int kShiftQuads = 4;
+__global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ x, float* __restrict__ xs,
+                                                      const int* __restrict__ found, int found_rows,
+                                                      int* __restrict__ one_term, unsigned total,
+                                                      unsigned n_items, unsigned c_in, int w_in, int h_in, int pad_w, int pad_h,
                                                       int ho)
 {
-    const int wp = w_in + 2 * pad_w, hq = ho >> 2;
+    const unsigned wp = w_in + 2 * pad_w, hq = ho >> 2;
     const float4* x4 = (const float4*)x;
-    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < total; e += (long long)gridDim.x * 256) {
-        // e = (((v * c_in + ci) * n_items + n) * wp + r) * hq + quad
-        long long t = e;
-        const int bq = (int)(t % hq);
-        t /= hq;
-        const int r = (int)(t % wp);
-        t /= wp;
-        const int n = (int)(t % n_items);
-        t /= n_items;
-        const int ci = (int)(t % c_in), v = (int)(t / c_in);
-        const int row = r - pad_w, c = 4 * bq + v - pad_h;  // input row, and input column of the first of the four
-        const int sh = c & 3, ca = c - sh;
-        const bool row_ok = row >= 0 && row < w_in;
-        const bool ok_a = row_ok && ca >= 0 && ca < h_in, ok_b = row_ok && sh != 0 && ca + 4 >= 0 && ca + 4 < h_in;
-        const long long at = ((((long long)n * c_in + ci) * w_in + row) * h_in + ca) >> 2;
-        float4 a = x4[ok_a ? at : 0], b = x4[ok_b ? at + 1 : 0];
-        if (!ok_a) a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (!ok_b) b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        ((float4*)xs)[e] = shifted_quad(a, b, sh);
+    const bool one = operands_are_bf16(found, found_rows);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *one_term = one;
+    // kShiftQuads quads per thread and trip, a block's width apart: their loads go out together
+    for (unsigned e0 = blockIdx.x * (256 * kShiftQuads) + threadIdx.x; e0 < total; e0 += gridDim.x * (256 * kShiftQuads)) {
+        float4 a[kShiftQuads], b[kShiftQuads];
+        int sh[kShiftQuads];
+        bool ok_a[kShiftQuads], ok_b[kShiftQuads];
+#pragma unroll
+        for (int q = 0; q < kShiftQuads; q++) {
+            const unsigned e = min(e0 + q * 256, total - 1);
+            // e = (((v * c_in + ci) * n_items + n) * wp + r) * hq + quad
+            unsigned t = e / hq;
+            const int bq = (int)(e - t * hq);
+            const unsigned pr = t / wp;
+            const int r = (int)(t - pr * wp);
+            t = pr / n_items;
+            const unsigned n = pr - t * n_items;
+            const int v = (int)(t / c_in);
+            const unsigned ci = t - v * c_in;
+            const int row = r - pad_w, c = 4 * bq + v - pad_h;  // input row, and input column of the first of the four
+            sh[q] = c & 3;
+            const int ca = c - sh[q];
+            const bool row_ok = row >= 0 && row < w_in;
+            ok_a[q] = row_ok && ca >= 0 && ca < h_in;
+            ok_b[q] = row_ok && sh[q] != 0 && ca + 4 >= 0 && ca + 4 < h_in;
+            const long long at = (((long long)(n * c_in + ci) * w_in + row) * h_in + ca) >> 2;
+            a[q] = x4[ok_a[q] ? at : 0];
+            b[q] = x4[ok_b[q] ? at + 1 : 0];
+        }
+#pragma unroll
+        for (int q = 0; q < kShiftQuads; q++) {
+            const unsigned e = e0 + q * 256;
+            if (!ok_a[q]) a[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (!ok_b[q]) b[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 quad = shifted_quad(a[q], b[q], sh[q]);
+            if (e >= total) break;
+            if (one)
+                ((uint2*)xs)[e] = exact_bf16(quad);
+            else
+                ((float4*)xs)[e] = quad;
+        }
     }
 }
 
@@ -1236,17 +1467,22 @@ __global__ __launch_bounds__(256) void k_weight_operands(const float* __restrict
 // by its operands ends at the element that makes it so.
 struct WgradOperands {
     const float* col;
+    const int* one_term;  // col holds bf16 numbers
     const float* e;
     long long m, col_ld, e_ld;
     size_t col_v, e_v;
 };
 __device__ __forceinline__ float wgrad_again(const WgradOperands& o, int group, int k, int j, long long begin, long long end)
 {
-    const float* c = o.col + group * o.col_v + k * o.col_ld;
+    const size_t c0 = group * o.col_v + k * o.col_ld;
+    const bool one = *o.one_term != 0;
     const float* e = o.e + group * o.e_v + j;
     float sum = 0.0f;
 #pragma unroll 1
-    for (long long m = begin; m < end && sum == sum; m++) sum = fmaf(c[m], e[m * o.e_ld], sum);
+    for (long long m = begin; m < end && sum == sum; m++) {
+        const float c = one ? __uint_as_float((unsigned)((const bf16_bits*)o.col)[c0 + m] << 16) : o.col[c0 + m];
+        sum = fmaf(c, e[m * o.e_ld], sum);
+    }
     return sum;
 }
 
@@ -1503,7 +1739,8 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restr
 //    apart (ShiftStager);
 //  * from the blocks of the round's first group: view_rows[g][k], where row k of group g's col starts in the
 //    planes of k_shift_planes (elements), for every group; and 64 zeros for the shifted view of E (a store
-//    rather than a memset, so that a caller may capture the launch sequence in a graph).
+//    rather than a memset, so that a caller may capture the launch sequence in a graph);
+//  * in rows of blocks of their own behind the groups': the scan of x and w.
 struct PrepParams {
     const float* __restrict__ w;
     float* __restrict__ wcat;
@@ -1516,9 +1753,19 @@ struct PrepParams {
     int view_groups, view_k_pad, ho;
     long long plane;
     float* zero;            // null: no block of zeros wanted
+    int groups;             // of the round: blockIdx.y below it
+    int scan_rows;          // rows of kScanBlocks blocks behind the groups' that scan x and w; 0: no scan wanted
+    const float* __restrict__ x;
+    long long x_total, w_total;
+    int* found;             // what the scan's blocks found
 };
 __global__ __launch_bounds__(256) void k_bwd_prep(PrepParams q)
 {
+    if (blockIdx.y >= q.groups) {
+        scan_operands(q.x, q.x_total, q.w, q.w_total, (blockIdx.y - q.groups) * kScanBlocks + blockIdx.x, q.scan_rows * kScanBlocks,
+                      q.found);
+        return;
+    }
     const int K = q.G.n_members, c_out = q.c_out;
     const int g = q.g0 + blockIdx.y;
     float* wcatg = q.wcat + (size_t)blockIdx.y * q.g_stride;
@@ -2259,7 +2506,7 @@ inline bool split_tiles_whole(int I, int J)
     return I % ti == 0 && J % tj == 0;
 }
 
-template <bool AK, bool BK, int EPI, bool VA = false, bool VB = false>
+template <bool AK, bool BK, int EPI, int PRODUCT, bool VA = false, bool VB = false>
 int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
 {
     GemmParams q = q0;
@@ -2289,13 +2536,13 @@ int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
             auto launch = [&](auto epi) {
                 constexpr int E = decltype(epi)::value;
                 if (nx == 4)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, VA, VB, 4>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 4>), grid, dim3(512), 0, s, q);
                 else if (nx == 3)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, VA, VB, 3>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 3>), grid, dim3(512), 0, s, q);
                 else if (kc2)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, VA, VB, 2, 2>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 2, 2>), grid, dim3(512), 0, s, q);
                 else
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, VA, VB, 2>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 2>), grid, dim3(512), 0, s, q);
             };
             if constexpr (EPI == EPI_EXP_TIMES_G) {
                 if (q.g_planes)
@@ -2337,21 +2584,21 @@ int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
     const bool b_vec = BK || rows_aligned(q.b, q.ldb, q.b_batch_stride);
     if constexpr (VB) {
         // (the caller has checked the view's alignment: rows of E and the runs of eight columns)
-        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, false, true>), grid, dim3(256), 0, s, q);
+        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, false, true>), grid, dim3(256), 0, s, q);
     } else if constexpr (VA) {
         if (!b_vec) return GEO_SC_ERR_UNSUPPORTED;
         if constexpr (EPI == EPI_EXP_TIMES_G) {
             if (q.g_planes)
-                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI_EXP_TIMES_G_PLANES, true>), grid, dim3(256), 0, s, q);
+                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI_EXP_TIMES_G_PLANES, PRODUCT, true>), grid, dim3(256), 0, s, q);
             else
-                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, true>), grid, dim3(256), 0, s, q);
+                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true>), grid, dim3(256), 0, s, q);
         } else {
-            hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, true>), grid, dim3(256), 0, s, q);
+            hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true>), grid, dim3(256), 0, s, q);
         }
     } else {
         // (the scratch layout aligns the rows)
         if (!a_vec || !b_vec) return GEO_SC_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI>), grid, dim3(256), 0, s, q);
+        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT>), grid, dim3(256), 0, s, q);
     }
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }
@@ -2373,6 +2620,7 @@ struct BwdLayout {
     bool dx_rows;        // the input-gradient GEMM sums the kernel rows itself (E read as a view shifted by image rows)
     bool dx_taps;        // it sums all kernel taps and writes dL/dx itself (E read as a view shifted by rows and columns)
     size_t off_zero;     // a block of zeros for that view
+    size_t off_scan;     // what the scan's blocks found, and behind it the word that the products read
     bool view_col;       // the GEMMs read col as a view of the shifted input planes (k_shift_planes) kept in col's space
     int view_k_pad;      // entries per group of the view's row table
     size_t off_rows;     // the row table
@@ -2458,7 +2706,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     if (rows > (size_t)b.G.n_groups) rows = b.G.n_groups;
     // the caller's cap on the add groups per round (less scratch, more launches)
     if (groups_per_round >= 1 && (size_t)groups_per_round < rows) rows = (size_t)groups_per_round;
-    if (rows * b.splits > 65535) rows = 65535 / b.splits;  // grid.z = rows * splits
+    if (rows * b.splits > 65535 - kScanRows) rows = (65535 - kScanRows) / b.splits;  // grid.y = rows and the scan's, grid.z = rows * splits
     if (rows < 1) rows = 1;
     b.rows_per_chunk = (int)rows;
     // col as a view: whole quads in every row on both sides, chunks of kChunk positions inside one item, an
@@ -2468,7 +2716,8 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     b.view_col = !b.fused_k && g.ho % 4 == 0 && g.h_in % 4 == 0 && (g.wo * g.ho) % kChunk == 0 && g.c_out % 2 == 0 &&
                  rows == (size_t)b.G.n_groups && !(g.mode == GEO_SC_ACC_YZ && g.c_in % g.z_unit != 0) &&
                  view_floats(g) <= rows * col_alloc &&
-                 (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho + (long long)g.w_k * g.ho < 0x7fffffffLL;
+                 (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho + (long long)g.w_k * g.ho < 0x7fffffffLL &&
+                 view_floats(g) < ((size_t)1 << 33);  // 32-bit numbers of their quads
     // the kernel rows summed inside the input-gradient GEMM: y accumulation (group = kernel column, members =
     // (channel, kernel row)), whole quads in the rows of input and output, whole chunks of rails, every group in
     // one round, and the per-column result inside dcol's space
@@ -2509,6 +2758,8 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     o += align256(sizeof(long long) * ((size_t)b.G.n_groups * b.view_k_pad + 2 * kChunk + 8));
     b.off_zero = o;
     o += 256;
+    b.off_scan = o;
+    o += align256(sizeof(int) * (kScanBlocks * kScanRows + 1));
     b.bytes = o;
     return b;
 }
@@ -2549,10 +2800,15 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
     const bool fused = L.fused_k;
     // col as a view of the shifted input planes (one round holds every group then)
     const bool view = L.view_col && ((uintptr_t)x & 15) == 0;
+    int* found = (int*)(ws + L.off_scan);
+    int* one_term = found + kScanBlocks * kScanRows;
+    const int n_scan_rows = scan_rows(x_total);
     // the position tables serve the gathers of im2col and of the fused kernels
-    if (fused || !view)
-        hipLaunchKernelGGL(k_position_table, dim3(m_blocks), dim3(256), 0, s, pos_base, pos_arow, pos_bcol, M,
+    auto position_tables = [&](const int* scanned) {
+        hipLaunchKernelGGL(k_position_table, dim3(m_blocks), dim3(256), 0, s, pos_base, pos_arow, pos_bcol, scanned, n_scan_rows, one_term, M,
                            g.c_in, g.c_out, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho);
+    };
+    if (fused) position_tables(nullptr);
     // Where the first product reads col as a view and its tiles are whole (the eight-wave kernel in every round,
     // or the 128 x 128 kernel), its epilogue reads the upstream gradient as it is (items of whole 32-position
     // blocks, 16-byte aligned): no transposed copy.
@@ -2656,26 +2912,8 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
     long long* view_rows = (long long*)(ws + L.off_rows);
-    if (view) {
-        const long long plane = (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho;
-        const long long quads = (long long)g.h_k * g.c_in * plane / 4;
-        hipLaunchKernelGGL(k_shift_planes, dim3(grid1d(quads)), dim3(256), 0, s, x, col, quads, g.n, g.c_in, g.w_in, g.h_in,
-                           g.pad_w, g.pad_h, g.ho);
-    }
     for (int v0 = 0; v0 < G.n_groups; v0 += L.rows_per_chunk) {
         const int nv = G.n_groups - v0 < L.rows_per_chunk ? G.n_groups - v0 : L.rows_per_chunk;
-        if (view) {
-            // nothing to copy
-        } else if (im2col_v4) {
-            const int q_blocks = grid1d(M / 4);
-            hipLaunchKernelGGL(k_im2col_rows_v4,
-                               dim3(q_blocks > 1024 ? 1024 : q_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
-                               dim3(256), 0, s, x, col, pos_base, pos_arow, pos_bcol, v0, M, G, g.w_in, g.h_in, L.col_v);
-        } else {
-            hipLaunchKernelGGL(k_im2col_rows,
-                               dim3(m_blocks > 1024 ? 1024 : m_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
-                               dim3(256), 0, s, x, col, pos_base, pos_arow, pos_bcol, v0, M, col_ld, G, g.w_in, g.h_in, L.col_v);
-        }
         const bool dx_taps = gx && L.dx_taps;
         const bool dx_rows = dx_taps || (gx && L.dx_rows && ((uintptr_t)gx & 15) == 0);
         {
@@ -2691,11 +2929,34 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             long long work = (long long)K * g.c_out;
             if (dx_rows && (long long)g.w_k * J * g.c_in > work) work = (long long)g.w_k * J * g.c_in;
             if (pp.view_rows && (long long)G.n_groups * L.view_k_pad > work) work = (long long)G.n_groups * L.view_k_pad;
-            const int wb = grid1d(work);
-            hipLaunchKernelGGL(k_bwd_prep, dim3(wb > 256 ? 256 : wb, nv), dim3(256), 0, s, pp);
+            pp.groups = nv;
+            int wb = std::min(grid1d(work), 256);
+            if (v0 == 0) {
+                pp.x = x; pp.x_total = x_total; pp.w_total = (long long)g.c_out * g.c_in * g.w_k * g.h_k; pp.found = found;
+                pp.scan_rows = n_scan_rows;
+                wb = kScanBlocks;
+            }
+            hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + pp.scan_rows), dim3(256), 0, s, pp);
+        }
+        if (!view && v0 == 0) position_tables(found);
+        if (view) {
+            const long long plane = (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho;
+            const long long quads = (long long)g.h_k * g.c_in * plane / 4;
+            hipLaunchKernelGGL(k_shift_planes, dim3(grid1d((quads + kShiftQuads - 1) / kShiftQuads)), dim3(256), 0, s, x, col, found, n_scan_rows, one_term, (unsigned)quads, g.n, g.c_in,
+                               g.w_in, g.h_in, g.pad_w, g.pad_h, g.ho);
+        } else if (im2col_v4) {
+            const int q_blocks = grid1d(M / 4);
+            hipLaunchKernelGGL(k_im2col_rows_v4,
+                               dim3(q_blocks > 1024 ? 1024 : q_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
+                               dim3(256), 0, s, x, col, one_term, pos_base, pos_arow, pos_bcol, v0, M, G, g.w_in, g.h_in, L.col_v);
+        } else {
+            hipLaunchKernelGGL(k_im2col_rows,
+                               dim3(m_blocks > 1024 ? 1024 : m_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
+                               dim3(256), 0, s, x, col, one_term, pos_base, pos_arow, pos_bcol, v0, M, col_ld, G, g.w_in, g.h_in, L.col_v);
         }
         // E[v][m][j] = g * exp(-(col_v^T . wcat_v)), col stored [K][M]
         GemmParams q1 = {};
+        q1.one_term = one_term;
         q1.a = col; q1.b = wcat; q1.c = e;
         q1.I = M; q1.J = J; q1.K = K;
         q1.lda = col_ld; q1.ldb = J; q1.ldc = e_ld;
@@ -2704,12 +2965,13 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         q1.c_batch_stride = (long long)L.e_v;
         q1.g = g_planes ? gy : gt; q1.g_planes = g_planes; q1.c_out = g.c_out; q1.npos = g.wo * g.ho;
         q1.a_rows = view_rows; q1.a_rows_batch = L.view_k_pad; q1.a_item = g.wo * g.ho; q1.a_skip = (g.w_k - 1) * g.ho;
-        rc = view ? launch_gemm<true, true, EPI_EXP_TIMES_G, true>(q1, nv, s)
-                  : launch_gemm<true, true, EPI_EXP_TIMES_G>(q1, nv, s);
+        rc = view ? launch_gemm<true, true, EPI_EXP_TIMES_G, PRODUCT_E, true>(q1, nv, s)
+                  : launch_gemm<true, true, EPI_EXP_TIMES_G, PRODUCT_E>(q1, nv, s);
         if (rc != GEO_SC_OK) return rc;
         if (gw) {
             // partial Gw[v][s][k][j] = sum_{m in split s} col_v[k][m] * E_v[m][j]
             GemmParams q2 = {};
+            q2.one_term = one_term;
             q2.a = col; q2.b = e; q2.c = part;
             q2.I = K; q2.J = J; q2.K = M;
             q2.lda = col_ld; q2.ldb = e_ld; q2.ldc = J;
@@ -2717,10 +2979,11 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             q2.a_batch_stride = (long long)L.col_v; q2.b_batch_stride = (long long)L.e_v;
             q2.c_batch_stride = (long long)L.part_v;
             q2.a_rows = view_rows; q2.a_rows_batch = L.view_k_pad; q2.a_item = g.wo * g.ho; q2.a_skip = (g.w_k - 1) * g.ho;
-            rc = view ? launch_gemm<false, true, EPI_STORE, true>(q2, nv, s) : launch_gemm<false, true, EPI_STORE>(q2, nv, s);
+            rc = view ? launch_gemm<false, true, EPI_STORE, PRODUCT_DW, true>(q2, nv, s)
+                      : launch_gemm<false, true, EPI_STORE, PRODUCT_DW>(q2, nv, s);
             if (rc != GEO_SC_OK) return rc;
             WgradOperands again = {};
-            if (!view) again = {col, e, M, col_ld, e_ld, L.col_v, L.e_v};
+            if (!view) again = {col, one_term, e, M, col_ld, e_ld, L.col_v, L.e_v};
             // Few partial sums and many weights: coalesced tiles (512 -> 512, 3 x 3, three partial sums: 50 -> 15.6 us;
             // the other kernel reads w and writes dL/dw one element per line).  Not where eight splits side by side are
             // what fills the GPU.
@@ -2741,6 +3004,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             const int k9 = g.w_k * g.h_k * J;
             const long long m2 = (long long)g.n * g.w_in * g.h_in;
             GemmParams q3 = {};
+            q3.one_term = one_term;
             q3.a = wd; q3.b = e; q3.c = gx;
             q3.I = g.c_in; q3.J = (int)m2; q3.K = k9;
             q3.lda = g.c_in; q3.ldb = e_ld; q3.ldc = m2;
@@ -2749,7 +3013,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             q3.sh_zero = zero; q3.sh_j = J; q3.sh_wo = g.wo; q3.sh_ho = g.ho; q3.sh_win = g.w_in; q3.sh_hin = g.h_in;
             q3.sh_pad = g.pad_w; q3.sh_padh = g.pad_h; q3.sh_wk = g.w_k; q3.sh_hk = g.h_k;
             q3.c_plane = g.w_in * g.h_in;
-            if ((rc = launch_gemm<true, false, EPI_STORE_ITEMS, false, true>(q3, 1, s)) != GEO_SC_OK) return rc;
+            if ((rc = launch_gemm<true, false, EPI_STORE_ITEMS, PRODUCT_DX, false, true>(q3, 1, s)) != GEO_SC_OK) return rc;
             continue;
         }
         if (dx_rows) {
@@ -2761,6 +3025,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             const int k3 = g.w_k * J;
             const long long m2 = (long long)g.n * g.w_in * g.ho;
             GemmParams q3 = {};
+            q3.one_term = one_term;
             q3.a = wd; q3.b = e; q3.c = dcol;
             q3.I = g.c_in; q3.J = (int)m2; q3.K = k3;
             q3.lda = g.c_in; q3.ldb = e_ld; q3.ldc = m2;
@@ -2769,7 +3034,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             q3.c_batch_stride = (long long)g.c_in * m2;
             q3.sh_zero = zero; q3.sh_j = J; q3.sh_wo = g.wo; q3.sh_ho = g.ho; q3.sh_win = g.w_in; q3.sh_hin = g.ho;
             q3.sh_pad = g.pad_w; q3.sh_padh = 0; q3.sh_wk = g.w_k; q3.sh_hk = 1;
-            if ((rc = launch_gemm<true, false, EPI_STORE, false, true>(q3, nv, s)) != GEO_SC_OK) return rc;
+            if ((rc = launch_gemm<true, false, EPI_STORE, PRODUCT_DX, false, true>(q3, nv, s)) != GEO_SC_OK) return rc;
             const long long quads = (long long)g.n * g.c_in * g.w_in * g.h_in / 4;
             hipLaunchKernelGGL(k_shift_sum_v4, dim3(grid1d(quads)), dim3(256), 0, s, dcol, gx, quads, g.n, g.c_in, g.w_in,
                                g.h_in, g.h_k, g.pad_h, g.ho);
@@ -2777,13 +3042,14 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         }
         // dcol[v][k][m] = sum_j wd_v[j][k] * E_v[m][j]
         GemmParams q3 = {};
+        q3.one_term = one_term;
         q3.a = wd; q3.b = e; q3.c = dcol;
         q3.I = K; q3.J = M; q3.K = J;
         q3.lda = K; q3.ldb = e_ld; q3.ldc = M;
         q3.splits = 1; q3.k_per_split = e_ld; q3.c_split_stride = 0;
         q3.a_batch_stride = (long long)L.w_v; q3.b_batch_stride = (long long)L.e_v;
         q3.c_batch_stride = (long long)L.col_v;
-        if ((rc = launch_gemm<true, false, EPI_STORE>(q3, nv, s)) != GEO_SC_OK) return rc;
+        if ((rc = launch_gemm<true, false, EPI_STORE, PRODUCT_DX>(q3, nv, s)) != GEO_SC_OK) return rc;
         const int plane_blocks = (g.w_in * g.h_in + 255) / 256;
         const int n_planes = g.n * g.c_in;
         const int pb = plane_blocks > 64 ? 64 : plane_blocks;

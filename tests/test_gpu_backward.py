@@ -533,3 +533,66 @@ def test_infinite_and_largest_gradients_at_sizes_of_no_whole_quads(capi, shape_x
     _, rw, _ = surrogate.surrogate_autograd(x * 0.04, w, gb, pad)
     _, bw = capi.conv2d_add_partial_backward((x * 0.04).cuda(), w.cuda(), gb.cuda(), 128, pad)
     check("grad_w of a gradient of 3.4e38", bw, rw)
+
+
+ONE_TERM_SHAPES = [
+    ((2, 32, 16, 16), (32, 32, 5, 5), 2, "y", 1),      # planes, 64-wide tiles
+    ((9, 64, 28, 28), (64, 64, 3, 3), 1, "y", 1),      # planes, whole 128-wide tiles, the gradient as it is
+    ((64, 128, 16, 16), (128, 128, 3, 3), 1, "y", 1),  # eight waves
+    ((16, 256, 8, 8), (256, 256, 3, 3), 1, "y", 1),    # eight waves, tiles of other heights
+    ((7, 45, 27, 19), (43, 45, 3, 3), 1, "yz", 16),    # im2col, ragged channel blocks
+    ((5, 40, 7, 9), (30, 40, 3, 3), 1, "full", 1),     # one group of 360 members
+    ((3, 12, 5, 3), (5, 12, 3, 1), 0, "y", 1),         # rows that are no whole quads
+    ((8, 24, 4, 4), (40, 24, 4, 4), 0, "y", 1),        # one output position per item: partial chunks of rows of bf16
+]
+
+
+def seven_bit(shape_x, shape_w, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = lambda t: (t * 128).round().clamp(-127, 127) / 128
+    x = q((torch.rand(shape_x, generator=g) * 1.6 - 0.6).clamp(0, 1))
+    w = q((torch.rand(shape_w, generator=g) * 2 - 1) * 3 / (shape_w[1] * shape_w[2] * shape_w[3]) ** 0.5)
+    return x, w, g
+
+
+@pytest.mark.parametrize("rounds", [0, 1])
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", ONE_TERM_SHAPES)
+def test_operands_of_one_term_give_the_bits_of_three(capi, shape_x, shape_w, pad, mode, zu, rounds):
+    """7-bit operands leave out the products with their zero terms.  An activation that is no bf16 number, in a channel
+    that no weight reads, takes the same problem to all six products: every other gradient has the same bits."""
+    x, w, g = seven_bit(shape_x, shape_w, 5)
+    w[:, 1] = 0.0
+    x, w = x.cuda(), w.cuda()
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gy = (torch.randn(capi.output_shape(d), generator=g) * 1e-2).cuda()
+    kw = dict(accumulate=mode, z_unit=zu, options=capi.make_options(backward_groups_per_round=rounds) if rounds else None)
+    gx, gw = capi.conv2d_add_partial_backward(x, w, gy, 128, (pad, pad), **kw)
+    other = x.clone()
+    other[0, 1, 2, 2] += 2.0 ** -20
+    gx3, gw3 = capi.conv2d_add_partial_backward(other, w, gy, 128, (pad, pad), **kw)
+    keep = [c for c in range(shape_x[1]) if c != 1]
+    assert torch.equal(gx, gx3) and torch.equal(gw[:, keep], gw3[:, keep])
+
+
+@pytest.mark.parametrize("where", ["first", "last", "weight", "none"])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+def test_one_element_of_more_than_eight_bits_is_found(capi, where, offset):
+    """The scan sees the ends of operands that start and end off a 16-byte boundary: as bf16 the element would be 2^-9 of
+    itself off."""
+    from oracle import surrogate
+    shape_x, shape_w = (3, 13, 7, 9), (5, 13, 3, 3)
+    x, w, g = seven_bit(shape_x, shape_w, 6)
+    x, w = x * 0, w.abs() * 0.5
+    x.view(-1)[0] = x.view(-1)[-1] = 0.5
+    if where == "first":
+        x.view(-1)[0] = 0.3
+    elif where == "last":
+        x.view(-1)[-1] = 0.3
+    elif where == "weight":
+        w.view(-1)[-1] = 0.3
+    hold = lambda t: torch.cat([torch.zeros(offset), t.reshape(-1)]).cuda()[offset:].view(t.shape)
+    gy = torch.randn((3, 5, 7, 9), generator=g)
+    gx, gw = capi.conv2d_add_partial_backward(hold(x), hold(w), gy.cuda(), 128, (1, 1))
+    rx, rw, _ = surrogate.surrogate_autograd(x, w, gy, (1, 1))
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
