@@ -1543,45 +1543,80 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad(const float* __restrict__ 
 
 // dL/dx[n][ci][p][q] (+)= sum over the kernel taps (u, v) whose group lies in [g0, g0 + ng) of
 // dcol[g][k][(n, p+pad_w-u, q+pad_h-v)] over the valid output positions; the first chunk of
-// groups writes, later chunks add.  Blocks stride over the planes (n, ci).
+// groups writes, later chunks add.  One grid-stride loop over the elements with the item inside the channel: neighbouring
+// threads read one row of dcol along its positions whatever the size of an item (blocks of whole planes left 252 of
+// 256 threads idle on 2 x 2 images; 512 channels of them, batch 128: 41 -> 4 us).
 __global__ __launch_bounds__(256) void k_col2im_rows(const float* __restrict__ dcol, float* __restrict__ gx, int g0,
-                                                     int ng, long long m_total, int n_planes, Groups G, int w_in,
+                                                     int ng, long long m_total, unsigned total, unsigned n_items, Groups G, int w_in,
                                                      int h_in, int pad_w, int pad_h, int wo, int ho, size_t g_stride)
 {
-    const int plane = w_in * h_in;
+    const unsigned plane = w_in * h_in;
     const int k_step = (G.mode == GEO_SC_ACC_Z || G.mode == GEO_SC_ACC_FULL) ? G.h_k : 1;
-    for (int nc = blockIdx.x; nc < n_planes; nc += gridDim.x) {
-        const int n = nc / G.c_in, ci = nc - n * G.c_in;
-        float* dst = gx + (size_t)nc * plane;
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const unsigned cn = i / plane, e = i - cn * plane;
+        const int ci = (int)(cn / n_items), n = (int)(cn - ci * n_items);
+        const int p = (int)e / h_in, qq = (int)e - p * h_in;
         const float* src = dcol + (size_t)n * wo * ho;
-        for (int e = blockIdx.y * 256 + threadIdx.x; e < plane; e += gridDim.y * 256) {
-            const int p = e / h_in, qq = e - p * h_in;
-            float s = 0.0f;
-            // kernel rows v whose output column b = qq + pad_h - v exists (a 1 x 256 kernel on a 256-wide
-            // input has one such row per element, not 256)
-            const int v_lo = max(0, qq + pad_h - (ho - 1)), v_hi = min(G.h_k - 1, qq + pad_h);
-            for (int v = v_lo; v <= v_hi; v++) {
-                const int b = qq + pad_h - v;
-                // the group does not depend on u, and the member index advances by k_step per tap
-                int g, k;
-                group_of(G, ci, 0, v, g, k);
-                if (g < g0 || g >= g0 + ng) continue;  // uniform
-                const bool b_ok = b >= 0 && b < ho;
-                const float* sg = src + (size_t)(g - g0) * g_stride + (size_t)k * m_total + (b_ok ? b : 0);
-                // four taps at a time: loads from clamped addresses first, then the sum
-                for (int u0 = 0; u0 < G.w_k; u0 += 4) {
-                    float t[4];
+        float* dst = gx + ((size_t)n * G.c_in + ci) * plane + e;
+        float s = 0.0f;
+        // kernel rows v whose output column b = qq + pad_h - v exists (a 1 x 256 kernel on a 256-wide
+        // input has one such row per element, not 256)
+        const int v_lo = max(0, qq + pad_h - (ho - 1)), v_hi = min(G.h_k - 1, qq + pad_h);
+        for (int v = v_lo; v <= v_hi; v++) {
+            const int b = qq + pad_h - v;
+            // the group does not depend on u, and the member index advances by k_step per tap
+            int g, k;
+            group_of(G, ci, 0, v, g, k);
+            if (g < g0 || g >= g0 + ng) continue;
+            const float* sg = src + (size_t)(g - g0) * g_stride + (size_t)k * m_total + b;
+            // four taps at a time: loads from clamped addresses first, then the sum
+            for (int u0 = 0; u0 < G.w_k; u0 += 4) {
+                float t[4];
 #pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const int u = u0 + q, a = p + pad_w - u;
-                        const bool ok = b_ok && u < G.w_k && a >= 0 && a < wo;
-                        const float val = sg[ok ? (size_t)u * k_step * m_total + a * ho : 0];
-                        t[q] = ok ? val : 0.0f;
-                    }
-                    s += (t[0] + t[1]) + (t[2] + t[3]);
+                for (int q = 0; q < 4; q++) {
+                    const int u = u0 + q, a = p + pad_w - u;
+                    const bool ok = u < G.w_k && a >= 0 && a < wo;
+                    const float val = sg[ok ? (size_t)u * k_step * m_total + a * ho : 0];
+                    t[q] = ok ? val : 0.0f;
                 }
+                s += (t[0] + t[1]) + (t[2] + t[3]);
             }
-            dst[e] = g0 == 0 ? s : dst[e] + s;
+        }
+        *dst = g0 == 0 ? s : *dst + s;
+    }
+}
+
+// The same for outputs of one position (a classifier, a linear layer): an element has the one term of the tap that lies on
+// it, and the sum is a transposition of dcol's rows [element][n] to dL/dx [n][element], in tiles of 32 x 32 through LDS.
+// The kernel above reads one element per cache line here (4096 elements in 256 groups, batch 1024: 47 -> 15 us).
+// blockIdx = (element tile, item tile); gridDim.y strides over the item tiles.
+__global__ __launch_bounds__(256) void k_col2im_one(const float* __restrict__ dcol, float* __restrict__ gx, int g0, int ng,
+                                                    int n_items, Groups G, int w_in, int h_in, int pad_w, int pad_h,
+                                                    size_t g_stride)
+{
+    __shared__ float tile[32][33];  // [element][item]
+    const int plane = w_in * h_in, elements = G.c_in * plane;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int e0 = blockIdx.x * 32;
+    for (int n0 = blockIdx.y * 32; n0 < n_items; n0 += gridDim.y * 32) {
+        __syncthreads();
+        for (int q = ty; q < 32; q += 8) {
+            const int e = min(e0 + q, elements - 1), n = min(n0 + tx, n_items - 1);
+            const int ci = e / plane, p = (e - ci * plane) / h_in, qq = e - ci * plane - p * h_in;
+            int g, k;
+            const int u = p + pad_w, v = qq + pad_h;
+            group_of(G, ci, u, v, g, k);
+            const bool ok = u < G.w_k && v < G.h_k && g >= g0 && g < g0 + ng;
+            const float val = dcol[ok ? (size_t)(g - g0) * g_stride + (size_t)k * n_items + n : 0];
+            tile[q][tx] = ok ? val : 0.0f;
+        }
+        __syncthreads();
+        for (int q = ty; q < 32; q += 8) {
+            const int n = n0 + q, e = e0 + tx;
+            if (n < n_items && e < elements) {
+                float* dst = gx + (size_t)n * elements + e;
+                *dst = g0 == 0 ? tile[tx][q] : *dst + tile[tx][q];
+            }
         }
     }
 }
@@ -1753,19 +1788,35 @@ struct PrepParams {
     int view_groups, view_k_pad, ho;
     long long plane;
     float* zero;            // null: no block of zeros wanted
-    int groups;             // of the round: blockIdx.y below it
+    int groups;             // rows of blocks (blockIdx.y) that make weight operands: one per group of the round
     int scan_rows;          // rows of kScanBlocks blocks behind the groups' that scan x and w; 0: no scan wanted
     const float* __restrict__ x;
     long long x_total, w_total;
     int* found;             // what the scan's blocks found
 };
+// what is no weight operand: the scan's blocks (true: the block is one of them), the view's row table, the zeros
+__device__ __forceinline__ bool prep_scans(const PrepParams& q)
+{
+    if ((int)blockIdx.y < q.groups) return false;
+    scan_operands(q.x, q.x_total, q.w, q.w_total, (blockIdx.y - q.groups) * kScanBlocks + blockIdx.x, q.scan_rows * kScanBlocks,
+                  q.found);
+    return true;
+}
+__device__ __forceinline__ void prep_tables(const PrepParams& q)
+{
+    if (blockIdx.y != 0) return;
+    if (q.view_rows)
+        for (int e = blockIdx.x * 256 + threadIdx.x; e < q.view_groups * q.view_k_pad; e += gridDim.x * 256) {
+            const int gi = e / q.view_k_pad, k = e - gi * q.view_k_pad;
+            const Member mb = member_of(q.G, gi, min(k, q.G.n_members - 1));
+            q.view_rows[e] = ((long long)mb.v * q.G.c_in + mb.ci) * q.plane + (long long)mb.u * q.ho;
+        }
+    if (q.zero && blockIdx.x == 0 && threadIdx.x < 64) q.zero[threadIdx.x] = 0.0f;
+}
+
 __global__ __launch_bounds__(256) void k_bwd_prep(PrepParams q)
 {
-    if (blockIdx.y >= q.groups) {
-        scan_operands(q.x, q.x_total, q.w, q.w_total, (blockIdx.y - q.groups) * kScanBlocks + blockIdx.x, q.scan_rows * kScanBlocks,
-                      q.found);
-        return;
-    }
+    if (prep_scans(q)) return;
     const int K = q.G.n_members, c_out = q.c_out;
     const int g = q.g0 + blockIdx.y;
     float* wcatg = q.wcat + (size_t)blockIdx.y * q.g_stride;
@@ -1799,15 +1850,106 @@ __global__ __launch_bounds__(256) void k_bwd_prep(PrepParams q)
                 wdg[e] = val;
         }
     }
-    if (blockIdx.y == 0) {
-        if (q.view_rows)
-            for (int e = blockIdx.x * 256 + threadIdx.x; e < q.view_groups * q.view_k_pad; e += gridDim.x * 256) {
-                const int gi = e / q.view_k_pad, k = e - gi * q.view_k_pad;
-                const Member mb = member_of(q.G, gi, k < K ? k : K - 1);
-                q.view_rows[e] = ((long long)mb.v * q.G.c_in + mb.ci) * q.plane + (long long)mb.u * q.ho;
+    prep_tables(q);
+}
+
+// The same operands in tiles of 32 output channels x `channels` input channels with all their taps, which pass through LDS:
+// w is read in the runs that it has along an output channel, and every operand is written along its innermost dimension
+// (element by element, k_bwd_prep reads one weight per cache line: 512 -> 512, 3 x 3: 35 -> 15 us with
+// the scan).  The
+// first q.groups rows of blocks take the tiles of all groups of the round.  For taps that fit (prep_tile_channels) and groups whose members all exist.
+constexpr int kPrepRow = 288;  // floats per output channel of a tile
+inline int prep_tile_channels(int c_in, int c_out, int taps)
+{
+    // (few weights are few tiles, one long pass each: 25 600 of 5 x 5 take 14 us in tiles, 7 element by element)
+    if ((long long)c_in * c_out * taps < 1 << 17) return 0;
+    int channels = 32;
+    while (channels > 1 && channels * taps > kPrepRow) channels /= 2;
+    if (channels * taps > kPrepRow) return 0;
+    // two tiles per CU, where narrower ones make them
+    while (channels > 4 && (long long)((c_out + 31) / 32) * ((c_in + channels - 1) / channels) < 512) channels /= 2;
+    return channels;
+}
+__global__ __launch_bounds__(256) void k_bwd_prep_tiled(PrepParams q, int n_groups, int channels_log2)
+{
+    __shared__ float tile[32][kPrepRow + 1];
+    __shared__ long long cat_at[kPrepRow];  // where weight i of a channel goes in wcat, and in wd without its channel; -1: nowhere
+    __shared__ int wd_at[kPrepRow];
+    if (prep_scans(q)) return;
+    const Groups& G = q.G;
+    const int K = G.n_members, c_out = q.c_out, J = 2 * c_out, c_in = G.c_in, taps = G.w_k * G.h_k;
+    const int channels = 1 << channels_log2;
+    const int ci_tiles = (c_in + channels - 1) >> channels_log2, tiles = ci_tiles * ((c_out + 31) / 32);
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int t = blockIdx.y * gridDim.x + blockIdx.x; t < tiles; t += q.groups * gridDim.x) {
+        const int ct = t / ci_tiles, c0 = (t - ct * ci_tiles) << channels_log2, o0 = ct * 32;
+        const int nc = min(channels, c_in - c0), no = min(32, c_out - o0), row = nc * taps;
+        __syncthreads();
+        for (int i = threadIdx.x; i < row; i += 256) {
+            const int c = i / taps, tap = i - c * taps, u = tap / G.h_k, v = tap - u * G.h_k;
+            int g, k;
+            group_of(G, c0 + c, u, v, g, k);
+            const bool mine = g >= q.g0 && g < q.g0 + n_groups;
+            cat_at[i] = mine ? (long long)(g - q.g0) * (long long)q.g_stride + (long long)k * J : -1;
+            wd_at[i] = k;
+        }
+        // (twelve loads in flight: one after the other they take most of the kernel's time)
+        for (int e0 = threadIdx.x; e0 < no * row; e0 += 12 * 256) {
+            float v[12];
+            int o[12], i[12];
+#pragma unroll
+            for (int n = 0; n < 12; n++) {
+                const int e = min(e0 + n * 256, no * row - 1);
+                o[n] = (int)((unsigned)e / (unsigned)row);
+                i[n] = e - o[n] * row;
+                v[n] = q.w[((size_t)(o0 + o[n]) * c_in + c0) * taps + i[n]];
             }
-        if (q.zero && blockIdx.x == 0 && threadIdx.x < 64) q.zero[threadIdx.x] = 0.0f;
+#pragma unroll
+            for (int n = 0; n < 12; n++) tile[o[n]][i[n]] = v[n];
+        }
+        __syncthreads();
+        // wcat: along the output channels
+        if (tx < no)
+#pragma unroll 4
+            for (int i = ty; i < row; i += 8) {
+                const long long at = cat_at[i];
+                if (at < 0) continue;
+                float* r = q.wcat + at + o0 + tx;
+                const float wv = tile[tx][i];
+                r[0] = fminf(fmaxf(wv, 0.0f), 100.0f);
+                r[c_out] = -fminf(fmaxf(wv, -100.0f), 0.0f);
+            }
+        if (!q.dx_rows) {
+            // wd: along the members
+            for (int o = ty; o < no; o += 8)
+#pragma unroll 4
+                for (int i = tx; i < row; i += 32) {
+                    if (cat_at[i] < 0) continue;
+                    float* r = q.wd + (cat_at[i] - (long long)wd_at[i] * J) + (size_t)(o0 + o) * K + wd_at[i];
+                    const float wv = tile[o][i];
+                    r[0] = fminf(fmaxf(wv, 0.0f), 100.0f);
+                    r[(size_t)c_out * K] = fminf(fmaxf(wv, -100.0f), 0.0f);
+                }
+            continue;
+        }
+        // wdx: along the input channels, 256 / channels (output channel, tap) pairs at a time (every group in the round)
+        const int c = threadIdx.x & (channels - 1), pair0 = threadIdx.x >> channels_log2, pairs = 256 >> channels_log2;
+        if (c < nc)
+            for (int tap = 0; tap < taps; tap++) {
+                const int u = tap / G.h_k, v = tap - u * G.h_k;
+                float* out = (q.dx_rows == 2 ? q.wd + ((size_t)v * G.w_k + u) * kChunk * c_in
+                                             : q.wd + (size_t)v * q.g_stride + (size_t)u * kChunk * c_in) + c0 + c;
+                const size_t jc_stride = (size_t)(q.dx_rows == 2 ? taps : G.w_k) * kChunk * c_in;
+#pragma unroll 4
+                for (int o = pair0; o < 2 * no; o += pairs) {
+                    const int rail = o >= no, oo = rail ? o - no : o;
+                    const float wv = tile[oo][c * taps + tap];
+                    const int j = rail * c_out + o0 + oo, jc = j / kChunk, jj = j % kChunk;
+                    out[jc * jc_stride + (size_t)jj * c_in] = rail ? fminf(fmaxf(wv, -100.0f), 0.0f) : fminf(fmaxf(wv, 0.0f), 100.0f);
+                }
+            }
     }
+    prep_tables(q);
 }
 
 // dL/dx[n][ci][p][q] = sum over the kernel columns v of d[v][ci][(n, p, q + pad_h - v)] where that output
@@ -2834,13 +2976,25 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                                g.c_out, npos);
         }
     }
+    // dL/dx from dcol of the groups [v0, v0 + nv)
+    auto col2im = [&](int v0, int nv) {
+        const int n_planes = g.n * g.c_in;
+        // (under two tiles of items the other kernel's single pass is no slower: 18 items of 592 elements 37 us in all, 38.5)
+        if (g.wo * g.ho == 1 && g.n >= 64) {
+            const int tiles = (g.c_in * g.w_in * g.h_in + 31) / 32, rows = (g.n + 31) / 32;
+            hipLaunchKernelGGL(k_col2im_one, dim3(tiles, std::min(rows, 1024)), dim3(256), 0, s, dcol, gx, v0, nv, g.n, G, g.w_in,
+                               g.h_in, g.pad_w, g.pad_h, L.col_v);
+        } else if (col2im_v4) {
+            hipLaunchKernelGGL(k_col2im_rows_v4, dim3(grid1d((long long)n_planes * (g.w_in * g.h_in / 4))), dim3(256), 0, s, dcol, gx,
+                               v0, nv, L.m_total, n_planes, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
+        } else {
+            hipLaunchKernelGGL(k_col2im_rows, dim3(grid1d(x_total)), dim3(256), 0, s, dcol, gx, v0, nv, L.m_total,
+                               (unsigned)x_total, (unsigned)g.n, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
+        }
+    };
     int rc;
     if (fused) {
         if (!gx && !gw) return GEO_SC_OK;
-        const int plane_blocks = (g.w_in * g.h_in + 255) / 256;
-        const int n_planes = g.n * g.c_in;
-        const int pb = plane_blocks > 64 ? 64 : plane_blocks;
-        const int want = 256 * 16 / pb;
         const int ks = (K + 1) / 2;
         const int jw = L.fused_jw;
         const size_t slice = (size_t)L.rows_per_chunk * L.col_v;
@@ -2902,12 +3056,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             if (gx && L.dcol_slices > 1)
                 hipLaunchKernelGGL(k_sum_slices, dim3(grid1d((long long)((size_t)nv * L.col_v / 4))), dim3(256), 0, s, dcol,
                                    (size_t)nv * L.col_v, L.dcol_slices, slice);
-            if (gx && col2im_v4)
-                hipLaunchKernelGGL(k_col2im_rows_v4, dim3(grid1d((long long)n_planes * (g.w_in * g.h_in / 4))), dim3(256), 0, s, dcol, gx,
-                                   v0, nv, L.m_total, n_planes, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
-            else if (gx)
-                hipLaunchKernelGGL(k_col2im_rows, dim3(n_planes < want ? n_planes : want, pb), dim3(256), 0, s, dcol, gx,
-                                   v0, nv, L.m_total, n_planes, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
+            if (gx) col2im(v0, nv);
         }
         return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
     }
@@ -2936,7 +3085,16 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                 pp.scan_rows = n_scan_rows;
                 wb = kScanBlocks;
             }
-            hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + pp.scan_rows), dim3(256), 0, s, pp);
+            const bool ragged = G.mode == GEO_SC_ACC_YZ && g.c_in % G.zu != 0;
+            const int channels = ragged ? 0 : prep_tile_channels(g.c_in, g.c_out, g.w_k * g.h_k);
+            if (channels) {
+                const long long tiles = (long long)((g.c_out + 31) / 32) * ((g.c_in + channels - 1) / channels);
+                pp.groups = (int)std::min<long long>((tiles + kScanBlocks - 1) / kScanBlocks, 8);  // rows of tiles
+                hipLaunchKernelGGL(k_bwd_prep_tiled, dim3(kScanBlocks, pp.groups + pp.scan_rows), dim3(256), 0, s, pp, nv,
+                                   __builtin_ctz((unsigned)channels));
+            } else {
+                hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + pp.scan_rows), dim3(256), 0, s, pp);
+            }
         }
         if (!view && v0 == 0) position_tables(found);
         if (view) {
@@ -3050,16 +3208,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         q3.a_batch_stride = (long long)L.w_v; q3.b_batch_stride = (long long)L.e_v;
         q3.c_batch_stride = (long long)L.col_v;
         if ((rc = launch_gemm<true, false, EPI_STORE, PRODUCT_DX>(q3, nv, s)) != GEO_SC_OK) return rc;
-        const int plane_blocks = (g.w_in * g.h_in + 255) / 256;
-        const int n_planes = g.n * g.c_in;
-        const int pb = plane_blocks > 64 ? 64 : plane_blocks;
-        const int want = 256 * 16 / pb;  // a few thousand blocks in all
-        if (col2im_v4)
-            hipLaunchKernelGGL(k_col2im_rows_v4, dim3(grid1d((long long)n_planes * (g.w_in * g.h_in / 4))), dim3(256), 0, s, dcol, gx, v0,
-                               nv, L.m_total, n_planes, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
-        else
-            hipLaunchKernelGGL(k_col2im_rows, dim3(n_planes < want ? n_planes : want, pb), dim3(256), 0, s, dcol, gx, v0,
-                               nv, L.m_total, n_planes, G, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho, L.col_v);
+        col2im(v0, nv);
     }
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
 }

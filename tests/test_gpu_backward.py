@@ -596,3 +596,51 @@ def test_one_element_of_more_than_eight_bits_is_found(capi, where, offset):
     rx, rw, _ = surrogate.surrogate_autograd(x, w, gy, (1, 1))
     check("grad_x", gx, rx)
     check("grad_w", gw, rw)
+
+
+@pytest.mark.parametrize("rounds", [0, 2])
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((2, 133, 5, 6), (115, 133, 3, 3), 1, "y", 1),     # 137655 weights: odd tiles of channels, operands per member
+    ((3, 96, 4, 8), (152, 96, 3, 3), 1, "y", 1),       # the input gradient's operand per kernel column
+    ((65, 72, 32, 32), (80, 72, 5, 5), 2, "y", 1),     # its operand of all taps; 8 channels a tile
+    ((2, 54, 7, 8), (51, 54, 7, 7), 3, "z", 1),        # groups of 49 members, one per channel
+    ((2, 128, 5, 5), (120, 128, 3, 3), 1, "yz", 16),
+    ((2, 128, 5, 5), (120, 128, 3, 3), 1, "full", 1),
+])
+def test_weight_operands_made_in_tiles(capi, shape_x, shape_w, pad, mode, zu, rounds):
+    """From 2^17 weights on the operands of the products are made in tiles of channels through LDS."""
+    from oracle import surrogate
+    x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_x[1])
+    w = (w * 3).contiguous()
+    w.view(-1)[::5] = 0.0
+    kw = dict(accumulate=mode, z_unit=zu, options=capi.make_options(backward_groups_per_round=rounds) if rounds else None)
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    g = torch.randn(capi.output_shape(d), generator=torch.Generator().manual_seed(7))
+    gx, gw = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), **kw)
+    rx, rw, _ = surrogate.surrogate_autograd(x.cuda(), w.cuda(), g.cuda(), (pad, pad), mode=mode, z_unit=zu)
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
+
+
+@pytest.mark.parametrize("rounds", [0, 1])
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((64, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),       # one output position: dL/dx by transposition
+    ((79, 20, 3, 5), (9, 20, 3, 5), 0, "y", 1),        # ragged tiles of elements and items
+    ((65, 16, 1, 40), (24, 16, 1, 40), 0, "y", 1),     # the linear mapping: small groups
+    ((67, 9, 3, 3), (7, 9, 5, 5), 1, "z", 1),          # taps in the padding
+    ((85, 40, 1, 1), (7, 40, 1, 1), 0, "yz", 16),
+    ((63, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),       # too few items for that
+    ((70, 24, 2, 2), (12, 24, 3, 3), 1, "y", 1),       # items of four elements
+    ((5, 13, 3, 3), (6, 13, 3, 3), 1, "full", 1),
+])
+def test_input_gradient_of_few_positions(capi, shape_x, shape_w, pad, mode, zu, rounds):
+    from oracle import surrogate
+    x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_x[1])
+    w = (w * 3).contiguous()
+    kw = dict(accumulate=mode, z_unit=zu, options=capi.make_options(backward_groups_per_round=rounds) if rounds else None)
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    g = torch.randn(capi.output_shape(d), generator=torch.Generator().manual_seed(8))
+    gx, gw = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), g.cuda(), 128, (pad, pad), **kw)
+    rx, rw, _ = surrogate.surrogate_autograd(x.cuda(), w.cuda(), g.cuda(), (pad, pad), mode=mode, z_unit=zu)
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
