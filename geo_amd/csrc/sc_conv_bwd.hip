@@ -1246,12 +1246,20 @@ __device__ __forceinline__ bool operands_are_bf16(const int* __restrict__ found,
 //   base[m] = ((n*c_in)*w_in + (a - pad_w))*h_in + (b - pad_h),  arow[m] = a - pad_w,  bcol[m] = b - pad_h
 // Built once per call; it keeps integer divisions out of the per-element kernels.
 // With `found`, the first block also turns what scan_operands found into *one_term.
+// With scan_x, rows of blocks behind the first scan x_total elements of x.
 __global__ __launch_bounds__(256) void k_position_table(int* __restrict__ base, int* __restrict__ arow,
                                                         int* __restrict__ bcol, const int* __restrict__ found, int found_rows,
-                                                        int* __restrict__ one_term, int m_total,
+                                                        int* __restrict__ one_term, const float* __restrict__ scan_x,
+                                                        long long x_total, int* __restrict__ scan_found, int m_total,
                                                         int c_in, int c_out, int w_in, int h_in, int pad_w, int pad_h,
                                                         int wo, int ho)
 {
+    if (blockIdx.y > 0) {
+        if (blockIdx.x < kScanBlocks)
+            scan_operands(scan_x, x_total, nullptr, 0, (blockIdx.y - 1) * kScanBlocks + blockIdx.x, (gridDim.y - 1) * kScanBlocks,
+                          scan_found);
+        return;
+    }
     if (found && blockIdx.x == 0) {
         const bool one = operands_are_bf16(found, found_rows);
         if (threadIdx.x == 0) *one_term = one;
@@ -2305,135 +2313,180 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
 }
 
-// The fused kernel on the bf16 matrix cores, for K <= 16 members and more than 128 rails.  The fp32
-// MFMAs of k_bwd_small_k run on the vector ALU's multipliers: while one executes, no wave of the SIMD
-// issues vector instructions, and the kernel's time is the sum of its MFMA and vector work.  The bf16
-// MFMAs have a pipe of their own.  Here every operand is split into three bf16 terms as in
-// k_gemm_split (six term products per product, fp32 accumulation): the weights once per workgroup,
-// col once per tile, E once per element (eleven vector instructions per pair), and all three
-// products take 72 bf16 MFMAs per wave and tile (1152 cycles of the matrix pipe, beside the vector
-// work) where the fp32 kernel takes 80 fp32 ones (3072 cycles of the vector pipe).
-//   first product   32x32x16: A = col[m][k] (csz), B = wcat[k][j] (registers)
-//   weight gradient 16x16x32: A = col[k][m] (csg), B = E[m][j] read from E^T[j][m]: 8 consecutive m
-//   input gradient  16x16x32: A = wd[k][j] (registers), B = E[m][j] for 8 consecutive j: eight 2-byte
-//                   reads down a column of E^T (rows of kBfEw words keep them free of bank conflicts)
-// Same grid, arguments, tiles and outputs as k_bwd_small_k<8, 2, DX>.
-constexpr int kBfEw = 18;  // words per row of E^T: 32 bf16 and padding
+// The fused kernel on the bf16 matrix cores, for K <= 16 members.  The fp32 MFMAs of k_bwd_small_k run on the vector
+// ALU's multipliers: while one executes, no wave of the SIMD issues vector instructions, and the kernel's time is the
+// sum of its MFMA and vector work.  The bf16 MFMAs have a pipe of their own; what bounds this kernel is the vector work
+// per element of E: the exponential, the factor g and the split into three bf16 terms (5.5 instructions).  So E makes
+// no detour that costs more of it.  All products are 16x16x32:
+//   first product    A = col[m][k] (csz), B = wcat[k][j] (registers).  The 16 members are half of the instruction's k:
+//                    operands of three terms put two term products into one instruction.  Row i of its two blocks is
+//                    position 16 (i / 8) + i % 8 and that + 8, so that a lane's eight results are eight consecutive
+//                    floats of the tiled gradient (k_tile_grad).
+//   weight gradient  A = col[k][m] (csg), B = E[m][j]: the lane's eight results as they are - the order of a
+//                    contraction is free, col's words are read in E's order.
+//   input gradient   A = wd[k][j] (registers), B = E[m][j] along j: one term of a 32 x 32 block at a time through an
+//                    LDS block of the wave's own, written as E^T[j][m] and read transposed (ds_read_b64_tr_b16), no
+//                    barrier.  The waves' sums meet in LDS, once per tile.
+// A wave has NB blocks of 32 columns.  Where x and the workgroup's weights are bf16 numbers (the layers' 7-bit operands)
+// they are one term, 1, 3 and 3 products instead of 6, 6 and 6; otherwise a wave takes its blocks one after the other,
+// each over all tiles (two blocks' operands of three terms need more than the 128 registers that four waves per SIMD
+// have), and adds to the dcol of the first.  4096 x 4096 linear layer, batch 1024: 1965 us with three terms
+// throughout and E in LDS for both gradients, 1096 now, of which the vector work of E is 630 (the sum of the slices of
+// dcol, 16 with NB = 2 and 32 with NB = 1: 119 -> 62); unquantised operands, step 4.20 -> 4.17 ms; first layer of the
+// 4-layer CNN 92 -> 69, half of that the gather's.
+// Same grid, arguments, tiles and outputs as k_bwd_small_k.
+constexpr int kBfEw = 18;  // words per row of E^T: 32 bf16 and padding (8-byte accesses of 16 rows meet no bank twice)
 constexpr int kBfCw = 20;  // words per row of col[k][m]: 16-byte aligned rows
 
-template <int NW, bool DX>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 3))) void k_bwd_small_k_bf16(
-    const float* __restrict__ x, const float* __restrict__ wcat, const float* __restrict__ gtt,
-    const int* __restrict__ base, const int* __restrict__ arow, const int* __restrict__ bcol, float* __restrict__ part,
-    float* __restrict__ dcol, Groups G, int g0, int M, int w_in, int h_in, int c_out, int jblocks, int splits,
-    int store_part, int gt_blocks, int gt_dedupe, size_t w_stride, size_t part_stride, size_t dcol_stride,
-    size_t dcol_slice)
-{
-    constexpr int KP = 16, TM = kFusedTile, JW = 32 * NW, EW = kBfEw, CW = kBfCw, NT = 64 * NW;
-    constexpr int JPARTS = NW / 2;   // waves that share one 16 x 16 block of dcol and split j
-    constexpr int GP = 256 / NT > 1 ? 256 / NT : 1;  // member pairs gathered per thread (256 (position, pair) slots)
-    // col of two tiles in turn: the next tile's is written while this tile's products run
-    __shared__ __attribute__((aligned(16))) uint4 csz[2][3][2][TM];      // first product: (term, k half, m) -> 8 bf16 along k
-    __shared__ __attribute__((aligned(16))) unsigned csg[2][3][KP][CW];  // weight gradient: [term][k][m], two m per word
-    __shared__ __attribute__((aligned(16))) unsigned est[3][JW][EW];  // E^T: [term][j][m], two m per word
-    __shared__ float red[JPARTS > 1 ? JPARTS - 1 : 1][2][16][17];     // the other j parts' partial dcol blocks
-    const int K = G.n_members, J = 2 * c_out;
-    const int g = g0 + blockIdx.y;
-    const int split = blockIdx.x / jblocks, jblock = blockIdx.x - split * jblocks;
-    const int j_begin = jblock * JW;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int l32 = lane & 31, lk = lane >> 5, l16 = lane & 15, lq = lane >> 4;
-    // smallest terms first; 0 = hi, 1 = mid, 2 = lo
-    constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+struct SmallKParams {
+    const float* __restrict__ x;
+    const float* __restrict__ wcat;
+    const float* __restrict__ gtt;
+    const int* __restrict__ base;
+    const int* __restrict__ arow;
+    const int* __restrict__ bcol;
+    const int* __restrict__ found;  // what the scan of x left (scan_operands)
+    float* __restrict__ part;
+    float* __restrict__ dcol;
+    Groups G;
+    int g0, M, w_in, h_in, c_out, jblocks, splits, store_part, gt_blocks, gt_dedupe, found_rows;
+    size_t w_stride, part_stride, dcol_stride, dcol_slice;
+};
 
-    // this group's wcat[k][j_begin .. j_begin + JW) through LDS (the space of est); zero outside the problem
-    constexpr int WLD = JW + 1;
-    float* wl = (float*)&est[0][0][0];
-    {
-        const float* wg = wcat + (size_t)blockIdx.y * w_stride;
-        for (int e = threadIdx.x; e < KP * JW; e += NT) {
-            const int k = e / JW, jl = e - k * JW, j = j_begin + jl;
-            const bool ok = k < K && j < J;
-            const float v = wg[ok ? (size_t)k * J + j : 0];
-            wl[k * WLD + jl] = ok ? v : 0.0f;
-        }
+template <int NW, int NB, bool DX>
+struct SmallKShared {
+    // col of two tiles in turn: the next tile's is written while this tile's products run
+    uint4 csz[2][3][2][kFusedTile];      // first product: (term, k half, m) -> 8 bf16 along k
+    unsigned csg[2][3][16][kBfCw];       // weight gradient: [term][k][m], two m per word
+    union {
+        float wl[16][32 * NW * NB + 1];  // the group's weights on their way into registers
+        struct {
+            uint2 est[DX ? NW : 1][32][kBfEw / 2];  // per wave: one term of E^T[j][m]
+            float4 red[2][DX ? NW : 1][2][64];      // per wave: its part of dcol, 16 x 16 blocks in the order of an MFMA result
+        } t;
+    } u;
+};
+
+// this group's wcat[k][j_begin ..] into wl; zero outside the problem.  Whether an element takes three terms.
+template <int NW, int NB, bool DX>
+__device__ __forceinline__ bool small_k_weights(const SmallKParams& q, SmallKShared<NW, NB, DX>& sh, int j_begin)
+{
+    constexpr int JW = 32 * NW * NB;
+    const int K = q.G.n_members, J = 2 * q.c_out;
+    const float* wg = q.wcat + (size_t)blockIdx.y * q.w_stride;
+    bool three = false;
+    for (int e = threadIdx.x; e < 16 * JW; e += 64 * NW) {
+        const int k = e / JW, jl = e - k * JW, j = j_begin + jl;
+        const bool ok = k < K && j < J;
+        const float v = wg[ok ? (size_t)k * J + j : 0];
+        sh.u.wl[k][jl] = ok ? v : 0.0f;
+        three |= ok && takes_three_terms(v);
     }
-    __syncthreads();
-    // first product, B operand: lane -> column 32 wave + l32, k = 8 lk .. + 7
-    bf16x8 wz[3];
-    {
-        unsigned h[4], m[4], l[4];
+    return three;
+}
+
+// columns c0 + 32 (b NW + wave) .. + 31, b < NB, of the workgroup's (from j_begin on, weights in wl) over its tiles; ADD: to
+// the dcol that is there
+template <int TERMS, int NW, int NB, bool DX, bool ADD, typename Shared>
+__device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& sh, int split, int jblock, int j_begin, int c0)
+{
+    constexpr int KP = 16, TM = kFusedTile, NT = 64 * NW;
+    constexpr int EP = NW == 8 ? 1 : 2;                    // members gathered per slot of a thread
+    constexpr int GP = KP * TM / EP / NT;                  // slots per thread
+    static_assert(GP * EP * NT == KP * TM, "every thread gathers");
+    const int K = q.G.n_members, J = 2 * q.c_out, M = q.M, c_out = q.c_out;
+    const int g = q.g0 + blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int l16 = lane & 15, lq = lane >> 4;
+
+    // first product, B operand of 16 columns: lane -> column l16, k = 8 (lq % 2) .. + 7 of one term; lanes from 32 on
+    // have the second of two terms (hi and lo, mid and hi), or zeros
+    constexpr int ZB = TERMS == 3 ? 2 : 1;
+    const unsigned first = lq < 2 ? ~0u : 0u;
+    bf16x8 wz[NB][2][ZB];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const float* src = wl + (8 * lk + 2 * c) * WLD + 32 * wave + l32;
-            split3(src[0], src[WLD], h[c], m[c], l[c]);
-        }
-        wz[0] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-        wz[1] = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
-        wz[2] = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
-    }
-    // input gradient: wave -> (position block mb, j part jpart of 64 columns); A operand of step st: wd[j][k = l16] for
-    // j = jd0 + 32 st + 8 lq .. + 7, which is wcat[k][j] with the negative rail (j >= c_out) negated
-    const int mb = wave & 1, jpart = wave >> 1;
-    const int jd0 = jpart * 64;
-    bf16x8 wdr[DX ? 2 : 1][3];
-    if (DX) {
+    for (int b = 0; b < NB; b++)
 #pragma unroll
-        for (int st = 0; st < 2; st++) {
-            unsigned h[4], m[4], l[4];
+        for (int s = 0; s < 2; s++) {
+            unsigned t3[3][4];
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const int jl = jd0 + 32 * st + 8 * lq + 2 * c;
-                float v0 = wl[l16 * WLD + jl], v1 = wl[l16 * WLD + jl + 1];
+                const int k = 8 * (lq & 1) + 2 * c, jl = c0 + 32 * (b * NW + wave) + 16 * s + l16;
+                split3(sh.u.wl[k][jl], sh.u.wl[k + 1][jl], t3[0][c], t3[1][c], t3[2][c]);
+            }
+            unsigned o[2][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                o[0][c] = (t3[0][c] & first) | (TERMS == 3 ? t3[2][c] & ~first : 0u);
+                o[1][c] = (t3[1][c] & first) | (t3[0][c] & ~first);
+            }
+#pragma unroll
+            for (int z = 0; z < ZB; z++) wz[b][s][z] = __builtin_bit_cast(bf16x8, make_uint4(o[z][0], o[z][1], o[z][2], o[z][3]));
+        }
+    // input gradient, A operand of 32 columns: lane -> wd[j][k = l16], j = 8 lq .. + 7, which is wcat[k][j] with the
+    // negative rail (j >= c_out) negated
+    bf16x8 wd[DX ? NB : 1][TERMS];
+    if constexpr (DX) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            unsigned t3[3][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int jl = c0 + 32 * (b * NW + wave) + 8 * lq + 2 * c;
+                float v0 = sh.u.wl[l16][jl], v1 = sh.u.wl[l16][jl + 1];
                 if (j_begin + jl >= c_out) v0 = -v0;
                 if (j_begin + jl + 1 >= c_out) v1 = -v1;
-                split3(v0, v1, h[c], m[c], l[c]);
+                split3(v0, v1, t3[0][c], t3[1][c], t3[2][c]);
             }
-            wdr[st][0] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-            wdr[st][1] = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
-            wdr[st][2] = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+#pragma unroll
+            for (int t = 0; t < TERMS; t++) wd[b][t] = __builtin_bit_cast(bf16x8, make_uint4(t3[t][0], t3[t][1], t3[t][2], t3[t][3]));
         }
     }
-    // (the tile loop's first barriers come before anything is written to est)
+    // (a barrier comes before anything else is written to wl's space: behind the first tile's gather)
 
-    // im2col gather: 256 slots (position t & 31 of the tile, member pair t >> 5: members 2 pair and 2 pair + 1),
-    // taken by the first four waves, or GP per thread in a smaller workgroup
+    // im2col gather: slot = (position t % 32 of the tile, members EP (t / 32) ..)
     const int ml = threadIdx.x & 31;
-    const bool gathers = threadIdx.x < 256;
-    int kg[GP];
-    int g_off[GP][2], g_u[GP][2], g_v[GP][2];
-    bool g_ok[GP][2];
+    int kg[GP], g_off[GP][EP], g_u[GP][EP], g_v[GP][EP];
+    bool g_ok[GP][EP];
 #pragma unroll
     for (int gp = 0; gp < GP; gp++) {
-        kg[gp] = ((threadIdx.x >> 5) + gp * (NT / 32)) & 7;
+        kg[gp] = (threadIdx.x >> 5) + gp * (NT / 32);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int k = 2 * kg[gp] + q;
-            const Member e = member_of(G, g, k < K ? k : 0);
-            g_ok[gp][q] = gathers && k < K && e.ok;
-            g_off[gp][q] = (e.ci * w_in + e.u) * h_in + e.v;
-            g_u[gp][q] = e.u;
-            g_v[gp][q] = e.v;
+        for (int p = 0; p < EP; p++) {
+            const int k = EP * kg[gp] + p;
+            const Member e = member_of(q.G, g, k < K ? k : 0);
+            g_ok[gp][p] = k < K && e.ok;
+            g_off[gp][p] = (e.ci * q.w_in + e.u) * q.h_in + e.v;
+            g_u[gp][p] = e.u;
+            g_v[gp][p] = e.v;
         }
     }
-    // this lane's 16 values of the wave's 32 x 32 block of the upstream gradient: offset in tile `split`, and
-    // the distance to the next tile of this workgroup
-    size_t g_at;
-    {
-        const int j0 = j_begin + 32 * wave;
-        int blk = gt_dedupe ? (j0 >= c_out ? j0 - c_out : j0) >> 5 : j0 >> 5;
-        if (j0 >= J) blk = 0;  // columns outside the problem: any finite values will do
-        g_at = ((size_t)split * gt_blocks + blk) * 1024 + lane * 16;
+    // where the upstream gradient of the wave's blocks lies in tile `split`: this lane's first eight values (columns 0 - 15;
+    // those of columns 16 - 31 are 256 floats further), and the distance to the next tile of this workgroup
+    int g_blk[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int j0 = j_begin + c0 + 32 * (b * NW + wave);
+        g_blk[b] = q.gt_dedupe ? (j0 >= c_out ? j0 - c_out : j0) >> 5 : j0 >> 5;
+        if (j0 >= J) g_blk[b] = 0;  // columns outside the problem: any finite values will do
     }
-    const size_t g_step = (size_t)splits * gt_blocks * 1024;
-
-    floatx4 gw_acc4[2];
+    const float* g_at = q.gtt + (size_t)split * q.gt_blocks * 1024 + ((lq & 1) * 32 + l16) * 16 + 8 * (lq >> 1);
+    const size_t g_step = (size_t)q.splits * q.gt_blocks * 1024;
+    float4 gv[2][2];
+    auto fetch_g = [&](int b) {
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+        for (int s = 0; s < 2; s++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) gw_acc4[b][r] = 0.0f;
+            for (int h = 0; h < 2; h++) gv[s][h] = *(const float4*)(g_at + (size_t)g_blk[b] * 1024 + 256 * s + 4 * h);
+    };
 
-    float* dg = dcol + (size_t)jblock * dcol_slice + (size_t)blockIdx.y * dcol_stride;
+    floatx4 gw_acc[NB][2];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) gw_acc[b][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    float* dg = q.dcol + (size_t)jblock * q.dcol_slice + (size_t)blockIdx.y * q.dcol_stride;
     const int n_tiles = (M + TM - 1) / TM;
     // The gather runs a tile ahead and its table entries two: a tile's columns of x are asked for at the
     // top of the tile before and its table entries at the top of the one before that, so that no tile
@@ -2444,168 +2497,224 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8
     };
     auto where = [&](int tile) {
         Where p;
-        p.ok = gathers && tile < n_tiles && tile * TM + ml < M;
+        p.ok = tile < n_tiles && tile * TM + ml < M;
         const int mc = p.ok ? tile * TM + ml : 0;
-        p.r0 = arow[mc];
-        p.c0 = bcol[mc];
-        p.b0 = base[mc];
+        p.r0 = q.arow[mc];
+        p.c0 = q.bcol[mc];
+        p.b0 = q.base[mc];
         return p;
     };
-    auto fetch = [&](const Where& p, float (&v)[GP][2], bool (&ok)[GP][2]) {
+    auto fetch = [&](const Where& p, float (&v)[GP][EP]) {  // returns which of them exist, one bit each
+        unsigned exist = 0;
 #pragma unroll
         for (int gp = 0; gp < GP; gp++)
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int rr = p.r0 + g_u[gp][q], cc = p.c0 + g_v[gp][q];
-                ok[gp][q] = p.ok && g_ok[gp][q] && cc >= 0 && cc < h_in && rr >= 0 && rr < w_in;
-                v[gp][q] = x[ok[gp][q] ? p.b0 + g_off[gp][q] : 0];
+            for (int e = 0; e < EP; e++) {
+                const int rr = p.r0 + g_u[gp][e], cc = p.c0 + g_v[gp][e];
+                const bool ok = p.ok && g_ok[gp][e] && cc >= 0 && cc < q.h_in && rr >= 0 && rr < q.w_in;
+                v[gp][e] = q.x[ok ? p.b0 + g_off[gp][e] : 0];
+                exist |= (unsigned)ok << (gp * EP + e);
             }
+        return exist;
     };
-    float x_next[GP][2], x_after[GP][2];
-    bool ok_next[GP][2], ok_after[GP][2];
-    Where w_after;
-    auto commit = [&](int buf, const float (&v)[GP][2], const bool (&ok)[GP][2]) {
+    auto commit = [&](int buf, const float (&v)[GP][EP], unsigned exist) {
 #pragma unroll
         for (int gp = 0; gp < GP; gp++) {
-            unsigned t3[3];
-            split3(ok[gp][0] ? v[gp][0] : 0.0f, ok[gp][1] ? v[gp][1] : 0.0f, t3[0], t3[1], t3[2]);
+            float v2[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int t = 0; t < 3; t++) {
-                ((unsigned*)&csz[buf][t][kg[gp] >> 2][ml])[kg[gp] & 3] = t3[t];
-                ((unsigned short*)&csg[buf][t][2 * kg[gp]][0])[ml] = (unsigned short)t3[t];
-                ((unsigned short*)&csg[buf][t][2 * kg[gp] + 1][0])[ml] = (unsigned short)(t3[t] >> 16);
+            for (int e = 0; e < EP; e++) v2[e] = exist >> (gp * EP + e) & 1 ? v[gp][e] : 0.0f;
+            unsigned t3[3];
+            split3(v2[0], v2[1], t3[0], t3[1], t3[2]);
+#pragma unroll
+            for (int t = 0; t < TERMS; t++) {
+                if constexpr (EP == 2) {
+                    ((unsigned*)&sh.csz[buf][t][kg[gp] >> 2][ml])[kg[gp] & 3] = t3[t];
+                    ((unsigned short*)&sh.csg[buf][t][2 * kg[gp] + 1][0])[ml] = (unsigned short)(t3[t] >> 16);
+                } else {
+                    ((unsigned short*)&sh.csz[buf][t][kg[gp] >> 3][ml])[kg[gp] & 7] = (unsigned short)t3[t];
+                }
+                ((unsigned short*)&sh.csg[buf][t][EP * kg[gp]][0])[ml] = (unsigned short)t3[t];
             }
         }
     };
+    float x_next[GP][EP], x_after[GP][EP];
+    unsigned ok_next, ok_after;
+    Where w_after;
     {
         const Where w0 = where(split);
-        fetch(w0, x_next, ok_next);
-        if (gathers) commit(0, x_next, ok_next);
-        const Where w1 = where(split + splits);
-        fetch(w1, x_next, ok_next);
-        w_after = where(split + 2 * splits);
+        ok_next = fetch(w0, x_next);
+        commit(0, x_next, ok_next);
+        const Where w1 = where(split + q.splits);
+        ok_next = fetch(w1, x_next);
+        w_after = where(split + 2 * q.splits);
     }
-    __syncthreads();  // the first tile's col is in place, and every wave has taken its weights out of est's space
+    fetch_g(0);
+    __syncthreads();  // the first tile's col is in place, and every wave has taken its weights out of wl
+    // row i of the first product's two blocks is position zrow + 8 h; lane's results: positions ep + r and ep + 8 + r
+    const int zrow = 16 * (l16 >> 3) + (l16 & 7), ep = 16 * (lq >> 1) + 4 * (lq & 1);
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4v* tr_ptr;
     int buf = 0;
-    for (int tile = split; tile < n_tiles; tile += splits, buf ^= 1) {
-        const int m0 = tile * TM;
-        float4 gv[4];
+    for (int tile = split; tile < n_tiles; tile += q.splits, buf ^= 1) {
+        ok_after = fetch(w_after, x_after);
+        w_after = where(tile + 3 * q.splits);
+        bf16x8 ag[TERMS];
 #pragma unroll
-        for (int q = 0; q < 4; q++) gv[q] = ((const float4*)(gtt + g_at))[q];
-        g_at += g_step;
-        fetch(w_after, x_after, ok_after);
-        w_after = where(tile + 3 * splits);
-        {
-            // Z[m][j] = sum_k col[k][m] * wcat[k][j] for the wave's 32 x 32 block; then E^T[j][m] =
-            // g[m][co] * exp(-Z), split into its terms: register r is position 8 (r / 4) + 4 lk + r % 4
-            bf16x8 az[3];
-#pragma unroll
-            for (int t = 0; t < 3; t++) az[t] = __builtin_bit_cast(bf16x8, csz[buf][t][lk][l32]);
-            floatx16 z;
-#pragma unroll
-            for (int r = 0; r < 16; r++) z[r] = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 6; t++) z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(az[ta[t]], wz[tb[t]], z, 0, 0, 0);
-            const int j = 32 * wave + l32;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float e0 = gv[q].x * exp_neg(z[4 * q + 0]), e1 = gv[q].y * exp_neg(z[4 * q + 1]);
-                const float e2 = gv[q].z * exp_neg(z[4 * q + 2]), e3 = gv[q].w * exp_neg(z[4 * q + 3]);
-                unsigned h0, m0w, l0, h1, m1w, l1;
-                split3(e0, e1, h0, m0w, l0);
-                split3(e2, e3, h1, m1w, l1);
-                *(uint2*)&est[0][j][4 * q + 2 * lk] = make_uint2(h0, h1);
-                *(uint2*)&est[1][j][4 * q + 2 * lk] = make_uint2(m0w, m1w);
-                *(uint2*)&est[2][j][4 * q + 2 * lk] = make_uint2(l0, l1);
-            }
+        for (int t = 0; t < TERMS; t++) {
+            const unsigned* row = sh.csg[buf][t][l16];
+            const uint2 p0 = *(const uint2*)(row + ep / 2), p1 = *(const uint2*)(row + ep / 2 + 4);
+            ag[t] = __builtin_bit_cast(bf16x8, make_uint4(p0.x, p0.y, p1.x, p1.y));
         }
-        __syncthreads();
-        {
-            // Gw[k][j] += sum_m col[k][m] * E[m][j]: two 16-column blocks of the wave, lane -> m = 8 lq .. + 7
-            bf16x8 ag[3];
+        floatx4 d[2] = {floatx4{0.0f, 0.0f, 0.0f, 0.0f}, floatx4{0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
-            for (int t = 0; t < 3; t++) ag[t] = __builtin_bit_cast(bf16x8, *(const uint4*)&csg[buf][t][l16][4 * lq]);
-            bf16x8 bg[2][3];
+        for (int b = 0; b < NB; b++) {
+            // Z[m][j] = sum_k col[k][m] * wcat[k][j], E = g * exp(-Z): eight positions of column 16 s + l16 per lane
+            float e[2][8];
 #pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int t = 0; t < 3; t++) {
-                    const unsigned* row = &est[t][32 * wave + 16 * b + l16][4 * lq];
-                    const uint2 p0 = *(const uint2*)row, p1 = *(const uint2*)(row + 2);
-                    bg[b][t] = __builtin_bit_cast(bf16x8, make_uint4(p0.x, p0.y, p1.x, p1.y));
+            for (int h = 0; h < 2; h++) {
+                // of three terms: lo hi + hi lo, mid mid + mid hi, hi mid + hi hi
+                bf16x8 az[TERMS];
+                if constexpr (TERMS == 3) {
+                    az[0] = __builtin_bit_cast(bf16x8, sh.csz[buf][lq < 2 ? 2 : 0][lq & 1][zrow + 8 * h]);
+                    az[1] = __builtin_bit_cast(bf16x8, sh.csz[buf][1][lq & 1][zrow + 8 * h]);
+                    az[2] = __builtin_bit_cast(bf16x8, sh.csz[buf][0][lq & 1][zrow + 8 * h]);
+                } else {
+                    // (lanes from 32 on meet zero weights; what they read is finite)
+                    az[0] = __builtin_bit_cast(bf16x8, sh.csz[buf][0][lq & 1][zrow + 8 * h]);
                 }
 #pragma unroll
-            for (int t = 0; t < 6; t++)
+                for (int s = 0; s < 2; s++) {
+                    floatx4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (TERMS == 3) {
+                        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(az[0], wz[b][s][0], z, 0, 0, 0);
+                        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(az[1], wz[b][s][1], z, 0, 0, 0);
+                        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(az[2], wz[b][s][1], z, 0, 0, 0);
+                    } else {
+                        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(az[0], wz[b][s][0], z, 0, 0, 0);
+                    }
+                    const float4 gq = gv[s][h];
+                    e[s][4 * h + 0] = gq.x * exp_neg(z[0]);
+                    e[s][4 * h + 1] = gq.y * exp_neg(z[1]);
+                    e[s][4 * h + 2] = gq.z * exp_neg(z[2]);
+                    e[s][4 * h + 3] = gq.w * exp_neg(z[3]);
+                }
+            }
+            // the next block's gradient, of this tile or of the workgroup's next one
+            if (b + 1 == NB && tile + q.splits < n_tiles) g_at += g_step;
+            fetch_g(b + 1 == NB ? 0 : b + 1);
+            unsigned et[3][2][4];  // term, half of the columns, pairs of positions
 #pragma unroll
-                for (int b = 0; b < 2; b++)
-                    gw_acc4[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ag[ta[t]], bg[b][tb[t]], gw_acc4[b], 0, 0, 0);
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) split3(e[s][2 * c], e[s][2 * c + 1], et[0][s][c], et[1][s][c], et[2][s][c]);
+            // Gw[k][j] += sum_m col[k][m] * E[m][j], smallest terms first
+            using Products = TermProducts<TERMS, 3>;
+#pragma unroll
+            for (int t = 0; t < Products::N; t++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const unsigned(&o)[4] = et[Products::b(t)][s];
+                    gw_acc[b][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        ag[Products::a(t)], __builtin_bit_cast(bf16x8, make_uint4(o[0], o[1], o[2], o[3])), gw_acc[b][s], 0, 0, 0);
+                }
+            if constexpr (DX) {
+                // dcol[k][m] = sum_j wd[j][k] * E[m][j] over this block's 32 columns, for positions 16 mb + l16; the wave
+                // is alone in its block of LDS, whose accesses stay in the order that they are written here
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    const int t = 2 - i;  // smallest first
+#pragma unroll
+                    for (int s = 0; s < 2; s++) {
+                        uint2* row = sh.u.t.est[wave][16 * s + l16];
+                        row[ep / 4] = make_uint2(et[t][s][0], et[t][s][1]);
+                        row[ep / 4 + 2] = make_uint2(et[t][s][2], et[t][s][3]);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int mb = 0; mb < 2; mb++) {
+                        // 16 lanes read four columns of 16 positions; each gets its position's four columns
+                        const uint2* at = &sh.u.t.est[wave][8 * lq + (l16 >> 2)][4 * mb + (l16 & 3)];
+                        const short4v j0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
+                        const short4v j4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * (kBfEw / 2)));
+                        const bf16x8 bd = __builtin_bit_cast(bf16x8, __builtin_shufflevector(j0, j4, 0, 1, 2, 3, 4, 5, 6, 7));
+                        if constexpr (TERMS == 3) {
+                            if (i > 1) d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wd[b][2], bd, d[mb], 0, 0, 0);
+                            if (i > 0) d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wd[b][1], bd, d[mb], 0, 0, 0);
+                        }
+                        d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wd[b][0], bd, d[mb], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
         }
         // the next tile's col, into the buffer whose readers finished before the last barrier
-        if (gathers) commit(buf ^ 1, x_next, ok_next);
-        floatx4 d[2];
-        if (DX) {
-            // dcol[k][m] = sum_j wd[j][k] * E[m][j]: one 16 x 16 block per wave over its quarter of j, lane ->
-            // position 16 mb + l16, j = jd0 + 32 st + 8 lq .. + 7; the two steps in accumulators of their own
-            const unsigned short* eh = (const unsigned short*)&est[0][jd0 + 8 * lq][0] + 16 * mb + l16;
-            bf16x8 bd[2][3];
+        commit(buf ^ 1, x_next, ok_next);
+        if constexpr (DX) {
 #pragma unroll
-            for (int st = 0; st < 2; st++)
-#pragma unroll
-                for (int t = 0; t < 3; t++) {
-                    unsigned wv[4];
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const unsigned short* pe = eh + ((t * JW + 32 * st + 2 * c) * EW) * 2;
-                        wv[c] = (unsigned)pe[0] | ((unsigned)pe[2 * EW] << 16);
-                    }
-                    bd[st][t] = __builtin_bit_cast(bf16x8, make_uint4(wv[0], wv[1], wv[2], wv[3]));
-                }
-#pragma unroll
-            for (int st = 0; st < 2; st++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) d[st][r] = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 6; t++)
-#pragma unroll
-                for (int st = 0; st < 2; st++)
-                    d[st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wdr[st][ta[t]], bd[st][tb[t]], d[st], 0, 0, 0);
-            if (JPARTS > 1 && jpart > 0) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) red[jpart - 1][mb][4 * lq + r][l16] = d[0][r] + d[1][r];
-            }
+            for (int mb = 0; mb < 2; mb++)
+                sh.u.t.red[buf][wave][mb][lane] = make_float4(d[mb][0], d[mb][1], d[mb][2], d[mb][3]);
         }
-        // every wave has read this tile's E and col, and written the next tile's col and its share of red
+        // every wave has read this tile's col, and written the next tile's and its share of red (whose other buffer
+        // was read before this barrier)
         __syncthreads();
-        if (DX && jpart == 0) {
-            const int m = m0 + 16 * mb + l16;
+        if constexpr (DX) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int k = 4 * lq + r;
-                float sum = d[0][r] + d[1][r];
+            for (int o = threadIdx.x; o < 2 * 64 * 4; o += NT) {
+                const float* r = (const float*)&sh.u.t.red[buf][0][0][0] + o;
+                float sum = r[0];
 #pragma unroll
-                for (int jp = 1; jp < JPARTS; jp++) sum += red[jp - 1][mb][k][l16];
-                if (k < K && m < M) dg[(size_t)k * M + m] = sum;
+                for (int w = 1; w < NW; w++) sum += r[w * 2 * 64 * 4];
+                const int k = 4 * (o >> 6 & 3) + (o & 3), m = tile * TM + 16 * (o >> 8) + (o >> 2 & 15);
+                if (k < K && m < M) {
+                    float* to = dg + (size_t)k * M + m;
+                    *to = ADD ? *to + sum : sum;
+                }
             }
         }
 #pragma unroll
         for (int gp = 0; gp < GP; gp++)
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                x_next[gp][q] = x_after[gp][q];
-                ok_next[gp][q] = ok_after[gp][q];
+            for (int e = 0; e < EP; e++) x_next[gp][e] = x_after[gp][e];
+        ok_next = ok_after;
+    }
+    if (q.store_part) {
+        float* pg = q.part + (size_t)blockIdx.y * q.part_stride + (size_t)split * K * J;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const int j = j_begin + c0 + 32 * (b * NW + wave) + 16 * s + l16;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int k = 4 * lq + r;
+                    if (k < K && j < J) pg[(size_t)k * J + j] = gw_acc[b][s][r];
+                }
             }
     }
-    if (store_part) {
-        float* pg = part + (size_t)blockIdx.y * part_stride + (size_t)split * K * J;
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int j = j_begin + 32 * wave + 16 * b + l16;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int k = 4 * lq + r;
-                if (k < K && j < J) pg[(size_t)k * J + j] = gw_acc4[b][r];
-            }
-        }
+}
+
+template <int NW, int NB, bool DX>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 3))) void k_bwd_small_k_bf16(SmallKParams q)
+{
+    constexpr int NT = 64 * NW, JW = 32 * NW * NB;
+    __shared__ __attribute__((aligned(16))) SmallKShared<NW, NB, DX> sh;
+    const int split = blockIdx.x / q.jblocks, jblock = blockIdx.x - split * q.jblocks, j_begin = jblock * JW;
+    // whether x and this workgroup's weights are bf16 numbers
+    bool three = small_k_weights(q, sh, j_begin);
+    for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
+    if (!__syncthreads_or(three)) {
+        small_k_columns<1, NW, NB, DX, false>(q, sh, split, jblock, j_begin, 0);
+        return;
+    }
+    small_k_columns<3, NW, 1, DX, false>(q, sh, split, jblock, j_begin, 0);
+    if constexpr (NB > 1) {
+        static_assert(NB == 2, "one more pass");
+        __syncthreads();
+        small_k_weights(q, sh, j_begin);
+        __syncthreads();
+        small_k_columns<3, NW, 1, DX, true>(q, sh, split, jblock, j_begin, 32 * NW);
     }
 }
 
@@ -2803,15 +2912,37 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     }
     const int K = b.G.n_members;
     b.fused_k = K <= kFusedK;
-    // the bf16 kernel (at most 16 members) comes with 2, 4 or 8 waves of 32 columns, the fp32 one with 128 or 256 columns
-    b.fused_jw = 2 * g.c_out <= 64 && K <= 16 ? 64 : 2 * g.c_out <= 128 ? 128 : 256;
+    // the bf16 kernel (at most 16 members) comes with 2, 4 or 8 waves of 32 columns, or 8 of 64 where under four of the
+    // waves' 16 blocks stay empty (with 260 columns, operands of three terms: 417 us against 398 of 256-wide ones for
+    // 64 -> 130 at 20 x 20, z_unit 4, batch 32) and a workgroup gets eight tiles (512 channels, 37 groups, batch 100:
+    // 109 against 97); the fp32 one with 128 or 256 columns
+    const long long fused_tiles = (b.m_total + kFusedTile - 1) / kFusedTile;
+    const bool wide = K <= 16 && (512 - 2 * g.c_out % 512) % 512 < 128 &&
+                      fused_tiles * b.G.n_groups * ((2 * g.c_out + 511) / 512) >= 8 * 512;
+    b.fused_jw = 2 * g.c_out <= 64 && K <= 16 ? 64 : 2 * g.c_out <= 128 ? 128 : wide ? 512 : 256;
     b.fused_jblocks = (2 * g.c_out + b.fused_jw - 1) / b.fused_jw;
     b.gt_dedupe = g.c_out % 32 == 0;
     b.gt_blocks = b.gt_dedupe ? g.c_out / 32 : (2 * g.c_out + 31) / 32;
     {
         // about eight workgroups per CU in all, each looping over its share of the tiles
-        const long long n_tiles = (b.m_total + kFusedTile - 1) / kFusedTile;
-        long long want = 2048 / ((long long)b.G.n_groups * b.fused_jblocks);
+        const long long n_tiles = fused_tiles;
+        const long long per_split = (long long)b.G.n_groups * b.fused_jblocks;
+        long long want = 2048 / per_split;
+        if (K <= 16) {
+            // the bf16 kernel: the number of full rounds of workgroups that takes least, where one begins with what costs
+            // it two tiles (its weights' terms).  12 -> 100, 1 x 1, 28 x 28, batch 64, step on floats: 161 us, 110; with
+            // 2048 workgroups whatever their tiles 12 -> 200 took 289, now 137
+            const long long at_once = b.fused_jw == 64 ? 1536 : b.fused_jw == 128 ? 768 : 512;
+            long long least = 0;
+            for (int rounds = 1; rounds <= 4; rounds++) {
+                const long long splits = std::max(1LL, std::min(n_tiles, at_once * rounds / per_split));
+                const long long cost = (splits * per_split + at_once - 1) / at_once * (2 + (n_tiles + splits - 1) / splits);
+                if (rounds == 1 || cost < least) {
+                    least = cost;
+                    want = splits;
+                }
+            }
+        }
         if (want > n_tiles) want = n_tiles;
         if (want > 65535) want = 65535;
         b.fused_splits = (int)(want < 1 ? 1 : want);
@@ -2946,11 +3077,13 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
     int* one_term = found + kScanBlocks * kScanRows;
     const int n_scan_rows = scan_rows(x_total);
     // the position tables serve the gathers of im2col and of the fused kernels
-    auto position_tables = [&](const int* scanned) {
-        hipLaunchKernelGGL(k_position_table, dim3(m_blocks), dim3(256), 0, s, pos_base, pos_arow, pos_bcol, scanned, n_scan_rows, one_term, M,
-                           g.c_in, g.c_out, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho);
+    auto position_tables = [&](const int* scanned, int scan_x_rows) {
+        const dim3 grid(scan_x_rows ? std::max(m_blocks, kScanBlocks) : m_blocks, 1 + scan_x_rows);
+        hipLaunchKernelGGL(k_position_table, grid, dim3(256), 0, s, pos_base, pos_arow, pos_bcol, scanned, n_scan_rows, one_term, x,
+                           x_total, found, M, g.c_in, g.c_out, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho);
     };
-    if (fused) position_tables(nullptr);
+    // (the kernel for up to 16 members takes operands of one term as such)
+    if (fused) position_tables(nullptr, K <= 16 ? n_scan_rows : 0);
     // Where the first product reads col as a view and its tiles are whole (the eight-wave kernel in every round,
     // or the 128 x 128 kernel), its epilogue reads the upstream gradient as it is (items of whole 32-position
     // blocks, 16-byte aligned): no transposed copy.
@@ -3025,22 +3158,28 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             if (gx) GEO_SC_FUSED_K(KS, 2, true); else GEO_SC_FUSED_K(KS, 2, false);                                    \
         }                                                                                                              \
     } while (0)
-#define GEO_SC_FUSED_BF16(NW, DX)                                                                                      \
-    hipLaunchKernelGGL((k_bwd_small_k_bf16<NW, DX>), grid, dim3(64 * NW), 0, s, x, wcat, gt, pos_base, pos_arow,        \
-                       pos_bcol, part, dcol, G, v0, M, g.w_in, g.h_in, g.c_out, L.fused_jblocks, L.fused_splits,        \
-                       gw ? 1 : 0, L.gt_blocks, L.gt_dedupe, L.w_v, L.part_v, L.col_v, slice)
                 if (ks <= 8) {
-                    if (jw == 64) {
-                        if (gx) GEO_SC_FUSED_BF16(2, true); else GEO_SC_FUSED_BF16(2, false);
-                    } else if (jw == 128) {
-                        if (gx) GEO_SC_FUSED_BF16(4, true); else GEO_SC_FUSED_BF16(4, false);
-                    } else {
-                        if (gx) GEO_SC_FUSED_BF16(8, true); else GEO_SC_FUSED_BF16(8, false);
-                    }
+                    SmallKParams p = {x, wcat, gt, pos_base, pos_arow, pos_bcol, found, part, dcol, G, v0, M, g.w_in, g.h_in,
+                                      g.c_out, L.fused_jblocks, L.fused_splits, gw ? 1 : 0, L.gt_blocks, L.gt_dedupe, n_scan_rows,
+                                      L.w_v, L.part_v, L.col_v, slice};
+                    auto launch = [&](auto dx) {
+                        constexpr bool DX = decltype(dx)::value;
+                        if (jw == 64)
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<2, 1, DX>), grid, dim3(128), 0, s, p);
+                        else if (jw == 128)
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<4, 1, DX>), grid, dim3(256), 0, s, p);
+                        else if (jw == 256)
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 1, DX>), grid, dim3(512), 0, s, p);
+                        else
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 2, DX>), grid, dim3(512), 0, s, p);
+                    };
+                    if (gx)
+                        launch(std::true_type());
+                    else
+                        launch(std::false_type());
                 }
                 else if (ks <= 12) GEO_SC_FUSED_NB_DX(12);
                 else GEO_SC_FUSED_NB_DX(16);
-#undef GEO_SC_FUSED_BF16
 #undef GEO_SC_FUSED_NB_DX
 #undef GEO_SC_FUSED_K
             }
@@ -3096,7 +3235,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                 hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + pp.scan_rows), dim3(256), 0, s, pp);
             }
         }
-        if (!view && v0 == 0) position_tables(found);
+        if (!view && v0 == 0) position_tables(found, 0);
         if (view) {
             const long long plane = (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho;
             const long long quads = (long long)g.h_k * g.c_in * plane / 4;

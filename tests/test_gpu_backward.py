@@ -644,3 +644,36 @@ def test_input_gradient_of_few_positions(capi, shape_x, shape_w, pad, mode, zu, 
     rx, rw, _ = surrogate.surrogate_autograd(x.cuda(), w.cuda(), g.cuda(), (pad, pad), mode=mode, z_unit=zu)
     check("grad_x", gx, rx)
     check("grad_w", gw, rw)
+
+
+SMALL_GROUPS = [
+    # shape_x, shape_w, pad, mode, z_unit: the fused kernel with 2, 4 and 8 waves, one and two blocks of columns per wave
+    ((1, 3, 1, 5), (5, 3, 1, 5), 0, "y", 1),        # one position, 10 of 64 columns
+    ((33, 16, 1, 6), (33, 16, 1, 6), 0, "y", 1),    # 33 positions, 66 of 128 columns
+    ((2, 3, 9, 11), (64, 3, 5, 5), 2, "y", 1),      # 15 members, 128 columns
+    ((3, 7, 6, 6), (130, 7, 3, 3), 1, "z", 1),      # 9 members, 260 of 512 columns in two sets of 256
+    ((31, 16, 1, 4), (200, 16, 1, 4), 0, "y", 1),   # 31 positions, 400 of 512 columns
+    ((65, 16, 1, 3), (256, 16, 1, 3), 0, "y", 1),   # 512 columns, whole tiles and one position
+    ((40, 6, 4, 4), (500, 6, 3, 3), 1, "yz", 4),    # 12 members, ragged channel blocks, two sets of 512 columns
+]
+
+
+@pytest.mark.parametrize("operands", ["seven bits", "floats", "float weights of the last channel"])
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", SMALL_GROUPS)
+def test_small_or_groups(capi, shape_x, shape_w, pad, mode, zu, operands):
+    """One term or three, which each workgroup finds for its columns; with and without the input gradient."""
+    from oracle import surrogate
+    x, w, g = seven_bit(shape_x, shape_w, 7)
+    if operands == "floats":
+        x, w = x * 0.93, w * 0.93
+    elif operands != "seven bits":
+        w[-1] *= 0.93
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gy = torch.randn(capi.output_shape(d), generator=g)
+    gx, gw = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, (pad, pad), accumulate=mode, z_unit=zu)
+    rx, rw, _ = surrogate.surrogate_autograd(x, w, gy, (pad, pad), mode=mode, z_unit=zu)
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
+    none, only = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, (pad, pad), accumulate=mode, z_unit=zu,
+                                                  need_grad_x=False)
+    assert none is None and torch.equal(only, gw)
