@@ -25,7 +25,8 @@
 // and reduced deterministically.  Where every x and w is a bf16 number, as the 7-bit operands of the layers are
 // (k / 128), eleven of the eighteen term products would multiply by zeros: a scan finds that out on the device and the
 // products are left out (GemmParams::one_term), the same results bit for bit.  Three products of 64 -> 64 at 56 x 56,
-// batch 128: 438 + 411 + 426 -> 349 + 303 + 349 us; 512 -> 512 at 4 x 4, batch 128, first product: 126 -> 61.
+// batch 128: 438 + 411 + 426 -> 349 + 303 + 349 us; 512 -> 512 at 4 x 4, batch 128, first product: 126 -> 61.  Up to 192
+// members the first two are one kernel then, k_bwd_e_wgrad: 314 us there.
 //
 // The other accumulation modes have the same surrogate with other add groups
 // (utils_functional.py:254-299): one exponential per add group, whose argument sums the OR
@@ -101,6 +102,7 @@ struct GemmParams {
     // operands made from them are one term of the split instead of three, and the rows that `a` of the first two products
     // points to hold bf16 numbers (the same elements at the same indexes).
     const int* __restrict__ one_term;
+    int one_term_elsewhere;  // another kernel (k_bwd_e_wgrad) does this product where they are
     // EPI_STORE_ITEMS: column j = (n, rest) of the result goes to c[(n * I + i) * c_plane + rest] (c_plane
     // columns per item): the input gradient in the caller's layout (n, c_in, w_in, h_in)
     int c_plane;
@@ -419,6 +421,9 @@ struct SplitStager {
 // AHEAD (K-major only): the table entries of a chunk are read when the chunk before it is fetched, so that a
 // fetch issues its loads without waiting for the table first; the entries read for the chunk behind the last
 // one (up to 2 * kChunk + 8 entries behind the member's part of the table) are never used.
+// Without AHEAD the table is read as constant memory (its kernel ran before): scalar loads, where the compiler otherwise
+// takes vector loads in some of the loops, which the data loads then wait for (first product of 64 -> 64 at 28 x 28, batch
+// 64, three terms: 69 us, now 57).
 template <bool KMAJOR, typename T = float, bool AHEAD = false>
 struct ViewStager {
     const T* base;
@@ -430,6 +435,10 @@ struct ViewStager {
     int half, ii;
     long long ahead[(KMAJOR && AHEAD) ? 8 : 1];  // the rows' starts of the chunk to fetch next
 
+    __device__ __forceinline__ long long row_at(int k) const
+    {
+        return ((const __attribute__((address_space(4))) long long*)rows)[k];
+    }
     __device__ __forceinline__ void read_ahead()
     {
         if constexpr (KMAJOR && AHEAD) {
@@ -492,7 +501,7 @@ struct ViewStager {
         }
         if (KMAJOR) {
 #pragma unroll
-            for (int c = 0; c < 8; c++) r[c] = (base + rows[kr + c])[off];
+            for (int c = 0; c < 8; c++) r[c] = (base + row_at(kr + c))[off];
         } else {
             load_row(p, r);
         }
@@ -506,7 +515,7 @@ struct ViewStager {
             for (int c = 0; c < 8; c++) {
                 // rows past the end of a partial chunk read the chunk's first row instead
                 const int row = (tail && 8 * half + c >= k_left) ? kr - 8 * half : kr + c;
-                r[c] = (base + rows[row])[off];
+                r[c] = (base + row_at(row))[off];
             }
         } else {
             if (!tail)
@@ -783,6 +792,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 {
     __shared__ uint4 as[2][3][2][kLdx];
     __shared__ uint4 bs[2][3][2][kLdx];
+    if (q.one_term_elsewhere && *q.one_term) return;
     int it, jt, z;
     gemm_tile_of(q, blockIdx.x, it, jt, z);
     const int i0 = it * q.tile_i, j0 = jt * q.tile_j;
@@ -1066,6 +1076,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 {
     __shared__ uint4 as[2][3][2 * KC][64 * NX + 4];
     __shared__ uint4 bs[2][3][2 * KC][kBigJ + 4];
+    if (q.one_term_elsewhere && *q.one_term) return;
     if (!(q.one_term && *q.one_term))
         gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 3, 3, float>(q, as, bs);
     else if constexpr (PRODUCT == PRODUCT_E)
@@ -1074,6 +1085,264 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 3, bf16_bits>(q, as, bs);
     else
         gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 3, float>(q, as, bs);
+}
+
+// ---- E and the weight gradient in one kernel, for operands of one term and up to 192 members ----
+// What the two products by themselves spend their time on is E (M x 2 c_out floats per group: written, read once per 128
+// members, split each time) and chunks of 16 members or positions, a barrier each, that hold four MFMAs per wave where
+// operands are one term.  Here a wave keeps 32 columns: their weights for all members in registers (first product, 32x32x16:
+// A = col[m][k], read transposed from LDS), and all members' sums of the weight gradient.  The first product's result
+// E[m][j] is the second one's B operand as it is: lane -> column j, and of each 16 positions the eight that the lane
+// holds (the order of a contraction is free; A = col[k][m] is read in the same order).  So E is split once and never read
+// back; it is stored for the input gradient, and the same bits as the first product stores.
+// A workgroup is persistent: 4 waves, one group, NWJ * 32 columns, one part of the positions in tiles of 32 (64 where two
+// waves cover the columns: the halves' sums meet at the end); col's next tile is loaded while this one is multiplied.
+// 64 -> 64 at 56 x 56, batch 128: 314 us, the two products 354 + 306; without the stores of E it takes 40 less, without the
+// gradient's loads 45 less, its matrix work is 108.  Ragged layer of 77 items, 45 -> 83, blocks of 32 channels: 89, 79 + 76.
+// Three terms need three times the registers: those operands take the two products (which return at once otherwise).
+struct EwParams {
+    const bf16_bits* __restrict__ col;
+    const float* __restrict__ wcat;
+    const float* __restrict__ g;  // the gradient: [m][c_out], or as the caller has it (GemmParams::g_planes)
+    float* __restrict__ e;
+    float* __restrict__ part;
+    const int* __restrict__ one_term;
+    const long long* __restrict__ rows;  // the view's row table, or NULL: rows col_ld apart
+    int rows_batch, item, skip;
+    long long col_ld;
+    size_t col_v, w_v, e_v, part_v;
+    int M, K, J, e_ld, c_out, npos, m_per_split, jtiles;
+};
+constexpr int kEwMembers = 192;     // six blocks of 32: 96 registers of sums
+constexpr int kEwWorkgroups = 512;  // two per CU
+
+// PLANES: the gradient as the caller has it, through LDS in runs along the positions (a lane's own loads, 16 bytes from
+// each of 32 channels, thrash the CU's cache: 483 us instead of 314); otherwise [m][c_out], read by the lanes as it is.
+template <int NKB, int NWJ, bool PLANES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_bwd_e_wgrad(EwParams q)
+{
+    static_assert(!PLANES || NWJ == 4, "tiles of 32 positions");
+    constexpr int NWM = 4 / NWJ, TM = 32 * NWM, KR = 32 * NKB;
+    constexpr int RQ = TM == 32 ? 9 : 18;            // 8-byte words per row of col: 8 or 16 and padding (no bank conflicts)
+    constexpr int QPR = TM / 4, RPP = 256 / QPR, NP = KR / RPP;  // quads per row; rows per pass over the workgroup, passes
+    __shared__ uint2 cs[2][KR][RQ];
+    __shared__ long long row_at[KR];
+    constexpr int GR = 128, GQ = 9;  // the gradient's rows in LDS (channels), 16-byte words per row: 8 and padding
+    __shared__ floatx4 gs[2][PLANES ? GR : 1][GQ];
+    static_assert(sizeof(cs) >= 2 * 16 * 64 * sizeof(float), "room for a block's sums of two waves");
+    if (!*q.one_term) return;
+    const int group = blockIdx.y;
+    const int split = blockIdx.x / q.jtiles, jt = blockIdx.x - split * q.jtiles;
+    const int m_begin = split * q.m_per_split, m_end = min(q.M, m_begin + q.m_per_split);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int l32 = lane & 31, lk = lane >> 5;
+    const int wj = wave % NWJ, wm = wave / NWJ;
+    const int j0 = (jt * NWJ + wj) * 32, j = j0 + l32;
+    const bool j_ok = j < q.J;
+    const bool has_columns = j0 < q.J;  // uniform
+
+    for (int k = threadIdx.x; k < KR; k += 256) {
+        const int kc = min(k, q.K - 1);
+        row_at[k] = q.rows ? q.rows[(size_t)group * q.rows_batch + kc] : kc * q.col_ld;
+    }
+    // first product, B operand of step s: lane -> column j, members 16 s + 8 lk .. + 7
+    bf16x8 wz[2 * NKB];
+    {
+        const float* wg = q.wcat + (size_t)group * q.w_v + min(j, q.J - 1);
+#pragma unroll
+        for (int s = 0; s < 2 * NKB; s++) {
+            unsigned h[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int k = 16 * s + 8 * lk + 2 * c;
+                const float v0 = wg[(size_t)min(k, q.K - 1) * q.J], v1 = wg[(size_t)min(k + 1, q.K - 1) * q.J];
+                h[c] = pack_bf16(j_ok && k < q.K ? v0 : 0.0f, j_ok && k + 1 < q.K ? v1 : 0.0f);
+            }
+            wz[s] = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+        }
+    }
+    // col's tile: a thread moves quad tq of the rows tr, tr + RPP, ...; positions from the part's end on and rows
+    // beyond the members are zero
+    const int tq = threadIdx.x % QPR, tr = threadIdx.x / QPR;
+    const bf16_bits* colg = q.col + (q.rows ? 0 : (size_t)group * q.col_v);
+    // (in two halves where a thread moves up to 24 quads: registers)
+    constexpr int HALVES = NWM, NH = NP / HALVES;
+    static_assert(NH * HALVES == NP, "whole halves");
+    uint2 keep;
+    auto fetch = [&](int m0, int half, uint2 (&v)[NH]) {
+        const int m = m0 + 4 * tq, left = m_end - m;
+        keep.x = left >= 2 ? ~0u : left == 1 ? 0xffffu : 0u;
+        keep.y = left >= 4 ? ~0u : left == 3 ? 0xffffu : 0u;
+        const int mc = left > 0 ? m : m_begin;
+        const long long at = q.rows ? mc + (long long)(mc / q.item) * q.skip : mc;
+#pragma unroll
+        for (int p = 0; p < NH; p++) v[p] = *(const uint2*)(colg + row_at[tr + RPP * (half * NH + p)] + at);
+    };
+    auto commit = [&](int buf, int half, const uint2 (&v)[NH]) {
+#pragma unroll
+        for (int p = 0; p < NH; p++) {
+            const int k = tr + RPP * (half * NH + p);
+            const bool in = k < q.K;
+            cs[buf][k][tq] = make_uint2(in ? v[p].x & keep.x : 0u, in ? v[p].y & keep.y : 0u);
+        }
+    };
+    floatx16 acc[NKB];
+#pragma unroll
+    for (int b = 0; b < NKB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[b][r] = 0.0f;
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4v* tr_ptr;
+    const int co = j_ok ? (j >= q.c_out ? j - q.c_out : j) : 0;
+    float* eg = q.e + (size_t)group * q.e_v;
+    // the upstream gradient at the wave's positions mb + 8 (r / 4) + 4 lk + r % 4 (register r), a tile ahead (behind the
+    // part's end: of its first positions)
+    float gv[16];
+    auto fetch_g = [&](int mb) {
+        const int mi = (mb < m_end ? mb : m_begin) + 4 * lk;
+#pragma unroll
+        for (int r = 0; r < 16; r++) gv[r] = q.g[(size_t)min(mi + 8 * (r >> 2) + (r & 3), m_end - 1) * q.c_out + co];
+    };
+    // the same by rows of 32 positions, one per channel that the workgroup's columns have: all of them where they are few
+    const int g_rows = min(q.c_out, GR), g_first = q.c_out <= GR ? 0 : jt * 128, g_row = q.c_out <= GR ? co : min(j, q.J - 1) - jt * 128;
+    floatx4 g_next[GR / 32];
+    auto fetch_planes = [&](int m0) {
+        const int mc = m0 < m_end ? m0 : m_begin, item = mc / q.npos;
+        const float* gp = q.g + (size_t)item * q.c_out * q.npos + (mc - item * q.npos) + 4 * (threadIdx.x & 7);
+#pragma unroll
+        for (int p = 0; p < GR / 32; p++) {
+            const int row = min((int)(threadIdx.x >> 3) + 32 * p, g_rows - 1), jr = min(g_first + row, q.J - 1);
+            g_next[p] = *(const floatx4*)(gp + (size_t)(jr >= q.c_out ? jr - q.c_out : jr) * q.npos);
+        }
+    };
+    auto commit_planes = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < GR / 32; p++)
+            gs[buf][(threadIdx.x >> 3) + 32 * p][threadIdx.x & 7] = g_next[p];
+    };
+    if constexpr (PLANES) {
+        fetch_planes(m_begin);
+        commit_planes(0);
+    } else {
+        fetch_g(m_begin + 32 * wm);
+    }
+    uint2 next[NH];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < HALVES; h++) {
+        fetch(m_begin, h, next);
+        commit(0, h, next);
+    }
+    __syncthreads();
+    constexpr int kMfma = 0x008, kDsRead = 0x100;  // of __builtin_amdgcn_sched_group_barrier
+    int buf = 0;
+    for (int m0 = m_begin; m0 < m_end; m0 += TM, buf ^= 1) {
+        const int mb = m0 + 32 * wm, mi = mb + 4 * lk;
+        fetch(m0 + TM, 0, next);  // (zeros behind the part's end)
+        if constexpr (PLANES) fetch_planes(m0 + TM);
+        floatx16 z;
+        if (has_columns) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) z[r] = 0.0f;
+#pragma unroll
+            for (int s = 0; s < 2 * NKB; s++) {
+                // 16 lanes read four members of 16 positions; each gets its position's four members
+                const uint2* at = &cs[buf][16 * s + 8 * lk + ((lane & 15) >> 2)][8 * wm + 4 * (lane >> 4 & 1) + (lane & 3)];
+                const short4v k0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
+                const short4v k4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * RQ));
+                const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(k0, k4, 0, 1, 2, 3, 4, 5, 6, 7));
+                z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wz[s], z, 0, 0, 0);
+            }
+            // operands four steps ahead: a step alone waits for LDS longer than it multiplies
+            constexpr int kAhead = 4;
+            __builtin_amdgcn_sched_group_barrier(kDsRead, 2 * kAhead, 0);
+#pragma unroll
+            for (int s = 0; s < 2 * NKB; s++) {
+                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                if (s + kAhead < 2 * NKB) __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+            }
+            if constexpr (PLANES) {
+#pragma unroll
+                for (int o = 0; o < 4; o++) {
+                    const floatx4 v = gs[buf][g_row][2 * o + lk];
+                    gv[4 * o] = v[0]; gv[4 * o + 1] = v[1]; gv[4 * o + 2] = v[2]; gv[4 * o + 3] = v[3];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) z[r] = gv[r] * exp_neg(z[r]);
+            if constexpr (!PLANES) fetch_g(mb + TM);
+            float* ep = eg + (size_t)mi * q.e_ld + j;
+            if (mb + 32 <= m_end && j0 + 32 <= q.J) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) ep[(size_t)(8 * (r >> 2) + (r & 3)) * q.e_ld] = z[r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int d = 8 * (r >> 2) + (r & 3);
+                    if (mi + d >= m_end)
+                        z[r] = 0.0f;
+                    else if (j_ok)
+                        ep[(size_t)d * q.e_ld] = z[r];
+                }
+            }
+        }
+        if constexpr (HALVES > 1) {
+            commit(buf ^ 1, 0, next);
+            fetch(m0 + TM, 1, next);
+        }
+        if (has_columns) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                unsigned t3[3][4];
+#pragma unroll
+                for (int o = 0; o < 4; o++) split3(z[8 * c + 2 * o], z[8 * c + 2 * o + 1], t3[0][o], t3[1][o], t3[2][o]);
+                bf16x8 bt[3];
+#pragma unroll
+                for (int t = 0; t < 3; t++) bt[t] = __builtin_bit_cast(bf16x8, make_uint4(t3[t][0], t3[t][1], t3[t][2], t3[t][3]));
+#pragma unroll
+                for (int b = 0; b < NKB; b++) {
+                    const uint2* row = &cs[buf][32 * b + l32][8 * wm + 4 * c + lk];
+                    const uint2 p0 = row[0], p1 = row[2];
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, make_uint4(p0.x, p0.y, p1.x, p1.y));
+#pragma unroll
+                    for (int t = 2; t >= 0; t--) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bt[t], acc[b], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 1);
+#pragma unroll
+            for (int b = 0; b < 2 * NKB; b++) {
+                __builtin_amdgcn_sched_group_barrier(kMfma, 3, 1);
+                if (b + 2 < 2 * NKB) __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 1);
+            }
+        }
+        commit(buf ^ 1, HALVES - 1, next);
+        if constexpr (PLANES) commit_planes(buf ^ 1);
+        __syncthreads();
+    }
+    float* pg = q.part + (size_t)group * q.part_v + (size_t)split * q.K * q.J;
+    float* meet = (float*)&cs[0][0][0];  // sums of the waves with the tile's other half, [column block][register][lane]
+#pragma unroll
+    for (int b = 0; b < NKB; b++) {
+        if constexpr (NWM == 2) {
+            __syncthreads();
+            if (wm == 1) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) meet[(wj * 16 + r) * 64 + lane] = acc[b][r];
+            }
+            __syncthreads();
+            if (wm == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[b][r] += meet[(wj * 16 + r) * 64 + lane];
+            }
+        }
+        if (wm == 0 && j_ok) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int k = 32 * b + 8 * (r >> 2) + 4 * lk + (r & 3);
+                if (k < q.K) pg[(size_t)k * q.J + j] = acc[b][r];
+            }
+        }
+    }
 }
 
 // gt[n*npos + pos][co] = g[n][co][pos]: the upstream gradient with the channel innermost, so that the
@@ -1480,6 +1749,12 @@ struct WgradOperands {
     long long m, col_ld, e_ld;
     size_t col_v, e_v;
 };
+// The partial sums to add: `splits`, or `one` where operands of one term take k_bwd_e_wgrad.
+struct WgradSplits {
+    int splits, one;
+    const int* one_term;  // NULL: they don't
+    __device__ __forceinline__ int count() const { return one_term && *one_term ? one : splits; }
+};
 __device__ __forceinline__ float wgrad_again(const WgradOperands& o, int group, int k, int j, long long begin, long long end)
 {
     const size_t c0 = group * o.col_v + k * o.col_ld;
@@ -1498,9 +1773,10 @@ __device__ __forceinline__ float wgrad_again(const WgradOperands& o, int group, 
 // block takes 32 consecutive (k, co) entries; 8 sets of threads each sum every 8th split, the
 // sets are then added in a fixed order, so the result does not depend on scheduling.
 __global__ __launch_bounds__(256) void k_reduce_wgrad(const float* __restrict__ part, const float* __restrict__ w,
-                                                      float* __restrict__ gw, int g0, int splits, int c_out, Groups G,
+                                                      float* __restrict__ gw, int g0, WgradSplits parts, int c_out, Groups G,
                                                       size_t g_stride, WgradOperands again)
 {
+    const int splits = parts.count();
     __shared__ float red[2][8][32];
     const int K = G.n_members;
     const int total = K * c_out;
@@ -1725,9 +2001,10 @@ __global__ __launch_bounds__(256) void k_weight_cat_tiled(const float* __restric
 // are read in 128-byte runs along the channel, added over the splits in their order, and dL/dw is
 // written in 128-byte runs along the weights of one channel.
 __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restrict__ part, const float* __restrict__ w,
-                                                            float* __restrict__ gw, int g0, int ng, int splits, int c_out,
+                                                            float* __restrict__ gw, int g0, int ng, WgradSplits parts, int c_out,
                                                             Groups G, size_t g_stride, WgradOperands again)
 {
+    const int splits = parts.count();
     __shared__ float tp[32][33], tn[32][33];  // [weight][channel]
     const int per_channel = G.c_in * G.w_k * G.h_k;
     const long long stride = (long long)G.n_members * 2 * c_out;
@@ -2866,6 +3143,8 @@ struct BwdLayout {
     int fused_splits;    // its workgroups per add group and column block
     int gt_dedupe;       // its upstream-gradient tiles serve both rails (c_out a multiple of 32)
     int gt_blocks;       // 32-column blocks of those tiles
+    int ew_splits;       // parts of the positions in k_bwd_e_wgrad; 0: more members than it takes
+    int ew_m_per_split;
     int rows_per_chunk;  // add groups processed by one round of launches
     int dcol_slices;     // partial dcol arrays per round (column blocks of the fused kernel), rows_per_chunk * col_v apart
     bool dx_rows;        // the input-gradient GEMM sums the kernel rows itself (E read as a view shifted by image rows)
@@ -2962,12 +3241,22 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     if (per < 256) per = 256;
     b.m_per_split = (int)(per > 0x7fffffffLL ? 0x7fffffffLL : per);
     b.splits = (int)((b.m_total + b.m_per_split - 1) / b.m_per_split);
+    // one round of persistent workgroups for E and the weight gradient of operands of one term
+    b.ew_splits = b.ew_m_per_split = 0;
+    if (!b.fused_k && K <= kEwMembers) {
+        const int tm = 2 * g.c_out <= 64 ? 64 : 32;
+        const long long jtiles = (2 * g.c_out + 127) / 128, m_tiles = (b.m_total + tm - 1) / tm;
+        const long long parts = std::max(1LL, std::min(kEwWorkgroups / (jtiles * b.G.n_groups), m_tiles / 2));
+        const long long tiles_each = (m_tiles + parts - 1) / parts;
+        b.ew_m_per_split = (int)std::min<long long>(tiles_each * tm, 0x7fffffc0);
+        b.ew_splits = (int)((b.m_total + b.ew_m_per_split - 1) / b.ew_m_per_split);
+    }
     // per-row scratch, each row's part padded to 64 floats so that float4 staging stays aligned
     auto pad64 = [](size_t v) { return (v + 63) & ~(size_t)63; };
     // (rows of col and of E start on 16-byte boundaries: the products that read them along a row do so four at a time)
     b.col_v = pad64((size_t)pad4(b.m_total) * K);
     b.e_v = pad64((size_t)b.m_total * pad4(2 * g.c_out));
-    b.part_v = pad64((size_t)(b.fused_k && b.fused_splits > b.splits ? b.fused_splits : b.splits) * K * 2 * g.c_out);
+    b.part_v = pad64((size_t)std::max(b.splits, b.fused_k ? b.fused_splits : b.ew_splits) * K * 2 * g.c_out);
     b.w_v = pad64((size_t)K * 2 * g.c_out);
     // the fused kernel needs neither col nor E
     const size_t col_alloc = b.fused_k ? 0 : b.col_v, e_alloc = b.fused_k ? 0 : b.e_v;
@@ -3186,11 +3475,11 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             if (gw) {
                 // few partial sums (wide layers): coalesced tiles; many: the kernel that adds eight splits side by side
                 if (L.fused_splits <= 4)
-                    hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, L.fused_splits,
-                                       g.c_out, G, L.part_v, WgradOperands{});
+                    hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv,
+                                       WgradSplits{L.fused_splits, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
                 else
                     hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                       L.fused_splits, g.c_out, G, L.part_v, WgradOperands{});
+                                       WgradSplits{L.fused_splits, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
             }
             if (gx && L.dcol_slices > 1)
                 hipLaunchKernelGGL(k_sum_slices, dim3(grid1d((long long)((size_t)nv * L.col_v / 4))), dim3(256), 0, s, dcol,
@@ -3261,6 +3550,34 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
         q1.a_batch_stride = (long long)L.col_v; q1.b_batch_stride = (long long)L.w_v;
         q1.c_batch_stride = (long long)L.e_v;
         q1.g = g_planes ? gy : gt; q1.g_planes = g_planes; q1.c_out = g.c_out; q1.npos = g.wo * g.ho;
+        const bool ew = gw && L.ew_splits;
+        if (ew) {
+            // E and the partial sums of the weight gradient at once where the operands are one term
+            EwParams p = {};
+            p.col = (const bf16_bits*)col; p.wcat = wcat; p.g = g_planes ? gy : gt; p.e = e; p.part = part; p.one_term = one_term;
+            p.rows = view ? view_rows : nullptr; p.rows_batch = L.view_k_pad; p.item = g.wo * g.ho; p.skip = (g.w_k - 1) * g.ho;
+            p.col_ld = col_ld; p.col_v = L.col_v; p.w_v = L.w_v; p.e_v = L.e_v; p.part_v = L.part_v;
+            p.M = M; p.K = K; p.J = J; p.e_ld = e_ld; p.c_out = g.c_out; p.npos = g.wo * g.ho;
+            p.m_per_split = L.ew_m_per_split; p.jtiles = (J + 127) / 128;
+            const dim3 grid((unsigned)(L.ew_splits * p.jtiles), nv);
+            auto launch = [&](auto blocks) {
+                constexpr int B = decltype(blocks)::value;
+                if (J <= 64)  // (never the gradient as it is: whole tiles of 128 columns)
+                    hipLaunchKernelGGL((k_bwd_e_wgrad<B, 2, false>), grid, dim3(256), 0, s, p);
+                else if (g_planes)
+                    hipLaunchKernelGGL((k_bwd_e_wgrad<B, 4, true>), grid, dim3(256), 0, s, p);
+                else
+                    hipLaunchKernelGGL((k_bwd_e_wgrad<B, 4, false>), grid, dim3(256), 0, s, p);
+            };
+            switch ((K + 31) / 32) {
+            case 2: launch(std::integral_constant<int, 2>()); break;
+            case 3: launch(std::integral_constant<int, 3>()); break;
+            case 4: launch(std::integral_constant<int, 4>()); break;
+            case 5: launch(std::integral_constant<int, 5>()); break;
+            default: launch(std::integral_constant<int, 6>()); break;
+            }
+            q1.one_term_elsewhere = 1;
+        }
         q1.a_rows = view_rows; q1.a_rows_batch = L.view_k_pad; q1.a_item = g.wo * g.ho; q1.a_skip = (g.w_k - 1) * g.ho;
         rc = view ? launch_gemm<true, true, EPI_EXP_TIMES_G, PRODUCT_E, true>(q1, nv, s)
                   : launch_gemm<true, true, EPI_EXP_TIMES_G, PRODUCT_E>(q1, nv, s);
@@ -3269,6 +3586,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             // partial Gw[v][s][k][j] = sum_{m in split s} col_v[k][m] * E_v[m][j]
             GemmParams q2 = {};
             q2.one_term = one_term;
+            q2.one_term_elsewhere = ew;
             q2.a = col; q2.b = e; q2.c = part;
             q2.I = K; q2.J = J; q2.K = M;
             q2.lda = col_ld; q2.ldb = e_ld; q2.ldc = J;
@@ -3285,12 +3603,13 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             // the other kernel reads w and writes dL/dw one element per line).  Not where eight splits side by side are
             // what fills the GPU.
             const dim3 w_tiles((g.c_in * g.w_k * g.h_k + 31) / 32, (g.c_out + 31) / 32);
-            if (L.splits <= 8 && (long long)w_tiles.x * w_tiles.y >= 512 && w_tiles.y <= 65535)
-                hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, L.splits, g.c_out,
-                                   G, L.part_v, again);
+            const WgradSplits parts = {L.splits, L.ew_splits, ew ? one_term : nullptr};
+            if (std::max(L.splits, L.ew_splits) <= 8 && (long long)w_tiles.x * w_tiles.y >= 512 && w_tiles.y <= 65535)
+                hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, parts,
+                                   g.c_out, G, L.part_v, again);
             else
-                hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                   L.splits, g.c_out, G, L.part_v, again);
+                hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0, parts,
+                                   g.c_out, G, L.part_v, again);
         }
         if (!gx) continue;
         if (dx_taps) {
