@@ -75,6 +75,7 @@ C_API = {
     "geo_sc_quantize_many": (ctypes.c_int, [ctypes.c_int, _P, _P, _P, ctypes.c_int, _P]),
     "geo_sc_copy_back_clamp": (ctypes.c_int, [ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, ctypes.c_float, _P]),
     "geo_sc_conv2d_add_partial_forward_q7": (ctypes.c_int, [_D, _P, _P, _P, _P, ctypes.c_size_t, _P]),
+    "geo_sc_counts_to_values": (ctypes.c_int, [_P, ctypes.c_size_t, ctypes.c_int, _P]),
     "geo_sc_quantize": (ctypes.c_int, [_P, _P, ctypes.c_size_t, ctypes.c_int, _P]),
     "geo_sc_weight_streams_finish": (ctypes.c_int, [_D, _P, _P]),
     "geo_sc_weight_streams_check": (ctypes.c_int, [_D, _P, _P]),

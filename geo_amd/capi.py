@@ -119,6 +119,19 @@ def conv2d_add_partial_forward(x, w, bit_length, padding=(0, 0), total_width=7, 
     return out
 
 
+def conv2d_add_partial_values(x, w, desc: ConvDesc, bit_length, stream=None):
+    """The forward's counts over ``bit_length`` as fp32: counts into the result's memory, then one pass in place
+    (geo_sc_counts_to_values)."""
+    _require_gpu_f32(x, "x")
+    _require_gpu_f32(w, "w")
+    workspace = torch.empty(workspace_size(desc), dtype=torch.uint8, device=x.device)
+    y = torch.empty(output_shape(desc), dtype=torch.float32, device=x.device)
+    conv2d_add_partial_forward(x, w, bit_length, out=y, workspace=workspace, desc=desc, stream=stream)
+    _check(_native.lib().geo_sc_counts_to_values(_ptr(y), y.numel(), int(bit_length), _stream_ptr(stream)),
+           "geo_sc_counts_to_values")
+    return y
+
+
 def static_workspace_bytes() -> int:
     """Size of the library's static device workspace (geo_sc_static_workspace_bytes)."""
     return int(_native.lib().geo_sc_static_workspace_bytes())

@@ -65,8 +65,9 @@ class _SCConv2dAddPartial(torch.autograd.Function):
         z_unit = max(1, min(int(z_unit), x.shape[1]))
         if generator != "lfsr":
             loading = dict(capi.NEUTRAL_LOADING)  # the random generators have no progressive loading
-        counts = capi.conv2d_add_partial_forward(x, w, int(bit_length), pad, accumulate=accumulate, z_unit=z_unit,
-                                                 generator=generator, seed=seed, **loading)
+        desc = capi.make_desc(x.shape, w.shape, int(bit_length), pad, accumulate=accumulate, z_unit=z_unit,
+                              generator=generator, seed=seed, **loading)
+        values = capi.conv2d_add_partial_values(x, w, desc, int(bit_length))
         ctx.save_for_backward(x, w)
         ctx.accumulate = accumulate
         ctx.z_unit = z_unit
@@ -76,8 +77,7 @@ class _SCConv2dAddPartial(torch.autograd.Function):
         ctx.act_dtype = activation.dtype
         ctx.w_dtype = weight.dtype
         ctx.w_device = weight.device
-        # int32 * python float -> float32 in one kernel; exact, the length is a power of two
-        return (counts * (1.0 / bit_length)).to(origin)
+        return values.to(origin)
 
     @staticmethod
     def backward(ctx, grad_out):

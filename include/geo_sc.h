@@ -403,6 +403,9 @@ GEO_SC_API int geo_sc_bn_fixed_eval_mean(const float* x, int n, int c, int plane
  * and to weight_org on every call (utils_class.py:32-33).  n fp32 elements on the device; dst may be src.
  */
 GEO_SC_API int geo_sc_quantize(const float* src, float* dst, size_t n, int prec, geo_sc_stream_t stream);
+/* Counts as the layer's values, in place: the n int32 at y become the fp32 numbers count * (1 / bit_length)
+ * (utils_functional.py:497-513 divide what the op returns). */
+GEO_SC_API int geo_sc_counts_to_values(int32_t* y, size_t n, int bit_length, geo_sc_stream_t stream);
 /* The same for `count` tensors in one launch per 24 of them (the weight_org buffers of all layers of a network
  * at the start of a forward): src, dst and elements are HOST arrays of `count` entries, the tensors are on the
  * device; a tensor of no elements may have null pointers. */

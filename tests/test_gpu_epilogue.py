@@ -374,6 +374,29 @@ def test_quantize_kernel_equals_the_torch_op_chain():
     assert capi.quantize(torch.empty(0, device="cuda"), 7).numel() == 0
 
 
+@pytest.mark.parametrize("offset", [0, 1, 2])
+@pytest.mark.parametrize("n", [1, 3, 4, 7, 1023, 2048, 2049, 4101, 8391687])
+def test_passes_in_quads_at_their_edges(n, offset):
+    """quantize and counts as values: remainders of a quad, of the two quads of a trip and of the grid, memory off a
+    16-byte boundary, and nothing written beyond the end."""
+    import ctypes
+    from geo_amd import _native, capi
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n + offset + 5, generator=g, device="cuda")
+    out = torch.full_like(x, 9.0)
+    capi.quantize(x[offset:offset + n], 7, out=out[offset:offset + n])
+    ref = torch.full_like(x, 9.0)
+    ref[offset:offset + n] = (x[offset:offset + n] * 128).round().clamp(-127, 127) / 128
+    assert torch.equal(out, ref)
+    counts = torch.randint(-2 ** 26, 2 ** 26, (n + offset + 5,), generator=g, device="cuda", dtype=torch.int32)
+    y = counts.clone()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    status = _native.lib().geo_sc_counts_to_values(ctypes.c_void_p(y.data_ptr() + 4 * offset), n, 256, stream)
+    assert status == 0
+    assert torch.equal(y[offset:offset + n].view(torch.float32), counts[offset:offset + n] * (1.0 / 256))
+    assert torch.equal(y[:offset], counts[:offset]) and torch.equal(y[offset + n:], counts[offset + n:])
+
+
 def test_quantize_many_equals_quantize_per_tensor(capi):
     """geo_sc_quantize_many: every tensor of the list as geo_sc_quantize gives it (odd sizes, an empty one, more
     tensors than one launch takes)."""
