@@ -1514,44 +1514,45 @@ __device__ __forceinline__ bool operands_are_bf16(const int* __restrict__ found,
 // Per output position m = (n, a, b): where its receptive field starts in the unpadded input.
 //   base[m] = ((n*c_in)*w_in + (a - pad_w))*h_in + (b - pad_h),  arow[m] = a - pad_w,  bcol[m] = b - pad_h
 // Built once per call; it keeps integer divisions out of the per-element kernels.
-// With `found`, the first block also turns what scan_operands found into *one_term.
-// With scan_x, rows of blocks behind the first scan x_total elements of x.
-__global__ __launch_bounds__(256) void k_position_table(int* __restrict__ base, int* __restrict__ arow,
-                                                        int* __restrict__ bcol, const int* __restrict__ found, int found_rows,
-                                                        int* __restrict__ one_term, const float* __restrict__ scan_x,
-                                                        long long x_total, int* __restrict__ scan_found, int m_total,
-                                                        int c_in, int c_out, int w_in, int h_in, int pad_w, int pad_h,
-                                                        int wo, int ho)
+struct PositionTable {
+    int* base;
+    int* arow;
+    int* bcol;
+    int m_total, c_in, w_in, h_in, pad_w, pad_h, wo, ho;
+    // by `blocks` blocks of 256
+    __device__ __forceinline__ void fill(int block, int blocks) const
+    {
+        for (int m = block * 256 + threadIdx.x; m < m_total; m += blocks * 256) {
+            const int b = m % ho;
+            const int t = m / ho;
+            const int a = t % wo;
+            const int n = t / wo;
+            base[m] = ((n * c_in) * w_in + (a - pad_w)) * h_in + (b - pad_h);
+            arow[m] = a - pad_w;
+            bcol[m] = b - pad_h;
+        }
+    }
+};
+// For the fused kernels; rows of blocks behind the first scan x_total elements of x.
+__global__ __launch_bounds__(256) void k_position_table(PositionTable p, const float* __restrict__ scan_x, long long x_total,
+                                                        int* __restrict__ scan_found)
 {
-    if (blockIdx.y > 0) {
-        if (blockIdx.x < kScanBlocks)
-            scan_operands(scan_x, x_total, nullptr, 0, (blockIdx.y - 1) * kScanBlocks + blockIdx.x, (gridDim.y - 1) * kScanBlocks,
-                          scan_found);
-        return;
-    }
-    if (found && blockIdx.x == 0) {
-        const bool one = operands_are_bf16(found, found_rows);
-        if (threadIdx.x == 0) *one_term = one;
-    }
-    for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
-        const int b = m % ho;
-        const int t = m / ho;
-        const int a = t % wo;
-        const int n = t / wo;
-        base[m] = ((n * c_in) * w_in + (a - pad_w)) * h_in + (b - pad_h);
-        arow[m] = a - pad_w;
-        bcol[m] = b - pad_h;
-    }
+    if (blockIdx.y == 0)
+        p.fill(blockIdx.x, gridDim.x);
+    else if (blockIdx.x < kScanBlocks)
+        scan_operands(scan_x, x_total, nullptr, 0, (blockIdx.y - 1) * kScanBlocks + blockIdx.x, (gridDim.y - 1) * kScanBlocks,
+                      scan_found);
 }
 
 // col[g][k][m] = x~[n, ci, a+u, b+v] for groups g0 + blockIdx.z, (ci, u, v) = member k of the
 // group, m = (n, a, b); x~ is the zero-padded activation, read straight from the unpadded
 // tensor.  blockIdx.y selects kIm2colMembers consecutive members; a thread reads its position's
-// table entry once and moves those members.  Reads and writes run along m; rows are ld elements apart.  Where *one_term
-// says that x holds bf16 numbers, so does col.
+// table entry once and moves those members.  Reads and writes run along m; rows are ld elements apart.  Where x and w hold
+// bf16 numbers, so does col, which the first block tells the products (*one_term).
 constexpr int kIm2colMembers = 12;
 __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x, float* __restrict__ col,
-                                                     const int* __restrict__ one_term,
+                                                     const int* __restrict__ found, int found_rows,
+                                                     int* __restrict__ one_term,
                                                      const int* __restrict__ base, const int* __restrict__ arow,
                                                      const int* __restrict__ bcol, int g0, int m_total, int ld,
                                                      Groups G, int w_in, int h_in, size_t g_stride)
@@ -1560,7 +1561,8 @@ __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x
     const int k0 = blockIdx.y * kIm2colMembers;
     const int k1 = min(G.n_members, k0 + kIm2colMembers);
     float* colg = col + (size_t)blockIdx.z * g_stride;
-    const bool bf16_col = *one_term != 0;
+    const bool bf16_col = operands_are_bf16(found, found_rows);
+    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
     for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
         // all loads first, from x[0] where the member lies in the padding (a load inside a branch is
@@ -1605,7 +1607,8 @@ __device__ __forceinline__ float4 shifted_quad(const float4& a, const float4& b,
 // quads (the kernel tap shifts them by v - pad_h) and stored as one quad: a quarter of the loads,
 // stores and table reads of the one-position kernel.
 __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict__ x, float* __restrict__ col,
-                                                        const int* __restrict__ one_term,
+                                                        const int* __restrict__ found, int found_rows,
+                                                        int* __restrict__ one_term,
                                                         const int* __restrict__ base, const int* __restrict__ arow,
                                                         const int* __restrict__ bcol, int g0, int m_total, Groups G,
                                                         int w_in, int h_in, size_t g_stride)
@@ -1616,7 +1619,8 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
     float* colg = col + (size_t)blockIdx.z * g_stride;
     const float4* x4 = (const float4*)x;
     const int quads = m_total >> 2;
-    const bool bf16_col = *one_term != 0;
+    const bool bf16_col = operands_are_bf16(found, found_rows);
+    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
     for (int mq = blockIdx.x * 256 + threadIdx.x; mq < quads; mq += gridDim.x * 256) {
         const int m = mq << 2;
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
@@ -2060,7 +2064,8 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restr
 //  * from the blocks of the round's first group: view_rows[g][k], where row k of group g's col starts in the
 //    planes of k_shift_planes (elements), for every group; and 64 zeros for the shifted view of E (a store
 //    rather than a memset, so that a caller may capture the launch sequence in a graph);
-//  * in rows of blocks of their own behind the groups': the scan of x and w.
+//  * in rows of blocks of their own behind the groups': the scan of x and w, and in the last row, if there is one more,
+//    the position table (a launch less in front of im2col: 4 us).
 struct PrepParams {
     const float* __restrict__ w;
     float* __restrict__ wcat;
@@ -2078,11 +2083,17 @@ struct PrepParams {
     const float* __restrict__ x;
     long long x_total, w_total;
     int* found;             // what the scan's blocks found
+    PositionTable positions;  // m_total 0: none wanted
 };
-// what is no weight operand: the scan's blocks (true: the block is one of them), the view's row table, the zeros
+// what is no weight operand: the blocks of the scan and the positions (true: the block is one of them), the view's row
+// table, the zeros
 __device__ __forceinline__ bool prep_scans(const PrepParams& q)
 {
     if ((int)blockIdx.y < q.groups) return false;
+    if ((int)blockIdx.y == q.groups + q.scan_rows) {
+        q.positions.fill(blockIdx.x, gridDim.x);
+        return true;
+    }
     scan_operands(q.x, q.x_total, q.w, q.w_total, (blockIdx.y - q.groups) * kScanBlocks + blockIdx.x, q.scan_rows * kScanBlocks,
                   q.found);
     return true;
@@ -3268,7 +3279,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     if (rows > (size_t)b.G.n_groups) rows = b.G.n_groups;
     // the caller's cap on the add groups per round (less scratch, more launches)
     if (groups_per_round >= 1 && (size_t)groups_per_round < rows) rows = (size_t)groups_per_round;
-    if (rows * b.splits > 65535 - kScanRows) rows = (65535 - kScanRows) / b.splits;  // grid.y = rows and the scan's, grid.z = rows * splits
+    if (rows * b.splits > 65534 - kScanRows) rows = (65534 - kScanRows) / b.splits;  // grid.y = rows, the scan's and the positions', grid.z = rows * splits
     if (rows < 1) rows = 1;
     b.rows_per_chunk = (int)rows;
     // col as a view: whole quads in every row on both sides, chunks of kChunk positions inside one item, an
@@ -3366,13 +3377,13 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
     int* one_term = found + kScanBlocks * kScanRows;
     const int n_scan_rows = scan_rows(x_total);
     // the position tables serve the gathers of im2col and of the fused kernels
-    auto position_tables = [&](const int* scanned, int scan_x_rows) {
-        const dim3 grid(scan_x_rows ? std::max(m_blocks, kScanBlocks) : m_blocks, 1 + scan_x_rows);
-        hipLaunchKernelGGL(k_position_table, grid, dim3(256), 0, s, pos_base, pos_arow, pos_bcol, scanned, n_scan_rows, one_term, x,
-                           x_total, found, M, g.c_in, g.c_out, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho);
-    };
-    // (the kernel for up to 16 members takes operands of one term as such)
-    if (fused) position_tables(nullptr, K <= 16 ? n_scan_rows : 0);
+    const PositionTable positions = {pos_base, pos_arow, pos_bcol, M, g.c_in, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho};
+    if (fused) {
+        // (the kernel for up to 16 members takes operands of one term as such)
+        const int rows = K <= 16 ? n_scan_rows : 0;
+        hipLaunchKernelGGL(k_position_table, dim3(rows ? std::max(m_blocks, kScanBlocks) : m_blocks, 1 + rows), dim3(256), 0, s,
+                           positions, x, x_total, found);
+    }
     // Where the first product reads col as a view and its tiles are whole (the eight-wave kernel in every round,
     // or the 128 x 128 kernel), its epilogue reads the upstream gradient as it is (items of whole 32-position
     // blocks, 16-byte aligned): no transposed copy.
@@ -3512,19 +3523,20 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                 pp.x = x; pp.x_total = x_total; pp.w_total = (long long)g.c_out * g.c_in * g.w_k * g.h_k; pp.found = found;
                 pp.scan_rows = n_scan_rows;
                 wb = kScanBlocks;
+                if (!view) pp.positions = positions;
             }
+            const int more_rows = pp.scan_rows + (pp.positions.m_total ? 1 : 0);
             const bool ragged = G.mode == GEO_SC_ACC_YZ && g.c_in % G.zu != 0;
             const int channels = ragged ? 0 : prep_tile_channels(g.c_in, g.c_out, g.w_k * g.h_k);
             if (channels) {
                 const long long tiles = (long long)((g.c_out + 31) / 32) * ((g.c_in + channels - 1) / channels);
                 pp.groups = (int)std::min<long long>((tiles + kScanBlocks - 1) / kScanBlocks, 8);  // rows of tiles
-                hipLaunchKernelGGL(k_bwd_prep_tiled, dim3(kScanBlocks, pp.groups + pp.scan_rows), dim3(256), 0, s, pp, nv,
+                hipLaunchKernelGGL(k_bwd_prep_tiled, dim3(kScanBlocks, pp.groups + more_rows), dim3(256), 0, s, pp, nv,
                                    __builtin_ctz((unsigned)channels));
             } else {
-                hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + pp.scan_rows), dim3(256), 0, s, pp);
+                hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + more_rows), dim3(256), 0, s, pp);
             }
         }
-        if (!view && v0 == 0) position_tables(found, 0);
         if (view) {
             const long long plane = (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho;
             const long long quads = (long long)g.h_k * g.c_in * plane / 4;
@@ -3534,11 +3546,11 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             const int q_blocks = grid1d(M / 4);
             hipLaunchKernelGGL(k_im2col_rows_v4,
                                dim3(q_blocks > 1024 ? 1024 : q_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
-                               dim3(256), 0, s, x, col, one_term, pos_base, pos_arow, pos_bcol, v0, M, G, g.w_in, g.h_in, L.col_v);
+                               dim3(256), 0, s, x, col, found, n_scan_rows, one_term, pos_base, pos_arow, pos_bcol, v0, M, G, g.w_in, g.h_in, L.col_v);
         } else {
             hipLaunchKernelGGL(k_im2col_rows,
                                dim3(m_blocks > 1024 ? 1024 : m_blocks, (K + kIm2colMembers - 1) / kIm2colMembers, nv),
-                               dim3(256), 0, s, x, col, one_term, pos_base, pos_arow, pos_bcol, v0, M, col_ld, G, g.w_in, g.h_in, L.col_v);
+                               dim3(256), 0, s, x, col, found, n_scan_rows, one_term, pos_base, pos_arow, pos_bcol, v0, M, col_ld, G, g.w_in, g.h_in, L.col_v);
         }
         // E[v][m][j] = g * exp(-(col_v^T . wcat_v)), col stored [K][M]
         GemmParams q1 = {};
