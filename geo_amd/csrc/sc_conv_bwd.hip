@@ -1097,7 +1097,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // back; it is stored for the input gradient, and the same bits as the first product stores.
 // A workgroup is persistent: 4 waves, one group, NWJ * 32 columns, one part of the positions in tiles of 32 (64 where two
 // waves cover the columns: the halves' sums meet at the end); col's next tile is loaded while this one is multiplied.
-// 64 -> 64 at 56 x 56, batch 128: 314 us, the two products 354 + 306; without the stores of E it takes 40 less, without the
+// 64 -> 64 at 56 x 56, batch 128: 314 us, the two products 354 + 306 us; without the stores of E it takes 40 less, without the
 // gradient's loads 45 less, its matrix work is 108.  Ragged layer of 77 items, 45 -> 83, blocks of 32 channels: 89, 79 + 76.
 // Three terms need three times the registers: those operands take the two products (which return at once otherwise).
 struct EwParams {
@@ -1112,6 +1112,7 @@ struct EwParams {
     long long col_ld;
     size_t col_v, w_v, e_v, part_v;
     int M, K, J, e_ld, c_out, npos, m_per_split, jtiles;
+    int splits, tiles_each, parts;  // partial sums as in SmallKParams
 };
 constexpr int kEwMembers = 192;     // six blocks of 32: 96 registers of sums
 constexpr int kEwWorkgroups = 512;  // two per CU
@@ -1129,7 +1130,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ long long row_at[KR];
     constexpr int GR = 128, GQ = 9;  // the gradient's rows in LDS (channels), 16-byte words per row: 8 and padding
     __shared__ floatx4 gs[2][PLANES ? GR : 1][GQ];
-    static_assert(sizeof(cs) >= 2 * 16 * 64 * sizeof(float), "room for a block's sums of two waves");
+    static_assert(NWM == 1 || sizeof(cs[0]) >= NWJ * 16 * 64 * sizeof(float), "room for a block's sums of the waves");
     if (!*q.one_term) return;
     const int group = blockIdx.y;
     const int split = blockIdx.x / q.jtiles, jt = blockIdx.x - split * q.jtiles;
@@ -1235,6 +1236,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     __syncthreads();
     constexpr int kMfma = 0x008, kDsRead = 0x100;  // of __builtin_amdgcn_sched_group_barrier
+    int part = 0, tiles_left = q.tiles_each;
+    // the sums so far into their place, through a buffer of col that nobody reads or writes meanwhile
+    auto store_part = [&](int free_buf) {
+        // (opaque to the compiler, which would keep the stores' addresses in registers over the loop)
+        int K = q.K, J = q.J;
+        asm volatile("" : "+s"(K), "+s"(J));
+        float* pg = q.part + (size_t)group * q.part_v + (size_t)(part * q.splits + split) * K * J;
+        float* meet = (float*)&cs[free_buf][0][0];  // of the waves with the tile's other half: [column block][register][lane]
+#pragma unroll
+        for (int b = 0; b < NKB; b++) {
+            if constexpr (NWM == 2) {
+                __syncthreads();
+                if (wm == 1) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) meet[(wj * 16 + r) * 64 + lane] = acc[b][r];
+                }
+                __syncthreads();
+                if (wm == 0) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[b][r] += meet[(wj * 16 + r) * 64 + lane];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int k = 32 * b + 8 * (r >> 2) + 4 * lk + (r & 3);
+                if (wm == 0 && j_ok && k < K) pg[(size_t)k * J + j] = acc[b][r];
+                acc[b][r] = 0.0f;
+            }
+        }
+        if constexpr (NWM == 2) __syncthreads();
+    };
     int buf = 0;
     for (int m0 = m_begin; m0 < m_end; m0 += TM, buf ^= 1) {
         const int mb = m0 + 32 * wm, mi = mb + 4 * lk;
@@ -1318,31 +1350,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         commit(buf ^ 1, HALVES - 1, next);
         if constexpr (PLANES) commit_planes(buf ^ 1);
         __syncthreads();
-    }
-    float* pg = q.part + (size_t)group * q.part_v + (size_t)split * q.K * q.J;
-    float* meet = (float*)&cs[0][0][0];  // sums of the waves with the tile's other half, [column block][register][lane]
-#pragma unroll
-    for (int b = 0; b < NKB; b++) {
-        if constexpr (NWM == 2) {
-            __syncthreads();
-            if (wm == 1) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) meet[(wj * 16 + r) * 64 + lane] = acc[b][r];
-            }
-            __syncthreads();
-            if (wm == 0) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[b][r] += meet[(wj * 16 + r) * 64 + lane];
-            }
-        }
-        if (wm == 0 && j_ok) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int k = 32 * b + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (k < q.K) pg[(size_t)k * q.J + j] = acc[b][r];
-            }
+        if (--tiles_left == 0) {
+            store_part(buf);
+            part++;
+            tiles_left = q.tiles_each;
         }
     }
+    for (; part < q.parts; part++) store_part(0);
 }
 
 // gt[n*npos + pos][co] = g[n][co][pos]: the upstream gradient with the channel innermost, so that the
@@ -2638,6 +2652,9 @@ struct SmallKParams {
     float* __restrict__ dcol;
     Groups G;
     int g0, M, w_in, h_in, c_out, jblocks, splits, store_part, gt_blocks, gt_dedupe, found_rows;
+    // partial sums of the weight gradient: one per `tiles_each` of a workgroup's tiles (longer sums in fp32 round more: 14
+    // items of 7 x 37, 31 -> 280, z accumulation: 2.4e-7 against float64 over 23 tiles, 1.3e-7 over 6), n of them per workgroup
+    int tiles_each, parts;
     size_t w_stride, part_stride, dcol_stride, dcol_slice;
 };
 
@@ -2674,8 +2691,8 @@ __device__ __forceinline__ bool small_k_weights(const SmallKParams& q, SmallKSha
 }
 
 // columns c0 + 32 (b NW + wave) .. + 31, b < NB, of the workgroup's (from j_begin on, weights in wl) over its tiles; ADD: to
-// the dcol that is there
-template <int TERMS, int NW, int NB, bool DX, bool ADD, typename Shared>
+// the dcol that is there; PARTS: more than one partial sum
+template <int TERMS, int NW, int NB, bool DX, bool ADD, bool PARTS, typename Shared>
 __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& sh, int split, int jblock, int j_begin, int c0)
 {
     constexpr int KP = 16, TM = kFusedTile, NT = 64 * NW;
@@ -2842,6 +2859,26 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
     const int zrow = 16 * (l16 >> 3) + (l16 & 7), ep = 16 * (lq >> 1) + 4 * (lq & 1);
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) short4v* tr_ptr;
+    int part = 0, tiles_left = q.tiles_each;
+    auto store_part = [&]() {
+        if (!q.store_part) return;
+        // (opaque to the compiler, which would keep the stores' addresses in registers over the loop)
+        int K = q.G.n_members, J = 2 * q.c_out;
+        if constexpr (PARTS) asm volatile("" : "+s"(K), "+s"(J));
+        float* pg = q.part + (size_t)blockIdx.y * q.part_stride + (size_t)(part * q.splits + split) * K * J;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const int j = j_begin + c0 + 32 * (b * NW + wave) + 16 * s + l16;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int k = 4 * lq + r;
+                    if (k < K && j < J) pg[(size_t)k * J + j] = gw_acc[b][s][r];
+                    if constexpr (PARTS) gw_acc[b][s][r] = 0.0f;
+                }
+            }
+    };
     int buf = 0;
     for (int tile = split; tile < n_tiles; tile += q.splits, buf ^= 1) {
         ok_after = fetch(w_after, x_after);
@@ -2966,21 +3003,16 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
 #pragma unroll
             for (int e = 0; e < EP; e++) x_next[gp][e] = x_after[gp][e];
         ok_next = ok_after;
+        if (PARTS && --tiles_left == 0) {
+            store_part();
+            part++;
+            tiles_left = q.tiles_each;
+        }
     }
-    if (q.store_part) {
-        float* pg = q.part + (size_t)blockIdx.y * q.part_stride + (size_t)split * K * J;
-#pragma unroll
-        for (int b = 0; b < NB; b++)
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                const int j = j_begin + c0 + 32 * (b * NW + wave) + 16 * s + l16;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int k = 4 * lq + r;
-                    if (k < K && j < J) pg[(size_t)k * J + j] = gw_acc[b][s][r];
-                }
-            }
-    }
+    if constexpr (PARTS)
+        for (; part < q.parts; part++) store_part();
+    else
+        store_part();
 }
 
 template <int NW, int NB, bool DX>
@@ -2993,16 +3025,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8
     bool three = small_k_weights(q, sh, j_begin);
     for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
     if (!__syncthreads_or(three)) {
-        small_k_columns<1, NW, NB, DX, false>(q, sh, split, jblock, j_begin, 0);
+        small_k_columns<1, NW, NB, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
         return;
     }
-    small_k_columns<3, NW, 1, DX, false>(q, sh, split, jblock, j_begin, 0);
+    small_k_columns<3, NW, 1, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
     if constexpr (NB > 1) {
         static_assert(NB == 2, "one more pass");
         __syncthreads();
         small_k_weights(q, sh, j_begin);
         __syncthreads();
-        small_k_columns<3, NW, 1, DX, true>(q, sh, split, jblock, j_begin, 32 * NW);
+        small_k_columns<3, NW, 1, DX, true, false>(q, sh, split, jblock, j_begin, 32 * NW);
     }
 }
 
@@ -3152,10 +3184,11 @@ struct BwdLayout {
     int fused_jw;        // columns of E per workgroup of that kernel
     int fused_jblocks;   // its column blocks: each writes a dcol slice of its own
     int fused_splits;    // its workgroups per add group and column block
+    int fused_tiles_each, fused_parts;  // of the bf16 kernel: tiles in a partial sum, partial sums per workgroup
     int gt_dedupe;       // its upstream-gradient tiles serve both rails (c_out a multiple of 32)
     int gt_blocks;       // 32-column blocks of those tiles
     int ew_splits;       // parts of the positions in k_bwd_e_wgrad; 0: more members than it takes
-    int ew_m_per_split;
+    int ew_m_per_split, ew_tiles_each, ew_parts;  // tiles in a partial sum, partial sums per part of the positions
     int rows_per_chunk;  // add groups processed by one round of launches
     int dcol_slices;     // partial dcol arrays per round (column blocks of the fused kernel), rows_per_chunk * col_v apart
     bool dx_rows;        // the input-gradient GEMM sums the kernel rows itself (E read as a view shifted by image rows)
@@ -3204,11 +3237,11 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     b.fused_k = K <= kFusedK;
     // the bf16 kernel (at most 16 members) comes with 2, 4 or 8 waves of 32 columns, or 8 of 64 where under four of the
     // waves' 16 blocks stay empty (with 260 columns, operands of three terms: 417 us against 398 of 256-wide ones for
-    // 64 -> 130 at 20 x 20, z_unit 4, batch 32) and a workgroup gets eight tiles (512 channels, 37 groups, batch 100:
-    // 109 against 97); the fp32 one with 128 or 256 columns
+    // 64 -> 130 at 20 x 20, z_unit 4, batch 32) and the groups alone are two rounds of workgroups (otherwise three terms lose
+    // more than one wins: 5 -> 250 at 28 x 28, batch 64: 405 us against 367); the fp32 one with 128 or 256 columns
     const long long fused_tiles = (b.m_total + kFusedTile - 1) / kFusedTile;
     const bool wide = K <= 16 && (512 - 2 * g.c_out % 512) % 512 < 128 &&
-                      fused_tiles * b.G.n_groups * ((2 * g.c_out + 511) / 512) >= 8 * 512;
+                      (long long)b.G.n_groups * ((2 * g.c_out + 511) / 512) >= 1024;
     b.fused_jw = 2 * g.c_out <= 64 && K <= 16 ? 64 : 2 * g.c_out <= 128 ? 128 : wide ? 512 : 256;
     b.fused_jblocks = (2 * g.c_out + b.fused_jw - 1) / b.fused_jw;
     b.gt_dedupe = g.c_out % 32 == 0;
@@ -3224,10 +3257,11 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
             // 2048 workgroups whatever their tiles 12 -> 200 took 289, now 137
             const long long at_once = b.fused_jw == 64 ? 1536 : b.fused_jw == 128 ? 768 : 512;
             long long least = 0;
+            // (64 columns per wave: one workgroup per group and block, one partial sum)
             for (int rounds = 1; rounds <= 4; rounds++) {
                 const long long splits = std::max(1LL, std::min(n_tiles, at_once * rounds / per_split));
                 const long long cost = (splits * per_split + at_once - 1) / at_once * (2 + (n_tiles + splits - 1) / splits);
-                if (rounds == 1 || cost < least) {
+                if (!least || cost < least) {
                     least = cost;
                     want = splits;
                 }
@@ -3236,6 +3270,11 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
         if (want > n_tiles) want = n_tiles;
         if (want > 65535) want = 65535;
         b.fused_splits = (int)(want < 1 ? 1 : want);
+        // (sums no longer than eight workgroups per CU would form)
+        const long long most = std::max(1LL, std::min(n_tiles, 2048 / per_split));
+        const long long each_wg = (n_tiles + b.fused_splits - 1) / b.fused_splits;
+        b.fused_tiles_each = K > 16 ? 0 : b.fused_jw == 512 ? (int)each_wg : (int)std::min(each_wg, (n_tiles + most - 1) / most);
+        b.fused_parts = K <= 16 ? (int)((each_wg + b.fused_tiles_each - 1) / b.fused_tiles_each) : 1;
     }
     // split the m-reduction of the weight gradient so that all groups' tiles together make about one
     // round of workgroups: three per CU for the 128 x 128 kernel (more splits only add partial sums to write
@@ -3253,7 +3292,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     b.m_per_split = (int)(per > 0x7fffffffLL ? 0x7fffffffLL : per);
     b.splits = (int)((b.m_total + b.m_per_split - 1) / b.m_per_split);
     // one round of persistent workgroups for E and the weight gradient of operands of one term
-    b.ew_splits = b.ew_m_per_split = 0;
+    b.ew_splits = b.ew_m_per_split = b.ew_tiles_each = b.ew_parts = 0;
     if (!b.fused_k && K <= kEwMembers) {
         const int tm = 2 * g.c_out <= 64 ? 64 : 32;
         const long long jtiles = (2 * g.c_out + 127) / 128, m_tiles = (b.m_total + tm - 1) / tm;
@@ -3261,13 +3300,16 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
         const long long tiles_each = (m_tiles + parts - 1) / parts;
         b.ew_m_per_split = (int)std::min<long long>(tiles_each * tm, 0x7fffffc0);
         b.ew_splits = (int)((b.m_total + b.ew_m_per_split - 1) / b.ew_m_per_split);
+        // (sums over no more positions than those of the weight gradient's own product)
+        b.ew_tiles_each = (int)std::min<long long>(tiles_each, std::max(1, b.m_per_split / tm));
+        b.ew_parts = (int)((tiles_each + b.ew_tiles_each - 1) / b.ew_tiles_each);
     }
     // per-row scratch, each row's part padded to 64 floats so that float4 staging stays aligned
     auto pad64 = [](size_t v) { return (v + 63) & ~(size_t)63; };
     // (rows of col and of E start on 16-byte boundaries: the products that read them along a row do so four at a time)
     b.col_v = pad64((size_t)pad4(b.m_total) * K);
     b.e_v = pad64((size_t)b.m_total * pad4(2 * g.c_out));
-    b.part_v = pad64((size_t)std::max(b.splits, b.fused_k ? b.fused_splits : b.ew_splits) * K * 2 * g.c_out);
+    b.part_v = pad64((size_t)std::max(b.splits, b.fused_k ? b.fused_splits * b.fused_parts : b.ew_splits * b.ew_parts) * K * 2 * g.c_out);
     b.w_v = pad64((size_t)K * 2 * g.c_out);
     // the fused kernel needs neither col nor E
     const size_t col_alloc = b.fused_k ? 0 : b.col_v, e_alloc = b.fused_k ? 0 : b.e_v;
@@ -3461,6 +3503,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
                 if (ks <= 8) {
                     SmallKParams p = {x, wcat, gt, pos_base, pos_arow, pos_bcol, found, part, dcol, G, v0, M, g.w_in, g.h_in,
                                       g.c_out, L.fused_jblocks, L.fused_splits, gw ? 1 : 0, L.gt_blocks, L.gt_dedupe, n_scan_rows,
+                                      L.fused_tiles_each, L.fused_parts,
                                       L.w_v, L.part_v, L.col_v, slice};
                     auto launch = [&](auto dx) {
                         constexpr bool DX = decltype(dx)::value;
@@ -3485,12 +3528,12 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             }
             if (gw) {
                 // few partial sums (wide layers): coalesced tiles; many: the kernel that adds eight splits side by side
-                if (L.fused_splits <= 4)
+                if (L.fused_splits * L.fused_parts <= 4)
                     hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv,
-                                       WgradSplits{L.fused_splits, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
+                                       WgradSplits{L.fused_splits * L.fused_parts, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
                 else
                     hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                       WgradSplits{L.fused_splits, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
+                                       WgradSplits{L.fused_splits * L.fused_parts, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
             }
             if (gx && L.dcol_slices > 1)
                 hipLaunchKernelGGL(k_sum_slices, dim3(grid1d((long long)((size_t)nv * L.col_v / 4))), dim3(256), 0, s, dcol,
@@ -3571,6 +3614,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             p.col_ld = col_ld; p.col_v = L.col_v; p.w_v = L.w_v; p.e_v = L.e_v; p.part_v = L.part_v;
             p.M = M; p.K = K; p.J = J; p.e_ld = e_ld; p.c_out = g.c_out; p.npos = g.wo * g.ho;
             p.m_per_split = L.ew_m_per_split; p.jtiles = (J + 127) / 128;
+            p.splits = L.ew_splits; p.tiles_each = L.ew_tiles_each; p.parts = L.ew_parts;
             const dim3 grid((unsigned)(L.ew_splits * p.jtiles), nv);
             auto launch = [&](auto blocks) {
                 constexpr int B = decltype(blocks)::value;
@@ -3615,8 +3659,8 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             // the other kernel reads w and writes dL/dw one element per line).  Not where eight splits side by side are
             // what fills the GPU.
             const dim3 w_tiles((g.c_in * g.w_k * g.h_k + 31) / 32, (g.c_out + 31) / 32);
-            const WgradSplits parts = {L.splits, L.ew_splits, ew ? one_term : nullptr};
-            if (std::max(L.splits, L.ew_splits) <= 8 && (long long)w_tiles.x * w_tiles.y >= 512 && w_tiles.y <= 65535)
+            const WgradSplits parts = {L.splits, L.ew_splits * L.ew_parts, ew ? one_term : nullptr};
+            if (std::max(L.splits, L.ew_splits * L.ew_parts) <= 8 && (long long)w_tiles.x * w_tiles.y >= 512 && w_tiles.y <= 65535)
                 hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv, parts,
                                    g.c_out, G, L.part_v, again);
             else

@@ -543,6 +543,8 @@ ONE_TERM_SHAPES = [
     ((7, 45, 27, 19), (43, 45, 3, 3), 1, "yz", 16),    # im2col, ragged channel blocks
     ((5, 40, 7, 9), (30, 40, 3, 3), 1, "full", 1),     # one group of 360 members
     ((3, 12, 5, 3), (5, 12, 3, 1), 0, "y", 1),         # rows that are no whole quads
+    ((40, 64, 24, 24), (60, 64, 3, 3), 1, "y", 1),     # 192 members, 120 columns, several partial sums per workgroup
+    ((130, 33, 17, 16), (20, 33, 1, 1), 0, "y", 1),    # 33 members, 40 columns: the halves of a tile's sums meet
     ((8, 24, 4, 4), (40, 24, 4, 4), 0, "y", 1),        # one output position per item: partial chunks of rows of bf16
 ]
 
@@ -657,10 +659,12 @@ SMALL_GROUPS = [
     ((1, 3, 1, 5), (5, 3, 1, 5), 0, "y", 1),        # one position, 10 of 64 columns
     ((33, 16, 1, 6), (33, 16, 1, 6), 0, "y", 1),    # 33 positions, 66 of 128 columns
     ((2, 3, 9, 11), (64, 3, 5, 5), 2, "y", 1),      # 15 members, 128 columns
-    ((3, 7, 6, 6), (130, 7, 3, 3), 1, "z", 1),      # 9 members, 260 of 512 columns in two sets of 256
-    ((31, 16, 1, 4), (200, 16, 1, 4), 0, "y", 1),   # 31 positions, 400 of 512 columns
+    ((3, 7, 6, 6), (130, 7, 3, 3), 1, "z", 1),      # 9 members, 260 columns in sets of 256
+    ((31, 16, 1, 4), (200, 16, 1, 4), 0, "y", 1),   # 31 positions, 400 columns
     ((65, 16, 1, 3), (256, 16, 1, 3), 0, "y", 1),   # 512 columns, whole tiles and one position
-    ((40, 6, 4, 4), (500, 6, 3, 3), 1, "yz", 4),    # 12 members, ragged channel blocks, two sets of 512 columns
+    ((40, 6, 4, 4), (500, 6, 3, 3), 1, "yz", 4),    # 12 members, ragged channel blocks
+    ((33, 2, 1, 520), (500, 2, 1, 520), 0, "y", 1), # two blocks of columns per wave, 1000 columns in sets of 512
+    ((40, 3, 40, 40), (20, 3, 3, 3), 1, "y", 1),    # several partial sums per workgroup
 ]
 
 
