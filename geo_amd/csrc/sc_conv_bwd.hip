@@ -2635,7 +2635,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // have), and adds to the dcol of the first.  4096 x 4096 linear layer, batch 1024: 1965 us with three terms
 // throughout and E in LDS for both gradients, 1096 now, of which the vector work of E is 630 (the sum of the slices of
 // dcol, 16 with NB = 2 and 32 with NB = 1: 119 -> 62); unquantised operands, step 4.20 -> 4.17 ms; first layer of the
-// 4-layer CNN 92 -> 69, half of that the gather's.
+// 4-layer CNN 92 -> 56, half of that the gather's.
 // Same grid, arguments, tiles and outputs as k_bwd_small_k.
 constexpr int kBfEw = 18;  // words per row of E^T: 32 bf16 and padding (8-byte accesses of 16 rows meet no bank twice)
 constexpr int kBfCw = 20;  // words per row of col[k][m]: 16-byte aligned rows
@@ -3254,7 +3254,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
         if (K <= 16) {
             // the bf16 kernel: the number of full rounds of workgroups that takes least, where one begins with what costs
             // it two tiles (its weights' terms).  12 -> 100, 1 x 1, 28 x 28, batch 64, step on floats: 161 us, 110; with
-            // 2048 workgroups whatever their tiles 12 -> 200 took 289, now 137
+            // 2048 workgroups whatever their tiles 12 -> 200 took 289, now 163 (182 before)
             const long long at_once = b.fused_jw == 64 ? 1536 : b.fused_jw == 128 ? 768 : 512;
             long long least = 0;
             // (64 columns per wave: one workgroup per group and block, one partial sum)
