@@ -49,13 +49,24 @@ def make_desc(x_shape, w_shape, bit_length, padding=(0, 0), total_width=7, load_
                     ctypes.c_int32(int(seed) & 0xffffffff).value)
 
 
-def make_options(forward_stream_bytes=0, backward_groups_per_round=0, forward_single_stream=False) -> Options:
+def make_options(forward_stream_bytes=0, backward_groups_per_round=0, forward_single_stream=False,
+                 backward_operand_bits=0) -> Options:
     """geo_sc_options: the budget (bytes) of the forward's activation stream buffer - a batch whose streams
     exceed it runs in chunks of items - and the cap on the add groups per round of backward launches;
     0 leaves a field at the library's default.  forward_single_stream keeps a cut batch on the caller's stream
-    (by default its odd chunks run on a second stream of the library)."""
+    (by default its odd chunks run on a second stream of the library).  backward_operand_bits: significant bits that the
+    backward's x and w are expected to have (up to 8: the library looks for operands that need fewer products)."""
     return Options(ctypes.sizeof(Options), int(forward_stream_bytes), int(backward_groups_per_round),
-                   1 if forward_single_stream else 0)
+                   1 if forward_single_stream else 0, int(backward_operand_bits))
+
+
+_SHORT_OPERANDS = make_options(backward_operand_bits=8)
+
+
+def operand_options(prec):
+    """Options of a backward whose x and w were quantised to ``prec`` bits (utils_functional.quantize); None where that is not
+    known or not short."""
+    return _SHORT_OPERANDS if isinstance(prec, int) and 1 <= prec <= 8 else None
 
 
 def _opt_ptr(options):

@@ -139,10 +139,13 @@ Options make_options(const geo_sc_options* o)
     r.forward_stream_bytes = kDefaultForwardStreamBytes;
     r.backward_groups_per_round = 0;
     r.forward_single_stream = false;
-    if (o && o->struct_bytes >= sizeof(geo_sc_options)) {
+    r.backward_operand_bits = 0;
+    if (o && o->struct_bytes >= offsetof(geo_sc_options, backward_operand_bits)) {
         if (o->forward_stream_bytes) r.forward_stream_bytes = o->forward_stream_bytes;
         if (o->backward_groups_per_round > 0) r.backward_groups_per_round = o->backward_groups_per_round;
         r.forward_single_stream = o->forward_single_stream != 0;
+        if (o->struct_bytes >= offsetof(geo_sc_options, backward_operand_bits) + sizeof(int32_t) && o->backward_operand_bits > 0)
+            r.backward_operand_bits = o->backward_operand_bits;
     }
     return r;
 }
@@ -551,7 +554,8 @@ int geo_sc_conv2d_add_partial_backward_workspace_size_ex(const geo_sc_conv_desc*
     if (!bytes) return GEO_SC_ERR_INVALID_ARGUMENT;
     const int rc = make_geometry(desc, &g);
     if (rc != GEO_SC_OK) return rc;
-    *bytes = backward_workspace_bytes(g, make_options(options).backward_groups_per_round);
+    const Options opt = make_options(options);
+    *bytes = backward_workspace_bytes(g, opt.backward_groups_per_round, opt.backward_operand_bits);
     return GEO_SC_OK;
 }
 
@@ -569,7 +573,8 @@ int geo_sc_conv2d_add_partial_backward_ex(const geo_sc_conv_desc* desc, const ge
     if (rc != GEO_SC_OK) return rc;
     if (!x || !w || !grad_y || (!grad_x && !grad_w)) return GEO_SC_ERR_INVALID_ARGUMENT;
     if (!workspace || ((uintptr_t)workspace & 255u)) return GEO_SC_ERR_WORKSPACE;
-    return launch_conv_backward(g, make_options(options).backward_groups_per_round, x, w, grad_y, grad_x, grad_w,
+    const Options opt = make_options(options);
+    return launch_conv_backward(g, opt.backward_groups_per_round, opt.backward_operand_bits, x, w, grad_y, grad_x, grad_w,
                                 workspace, workspace_bytes, (hipStream_t)stream);
 }
 

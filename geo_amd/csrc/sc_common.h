@@ -120,6 +120,7 @@ struct Options {
     size_t forward_stream_bytes;    // budget of the forward's activation stream buffer
     int backward_groups_per_round;  // cap on the add groups per round of backward launches; 0: none
     bool forward_single_stream;     // a cut batch runs on the caller's stream alone
+    int backward_operand_bits;      // significant bits that x and w of the backward are expected to have; 0: not known
 };
 constexpr size_t kDefaultForwardStreamBytes = (size_t)256 << 20;
 
@@ -141,9 +142,10 @@ double conv_forward_cost(const Geometry& g);
 int launch_rail_pack(const Geometry& g, uint32_t* wgt, hipStream_t s, bool from_generator);
 // the LFSR weight generator writes the rail-packed copy (and clears the flag area) itself
 inline bool generator_packs_rails(const Geometry& g) { return g.generator == GEO_SC_GEN_LFSR; }
-size_t backward_workspace_bytes(const Geometry& g, int groups_per_round);
-// GEO_SC_ERR_WORKSPACE when workspace_bytes is below backward_workspace_bytes(g, groups_per_round)
-int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x, const float* w, const float* gy,
-                         float* gx, float* gw, void* workspace, size_t workspace_bytes, hipStream_t s);
+// operand_bits: Options::backward_operand_bits
+size_t backward_workspace_bytes(const Geometry& g, int groups_per_round, int operand_bits);
+// GEO_SC_ERR_WORKSPACE when workspace_bytes is below backward_workspace_bytes(g, groups_per_round, operand_bits)
+int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bits, const float* x, const float* w,
+                         const float* gy, float* gx, float* gw, void* workspace, size_t workspace_bytes, hipStream_t s);
 
 }  // namespace geo_sc

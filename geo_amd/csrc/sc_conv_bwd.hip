@@ -98,7 +98,7 @@ struct GemmParams {
     // exists, zero elsewhere (read from sh_zero).
     const float* __restrict__ sh_zero;
     int sh_j, sh_wo, sh_ho, sh_win, sh_hin, sh_pad, sh_padh, sh_wk, sh_hk;
-    // not null: a word that says whether every x and w is a bf16 number (k_bwd_prep).  Where it is not zero, the
+    // not null (LOOK): a word that says whether every x and w is a bf16 number (k_bwd_prep).  Where it is not zero, the
     // operands made from them are one term of the split instead of three, and the rows that `a` of the first two products
     // points to hold bf16 numbers (the same elements at the same indexes).
     const int* __restrict__ one_term;
@@ -785,14 +785,16 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
     store_tile<EPI, NX, NY>(q, acc, q.c + batch * q.c_batch_stride + split * q.c_split_stride, i0 + wi, j0 + wj, l32, lk);
 }
 
-// Operands with 16-byte aligned rows and chunks (launch_gemm checks).
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA = false, bool VB = false>
+// Operands with 16-byte aligned rows and chunks (launch_gemm checks).  LOOK: one_term is there, operands of one term are
+// taken as such; without it three terms are all there is (one body, and the code and registers that it had alone: the
+// last product of 64 -> 64 channels in blocks of 16, 5 x 5, 16 x 16, 64 items takes 45 us beside the other body, 41 alone).
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA, bool VB, bool LOOK>
 // three waves per SIMD (at most 168 registers; three workgroups' LDS fit a CU)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_gemm_split(GemmParams q)
 {
     __shared__ uint4 as[2][3][2][kLdx];
     __shared__ uint4 bs[2][3][2][kLdx];
-    if (q.one_term_elsewhere && *q.one_term) return;
+    if (LOOK && q.one_term_elsewhere && *q.one_term) return;
     int it, jt, z;
     gemm_tile_of(q, blockIdx.x, it, jt, z);
     const int i0 = it * q.tile_i, j0 = jt * q.tile_j;
@@ -823,8 +825,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     };
     using One = std::integral_constant<int, 1>;
     using Three = std::integral_constant<int, 3>;
-    if (!(q.one_term && *q.one_term))
+    if (!LOOK || !*q.one_term)
         tile(Three(), Three(), 0.0f);
+    else if constexpr (!LOOK)
+        ;
     else if constexpr (PRODUCT == PRODUCT_E)
         tile(One(), One(), bf16_bits());
     else if constexpr (PRODUCT == PRODUCT_DW)
@@ -1071,14 +1075,16 @@ __device__ __forceinline__ void gemm_big_tiles(const GemmParams& q, uint4 (*as)[
     }
 }
 
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA, bool VB, int NX, int KC = 1>
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, int PRODUCT, bool VA, bool VB, bool LOOK, int NX, int KC = 1>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_big(GemmParams q)
 {
     __shared__ uint4 as[2][3][2 * KC][64 * NX + 4];
     __shared__ uint4 bs[2][3][2 * KC][kBigJ + 4];
-    if (q.one_term_elsewhere && *q.one_term) return;
-    if (!(q.one_term && *q.one_term))
+    if (LOOK && q.one_term_elsewhere && *q.one_term) return;
+    if (!LOOK || !*q.one_term)
         gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 3, 3, float>(q, as, bs);
+    else if constexpr (!LOOK)
+        ;
     else if constexpr (PRODUCT == PRODUCT_E)
         gemm_big_tiles<A_KMAJOR, B_KMAJOR, EPI, VA, VB, NX, KC, 1, 1, bf16_bits>(q, as, bs);
     else if constexpr (PRODUCT == PRODUCT_DW)
@@ -1477,6 +1483,17 @@ __device__ __forceinline__ bool takes_three_terms(float v)
     return (u & 0xffffu) != 0 || (u & 0x7f800000u) == 0x7f800000u;
 }
 
+// Whether a call looks for operands of one term: what the caller expects says so (geo_sc_options.backward_operand_bits), and
+// where it says nothing the products' size does (multiply-adds of one of them, both rails).  Other operands pay for the scan,
+// for kernels that ask what it found and for one that returns at once: 40 -> 128, 1 x 1, 32 x 32, 256 items (2.7e9) 355 -> 373
+// us, 64 -> 64 at 28 x 28, 128 items (7.4e9) 430 -> 443, at 56 x 56, 64 items (1.5e10) 788 -> 799, 128 items (3e10) 1469 ->
+// 1472; small ones 3 - 7 us of 24 - 90.  7-bit operands gain 1 - 25 % of 35 - 130 us (33 members and more), more when larger.
+constexpr double kLookWork = 2e10;
+inline bool looks_for_one_term(int operand_bits, double products)
+{
+    return operand_bits ? operand_bits <= 8 : products >= kLookWork;
+}
+
 // Whether x and w are bf16 numbers throughout, which 7-bit operands (k / 128) are: the scan's blocks leave what they found
 // (scan_operands), the launch behind them agrees on it (operands_are_bf16) and keeps it for those that follow, which
 // read one word.  A thread stops at its first element that is none, so that the scan of other operands costs next to
@@ -1516,9 +1533,10 @@ __device__ __forceinline__ void scan_operands(const float* __restrict__ x, long 
     const int any = __syncthreads_or(three);
     if (threadIdx.x == 0) found[block] = any;
 }
-// every thread of a block of 256; rows of the scan
+// every thread of a block of 256; rows of the scan; found NULL: nobody looked
 __device__ __forceinline__ bool operands_are_bf16(const int* __restrict__ found, int rows)
 {
+    if (!found) return false;
     static_assert(kScanBlocks == 256, "one word per thread and row");
     int any = 0;
     for (int r = 0; r < rows; r++) any |= found[r * 256 + threadIdx.x];
@@ -1576,7 +1594,7 @@ __global__ __launch_bounds__(256) void k_im2col_rows(const float* __restrict__ x
     const int k1 = min(G.n_members, k0 + kIm2colMembers);
     float* colg = col + (size_t)blockIdx.z * g_stride;
     const bool bf16_col = operands_are_bf16(found, found_rows);
-    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
+    if (found && blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
     for (int m = blockIdx.x * 256 + threadIdx.x; m < m_total; m += gridDim.x * 256) {
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
         // all loads first, from x[0] where the member lies in the padding (a load inside a branch is
@@ -1634,7 +1652,7 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
     const float4* x4 = (const float4*)x;
     const int quads = m_total >> 2;
     const bool bf16_col = operands_are_bf16(found, found_rows);
-    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
+    if (found && blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *one_term = bf16_col;
     for (int mq = blockIdx.x * 256 + threadIdx.x; mq < quads; mq += gridDim.x * 256) {
         const int m = mq << 2;
         const int r0 = arow[m], c0 = bcol[m], b0 = base[m];
@@ -1685,7 +1703,7 @@ __global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ 
     const unsigned wp = w_in + 2 * pad_w, hq = ho >> 2;
     const float4* x4 = (const float4*)x;
     const bool one = operands_are_bf16(found, found_rows);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *one_term = one;
+    if (found && blockIdx.x == 0 && threadIdx.x == 0) *one_term = one;
     // kShiftQuads quads per thread and trip, a block's width apart: their loads go out together
     for (unsigned e0 = blockIdx.x * (256 * kShiftQuads) + threadIdx.x; e0 < total; e0 += gridDim.x * (256 * kShiftQuads)) {
         float4 a[kShiftQuads], b[kShiftQuads];
@@ -1776,7 +1794,7 @@ struct WgradSplits {
 __device__ __forceinline__ float wgrad_again(const WgradOperands& o, int group, int k, int j, long long begin, long long end)
 {
     const size_t c0 = group * o.col_v + k * o.col_ld;
-    const bool one = *o.one_term != 0;
+    const bool one = o.one_term && *o.one_term;
     const float* e = o.e + group * o.e_v + j;
     float sum = 0.0f;
 #pragma unroll 1
@@ -3023,10 +3041,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8
     const int split = blockIdx.x / q.jblocks, jblock = blockIdx.x - split * q.jblocks, j_begin = jblock * JW;
     // whether x and this workgroup's weights are bf16 numbers
     bool three = small_k_weights(q, sh, j_begin);
-    for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
-    if (!__syncthreads_or(three)) {
-        small_k_columns<1, NW, NB, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
-        return;
+    if (q.found_rows) {
+        for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
+        if (!__syncthreads_or(three)) {
+            small_k_columns<1, NW, NB, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
+            return;
+        }
+    } else {
+        __syncthreads();
     }
     small_k_columns<3, NW, 1, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
     if constexpr (NB > 1) {
@@ -3077,8 +3099,8 @@ inline bool split_tiles_whole(int I, int J)
     return I % ti == 0 && J % tj == 0;
 }
 
-template <bool AK, bool BK, int EPI, int PRODUCT, bool VA = false, bool VB = false>
-int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
+template <bool AK, bool BK, int EPI, int PRODUCT, bool VA, bool VB, bool LOOK>
+int launch_gemm_of(const GemmParams& q0, int batch, hipStream_t s)
 {
     GemmParams q = q0;
     if constexpr (VA || VB) {
@@ -3107,13 +3129,13 @@ int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
             auto launch = [&](auto epi) {
                 constexpr int E = decltype(epi)::value;
                 if (nx == 4)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 4>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, LOOK, 4>), grid, dim3(512), 0, s, q);
                 else if (nx == 3)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 3>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, LOOK, 3>), grid, dim3(512), 0, s, q);
                 else if (kc2)
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 2, 2>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, LOOK, 2, 2>), grid, dim3(512), 0, s, q);
                 else
-                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, 2>), grid, dim3(512), 0, s, q);
+                    hipLaunchKernelGGL((k_gemm_big<AK, BK, E, PRODUCT, VA, VB, LOOK, 2>), grid, dim3(512), 0, s, q);
             };
             if constexpr (EPI == EPI_EXP_TIMES_G) {
                 if (q.g_planes)
@@ -3155,23 +3177,30 @@ int launch_gemm(const GemmParams& q0, int batch, hipStream_t s)
     const bool b_vec = BK || rows_aligned(q.b, q.ldb, q.b_batch_stride);
     if constexpr (VB) {
         // (the caller has checked the view's alignment: rows of E and the runs of eight columns)
-        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, false, true>), grid, dim3(256), 0, s, q);
+        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, false, true, LOOK>), grid, dim3(256), 0, s, q);
     } else if constexpr (VA) {
         if (!b_vec) return GEO_SC_ERR_UNSUPPORTED;
         if constexpr (EPI == EPI_EXP_TIMES_G) {
             if (q.g_planes)
-                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI_EXP_TIMES_G_PLANES, PRODUCT, true>), grid, dim3(256), 0, s, q);
+                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI_EXP_TIMES_G_PLANES, PRODUCT, true, false, LOOK>), grid, dim3(256), 0, s, q);
             else
-                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true>), grid, dim3(256), 0, s, q);
+                hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true, false, LOOK>), grid, dim3(256), 0, s, q);
         } else {
-            hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true>), grid, dim3(256), 0, s, q);
+            hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, true, false, LOOK>), grid, dim3(256), 0, s, q);
         }
     } else {
         // (the scratch layout aligns the rows)
         if (!a_vec || !b_vec) return GEO_SC_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT>), grid, dim3(256), 0, s, q);
+        hipLaunchKernelGGL((k_gemm_split<AK, BK, EPI, PRODUCT, false, false, LOOK>), grid, dim3(256), 0, s, q);
     }
     return hipGetLastError() == hipSuccess ? GEO_SC_OK : GEO_SC_ERR_LAUNCH;
+}
+
+template <bool AK, bool BK, int EPI, int PRODUCT, bool VA = false, bool VB = false>
+int launch_gemm(const GemmParams& q, int batch, hipStream_t s)
+{
+    return q.one_term ? launch_gemm_of<AK, BK, EPI, PRODUCT, VA, VB, true>(q, batch, s)
+                      : launch_gemm_of<AK, BK, EPI, PRODUCT, VA, VB, false>(q, batch, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -3180,6 +3209,7 @@ struct BwdLayout {
     long long m_total;
     int splits, m_per_split;
     Groups G;
+    bool look;           // whether x and w are bf16 numbers is found out on the device
     bool fused_k;        // OR groups of at most 32 members: whole backward in one kernel, no col / E scratch
     int fused_jw;        // columns of E per workgroup of that kernel
     int fused_jblocks;   // its column blocks: each writes a dcol slice of its own
@@ -3211,7 +3241,7 @@ size_t view_floats(const Geometry& g)
 
 inline long long pad4(long long v) { return (v + 3) & ~3LL; }
 
-BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
+BwdLayout bwd_layout(const Geometry& g, int groups_per_round, int operand_bits)
 {
     BwdLayout b;
     b.m_total = (long long)g.n * g.wo * g.ho;
@@ -3234,13 +3264,14 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
         b.G.n_members = g.k_or;
     }
     const int K = b.G.n_members;
+    b.look = looks_for_one_term(operand_bits, 2.0 * b.m_total * g.c_out * K * b.G.n_groups);
     b.fused_k = K <= kFusedK;
     // the bf16 kernel (at most 16 members) comes with 2, 4 or 8 waves of 32 columns, or 8 of 64 where under four of the
     // waves' 16 blocks stay empty (with 260 columns, operands of three terms: 417 us against 398 of 256-wide ones for
     // 64 -> 130 at 20 x 20, z_unit 4, batch 32) and the groups alone are two rounds of workgroups (otherwise three terms lose
     // more than one wins: 5 -> 250 at 28 x 28, batch 64: 405 us against 367); the fp32 one with 128 or 256 columns
     const long long fused_tiles = (b.m_total + kFusedTile - 1) / kFusedTile;
-    const bool wide = K <= 16 && (512 - 2 * g.c_out % 512) % 512 < 128 &&
+    const bool wide = b.look && K <= 16 && (512 - 2 * g.c_out % 512) % 512 < 128 &&
                       (long long)b.G.n_groups * ((2 * g.c_out + 511) / 512) >= 1024;
     b.fused_jw = 2 * g.c_out <= 64 && K <= 16 ? 64 : 2 * g.c_out <= 128 ? 128 : wide ? 512 : 256;
     b.fused_jblocks = (2 * g.c_out + b.fused_jw - 1) / b.fused_jw;
@@ -3293,7 +3324,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
     b.splits = (int)((b.m_total + b.m_per_split - 1) / b.m_per_split);
     // one round of persistent workgroups for E and the weight gradient of operands of one term
     b.ew_splits = b.ew_m_per_split = b.ew_tiles_each = b.ew_parts = 0;
-    if (!b.fused_k && K <= kEwMembers) {
+    if (b.look && !b.fused_k && K <= kEwMembers) {
         const int tm = 2 * g.c_out <= 64 ? 64 : 32;
         const long long jtiles = (2 * g.c_out + 127) / 128, m_tiles = (b.m_total + tm - 1) / tm;
         const long long parts = std::max(1LL, std::min(kEwWorkgroups / (jtiles * b.G.n_groups), m_tiles / 2));
@@ -3381,12 +3412,15 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round)
 
 }  // namespace
 
-size_t backward_workspace_bytes(const Geometry& g, int groups_per_round) { return bwd_layout(g, groups_per_round).bytes; }
-
-int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x, const float* w, const float* gy,
-                         float* gx, float* gw, void* workspace, size_t workspace_bytes, hipStream_t s)
+size_t backward_workspace_bytes(const Geometry& g, int groups_per_round, int operand_bits)
 {
-    const BwdLayout L = bwd_layout(g, groups_per_round);  // once per call: sizes the check and the launches alike
+    return bwd_layout(g, groups_per_round, operand_bits).bytes;
+}
+
+int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bits, const float* x, const float* w,
+                         const float* gy, float* gx, float* gw, void* workspace, size_t workspace_bytes, hipStream_t s)
+{
+    const BwdLayout L = bwd_layout(g, groups_per_round, operand_bits);  // once per call: sizes the check and the launches alike
     if (workspace_bytes < L.bytes) return GEO_SC_ERR_WORKSPACE;
     if (L.m_total > 0x7fffffffLL) return GEO_SC_ERR_INVALID_ARGUMENT;
     char* ws = (char*)workspace;
@@ -3415,9 +3449,11 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
     const bool fused = L.fused_k;
     // col as a view of the shifted input planes (one round holds every group then)
     const bool view = L.view_col && ((uintptr_t)x & 15) == 0;
-    int* found = (int*)(ws + L.off_scan);
-    int* one_term = found + kScanBlocks * kScanRows;
-    const int n_scan_rows = scan_rows(x_total);
+    // what the scan of the operands leaves, and the word that it comes down to; NULL: three terms, nobody looks
+    const bool look = L.look;
+    int* found = look ? (int*)(ws + L.off_scan) : nullptr;
+    int* one_term = look ? found + kScanBlocks * kScanRows : nullptr;
+    const int n_scan_rows = look ? scan_rows(x_total) : 0;
     // the position tables serve the gathers of im2col and of the fused kernels
     const PositionTable positions = {pos_base, pos_arow, pos_bcol, M, g.c_in, g.w_in, g.h_in, g.pad_w, g.pad_h, g.wo, g.ho};
     if (fused) {
@@ -3565,8 +3601,8 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, const float* x
             if (v0 == 0) {
                 pp.x = x; pp.x_total = x_total; pp.w_total = (long long)g.c_out * g.c_in * g.w_k * g.h_k; pp.found = found;
                 pp.scan_rows = n_scan_rows;
-                wb = kScanBlocks;
                 if (!view) pp.positions = positions;
+                if (look || !view) wb = kScanBlocks;
             }
             const int more_rows = pp.scan_rows + (pp.positions.m_total ? 1 : 0);
             const bool ragged = G.mode == GEO_SC_ACC_YZ && g.c_in % G.zu != 0;

@@ -25,7 +25,7 @@ class Conv2d_Add_Partial(nn.Conv2d):
         return utils_functional.conv2d_generic(
             input, self.weight, bit_length=2 ** err, padding=self.padding, stride=self.stride, forward=forward,
             generator=generator, legacy=legacy, z_unit=z_unit, load_unit=load_unit, load_wait_w=load_wait_w,
-            load_wait_a=load_wait_a)
+            load_wait_a=load_wait_a, prec=prec)
 
 
 def _fixed_affine(module, x, mean, var):
@@ -129,7 +129,8 @@ class _SCConvBlock(torch.autograd.Function):
         x = activation.detach().float().contiguous()
         w = weight.detach().float().contiguous()
         torch_stats = conv_kw.get("torch_stats", False)
-        conv_kw = {k: v for k, v in conv_kw.items() if k != "torch_stats"}
+        ctx.prec = conv_kw.get("prec")
+        conv_kw = {k: v for k, v in conv_kw.items() if k not in ("torch_stats", "prec")}
         L = conv_kw["bit_length"]
         counts = capi.conv2d_add_partial_forward(x, w, **conv_kw)
         gm = gamma.detach().float().contiguous() if gamma is not None else None
@@ -169,7 +170,8 @@ class _SCConvBlock(torch.autograd.Function):
         gx = gw = None
         if need_x or need_w:
             gx, gw = capi.conv2d_add_partial_backward(x, w, gy, kw["bit_length"], kw["padding"], need_x, need_w,
-                                                      accumulate=kw["accumulate"], z_unit=kw["z_unit"])
+                                                      accumulate=kw["accumulate"], z_unit=kw["z_unit"],
+                                                      options=capi.operand_options(ctx.prec))
         return (gx, gw, gg if ctx.has_gamma else None, gb if ctx.has_gamma else None, None, None, None, None, None,
                 None)
 
@@ -209,7 +211,7 @@ def sc_conv_block(conv, bn, input, *, err=7, forward="1d_bin", z_unit=8, load_un
     kw = dict(bit_length=2 ** err, padding=(int(conv.padding[0]), int(conv.padding[1])),
               total_width=utils_functional.prec_default, load_width=int(load_unit), load_wait_w=int(load_wait_w),
               load_wait_a=int(load_wait_a if mode == "yz" else load_wait_w), accumulate=mode,
-              z_unit=max(1, min(int(z_unit), conv.weight.shape[1])), torch_stats=bool(torch_stats))
+              z_unit=max(1, min(int(z_unit), conv.weight.shape[1])), torch_stats=bool(torch_stats), prec=prec)
     gamma, beta = (bn.weight, bn.bias) if bn.affine else (None, None)
     out = _SCConvBlock.apply(input, conv.weight, gamma, beta, bn, kw, relu, pool, hardtanh, quant7)
     if quant7 and hardtanh:

@@ -46,7 +46,7 @@ class _SCConv2dAddPartial(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, activation, weight, bit_length, padding, load_unit, load_wait, accumulate="y", z_unit=1,
-                load_wait_a=None, generator="lfsr", seed=0):
+                load_wait_a=None, generator="lfsr", seed=0, prec=None):
         origin = activation.device
         dev = origin if activation.is_cuda else torch.device("cuda", torch.cuda.current_device())
         x = activation.detach().to(dev, torch.float32).contiguous()
@@ -74,6 +74,7 @@ class _SCConv2dAddPartial(torch.autograd.Function):
         ctx.pad = pad
         ctx.origin = origin
         ctx.bit_length = int(bit_length)
+        ctx.prec = prec
         ctx.act_dtype = activation.dtype
         ctx.w_dtype = weight.dtype
         ctx.w_device = weight.device
@@ -87,19 +88,21 @@ class _SCConv2dAddPartial(torch.autograd.Function):
         gx = gw = None
         if need_x or need_w:
             gx, gw = capi.conv2d_add_partial_backward(x, w, g, ctx.bit_length, ctx.pad, need_x, need_w,
-                                                      accumulate=ctx.accumulate, z_unit=ctx.z_unit)
+                                                      accumulate=ctx.accumulate, z_unit=ctx.z_unit,
+                                                      options=capi.operand_options(ctx.prec))
         if gx is not None:
             gx = gx.to(ctx.origin, ctx.act_dtype)
         if gw is not None:
             gw = gw.to(ctx.w_device, ctx.w_dtype)
-        return gx, gw, None, None, None, None, None, None, None, None, None
+        return gx, gw, None, None, None, None, None, None, None, None, None, None
 
 
 def conv2d_generic(activation, weight, padding, stride, **kwargs):
     """Generic SC conv2d layer, same call as the reference's (utils_functional.py:406-634).
 
     Keyword arguments read: bit_length (128), generator (None), forward ('full_or'), legacy
-    (False), load_unit (8), load_wait_w (1), load_wait_a (1), z_unit (1024); prec/acc/share are
+    (False), load_unit (8), load_wait_w (1), load_wait_a (1), z_unit (1024), prec (None: not known; the bits that activation
+    and weight were quantised to, which the backward may take to look for operands of few bits); acc/share are
     accepted and unused on these paths.  Implemented: forward='1d_bin' with generator='lfsr' or,
     on GPU tensors, 'acc'; forward='z_bin' / 'yz_bin' on GPU tensors (the reference sends those to
     its LFSR GPU ops whatever the generator, utils_functional.py:503-510); forward='full_or' on GPU
@@ -114,6 +117,7 @@ def conv2d_generic(activation, weight, padding, stride, **kwargs):
     load_wait_w = kwargs.get("load_wait_w", 1)
     load_wait_a = kwargs.get("load_wait_a", 1)
     z_unit = kwargs.get("z_unit", 1024)
+    prec = kwargs.get("prec", None)
     ok_1d = forward == "1d_bin" and (generator == "lfsr" or (generator == "acc" and activation.is_cuda))
     ok_zyz = forward in ("z_bin", "yz_bin", "full_or") and activation.is_cuda
     if legacy or not (ok_1d or ok_zyz):
@@ -131,16 +135,19 @@ def conv2d_generic(activation, weight, padding, stride, **kwargs):
         # sc_extension_cuda.conv2d_or_acc: Bernoulli random streams, OR over everything
         # (utils_functional.py:511-514); surrogate conv2d_or_approx (:616-617)
         return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), 8, 1, "full", 1, None, "rand",
-                                         0)
+                                         0, prec)
     if forward == "1d_bin" and generator == "acc":
         # sc_extension_cuda.conv2d_add_partial_acc_acc (utils_functional.py:499-502)
-        return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), 8, 1, "y", 1, None, "acc", 37)
+        return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), 8, 1, "y", 1, None, "acc", 37,
+                                         prec)
     if forward == "z_bin":
-        return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), load_unit, load_wait_w, "z")
+        return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), load_unit, load_wait_w, "z",
+                                         1, None, "lfsr", 0, prec)
     if forward == "yz_bin":
         return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), load_unit, load_wait_w,
-                                         "yz", z_unit, load_wait_a)
-    return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), load_unit, load_wait_w)
+                                         "yz", z_unit, load_wait_a, "lfsr", 0, prec)
+    return _SCConv2dAddPartial.apply(activation, weight, bit_length, tuple(padding), load_unit, load_wait_w, "y", 1, None,
+                                     "lfsr", 0, prec)
 
 
 def sc_counts(activation, weight, bit_length, padding, forward="1d_bin", load_unit=8, load_wait_w=1, load_wait_a=1,

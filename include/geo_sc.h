@@ -129,6 +129,12 @@ typedef struct geo_sc_conv_desc {
  *   backward_groups_per_round  the backward processes its add groups (kernel rows in mode Y) in rounds of
  *                              launches of as many groups as fit about 3 GB of scratch; this lowers that
  *                              number and the workspace size with it.  Default: no further cap.
+ *   backward_operand_bits      how many significant bits the caller expects x and w of the backward to have: up
+ *                              to 8 (the layers' operands k / 128 have 7), or more.  Operands of up to 8 bits
+ *                              throughout are found on the device and take fewer products; this says whether to look.
+ *                              It is no promise: results do not depend on it beyond the rounding of sums.  Default:
+ *                              calls look where that costs other operands next to nothing (large ones).
+ *                              (A caller built without this field passes the smaller struct_bytes.)
  * The same options must be given to a size query and to the call that uses the workspace.
  */
 typedef struct geo_sc_options {
@@ -136,6 +142,7 @@ typedef struct geo_sc_options {
     size_t forward_stream_bytes;
     int32_t backward_groups_per_round;
     int32_t forward_single_stream;
+    int32_t backward_operand_bits;
 } geo_sc_options;
 
 /* Library version (GEO_SC_VERSION of the build). */

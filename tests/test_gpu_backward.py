@@ -26,6 +26,18 @@ def capi():
     return m
 
 
+@pytest.fixture
+def looking(capi, monkeypatch):
+    """Every backward of the test looks for operands of one term, whatever its size."""
+    real = capi.conv2d_add_partial_backward
+
+    def looks(*args, options=None, **kw):
+        rounds = options.backward_groups_per_round if options is not None else 0
+        return real(*args, options=capi.make_options(backward_groups_per_round=rounds, backward_operand_bits=8), **kw)
+
+    monkeypatch.setattr(capi, "conv2d_add_partial_backward", looks)
+
+
 def rel_err(got, ref):
     ref = ref.double().cpu()
     return ((got.double().cpu() - ref).abs().max() / ref.abs().max().clamp_min(1e-30)).item()
@@ -557,6 +569,7 @@ def seven_bit(shape_x, shape_w, seed):
     return x, w, g
 
 
+@pytest.mark.usefixtures("looking")
 @pytest.mark.parametrize("rounds", [0, 1])
 @pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", ONE_TERM_SHAPES)
 def test_operands_of_one_term_give_the_results_of_three(capi, shape_x, shape_w, pad, mode, zu, rounds):
@@ -582,6 +595,7 @@ def test_operands_of_one_term_give_the_results_of_three(capi, shape_x, shape_w, 
         check("grad_w", gw[:, keep], gw3[:, keep])
 
 
+@pytest.mark.usefixtures("looking")
 @pytest.mark.parametrize("where", ["first", "last", "weight", "none"])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 def test_one_element_of_more_than_eight_bits_is_found(capi, where, offset):
@@ -668,6 +682,7 @@ SMALL_GROUPS = [
 ]
 
 
+@pytest.mark.usefixtures("looking")
 @pytest.mark.parametrize("operands", ["seven bits", "floats", "float weights of the last channel"])
 @pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", SMALL_GROUPS)
 def test_small_or_groups(capi, shape_x, shape_w, pad, mode, zu, operands):
@@ -687,3 +702,79 @@ def test_small_or_groups(capi, shape_x, shape_w, pad, mode, zu, operands):
     none, only = capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, (pad, pad), accumulate=mode, z_unit=zu,
                                                   need_grad_x=False)
     assert none is None and torch.equal(only, gw)
+
+
+def launches(fn):
+    """Kernel launches of ``fn``: nodes of its captured graph."""
+    import ctypes
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out = fn()
+    with open("/proc/self/maps") as f:  # the runtime that is loaded already
+        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
+    nodes = ctypes.c_size_t(0)
+    status = ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes))
+    assert status == 0 and out is not None
+    return nodes.value
+
+
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((1, 16, 8, 8), (16, 16, 3, 3), 1, "y", 1),        # planes
+    ((2, 64, 8, 8), (128, 64, 3, 3), 1, "y", 1),       # planes and the gradient as it is
+    ((2, 45, 9, 7), (83, 45, 3, 3), 1, "yz", 32),      # im2col
+    ((2, 100, 8, 8), (40, 100, 3, 3), 1, "y", 1),      # more members than E and the weight gradient take together
+    ((40, 16, 1, 40), (300, 16, 1, 40), 0, "y", 1),    # small groups, one output position
+])
+def test_only_calls_that_expect_short_operands_pay_for_the_look(capi, shape_x, shape_w, pad, mode, zu):
+    """A call of this size that says nothing about its operands launches what three terms need.  Results do not depend on
+    what a call expects."""
+    from oracle import surrogate
+    x, w, g = seven_bit(shape_x, shape_w, 11)
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gy = torch.randn(capi.output_shape(d), generator=g)
+    rx, rw, _ = surrogate.surrogate_autograd(x, w, gy, (pad, pad), mode=mode, z_unit=zu)
+    x, w, gy = x.cuda(), w.cuda(), gy.cuda()
+    count = {}
+    for bits in (None, 0, 8, 9, 24):
+        options = None if bits is None else capi.make_options(backward_operand_bits=bits)
+        run = lambda: capi.conv2d_add_partial_backward(x, w, gy, 128, (pad, pad), accumulate=mode, z_unit=zu, options=options)
+        count[bits] = launches(run)
+        for xs in (x, x * 0.93):
+            gx, gw = capi.conv2d_add_partial_backward(xs, w, gy, 128, (pad, pad), accumulate=mode, z_unit=zu, options=options)
+            if xs is x:
+                check("grad_x", gx, rx)
+                check("grad_w", gw, rw)
+            elif bits is None:
+                other = gx, gw
+            else:
+                check("grad_x of floats", gx, other[0])
+                check("grad_w of floats", gw, other[1])
+    members = {"y": shape_x[1] * shape_w[2], "yz": zu * shape_w[2]}[mode]
+    assert count[None] == count[0] == count[9] == count[24]
+    assert count[8] == count[0] + (1 if 32 < members <= 192 else 0)
+
+
+def test_layers_say_what_their_operands_are(capi, monkeypatch):
+    from geo_amd import utils_class, utils_functional
+    seen = []
+    real = capi.conv2d_add_partial_backward
+
+    def watch(*args, options=None, **kw):
+        seen.append(0 if options is None else options.backward_operand_bits)
+        return real(*args, options=options, **kw)
+
+    monkeypatch.setattr(capi, "conv2d_add_partial_backward", watch)
+    conv = utils_class.Conv2d_Add_Partial(8, 6, kernel_size=3, padding=1, bias=False).cuda()
+    bn = utils_class.BatchNorm2d_fixed(6).cuda()
+    for prec in (7, 8, 9):
+        for forward in ("1d_bin", "z_bin", "yz_bin"):
+            conv(torch.rand(2, 8, 8, 8, device="cuda", requires_grad=True), prec=prec, forward=forward).sum().backward()
+        utils_class.sc_conv_block(conv, bn, torch.rand(2, 8, 8, 8, device="cuda", requires_grad=True), prec=prec).sum().backward()
+    assert seen == [8] * 8 + [0] * 4
+    seen.clear()
+    x, w = torch.rand(2, 8, 8, 8, device="cuda", requires_grad=True), torch.rand(6, 8, 3, 3, device="cuda")
+    for kw in ({}, dict(prec=7), dict(prec=None), dict(prec=128), dict(prec=7.0)):
+        utils_functional.conv2d_generic(x, w, 1, 1, forward="1d_bin", generator="lfsr", **kw).sum().backward()
+    assert seen == [0, 8, 0, 0, 0]

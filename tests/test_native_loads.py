@@ -83,6 +83,21 @@ def test_forward_scratch_is_bounded_by_the_stream_budget():
         assert capi.workspace_size(d, o) == capi.workspace_size(d, capi.make_options(budget, 0, True))
 
 
+def test_options_of_a_caller_that_knows_fewer_fields():
+    """struct_bytes says how much of geo_sc_options the caller has: what lies behind is not read, what lies in front counts."""
+    from geo_amd import _native, capi
+    d = capi.make_desc((64, 45, 27, 19), (83, 45, 3, 3), 128, (1, 1), accumulate="yz", z_unit=32)
+    size = lambda **kw: capi.backward_workspace_size(d, capi.make_options(**kw))
+    whole, rounds, short = size(), size(backward_groups_per_round=1), size(backward_operand_bits=8)
+    assert rounds < whole != short
+    assert size(backward_operand_bits=24) == whole
+    old = capi.make_options(backward_groups_per_round=1, backward_operand_bits=8)
+    old.struct_bytes = _native.Options.backward_operand_bits.offset
+    assert old.struct_bytes == 24 and capi.backward_workspace_size(d, old) == rounds
+    old.struct_bytes = 16
+    assert capi.backward_workspace_size(d, old) == whole
+
+
 def test_descriptors_around_four_gib_of_activation_streams():
     """Stage entry points hold the streams of the whole batch.  From 4 GiB on the kernels with 32-bit byte offsets
     are not used: the layout query stops answering item-innermost.  The whole-op forward never gets there: it
