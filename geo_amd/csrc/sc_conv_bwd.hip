@@ -422,8 +422,10 @@ struct SplitStager {
 // fetch issues its loads without waiting for the table first; the entries read for the chunk behind the last
 // one (up to 2 * kChunk + 8 entries behind the member's part of the table) are never used.
 // Without AHEAD the table is read as constant memory (its kernel ran before): scalar loads, where the compiler otherwise
-// takes vector loads in some of the loops, which the data loads then wait for (first product of 64 -> 64 at 28 x 28, batch
-// 64, three terms: 69 us, now 57).
+// takes vector loads, which the data loads then wait for (waves of 2 x 2 blocks, first product of 64 -> 64 at 28 x 28, batch
+// 64, three terms: 69 us, now 57).  Waves of fewer blocks have registers for the entries ahead: a scalar load's wait takes
+// in the LDS reads and each chunk's entries are a cache line of their own, a round trip to L2 per chunk in a short trip
+// (256 -> 256 at 8 x 8, one item: 44 us, now 35; 512 -> 512 at 4 x 4, two items: 70, 53).
 template <bool KMAJOR, typename T = float, bool AHEAD = false>
 struct ViewStager {
     const T* base;
@@ -523,7 +525,7 @@ struct ViewStager {
             else
                 load_row_part(p, 8 * half, k_left, r);
         }
-        advance();
+        skip_chunk();
     }
     template <int TERMS>
     __device__ __forceinline__ void commit(uint4 (*s)[2][kLdx], raw_of<T> (&r)[8], int k_left) const
@@ -626,7 +628,7 @@ __device__ __forceinline__ void gemm_wave_split(const GemmParams& q, uint4 (*as)
             for (int r = 0; r < 16; r++) acc[x][y][r] = 0.0f;
 
     constexpr bool BK = B_KMAJOR && !VB;
-    typename std::conditional<VA, ViewStager<A_KMAJOR, A>, SplitStager<A_KMAJOR, A>>::type sa;
+    typename std::conditional<VA, ViewStager<A_KMAJOR, A, NX * NY < 4>, SplitStager<A_KMAJOR, A>>::type sa;
     typename std::conditional<VB, ShiftStager, SplitStager<B_KMAJOR>>::type sb;
     // K-major operand: waves 0, 1 stage the first k half of the 128 rows, waves 2, 3 the second;
     // I-major operand: two threads per row, one k half each
