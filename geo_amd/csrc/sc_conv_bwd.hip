@@ -1102,7 +1102,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // A = col[m][k], read transposed from LDS), and all members' sums of the weight gradient.  The first product's result
 // E[m][j] is the second one's B operand as it is: lane -> column j, and of each 16 positions the eight that the lane
 // holds (the order of a contraction is free; A = col[k][m] is read in the same order).  So E is split once and never read
-// back; it is stored for the input gradient, and the same bits as the first product stores.
+// back; it is stored for the input gradient, and the same bits as the first product stores (not where nobody reads it:
+// the weight gradient alone of 64 -> 64 at 56 x 56, batch 128: 430 us in all with the stores, 348).
 // A workgroup is persistent: 4 waves, one group, NWJ * 32 columns, one part of the positions in tiles of 32 (64 where two
 // waves cover the columns: the halves' sums meet at the end); col's next tile is loaded while this one is multiplied.
 // 64 -> 64 at 56 x 56, batch 128: 314 us, the two products 354 + 306 us; without the stores of E it takes 40 less, without the
@@ -1121,6 +1122,7 @@ struct EwParams {
     size_t col_v, w_v, e_v, part_v;
     int M, K, J, e_ld, c_out, npos, m_per_split, jtiles;
     int splits, tiles_each, parts;  // partial sums as in SmallKParams
+    int store_e;                    // somebody reads E: the input gradient, or wgrad_again
 };
 constexpr int kEwMembers = 192;     // six blocks of 32: 96 registers of sums
 constexpr int kEwWorkgroups = 512;  // two per CU
@@ -1313,15 +1315,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if constexpr (!PLANES) fetch_g(mb + TM);
             float* ep = eg + (size_t)mi * q.e_ld + j;
             if (mb + 32 <= m_end && j0 + 32 <= q.J) {
+                if (q.store_e) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) ep[(size_t)(8 * (r >> 2) + (r & 3)) * q.e_ld] = z[r];
+                    for (int r = 0; r < 16; r++) ep[(size_t)(8 * (r >> 2) + (r & 3)) * q.e_ld] = z[r];
+                }
             } else {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int d = 8 * (r >> 2) + (r & 3);
                     if (mi + d >= m_end)
                         z[r] = 0.0f;
-                    else if (j_ok)
+                    else if (j_ok && q.store_e)
                         ep[(size_t)d * q.e_ld] = z[r];
                 }
             }
@@ -3653,6 +3657,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
             p.M = M; p.K = K; p.J = J; p.e_ld = e_ld; p.c_out = g.c_out; p.npos = g.wo * g.ho;
             p.m_per_split = L.ew_m_per_split; p.jtiles = (J + 127) / 128;
             p.splits = L.ew_splits; p.tiles_each = L.ew_tiles_each; p.parts = L.ew_parts;
+            p.store_e = gx || !view;
             const dim3 grid((unsigned)(L.ew_splits * p.jtiles), nv);
             auto launch = [&](auto blocks) {
                 constexpr int B = decltype(blocks)::value;
