@@ -1699,7 +1699,11 @@ __global__ __launch_bounds__(256) void k_im2col_rows_v4(const float* __restrict_
 // their cache lines.  Four columns per thread (ho and h_in multiples of four, 16-byte aligned x), as in
 // k_im2col_rows_v4.  `total` quads; the (w_k - 1) * ho elements behind the last plane are never read.  Planes of bf16
 // numbers where x and w are such throughout, which the first block tells the products.
-constexpr int kShiftQuads = 4;
+// Q quads per thread and trip, a block's width apart: their loads go out together.  Four where that leaves every CU two
+// workgroups, one below: 20 M quads (64 x 56 x 56, 128 items) 98 us with one, 94 with four; 645 k 7.1 and 6.6; 322 k 6.2
+// and 7.5; 15 k 2.8 and 4.5 (bf16 planes 3.2 and 4.8).
+constexpr long long kShiftMany = 1 << 19;
+template <int Q>
 __global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ x, float* __restrict__ xs,
                                                       const int* __restrict__ found, int found_rows,
                                                       int* __restrict__ one_term, unsigned total,
@@ -1710,13 +1714,12 @@ __global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ 
     const float4* x4 = (const float4*)x;
     const bool one = operands_are_bf16(found, found_rows);
     if (found && blockIdx.x == 0 && threadIdx.x == 0) *one_term = one;
-    // kShiftQuads quads per thread and trip, a block's width apart: their loads go out together
-    for (unsigned e0 = blockIdx.x * (256 * kShiftQuads) + threadIdx.x; e0 < total; e0 += gridDim.x * (256 * kShiftQuads)) {
-        float4 a[kShiftQuads], b[kShiftQuads];
-        int sh[kShiftQuads];
-        bool ok_a[kShiftQuads], ok_b[kShiftQuads];
+    for (unsigned e0 = blockIdx.x * (256 * Q) + threadIdx.x; e0 < total; e0 += gridDim.x * (256 * Q)) {
+        float4 a[Q], b[Q];
+        int sh[Q];
+        bool ok_a[Q], ok_b[Q];
 #pragma unroll
-        for (int q = 0; q < kShiftQuads; q++) {
+        for (int q = 0; q < Q; q++) {
             const unsigned e = min(e0 + q * 256, total - 1);
             // e = (((v * c_in + ci) * n_items + n) * wp + r) * hq + quad
             unsigned t = e / hq;
@@ -1738,7 +1741,7 @@ __global__ __launch_bounds__(256) void k_shift_planes(const float* __restrict__ 
             b[q] = x4[ok_b[q] ? at + 1 : 0];
         }
 #pragma unroll
-        for (int q = 0; q < kShiftQuads; q++) {
+        for (int q = 0; q < Q; q++) {
             const unsigned e = e0 + q * 256;
             if (!ok_a[q]) a[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (!ok_b[q]) b[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -3625,8 +3628,15 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
         if (view) {
             const long long plane = (long long)g.n * (g.w_in + 2 * g.pad_w) * g.ho;
             const long long quads = (long long)g.h_k * g.c_in * plane / 4;
-            hipLaunchKernelGGL(k_shift_planes, dim3(grid1d((quads + kShiftQuads - 1) / kShiftQuads)), dim3(256), 0, s, x, col, found, n_scan_rows, one_term, (unsigned)quads, g.n, g.c_in,
-                               g.w_in, g.h_in, g.pad_w, g.pad_h, g.ho);
+            auto shift = [&](auto per_thread) {
+                constexpr int Q = decltype(per_thread)::value;
+                hipLaunchKernelGGL((k_shift_planes<Q>), dim3(grid1d((quads + Q - 1) / Q)), dim3(256), 0, s, x, col, found,
+                                   n_scan_rows, one_term, (unsigned)quads, g.n, g.c_in, g.w_in, g.h_in, g.pad_w, g.pad_h, g.ho);
+            };
+            if (quads >= kShiftMany)
+                shift(std::integral_constant<int, 4>());
+            else
+                shift(std::integral_constant<int, 1>());
         } else if (im2col_v4) {
             const int q_blocks = grid1d(M / 4);
             hipLaunchKernelGGL(k_im2col_rows_v4,
