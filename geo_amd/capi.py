@@ -74,8 +74,11 @@ def _opt_ptr(options):
 
 
 def _stream_ptr(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    # torch.cuda.current_stream().cuda_stream without the Stream object (0.2 us of host time instead of 2.8 and more in the
+    # backward's thread: 220 -> 181 us for a small layer forward and backward, 62 -> 49 forward alone)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _ptr(t):
@@ -137,9 +140,10 @@ def conv2d_add_partial_values(x, w, desc: ConvDesc, bit_length, stream=None):
     _require_gpu_f32(w, "w")
     workspace = torch.empty(workspace_size(desc), dtype=torch.uint8, device=x.device)
     y = torch.empty(output_shape(desc), dtype=torch.float32, device=x.device)
-    conv2d_add_partial_forward(x, w, bit_length, out=y, workspace=workspace, desc=desc, stream=stream)
-    _check(_native.lib().geo_sc_counts_to_values(_ptr(y), y.numel(), int(bit_length), _stream_ptr(stream)),
-           "geo_sc_counts_to_values")
+    lib, y_ptr, stream_ptr = _native.lib(), _ptr(y), _stream_ptr(stream)
+    _check(lib.geo_sc_conv2d_add_partial_forward_ex(ctypes.byref(desc), None, _ptr(x), _ptr(w), y_ptr, _ptr(workspace),
+                                                    workspace.numel(), stream_ptr), "geo_sc_conv2d_add_partial_forward")
+    _check(lib.geo_sc_counts_to_values(y_ptr, y.numel(), int(bit_length), stream_ptr), "geo_sc_counts_to_values")
     return y
 
 

@@ -397,6 +397,32 @@ def test_passes_in_quads_at_their_edges(n, offset):
     assert torch.equal(y[:offset], counts[:offset]) and torch.equal(y[offset + n:], counts[offset + n:])
 
 
+def test_values_of_a_layer_look_the_stream_up_once(capi, monkeypatch):
+    """Counts and their values go to the current stream, whichever it is, from one look at it."""
+    seen = []
+    real = capi._stream_ptr
+
+    def watch(stream=None):
+        seen.append(real(stream).value or 0)
+        return real(stream)
+
+    x, w = torch.rand(3, 5, 6, 7, device="cuda"), torch.rand(4, 5, 3, 3, device="cuda") - 0.5
+    d = capi.make_desc(x.shape, w.shape, 64, (1, 1))
+    ref = capi.conv2d_add_partial_forward(x, w, 64, (1, 1)) * (1.0 / 64)
+    monkeypatch.setattr(capi, "_stream_ptr", watch)
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), side, torch.cuda.ExternalStream(side.cuda_stream)):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            y = capi.conv2d_add_partial_values(x, w, d, 64)
+        assert seen == [stream.cuda_stream]
+        seen.clear()
+        stream.synchronize()
+        assert torch.equal(y, ref)
+        assert torch.equal(capi.conv2d_add_partial_values(x, w, d, 64, stream=stream), ref) and seen == [stream.cuda_stream]
+        seen.clear()
+
+
 def test_quantize_many_equals_quantize_per_tensor(capi):
     """geo_sc_quantize_many: every tensor of the list as geo_sc_quantize gives it (odd sizes, an empty one, more
     tensors than one launch takes)."""
