@@ -583,7 +583,9 @@ def test_operands_of_one_term_give_the_results_of_three(capi, shape_x, shape_w, 
     kw = dict(accumulate=mode, z_unit=zu, options=capi.make_options(backward_groups_per_round=rounds) if rounds else None)
     gx, gw = capi.conv2d_add_partial_backward(x, w, gy, 128, (pad, pad), **kw)
     other = x.clone()
-    other[0, 1, 2, 2] += 2.0 ** -20
+    other[0, 1, 2, 2] = 0.3
+    beyond_bf16 = lambda t: bool((t.view(torch.int32) & 0xffff).any())
+    assert not beyond_bf16(x) and not beyond_bf16(w) and beyond_bf16(other)
     gx3, gw3 = capi.conv2d_add_partial_backward(other, w, gy, 128, (pad, pad), **kw)
     keep = [c for c in range(shape_x[1]) if c != 1]
     assert torch.equal(gx, gx3)
