@@ -508,6 +508,7 @@ def test_backward_of_many_channels_at_few_positions(capi, shape_x, shape_w, pad,
     assert torch.equal(gx2, gx) and torch.equal(gw2, gw)
 
 
+@pytest.mark.parametrize("operands", ["floats", "seven bits"])
 @pytest.mark.parametrize("shape_x,shape_w", [
     ((3, 20, 5, 7), (45, 20, 3, 3)),   # 105 positions, 90 rail columns: neither in whole quads
     ((3, 20, 5, 7), (46, 20, 3, 3)),   # odd positions
@@ -515,17 +516,23 @@ def test_backward_of_many_channels_at_few_positions(capi, shape_x, shape_w, pad,
     ((9, 40, 11, 13), (71, 40, 3, 3)), # several tiles and splits of each product
     ((3, 150, 5, 7), (360, 150, 3, 3)),  # partial sums added in tiles of weights x channels
 ])
-def test_infinite_and_largest_gradients_at_sizes_of_no_whole_quads(capi, shape_x, shape_w):
+def test_infinite_and_largest_gradients_at_sizes_of_no_whole_quads(capi, shape_x, shape_w, operands):
     """An infinite element of the upstream gradient makes its channel's weight gradient infinite, not NaN, and leaves the
-    other channels' bits alone; a NaN stays one; a finite gradient that a bf16 would round to infinity stays finite."""
+    other channels' bits alone; a NaN stays one; a finite gradient that a bf16 would round to infinity stays finite.  With
+    operands of one term E and the partial sums come from another kernel, and col's rows are bf16."""
     from oracle import surrogate
     x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_w[0])
     x = (x * 0.9 + 0.05).contiguous()
     w = (w * 2).contiguous()
     w.view(-1)[::7] = 0.0
     w[9] = 0.0
+    options = None
+    if operands == "seven bits":
+        x, w = (x * 128).round().clamp(1, 127) / 128, (w * 128).round().clamp(-127, 127) / 128
+        options = capi.make_options(backward_operand_bits=8)
     pad = (1, 1)
-    back = lambda gy: capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, pad)
+    small = x * 0.04 if operands == "floats" else x / 32
+    back = lambda gy, x=x: capi.conv2d_add_partial_backward(x.cuda(), w.cuda(), gy.cuda(), 128, pad, options=options)
     g = torch.randn((shape_x[0], shape_w[0]) + shape_x[2:], generator=torch.Generator().manual_seed(4))
     gx, gw = back(g)
     near = torch.zeros(shape_x, dtype=torch.bool)
@@ -542,14 +549,14 @@ def test_infinite_and_largest_gradients_at_sizes_of_no_whole_quads(capi, shape_x
     # without weights E is the gradient itself
     gb = g * 0
     gb[1, 9, 2, 3] = 3.4e38
-    _, rw, _ = surrogate.surrogate_autograd(x * 0.04, w, gb, pad)
-    _, bw = capi.conv2d_add_partial_backward((x * 0.04).cuda(), w.cuda(), gb.cuda(), 128, pad)
+    _, rw, _ = surrogate.surrogate_autograd(small, w, gb, pad)
+    _, bw = back(gb, small)
     check("grad_w of a gradient of 3.4e38", bw, rw)
 
 
 ONE_TERM_SHAPES = [
     ((2, 32, 16, 16), (32, 32, 5, 5), 2, "y", 1),      # planes, 64-wide tiles
-    ((9, 64, 28, 28), (64, 64, 3, 3), 1, "y", 1),      # planes, whole 128-wide tiles, the gradient as it is
+    ((9, 64, 28, 28), (64, 64, 3, 3), 1, "y", 1),      # planes, whole 128-wide tiles, items of 24.5 x 32 positions
     ((64, 128, 16, 16), (128, 128, 3, 3), 1, "y", 1),  # eight waves
     ((16, 256, 8, 8), (256, 256, 3, 3), 1, "y", 1),    # eight waves, tiles of other heights
     ((7, 45, 27, 19), (43, 45, 3, 3), 1, "yz", 16),    # im2col, ragged channel blocks
