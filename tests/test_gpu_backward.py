@@ -605,6 +605,44 @@ def test_operands_of_one_term_give_the_results_of_three(capi, shape_x, shape_w, 
 
 
 @pytest.mark.usefixtures("looking")
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((8, 64, 8, 8), (64, 64, 3, 3), 1, "y", 1),     # one tile of columns
+    ((8, 64, 8, 8), (128, 64, 3, 3), 1, "y", 1),    # two, which read the same channels
+    ((8, 64, 8, 8), (192, 64, 3, 3), 1, "y", 1),    # three, the middle one of both rails
+    ((8, 16, 8, 8), (256, 16, 3, 3), 1, "y", 1),    # four; two blocks of members
+    ((8, 96, 8, 8), (128, 96, 3, 3), 1, "yz", 32),  # three blocks, nine groups
+    ((8, 40, 8, 8), (128, 40, 3, 3), 1, "y", 1),    # four, the last one ragged
+    ((8, 32, 8, 8), (64, 32, 5, 5), 2, "y", 1),     # five
+    ((4, 64, 24, 32), (64, 64, 3, 3), 1, "y", 1),   # parts that begin and end inside items
+])
+def test_one_term_takes_the_gradient_as_the_caller_has_it(capi, shape_x, shape_w, pad, mode, zu):
+    """E and the weight gradient from the upstream gradient in the caller's layout (items of whole 32 positions, whole tiles
+    of 128 x 128), against float64, against the transposed copy that a gradient off its 16-byte boundary takes (the same
+    bits, one launch more) and against operands of three terms."""
+    x, w, g = seven_bit(shape_x, shape_w, 5)
+    w[:, 1] = 0.0
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gy = torch.randn(capi.output_shape(d), generator=g) * 1e-2
+    rx, rw = _fp64_reference_on_gpu(x, w, gy, pad, mode, zu)
+    x, w, gy = x.cuda(), w.cuda(), gy.cuda()
+    back = lambda x, gy: capi.conv2d_add_partial_backward(x, w, gy, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gx, gw = back(x, gy)
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
+    off = torch.empty(gy.numel() + 1, device="cuda")[1:].view(gy.shape)
+    off.copy_(gy)
+    assert launches(lambda: back(x, off)) == launches(lambda: back(x, gy)) + 1
+    for got, ref in zip(back(x, off), (gx, gw)):
+        assert torch.equal(got, ref)
+    other = x.clone()
+    other[0, 1, 2, 2] = 0.3
+    gx3, gw3 = back(other, gy)
+    keep = [c for c in range(shape_x[1]) if c != 1]
+    assert torch.equal(gx, gx3)
+    check("grad_w of three terms", gw[:, keep], gw3[:, keep])
+
+
+@pytest.mark.usefixtures("looking")
 @pytest.mark.parametrize("where", ["first", "last", "weight", "none"])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 def test_one_element_of_more_than_eight_bits_is_found(capi, where, offset):
