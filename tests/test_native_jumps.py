@@ -134,3 +134,22 @@ def test_weight_packing_counts_in_integers(tmp_path):
             seen += 1
             assert not [op for _, op, _ in code if "_f64" in op], name
     assert seen >= 2
+
+
+def test_small_group_backward_keeps_its_registers(tmp_path):
+    """k_bwd_small_k_bf16<8, 2, DX> lives within the 128 registers of four waves per SIMD.  What moved to scratch memory when its
+    two bodies had a branch more in front of them (184 and 48 bytes) cost it a fifth of its time."""
+    from geo_amd import _native
+    readobj = OBJDUMP.replace("objdump", "readobj")
+    if not os.path.exists(readobj):
+        pytest.skip("no disassembler here")
+    scratch = {}
+    for i, obj in enumerate(code_objects(_native.lib_path())):
+        f = tmp_path / f"{i}.co"
+        f.write_bytes(obj)
+        notes = subprocess.run([readobj, "--notes", str(f)], check=True, capture_output=True, text=True).stdout
+        for kernel in notes.split(".agpr_count")[1:]:
+            m = re.search(r"k_bwd_small_k_bf16ILi8ELi2ELb([01])E\S*\.kd", kernel)
+            if m:
+                scratch[m.group(1)] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1))
+    assert scratch["0"] == 0 and scratch["1"] <= 160, scratch
