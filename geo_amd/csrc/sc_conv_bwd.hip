@@ -2196,16 +2196,23 @@ __global__ __launch_bounds__(256) void k_bwd_prep(PrepParams q)
 // the scan).  The
 // first q.groups rows of blocks take the tiles of all groups of the round.  For taps that fit (prep_tile_channels) and groups whose members all exist.
 constexpr int kPrepRow = 288;  // floats per output channel of a tile
-inline int prep_tile_channels(int c_in, int c_out, int taps)
+// What it takes is one long pass per tile, element by element a line per weight.  Few weights are few tiles: from 2^18 weights on
+// (25 600 of 5 x 5: 14 us in tiles, 7 element by element; 205 k: 11 and 7.4; 410 k: 12 and 13), or 2^17 in tiles of few
+// weights per output channel (230 k of 3 x 3: 6.6 and 7.9; 147 k, channel blocks of 32: 6.1 and 8.1).  Where the input gradient's
+// operand is that of several taps (dx_rows) a tile writes it tap by tap: from two tiles per CU on (3 x 3, 128 -> 128, 128 tiles: 8.0
+// and 5.0; 224 -> 224, 392: 9.1 and 8.1; 256 -> 256, 512: 10.0 and 10.6; 512 -> 512: 18.5 and 25.4; 5 x 5, 128 -> 256, 256 tiles: 15.4
+// and 13.6; 128 -> 512, 512: 18.4 and 20.8).
+inline int prep_tile_channels(int c_in, int c_out, int taps, bool dx_rows)
 {
-    // (few weights are few tiles, one long pass each: 25 600 of 5 x 5 take 14 us in tiles, 7 element by element)
-    if ((long long)c_in * c_out * taps < 1 << 17) return 0;
+    const long long weights = (long long)c_in * c_out * taps;
+    if (weights < 1 << 17) return 0;
     int channels = 32;
     while (channels > 1 && channels * taps > kPrepRow) channels /= 2;
     if (channels * taps > kPrepRow) return 0;
     // two tiles per CU, where narrower ones make them
-    while (channels > 4 && (long long)((c_out + 31) / 32) * ((c_in + channels - 1) / channels) < 512) channels /= 2;
-    return channels;
+    auto tiles = [&] { return (long long)((c_out + 31) / 32) * ((c_in + channels - 1) / channels); };
+    while (channels > 4 && tiles() < 512) channels /= 2;
+    return (dx_rows ? weights >= 1 << 18 && tiles() >= 512 : weights >= 1 << 18 || channels * taps <= 48) ? channels : 0;
 }
 __global__ __launch_bounds__(256) void k_bwd_prep_tiled(PrepParams q, int n_groups, int channels_log2)
 {
@@ -3612,7 +3619,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
             }
             const int more_rows = pp.scan_rows + (pp.positions.m_total ? 1 : 0);
             const bool ragged = G.mode == GEO_SC_ACC_YZ && g.c_in % G.zu != 0;
-            const int channels = ragged ? 0 : prep_tile_channels(g.c_in, g.c_out, g.w_k * g.h_k);
+            const int channels = ragged ? 0 : prep_tile_channels(g.c_in, g.c_out, g.w_k * g.h_k, dx_rows);
             if (channels) {
                 const long long tiles = (long long)((g.c_out + 31) / 32) * ((g.c_in + channels - 1) / channels);
                 pp.groups = (int)std::min<long long>((tiles + kScanBlocks - 1) / kScanBlocks, 8);  // rows of tiles

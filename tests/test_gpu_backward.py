@@ -675,9 +675,13 @@ def test_one_element_of_more_than_eight_bits_is_found(capi, where, offset):
     ((2, 54, 7, 8), (51, 54, 7, 7), 3, "z", 1),        # groups of 49 members, one per channel
     ((2, 128, 5, 5), (120, 128, 3, 3), 1, "yz", 16),
     ((2, 128, 5, 5), (120, 128, 3, 3), 1, "full", 1),
+    ((3, 264, 4, 8), (264, 264, 3, 3), 1, "y", 1),     # the input gradient's operand per kernel column, in tiles
+    ((24, 264, 30, 32), (264, 264, 3, 3), 1, "y", 1),  # of all taps, in tiles
+    ((2, 520, 4, 4), (520, 520, 1, 1), 0, "y", 1),     # of one tap, 16 channels a tile
 ])
 def test_weight_operands_made_in_tiles(capi, shape_x, shape_w, pad, mode, zu, rounds):
-    """From 2^17 weights on the operands of the products are made in tiles of channels through LDS."""
+    """From 2^17 or 2^18 weights and some number of tiles on the operands of the products are made in tiles of channels
+    through LDS, element by element below."""
     from oracle import surrogate
     x, w = wl.make_inputs(shape_x, shape_w, "kaiming", seed=shape_x[1])
     w = (w * 3).contiguous()
