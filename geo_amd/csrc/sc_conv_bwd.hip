@@ -2670,7 +2670,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // throughout and E in LDS for both gradients, 1096 now, of which the vector work of E is 630 (the sum of the slices of
 // dcol, 16 with NB = 2 and 32 with NB = 1: 119 -> 62); unquantised operands, step 4.20 -> 4.17 ms; first layer of the
 // 4-layer CNN 92 -> 56, half of that the gather's.
-// Same grid, arguments, tiles and outputs as k_bwd_small_k.
+// Same grid, tiles and outputs as k_bwd_small_k.  LOOK: the call has scanned x; without it three terms are all there is.
 constexpr int kBfEw = 18;  // words per row of E^T: 32 bf16 and padding (8-byte accesses of 16 rows meet no bank twice)
 constexpr int kBfCw = 20;  // words per row of col[k][m]: 16-byte aligned rows
 
@@ -2738,51 +2738,6 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int l16 = lane & 15, lq = lane >> 4;
 
-    // first product, B operand of 16 columns: lane -> column l16, k = 8 (lq % 2) .. + 7 of one term; lanes from 32 on
-    // have the second of two terms (hi and lo, mid and hi), or zeros
-    constexpr int ZB = TERMS == 3 ? 2 : 1;
-    const unsigned first = lq < 2 ? ~0u : 0u;
-    bf16x8 wz[NB][2][ZB];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            unsigned t3[3][4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int k = 8 * (lq & 1) + 2 * c, jl = c0 + 32 * (b * NW + wave) + 16 * s + l16;
-                split3(sh.u.wl[k][jl], sh.u.wl[k + 1][jl], t3[0][c], t3[1][c], t3[2][c]);
-            }
-            unsigned o[2][4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                o[0][c] = (t3[0][c] & first) | (TERMS == 3 ? t3[2][c] & ~first : 0u);
-                o[1][c] = (t3[1][c] & first) | (t3[0][c] & ~first);
-            }
-#pragma unroll
-            for (int z = 0; z < ZB; z++) wz[b][s][z] = __builtin_bit_cast(bf16x8, make_uint4(o[z][0], o[z][1], o[z][2], o[z][3]));
-        }
-    // input gradient, A operand of 32 columns: lane -> wd[j][k = l16], j = 8 lq .. + 7, which is wcat[k][j] with the
-    // negative rail (j >= c_out) negated
-    bf16x8 wd[DX ? NB : 1][TERMS];
-    if constexpr (DX) {
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            unsigned t3[3][4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int jl = c0 + 32 * (b * NW + wave) + 8 * lq + 2 * c;
-                float v0 = sh.u.wl[l16][jl], v1 = sh.u.wl[l16][jl + 1];
-                if (j_begin + jl >= c_out) v0 = -v0;
-                if (j_begin + jl + 1 >= c_out) v1 = -v1;
-                split3(v0, v1, t3[0][c], t3[1][c], t3[2][c]);
-            }
-#pragma unroll
-            for (int t = 0; t < TERMS; t++) wd[b][t] = __builtin_bit_cast(bf16x8, make_uint4(t3[t][0], t3[t][1], t3[t][2], t3[t][3]));
-        }
-    }
-    // (a barrier comes before anything else is written to wl's space: behind the first tile's gather)
-
     // im2col gather: slot = (position t % 32 of the tile, members EP (t / 32) ..)
     const int ml = threadIdx.x & 31;
     int kg[GP], g_off[GP][EP], g_u[GP][EP], g_v[GP][EP];
@@ -2800,36 +2755,12 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
             g_v[gp][p] = e.v;
         }
     }
-    // where the upstream gradient of the wave's blocks lies in tile `split`: this lane's first eight values (columns 0 - 15;
-    // those of columns 16 - 31 are 256 floats further), and the distance to the next tile of this workgroup
-    int g_blk[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const int j0 = j_begin + c0 + 32 * (b * NW + wave);
-        g_blk[b] = q.gt_dedupe ? (j0 >= c_out ? j0 - c_out : j0) >> 5 : j0 >> 5;
-        if (j0 >= J) g_blk[b] = 0;  // columns outside the problem: any finite values will do
-    }
-    const float* g_at = q.gtt + (size_t)split * q.gt_blocks * 1024 + ((lq & 1) * 32 + l16) * 16 + 8 * (lq >> 1);
-    const size_t g_step = (size_t)q.splits * q.gt_blocks * 1024;
-    float4 gv[2][2];
-    auto fetch_g = [&](int b) {
-#pragma unroll
-        for (int s = 0; s < 2; s++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) gv[s][h] = *(const float4*)(g_at + (size_t)g_blk[b] * 1024 + 256 * s + 4 * h);
-    };
-
-    floatx4 gw_acc[NB][2];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-        for (int s = 0; s < 2; s++) gw_acc[b][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
     float* dg = q.dcol + (size_t)jblock * q.dcol_slice + (size_t)blockIdx.y * q.dcol_stride;
     const int n_tiles = (M + TM - 1) / TM;
     // The gather runs a tile ahead and its table entries two: a tile's columns of x are asked for at the
     // top of the tile before and its table entries at the top of the one before that, so that no tile
-    // waits for two dependent loads in a row.
+    // waits for two dependent loads in a row.  The first tile's are on their way while the weights become operands: with few
+    // tiles per workgroup that is most of its time (16 x 1 x 256 -> 1000, 8 items, three terms: 48 us, now 41).
     struct Where {
         int r0, c0, b0;
         bool ok;
@@ -2876,18 +2807,82 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
             }
         }
     };
-    float x_next[GP][EP], x_after[GP][EP];
-    unsigned ok_next, ok_after;
-    Where w_after;
-    {
-        const Where w0 = where(split);
-        ok_next = fetch(w0, x_next);
-        commit(0, x_next, ok_next);
-        const Where w1 = where(split + q.splits);
-        ok_next = fetch(w1, x_next);
-        w_after = where(split + 2 * q.splits);
+    float x_next[GP][EP], x_after[GP][EP], x_first[GP][EP];
+    const Where w_first = where(split), w_next = where(split + q.splits);
+    Where w_after = where(split + 2 * q.splits);
+    const unsigned ok_first = fetch(w_first, x_first);
+    unsigned ok_next = fetch(w_next, x_next), ok_after;
+    // first product, B operand of 16 columns: lane -> column l16, k = 8 (lq % 2) .. + 7 of one term; lanes from 32 on
+    // have the second of two terms (hi and lo, mid and hi), or zeros
+    constexpr int ZB = TERMS == 3 ? 2 : 1;
+    const unsigned first = lq < 2 ? ~0u : 0u;
+    bf16x8 wz[NB][2][ZB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            unsigned t3[3][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int k = 8 * (lq & 1) + 2 * c, jl = c0 + 32 * (b * NW + wave) + 16 * s + l16;
+                split3(sh.u.wl[k][jl], sh.u.wl[k + 1][jl], t3[0][c], t3[1][c], t3[2][c]);
+            }
+            unsigned o[2][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                o[0][c] = (t3[0][c] & first) | (TERMS == 3 ? t3[2][c] & ~first : 0u);
+                o[1][c] = (t3[1][c] & first) | (t3[0][c] & ~first);
+            }
+#pragma unroll
+            for (int z = 0; z < ZB; z++) wz[b][s][z] = __builtin_bit_cast(bf16x8, make_uint4(o[z][0], o[z][1], o[z][2], o[z][3]));
+        }
+    // input gradient, A operand of 32 columns: lane -> wd[j][k = l16], j = 8 lq .. + 7, which is wcat[k][j] with the
+    // negative rail (j >= c_out) negated
+    bf16x8 wd[DX ? NB : 1][TERMS];
+    if constexpr (DX) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            unsigned t3[3][4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int jl = c0 + 32 * (b * NW + wave) + 8 * lq + 2 * c;
+                float v0 = sh.u.wl[l16][jl], v1 = sh.u.wl[l16][jl + 1];
+                if (j_begin + jl >= c_out) v0 = -v0;
+                if (j_begin + jl + 1 >= c_out) v1 = -v1;
+                split3(v0, v1, t3[0][c], t3[1][c], t3[2][c]);
+            }
+#pragma unroll
+            for (int t = 0; t < TERMS; t++) wd[b][t] = __builtin_bit_cast(bf16x8, make_uint4(t3[t][0], t3[t][1], t3[t][2], t3[t][3]));
+        }
     }
+    // where the upstream gradient of the wave's blocks lies in tile `split`: this lane's first eight values (columns 0 - 15;
+    // those of columns 16 - 31 are 256 floats further), and the distance to the next tile of this workgroup
+    int g_blk[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int j0 = j_begin + c0 + 32 * (b * NW + wave);
+        g_blk[b] = q.gt_dedupe ? (j0 >= c_out ? j0 - c_out : j0) >> 5 : j0 >> 5;
+        if (j0 >= J) g_blk[b] = 0;  // columns outside the problem: any finite values will do
+    }
+    const float* g_at = q.gtt + (size_t)split * q.gt_blocks * 1024 + ((lq & 1) * 32 + l16) * 16 + 8 * (lq >> 1);
+    const size_t g_step = (size_t)q.splits * q.gt_blocks * 1024;
+    float4 gv[2][2];
+    auto fetch_g = [&](int b) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) gv[s][h] = *(const float4*)(g_at + (size_t)g_blk[b] * 1024 + 256 * s + 4 * h);
+    };
+
     fetch_g(0);
+
+    floatx4 gw_acc[NB][2];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) gw_acc[b][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    commit(0, x_first, ok_first);
     __syncthreads();  // the first tile's col is in place, and every wave has taken its weights out of wl
     // row i of the first product's two blocks is position zrow + 8 h; lane's results: positions ep + r and ep + 8 + r
     const int zrow = 16 * (l16 >> 3) + (l16 & 7), ep = 16 * (lq >> 1) + 4 * (lq & 1);
@@ -3049,19 +3044,22 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
         store_part();
 }
 
-template <int NW, int NB, bool DX>
+template <int NW, int NB, bool DX, bool LOOK>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 3))) void k_bwd_small_k_bf16(SmallKParams q)
 {
     constexpr int NT = 64 * NW, JW = 32 * NW * NB;
     __shared__ __attribute__((aligned(16))) SmallKShared<NW, NB, DX> sh;
     const int split = blockIdx.x / q.jblocks, jblock = blockIdx.x - split * q.jblocks, j_begin = jblock * JW;
-    // whether x and this workgroup's weights are bf16 numbers (without a scan of x nobody knows).  No branch around the look:
-    // with it <8, 2, true> had 76 registers in scratch memory instead of 51 and took 1233 us for the linear layer instead of 1035.
-    bool three = small_k_weights(q, sh, j_begin) || !q.found_rows;
-    for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
-    if (!__syncthreads_or(three)) {
-        small_k_columns<1, NW, NB, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
-        return;
+    bool three = small_k_weights(q, sh, j_begin);
+    if constexpr (LOOK) {
+        // whether x and this workgroup's weights are bf16 numbers
+        for (int e = threadIdx.x; e < q.found_rows * kScanBlocks; e += NT) three |= q.found[e] != 0;
+        if (!__syncthreads_or(three)) {
+            small_k_columns<1, NW, NB, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
+            return;
+        }
+    } else {
+        __syncthreads();
     }
     small_k_columns<3, NW, 1, DX, false, NB == 1>(q, sh, split, jblock, j_begin, 0);
     if constexpr (NB > 1) {
@@ -3554,21 +3552,25 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
                                       g.c_out, L.fused_jblocks, L.fused_splits, gw ? 1 : 0, L.gt_blocks, L.gt_dedupe, n_scan_rows,
                                       L.fused_tiles_each, L.fused_parts,
                                       L.w_v, L.part_v, L.col_v, slice};
-                    auto launch = [&](auto dx) {
-                        constexpr bool DX = decltype(dx)::value;
+                    auto launch = [&](auto dx, auto looks) {
+                        constexpr bool DX = decltype(dx)::value, LOOK = decltype(looks)::value;
                         if (jw == 64)
-                            hipLaunchKernelGGL((k_bwd_small_k_bf16<2, 1, DX>), grid, dim3(128), 0, s, p);
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<2, 1, DX, LOOK>), grid, dim3(128), 0, s, p);
                         else if (jw == 128)
-                            hipLaunchKernelGGL((k_bwd_small_k_bf16<4, 1, DX>), grid, dim3(256), 0, s, p);
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<4, 1, DX, LOOK>), grid, dim3(256), 0, s, p);
                         else if (jw == 256)
-                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 1, DX>), grid, dim3(512), 0, s, p);
-                        else
-                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 2, DX>), grid, dim3(512), 0, s, p);
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 1, DX, LOOK>), grid, dim3(512), 0, s, p);
+                        else  // (only where a call looks)
+                            hipLaunchKernelGGL((k_bwd_small_k_bf16<8, 2, DX, true>), grid, dim3(512), 0, s, p);
                     };
-                    if (gx)
-                        launch(std::true_type());
+                    if (gx && look)
+                        launch(std::true_type(), std::true_type());
+                    else if (gx)
+                        launch(std::true_type(), std::false_type());
+                    else if (look)
+                        launch(std::false_type(), std::true_type());
                     else
-                        launch(std::false_type());
+                        launch(std::false_type(), std::false_type());
                 }
                 else if (ks <= 12) GEO_SC_FUSED_NB_DX(12);
                 else GEO_SC_FUSED_NB_DX(16);
