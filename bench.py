@@ -201,13 +201,14 @@ def network_step_result(args, torch):
         xa, wa = xa.cuda(), wa.cuda()
         d = capi.make_desc(sx, sw, L, (pad, pad), 7, 2, 2, 2)
         ws = torch.empty(capi.workspace_size(d), dtype=torch.uint8, device="cuda")
-        wsb = torch.empty(capi.backward_workspace_size(d), dtype=torch.uint8, device="cuda")
+        opt = capi.operand_options(7)   # what the layers say of their operands
+        wsb = torch.empty(capi.backward_workspace_size(d, opt), dtype=torch.uint8, device="cuda")
         out = torch.empty(capi.output_shape(d), dtype=torch.int32, device="cuda")
         gy = torch.randn(out.shape, device="cuda")
         f = time_events(lambda: capi.conv2d_add_partial_forward(xa, wa, L, (pad, pad), out=out, workspace=ws, desc=d),
                         args.steps, 2, torch)
         b = time_events(lambda: capi.conv2d_add_partial_backward(xa, wa, gy, L, (pad, pad), workspace=wsb, desc=d,
-                                                                 need_grad_x=(name != "conv1")), args.steps, 2, torch)
+                                                                 need_grad_x=(name != "conv1"), options=opt), args.steps, 2, torch)
         act = capi.act_streams(xa, d)
         wgt = capi.weight_streams(wa, d)
         k = time_events(lambda: capi.conv2d_add_partial_from_streams(act, wgt, d, out=out), args.steps, 2, torch)

@@ -1107,7 +1107,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // A workgroup is persistent: 4 waves, one group, NWJ * 32 columns, one part of the positions in tiles of 32 (64 where two
 // waves cover the columns: the halves' sums meet at the end); col's next tile is loaded while this one is multiplied.
 // 64 -> 64 at 56 x 56, batch 128: 314 us, the two products 354 + 306 us; without the stores of E it takes 40 less, without the
-// gradient's loads 45 less, its matrix work is 108.  Ragged layer of 77 items, 45 -> 83, blocks of 32 channels: 89, 79 + 76.
+// gradient's loads 45 less, its matrix work is 108.  Ragged layer of 77 items, 45 -> 83, blocks of 32 channels: 93, 79 + 76.
 // Three terms need three times the registers: those operands take the two products (which return at once otherwise).
 struct EwParams {
     const bf16_bits* __restrict__ col;
@@ -1503,7 +1503,7 @@ inline bool looks_for_one_term(int operand_bits, double products)
 // Whether x and w are bf16 numbers throughout, which 7-bit operands (k / 128) are: the scan's blocks leave what they found
 // (scan_operands), the launch behind them agrees on it (operands_are_bf16) and keeps it for those that follow, which
 // read one word.  A thread stops at its first element that is none, so that the scan of other operands costs next to
-// nothing; 25.7 M floats of x take 20 us (64 -> 64 at 56 x 56, batch 128), of which bf16 planes alone give 16 back.
+// nothing; 25.7 M floats of x take 20 us (64 -> 64 at 56 x 56, batch 128), and bf16 planes alone give 24 back (94 -> 70).
 // One row of kScanBlocks blocks, kScanRows from kScanFew elements on (36 us with 256 blocks).
 constexpr int kScanRows = 4;
 constexpr long long kScanFew = 1 << 21;
