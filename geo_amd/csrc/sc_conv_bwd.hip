@@ -3501,8 +3501,9 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
     // dL/dx from dcol of the groups [v0, v0 + nv)
     auto col2im = [&](int v0, int nv) {
         const int n_planes = g.n * g.c_in;
-        // (under two tiles of items the other kernel's single pass is no slower: 18 items of 592 elements 37 us in all, 38.5)
-        if (g.wo * g.ho == 1 && g.n >= 64) {
+        // (from two tiles of items and 2^18 elements on: 1024 elements, 64 items 4.6 us and 3.5 with the other kernel, 128 items 4.2
+        // and 3.9, 256 items 4.9 and 5.4, 1024 items 5.2 and 11.5; 4096 elements, 64 items 4.6 and 6.3)
+        if (g.wo * g.ho == 1 && g.n >= 64 && x_total >= 1 << 18) {
             const int tiles = (g.c_in * g.w_in * g.h_in + 31) / 32, rows = (g.n + 31) / 32;
             hipLaunchKernelGGL(k_col2im_one, dim3(tiles, std::min(rows, 1024)), dim3(256), 0, s, dcol, gx, v0, nv, g.n, G, g.w_in,
                                g.h_in, g.pad_w, g.pad_h, L.col_v);

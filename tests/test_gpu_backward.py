@@ -697,14 +697,19 @@ def test_weight_operands_made_in_tiles(capi, shape_x, shape_w, pad, mode, zu, ro
 
 @pytest.mark.parametrize("rounds", [0, 1])
 @pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
-    ((64, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),       # one output position: dL/dx by transposition
-    ((79, 20, 3, 5), (9, 20, 3, 5), 0, "y", 1),        # ragged tiles of elements and items
+    ((64, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),       # one output position
+    ((79, 20, 3, 5), (9, 20, 3, 5), 0, "y", 1),
     ((65, 16, 1, 40), (24, 16, 1, 40), 0, "y", 1),     # the linear mapping: small groups
     ((67, 9, 3, 3), (7, 9, 5, 5), 1, "z", 1),          # taps in the padding
     ((85, 40, 1, 1), (7, 40, 1, 1), 0, "yz", 16),
-    ((63, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),       # too few items for that
+    ((63, 12, 4, 4), (10, 12, 4, 4), 0, "y", 1),
     ((70, 24, 2, 2), (12, 24, 3, 3), 1, "y", 1),       # items of four elements
     ((5, 13, 3, 3), (6, 13, 3, 3), 1, "full", 1),
+    ((64, 16, 1, 256), (9, 16, 1, 256), 0, "y", 1),    # one output position, 2^18 elements: dL/dx by transposition
+    ((69, 61, 8, 8), (7, 61, 8, 8), 0, "y", 1),        # ragged tiles of items
+    ((260, 113, 3, 3), (7, 113, 5, 5), 1, "z", 1),     # ragged tiles of elements, taps in the padding
+    ((270, 1000, 1, 1), (7, 1000, 1, 1), 0, "yz", 16),
+    ((63, 70, 8, 8), (7, 70, 8, 8), 0, "y", 1),        # too few items for that
 ])
 def test_input_gradient_of_few_positions(capi, shape_x, shape_w, pad, mode, zu, rounds):
     from oracle import surrogate
