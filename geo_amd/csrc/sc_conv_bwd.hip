@@ -2105,8 +2105,9 @@ __global__ __launch_bounds__(256) void k_reduce_wgrad_tiled(const float* __restr
 //  * from the blocks of the round's first group: view_rows[g][k], where row k of group g's col starts in the
 //    planes of k_shift_planes (elements), for every group; and 64 zeros for the shifted view of E (a store
 //    rather than a memset, so that a caller may capture the launch sequence in a graph);
-//  * in rows of blocks of their own behind the groups': the scan of x and w, and in the last row, if there is one more,
-//    the position table (a launch less in front of im2col: 4 us).
+//  * by blocks of their own in rows behind the groups': the scan of x and w, and the position table (a launch less in front of
+//    im2col: 4 us).  They are as many as they take, in rows as wide as the weight operands' (rows of 256 blocks for every
+//    group, nearly all of them without work: 5 x 5, 468 -> 26, 295 groups, 29 us for 5.6).
 struct PrepParams {
     const float* __restrict__ w;
     float* __restrict__ wcat;
@@ -2120,23 +2121,25 @@ struct PrepParams {
     long long plane;
     float* zero;            // null: no block of zeros wanted
     int groups;             // rows of blocks (blockIdx.y) that make weight operands: one per group of the round
-    int scan_rows;          // rows of kScanBlocks blocks behind the groups' that scan x and w; 0: no scan wanted
+    int scan_blocks;        // blocks that scan x and w; 0: no scan wanted
     const float* __restrict__ x;
     long long x_total, w_total;
     int* found;             // what the scan's blocks found
-    PositionTable positions;  // m_total 0: none wanted
+    PositionTable positions;
+    int position_blocks;    // blocks that fill it; 0: none wanted
 };
+constexpr int kPrepColumns = 8;  // least blocks in a row, so that those rows are few
+constexpr int kPrepRows = (kScanRows * kScanBlocks + kScanBlocks) / kPrepColumns;
 // what is no weight operand: the blocks of the scan and the positions (true: the block is one of them), the view's row
 // table, the zeros
 __device__ __forceinline__ bool prep_scans(const PrepParams& q)
 {
     if ((int)blockIdx.y < q.groups) return false;
-    if ((int)blockIdx.y == q.groups + q.scan_rows) {
-        q.positions.fill(blockIdx.x, gridDim.x);
-        return true;
-    }
-    scan_operands(q.x, q.x_total, q.w, q.w_total, (blockIdx.y - q.groups) * kScanBlocks + blockIdx.x, q.scan_rows * kScanBlocks,
-                  q.found);
+    const int block = (blockIdx.y - q.groups) * gridDim.x + blockIdx.x;
+    if (block < q.scan_blocks)
+        scan_operands(q.x, q.x_total, q.w, q.w_total, block, q.scan_blocks, q.found);
+    else if (block < q.scan_blocks + q.position_blocks)
+        q.positions.fill(block - q.scan_blocks, q.position_blocks);
     return true;
 }
 __device__ __forceinline__ void prep_tables(const PrepParams& q)
@@ -3363,7 +3366,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round, int operand_bits)
     if (rows > (size_t)b.G.n_groups) rows = b.G.n_groups;
     // the caller's cap on the add groups per round (less scratch, more launches)
     if (groups_per_round >= 1 && (size_t)groups_per_round < rows) rows = (size_t)groups_per_round;
-    if (rows * b.splits > 65534 - kScanRows) rows = (65534 - kScanRows) / b.splits;  // grid.y = rows, the scan's and the positions', grid.z = rows * splits
+    if (rows * b.splits > 65535 - kPrepRows) rows = (65535 - kPrepRows) / b.splits;  // grid.y = rows, the scan's and the positions', grid.z = rows * splits
     if (rows < 1) rows = 1;
     b.rows_per_chunk = (int)rows;
     // col as a view: whole quads in every row on both sides, chunks of kChunk positions inside one item, an
@@ -3616,20 +3619,21 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
             int wb = std::min(grid1d(work), 256);
             if (v0 == 0) {
                 pp.x = x; pp.x_total = x_total; pp.w_total = (long long)g.c_out * g.c_in * g.w_k * g.h_k; pp.found = found;
-                pp.scan_rows = n_scan_rows;
-                if (!view) pp.positions = positions;
-                if (look || !view) wb = kScanBlocks;
+                pp.scan_blocks = n_scan_rows * kScanBlocks;
+                pp.positions = positions;
+                pp.position_blocks = view ? 0 : std::min(m_blocks, kScanBlocks);
+                wb = std::max(wb, kPrepColumns);
             }
-            const int more_rows = pp.scan_rows + (pp.positions.m_total ? 1 : 0);
+            auto more_rows = [&](int columns) { return (pp.scan_blocks + pp.position_blocks + columns - 1) / columns; };
             const bool ragged = G.mode == GEO_SC_ACC_YZ && g.c_in % G.zu != 0;
             const int channels = ragged ? 0 : prep_tile_channels(g.c_in, g.c_out, g.w_k * g.h_k, dx_rows);
             if (channels) {
                 const long long tiles = (long long)((g.c_out + 31) / 32) * ((g.c_in + channels - 1) / channels);
                 pp.groups = (int)std::min<long long>((tiles + kScanBlocks - 1) / kScanBlocks, 8);  // rows of tiles
-                hipLaunchKernelGGL(k_bwd_prep_tiled, dim3(kScanBlocks, pp.groups + more_rows), dim3(256), 0, s, pp, nv,
+                hipLaunchKernelGGL(k_bwd_prep_tiled, dim3(kScanBlocks, pp.groups + more_rows(kScanBlocks)), dim3(256), 0, s, pp, nv,
                                    __builtin_ctz((unsigned)channels));
             } else {
-                hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + more_rows), dim3(256), 0, s, pp);
+                hipLaunchKernelGGL(k_bwd_prep, dim3(wb, nv + more_rows(wb)), dim3(256), 0, s, pp);
             }
         }
         if (view) {

@@ -793,20 +793,38 @@ def test_small_or_groups(capi, shape_x, shape_w, pad, mode, zu, operands):
     assert none is None and torch.equal(only, gw)
 
 
-def launches(fn):
-    """Kernel launches of ``fn``: nodes of its captured graph."""
+def workgroups(fn):
+    """Workgroups of each kernel launch of ``fn``, from the nodes of its captured graph."""
     import ctypes
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_uint32), ("y", ctypes.c_uint32), ("z", ctypes.c_uint32)]
+
+    class KernelNodeParams(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("block", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim3),
+                    ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
     fn()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph(keep_graph=True)
     with torch.cuda.graph(graph):
         out = fn()
     with open("/proc/self/maps") as f:  # the runtime that is loaded already
-        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
-    nodes = ctypes.c_size_t(0)
-    status = ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes))
-    assert status == 0 and out is not None
-    return nodes.value
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+    handle, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0 and out is not None
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
+    grids = []
+    for node in nodes:
+        q = KernelNodeParams()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(q)) == 0
+        grids.append(q.grid.x * q.grid.y * q.grid.z)
+    return grids
+
+
+def launches(fn):
+    return len(workgroups(fn))
 
 
 @pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
@@ -867,3 +885,31 @@ def test_layers_say_what_their_operands_are(capi, monkeypatch):
     for kw in ({}, dict(prec=7), dict(prec=None), dict(prec=128), dict(prec=7.0)):
         utils_functional.conv2d_generic(x, w, 1, 1, forward="1d_bin", generator="lfsr", **kw).sum().backward()
     assert seen == [0, 8, 0, 0, 0]
+
+
+@pytest.mark.parametrize("bits", [0, 8])
+@pytest.mark.parametrize("shape_x,shape_w,pad,mode,zu", [
+    ((3, 90, 5, 5), (26, 90, 5, 5), 2, "yz", 8),     # 60 groups of 40 members, ragged channel blocks
+    ((3, 64, 9, 7), (20, 64, 3, 5), 1, "yz", 16),    # 20 groups of 48
+    ((40, 33, 33, 35), (9, 33, 3, 3), 1, "y", 1),    # 46 200 positions, the table in 181 blocks
+    ((1, 40, 2, 3), (5, 40, 1, 1), 0, "y", 1),       # six positions
+])
+def test_preparation_has_no_more_workgroups_than_work(capi, shape_x, shape_w, pad, mode, zu, bits):
+    """The scan and the position table are some blocks in rows of their own; they don't widen the rows of the groups."""
+    from oracle import surrogate
+    x, w, g = seven_bit(shape_x, shape_w, 13)
+    d = capi.make_desc(x.shape, w.shape, 128, (pad, pad), accumulate=mode, z_unit=zu)
+    gy = torch.randn(capi.output_shape(d), generator=g)
+    rx, rw, _ = surrogate.surrogate_autograd(x, w, gy, (pad, pad), mode=mode, z_unit=zu)
+    x, w, gy = x.cuda(), w.cuda(), gy.cuda()
+    options = capi.make_options(backward_operand_bits=bits)
+    back = lambda: capi.conv2d_add_partial_backward(x, w, gy, 128, (pad, pad), accumulate=mode, z_unit=zu, options=options)
+    groups = {"y": 1, "yz": -(-shape_x[1] // zu)}[mode] * shape_w[3]
+    n, c_out, wo, ho = capi.output_shape(d)
+    row = max(8, -(-(shape_x[1] if mode == "y" else zu) * shape_w[2] * c_out // 256))
+    most = row * groups + min(256, -(-n * wo * ho // 256)) + (256 if bits == 8 else 0) + row
+    prepared = workgroups(back)[1]   # behind the transposed gradient
+    assert prepared <= most, (prepared, most)
+    gx, gw = back()
+    check("grad_x", gx, rx)
+    check("grad_w", gw, rw)
