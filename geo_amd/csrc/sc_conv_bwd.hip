@@ -2691,7 +2691,7 @@ struct SmallKParams {
     int g0, M, w_in, h_in, c_out, jblocks, splits, store_part, gt_blocks, gt_dedupe, found_rows;
     // partial sums of the weight gradient: one per `tiles_each` of a workgroup's tiles (longer sums in fp32 round more: 14
     // items of 7 x 37, 31 -> 280, z accumulation: 2.4e-7 against float64 over 23 tiles, 1.3e-7 over 6), n of them per workgroup
-    int tiles_each, parts;
+    int tiles_each, parts, sums;  // sums: those with tiles at all, the first ones
     size_t w_stride, part_stride, dcol_stride, dcol_slice;
 };
 
@@ -3042,7 +3042,7 @@ __device__ __forceinline__ void small_k_columns(const SmallKParams& q, Shared& s
         }
     }
     if constexpr (PARTS)
-        for (; part < q.parts; part++) store_part();
+        for (; part < q.parts && part * q.splits + split < q.sums; part++) store_part();
     else
         store_part();
 }
@@ -3229,6 +3229,7 @@ struct BwdLayout {
     int fused_jblocks;   // its column blocks: each writes a dcol slice of its own
     int fused_splits;    // its workgroups per add group and column block
     int fused_tiles_each, fused_parts;  // of the bf16 kernel: tiles in a partial sum, partial sums per workgroup
+    int fused_sums;      // partial sums with tiles at all
     int gt_dedupe;       // its upstream-gradient tiles serve both rails (c_out a multiple of 32)
     int gt_blocks;       // 32-column blocks of those tiles
     int ew_splits;       // parts of the positions in k_bwd_e_wgrad; 0: more members than it takes
@@ -3320,6 +3321,11 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round, int operand_bits)
         const long long each_wg = (n_tiles + b.fused_splits - 1) / b.fused_splits;
         b.fused_tiles_each = K > 16 ? 0 : b.fused_jw == 512 ? (int)each_wg : (int)std::min(each_wg, (n_tiles + most - 1) / most);
         b.fused_parts = K <= 16 ? (int)((each_wg + b.fused_tiles_each - 1) / b.fused_tiles_each) : 1;
+        // Partial sum (part, split) has tiles where split + splits * part * tiles_each is one; they are numbered part * splits +
+        // split, so those that have are the first ones, and what is left of the last parts is neither written nor read
+        // (54 items of 3 x 22 x 17 -> 11, 632 tiles in 512 workgroups: 1024 sums 36 us to add, 632 of them 23)
+        const long long before_last = (long long)b.fused_splits * (b.fused_parts - 1);
+        b.fused_sums = (int)(before_last + std::min<long long>(b.fused_splits, n_tiles - before_last * b.fused_tiles_each));
     }
     // split the m-reduction of the weight gradient so that all groups' tiles together make about one
     // round of workgroups: three per CU for the 128 x 128 kernel (more splits only add partial sums to write
@@ -3354,7 +3360,7 @@ BwdLayout bwd_layout(const Geometry& g, int groups_per_round, int operand_bits)
     // (rows of col and of E start on 16-byte boundaries: the products that read them along a row do so four at a time)
     b.col_v = pad64((size_t)pad4(b.m_total) * K);
     b.e_v = pad64((size_t)b.m_total * pad4(2 * g.c_out));
-    b.part_v = pad64((size_t)std::max(b.splits, b.fused_k ? b.fused_splits * b.fused_parts : b.ew_splits * b.ew_parts) * K * 2 * g.c_out);
+    b.part_v = pad64((size_t)std::max(b.splits, b.fused_k ? b.fused_sums : b.ew_splits * b.ew_parts) * K * 2 * g.c_out);
     b.w_v = pad64((size_t)K * 2 * g.c_out);
     // the fused kernel needs neither col nor E
     const size_t col_alloc = b.fused_k ? 0 : b.col_v, e_alloc = b.fused_k ? 0 : b.e_v;
@@ -3554,7 +3560,7 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
                 if (ks <= 8) {
                     SmallKParams p = {x, wcat, gt, pos_base, pos_arow, pos_bcol, found, part, dcol, G, v0, M, g.w_in, g.h_in,
                                       g.c_out, L.fused_jblocks, L.fused_splits, gw ? 1 : 0, L.gt_blocks, L.gt_dedupe, n_scan_rows,
-                                      L.fused_tiles_each, L.fused_parts,
+                                      L.fused_tiles_each, L.fused_parts, L.fused_sums,
                                       L.w_v, L.part_v, L.col_v, slice};
                     auto launch = [&](auto dx, auto looks) {
                         constexpr bool DX = decltype(dx)::value, LOOK = decltype(looks)::value;
@@ -3583,12 +3589,12 @@ int launch_conv_backward(const Geometry& g, int groups_per_round, int operand_bi
             }
             if (gw) {
                 // few partial sums (wide layers): coalesced tiles; many: the kernel that adds eight splits side by side
-                if (L.fused_splits * L.fused_parts <= 4)
+                if (L.fused_sums <= 4)
                     hipLaunchKernelGGL(k_reduce_wgrad_tiled, w_tiles, dim3(256), 0, s, part, w, gw, v0, nv,
-                                       WgradSplits{L.fused_splits * L.fused_parts, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
+                                       WgradSplits{L.fused_sums, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
                 else
                     hipLaunchKernelGGL(k_reduce_wgrad, dim3((K * g.c_out + 31) / 32, nv), dim3(256), 0, s, part, w, gw, v0,
-                                       WgradSplits{L.fused_splits * L.fused_parts, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
+                                       WgradSplits{L.fused_sums, 0, nullptr}, g.c_out, G, L.part_v, WgradOperands{});
             }
             if (gx && L.dcol_slices > 1)
                 hipLaunchKernelGGL(k_sum_slices, dim3(grid1d((long long)((size_t)nv * L.col_v / 4))), dim3(256), 0, s, dcol,

@@ -768,6 +768,8 @@ SMALL_GROUPS = [
     ((40, 6, 4, 4), (500, 6, 3, 3), 1, "yz", 4),    # 12 members, ragged channel blocks
     ((33, 2, 1, 520), (500, 2, 1, 520), 0, "y", 1), # two blocks of columns per wave, 1000 columns in sets of 512
     ((40, 3, 40, 40), (20, 3, 3, 3), 1, "y", 1),    # several partial sums per workgroup
+    ((54, 3, 22, 17), (11, 3, 3, 3), 1, "y", 1),    # 632 tiles, two partial sums in some of the workgroups
+    ((19, 5, 64, 8), (53, 5, 3, 3), 1, "y", 1),     # 304 tiles, likewise with four waves
 ]
 
 

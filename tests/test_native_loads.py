@@ -83,6 +83,24 @@ def test_forward_scratch_is_bounded_by_the_stream_budget():
         assert capi.workspace_size(d, o) == capi.workspace_size(d, capi.make_options(budget, 0, True))
 
 
+def test_no_more_partial_sums_than_tiles():
+    """Small OR groups: the weight gradient's partial sums, which a kernel adds one after the other, are at most one per tile
+    of 32 positions."""
+    from geo_amd import capi
+    for x, w in (((54, 3, 22, 17), (11, 3, 3, 3)), ((19, 5, 64, 8), (53, 5, 3, 3)), ((40, 3, 40, 40), (20, 3, 3, 3))):
+        d = capi.make_desc(x, w, 128, (1, 1))
+        n, c_out, wo, ho = capi.output_shape(d)
+        members, groups, positions = x[1] * w[2], w[3], n * wo * ho
+        tiles = -(-positions // 32)
+        columns = -(-2 * c_out // 32)
+        floats = groups * (tiles * members * 2 * c_out           # partial sums
+                           + members * (positions + 3)           # dcol, one slice
+                           + 2 * members * 2 * c_out) \
+            + max(tiles * columns * 1024, positions * c_out) \
+            + 3 * positions
+        assert capi.backward_workspace_size(d) <= 4 * floats + 16384, x
+
+
 def test_options_of_a_caller_that_knows_fewer_fields():
     """struct_bytes says how much of geo_sc_options the caller has: what lies behind is not read, what lies in front counts."""
     from geo_amd import _native, capi
